@@ -18,12 +18,17 @@
 //
 // On the device one V(1,1)-cycle with damped-Jacobi smoothing (same weight
 // before and after, so the preconditioner is symmetric; the weight is 1.3 w)
-// is, per level:
-//   k_amg_pre      x = w D^-1 b and r = b - A x fused (x gathered on the fly)
-//   k_amg_spmv     b_c = P^T r
-//   ...            coarser levels / dense coarse solve
-//   k_amg_prolong  x += P x_c
-//   k_amg_post     x' = x + w D^-1 (b - A x)  (+ (r, z) partial on level 0)
+// is one sparse product per level on the way down and one on the way up:
+//   down   b_c = R (I - A w D^-1) b    pre-smoothing from zero and restriction
+//   coarsest level: its down product and the dense inverse as one dense
+//          matrix where that is small, else one after the other
+//   up     z = (2 w D^-1 - w D^-1 A w D^-1) b + (I - w D^-1 A) P x_c
+//          prolongation and post-smoothing, as one product with [b | x_c]
+// The cycle of a single magnetisation is a chain of kernels of a few
+// microseconds each: what bounds it is their number, not their bytes.  Only
+// level 0 of a large system (see kLaneRows) goes up in two steps, prolongation and
+// post-smoothing, which read fewer bytes than the product with the wider rows
+// of (I - w D^-1 A) P.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -225,19 +230,16 @@ bool dense_inverse(std::vector<double>& a, int n) {
                 std::swap(a[(size_t)p * n + k], a[(size_t)c * n + k]);
                 std::swap(inv[(size_t)p * n + k], inv[(size_t)c * n + k]);
             }
+        // columns of a before c are zero in row c already
         const double piv = 1.0 / a[(size_t)c * n + c];
-        for (int k = 0; k < n; ++k) {
-            a[(size_t)c * n + k] *= piv;
-            inv[(size_t)c * n + k] *= piv;
-        }
+        for (int k = c; k < n; ++k) a[(size_t)c * n + k] *= piv;
+        for (int k = 0; k < n; ++k) inv[(size_t)c * n + k] *= piv;
         for (int r = 0; r < n; ++r) {
             if (r == c) continue;
             const double f = a[(size_t)r * n + c];
             if (f == 0.0) continue;
-            for (int k = 0; k < n; ++k) {
-                a[(size_t)r * n + k] -= f * a[(size_t)c * n + k];
-                inv[(size_t)r * n + k] -= f * inv[(size_t)c * n + k];
-            }
+            for (int k = c; k < n; ++k) a[(size_t)r * n + k] -= f * a[(size_t)c * n + k];
+            for (int k = 0; k < n; ++k) inv[(size_t)r * n + k] -= f * inv[(size_t)c * n + k];
         }
     }
     a.swap(inv);
@@ -254,40 +256,114 @@ bool dense_inverse(std::vector<double>& a, int n) {
     const int s0_ = xcd_block() * spb_, s1_ = min(nsl, s0_ + spb_);                                   \
     for (int s = s0_ + (int)threadIdx.x / kWave; s < s1_; s += kBlock / kWave)
 
-// x = w D^-1 b ;  r = b - A x   (x gathered on the fly as w dinv_j b_j)
 // With rr_part, every block first sums the CG update's (r, r) partials (G of
 // them) and all take the same decision: a CG that has reached its tolerance
 // stops here (block 0 records it) instead of after a V-cycle whose z it
 // would not use.
-__global__ __launch_bounds__(kBlock) void k_amg_pre(CgState* st, SellView A, const double* __restrict__ val,
-                                                    const double* __restrict__ dinv, const double* __restrict__ b,
-                                                    double w, double* __restrict__ x, double* __restrict__ r,
-                                                    const double* rr_part, int G) {
-    if (st && st->done) return;
-    if (st && rr_part) {
-        double t[1];
-        reduce_partials_all<1>(rr_part, G, G, t);
-        if (t[0] <= st->tol2bb) {
-            if (blockIdx.x == 0 && threadIdx.x == 0) {
-                st->rr = t[0];
-                st->done = 1;
-            }
-            return;
-        }
+__device__ inline bool cg_converged(CgState* st, const double* rr_part, int G) {
+    if (!st || !rr_part) return false;
+    double t[1];
+    reduce_partials_all<1>(rr_part, G, G, t);
+    if (!(t[0] <= st->tol2bb)) return false;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->rr = t[0];
+        st->done = 1;
     }
-    AMG_SLICE_LOOP(A) {
-        double acc = 0.0;
-        sell_row(A, s, lane, [&](int64_t e, int c) { acc += val[e] * (w * dinv[c] * b[c]); });
-        const int row = s * kWave + lane;
-        if (row < A.n) {
-            const double bi = b[row];
-            x[row] = w * dinv[row] * bi;
-            r[row] = bi - acc;
+    return true;
+}
+
+// y = M x, LPR lanes per row, one row per lane group.  The row is summed
+// before the convergence test of cg_converged, whose loads and LDS pass then
+// run under the gathers.
+template <int LPR>
+__global__ __launch_bounds__(kBlock) void k_amg_mv(CgState* st, const double* rr_part, int G, int n,
+                                                   const int* __restrict__ rp, const int* __restrict__ ci,
+                                                   const double* __restrict__ v, const double* x, double* y) {
+    if (st && st->done) return;
+    const int row = (blockIdx.x * kBlock + threadIdx.x) / LPR, sub = threadIdx.x & (LPR - 1);
+    double s[1] = {0.0};
+    if (row < n) csr_row<LPR, 1>(rp, ci, v, {x}, row, sub, s);
+    if (cg_converged(st, rr_part, G)) return;
+    if (row < n && sub == 0) y[row] = s[0];
+}
+
+// y = D x for a dense row-major n x m matrix, one block per row
+__global__ __launch_bounds__(kBlock) void k_amg_dmv(CgState* st, const double* rr_part, int G, int m,
+                                                    const double* __restrict__ D, const double* x, double* y) {
+    __shared__ double sp[kBlock / kWave];
+    if (st && st->done) return;
+    const double* d = D + (size_t)blockIdx.x * m;
+    double acc = 0.0;
+    int j = threadIdx.x;
+    for (; j + 3 * kBlock < m; j += 4 * kBlock) {
+        double a[4], b[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            a[k] = d[j + k * kBlock];
+            b[k] = x[j + k * kBlock];
         }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) acc += a[k] * b[k];
+    }
+    for (; j < m; j += kBlock) acc += d[j] * x[j];
+    if (cg_converged(st, rr_part, G)) return;
+    acc = wave_sum(acc);
+    if ((threadIdx.x & (kWave - 1)) == 0) sp[threadIdx.x / kWave] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int k = 0; k < kBlock / kWave; ++k) t += sp[k];
+        y[blockIdx.x] = t;
     }
 }
 
+// Level 0 upwards in one product: z = U [r | x_c] and the partials of (r, z)
+template <int LPR>
+__global__ __launch_bounds__(kBlock) void k_amg_up0(CgState* st, const double* rr_part, int n,
+                                                    const int* __restrict__ rp, const int* __restrict__ ci,
+                                                    const double* __restrict__ v, const double* __restrict__ x,
+                                                    double* __restrict__ z, double* part) {
+    __shared__ double sp[kBlock / kWave];
+    if (st && st->done) return;
+    const RowShare R = row_share<LPR>(n, xcd_block(), gridDim.x);
+    const int sub = threadIdx.x & (LPR - 1);
+    int row = R.r0 + threadIdx.x / LPR;
+    double s[1] = {0.0};
+    if (row < R.r1) csr_row<LPR, 1>(rp, ci, v, {x}, row, sub, s);
+    if (cg_converged(st, rr_part, gridDim.x)) return;
+    double dot = 0.0;
+    while (row < R.r1) {
+        if (sub == 0) {
+            z[row] = s[0];
+            dot += x[row] * s[0];
+        }
+        row += kBlock / LPR;
+        if (row < R.r1) csr_row<LPR, 1>(rp, ci, v, {x}, row, sub, s);
+    }
+    dot = wave_sum(dot);
+    if ((threadIdx.x & (kWave - 1)) == 0) sp[threadIdx.x / kWave] = dot;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int k = 0; k < kBlock / kWave; ++k) t += sp[k];
+        part[blockIdx.x] = t;
+    }
+}
 
+// x = w D^-1 b + P xc
+template <int LPR>
+__global__ __launch_bounds__(kBlock) void k_amg_prolong(const CgState* st, int n, const int* __restrict__ rp,
+                                                        const int* __restrict__ ci, const double* __restrict__ v,
+                                                        const double* __restrict__ dinv, const double* __restrict__ b,
+                                                        double w, const double* __restrict__ xc,
+                                                        double* __restrict__ x) {
+    if (st && st->done) return;
+    const int row = (blockIdx.x * kBlock + threadIdx.x) / LPR, sub = threadIdx.x & (LPR - 1);
+    if (row >= n) return;  // whole groups leave together
+    double s[1];
+    csr_row<LPR, 1>(rp, ci, v, {xc}, row, sub, s);
+    if (sub == 0) x[row] = w * dinv[row] * b[row] + s[0];
+}
 
 // xo = x + w D^-1 (b - A x); optionally partial (b, xo) per block into part.
 __global__ __launch_bounds__(kBlock) void k_amg_post(const CgState* st, SellView A, const double* __restrict__ val,
@@ -349,58 +425,6 @@ __global__ __launch_bounds__(kBlock) void k_amg_dot(const CgState* st, int n, co
     }
 }
 
-// ---- lanes-per-row CSR kernels (LPR lanes of a wavefront share one row) ----
-template <int LPR>
-__device__ inline double group_sum(double v) {
-#pragma unroll
-    for (int o = LPR / 2; o > 0; o >>= 1) v += __shfl_down(v, o, LPR);
-    return v;
-}
-
-// MODE 0: y = A x      MODE 1: y += A x (prolongation)
-// MODE 2: x = w dinv b, r = b - A(w dinv b)   (pre-smoothing + residual)
-// MODE 3: xo = x + w dinv (b - A x)           (post-smoothing)
-template <int LPR, int MODE>
-__global__ __launch_bounds__(kBlock) void k_csrv(const CgState* st, int n, const int* __restrict__ rp,
-                                                 const int* __restrict__ ci, const double* __restrict__ v,
-                                                 const double* __restrict__ x, const double* __restrict__ dinv,
-                                                 const double* __restrict__ b, double w, double* __restrict__ y,
-                                                 double* __restrict__ y2) {
-    if (st && st->done) return;  // the CG this V-cycle serves has converged
-    const int row = (blockIdx.x * kBlock + threadIdx.x) / LPR;
-    const int sub = threadIdx.x & (LPR - 1);
-    if (row >= n) return;  // whole groups exit together (LPR divides kBlock)
-    double acc = 0.0;
-    for (int q = rp[row] + sub; q < rp[row + 1]; q += LPR) {
-        const int c = ci[q];
-        acc += MODE == 2 ? v[q] * (w * dinv[c] * b[c]) : v[q] * x[c];
-    }
-    acc = group_sum<LPR>(acc);
-    if (sub != 0) return;
-    if (MODE == 0) y[row] = acc;
-    if (MODE == 1) y[row] += acc;
-    if (MODE == 2) {
-        const double bi = b[row];
-        y[row] = w * dinv[row] * bi;
-        y2[row] = bi - acc;
-    }
-    if (MODE == 3) y2[row] = x[row] + w * dinv[row] * (b[row] - acc);
-}
-
-template <int MODE>
-void csrv_launch(const CgState* st, const AmgPrecond::CsrDev& M, const double* x, const double* dinv,
-                 const double* b, double w, double* y, double* y2, hipStream_t s) {
-    const int rows_per_block = kBlock / M.lpr;
-    const dim3 g((M.n + rows_per_block - 1) / rows_per_block);
-    switch (M.lpr) {
-        case 4: hipLaunchKernelGGL((k_csrv<4, MODE>), g, dim3(kBlock), 0, s, st, M.n, M.rp.p, M.ci.p, M.v.p, x, dinv, b, w, y, y2); break;
-        case 8: hipLaunchKernelGGL((k_csrv<8, MODE>), g, dim3(kBlock), 0, s, st, M.n, M.rp.p, M.ci.p, M.v.p, x, dinv, b, w, y, y2); break;
-        case 16: hipLaunchKernelGGL((k_csrv<16, MODE>), g, dim3(kBlock), 0, s, st, M.n, M.rp.p, M.ci.p, M.v.p, x, dinv, b, w, y, y2); break;
-        case 32: hipLaunchKernelGGL((k_csrv<32, MODE>), g, dim3(kBlock), 0, s, st, M.n, M.rp.p, M.ci.p, M.v.p, x, dinv, b, w, y, y2); break;
-        default: hipLaunchKernelGGL((k_csrv<64, MODE>), g, dim3(kBlock), 0, s, st, M.n, M.rp.p, M.ci.p, M.v.p, x, dinv, b, w, y, y2); break;
-    }
-}
-
 int upload_csrv(const Csr& M, AmgPrecond::CsrDev& D, hipStream_t s) {
     D.n = M.n;
     const double avg = M.n ? (double)M.rp[M.n] / M.n : 1.0;
@@ -414,22 +438,50 @@ int upload_csrv(const Csr& M, AmgPrecond::CsrDev& D, hipStream_t s) {
     return TM_OK;
 }
 
-int upload_csr(const Csr& M, SellPattern& P, DevBuf<double>& val, hipStream_t s) {
-    P.build(M.n, M.m, M.rp.data(), M.ci.data());
-    std::vector<double> sv;
-    TM_CHECK(P.scatter(M.rp.data(), M.ci.data(), M.v.data(), sv));
-    TM_CHECK(P.upload(s));
-    TM_CHECK(val.upload(sv.data(), sv.size(), s));
-    TM_HIP(hipStreamSynchronize(s));
-    return TM_OK;
+// [2 w D^-1 - w D^-1 A w D^-1 | Q] with Q = (I - w D^-1 A) P
+Csr up_operator(const Csr& A, const std::vector<double>& d, double w, const Csr& Q) {
+    Csr U;
+    U.n = A.n;
+    U.m = A.n + Q.m;
+    U.rp.assign((size_t)A.n + 1, 0);
+    U.ci.reserve(A.ci.size() + Q.ci.size());
+    U.v.reserve(A.ci.size() + Q.ci.size());
+    for (int i = 0; i < A.n; ++i) {
+        const double f = d[i] != 0.0 ? w / d[i] : 0.0;
+        for (int q = A.rp[i]; q < A.rp[i + 1]; ++q) {
+            const int j = A.ci[q];
+            const double g = d[j] != 0.0 ? w / d[j] : 0.0;
+            U.ci.push_back(j);
+            U.v.push_back((j == i ? 2.0 * f : 0.0) - f * A.v[q] * g);
+        }
+        for (int q = Q.rp[i]; q < Q.rp[i + 1]; ++q) {
+            U.ci.push_back(A.n + Q.ci[q]);
+            U.v.push_back(Q.v[q]);
+        }
+        U.rp[i + 1] = (int)U.ci.size();
+    }
+    return U;
 }
 
+// Q = P - w D^-1 (A P), the rows of P being part of those of A P
+Csr smoothed(const Csr& P, const Csr& AP, const std::vector<double>& d, double w) {
+    Csr Q = AP;
+    for (int i = 0; i < P.n; ++i) {
+        const double f = d[i] != 0.0 ? w / d[i] : 0.0;
+        int t = P.rp[i];
+        for (int q = AP.rp[i]; q < AP.rp[i + 1]; ++q) {
+            Q.v[q] = -f * AP.v[q];
+            if (t < P.rp[i + 1] && P.ci[t] == AP.ci[q]) Q.v[q] += P.v[t++];
+        }
+    }
+    return Q;
+}
 
 }  // namespace
 
 int AmgPrecond::setup(int n, const int* rowptr, const int* colidx, const double* vals,
                       const std::vector<unsigned char>& fixed, const SellPattern* A0, const double* A0val,
-                      const double* A0dinv, hipStream_t s) {
+                      const double* A0dinv, int up0_lpr, hipStream_t s) {
     // symmetric operator seen by CG: free-free block, identity on fixed rows
     Csr A;
     A.n = A.m = n;
@@ -449,7 +501,8 @@ int AmgPrecond::setup(int n, const int* rowptr, const int* colidx, const double*
     }
     levels.clear();
     std::vector<char> excl(fixed.begin(), fixed.end());
-    Csr cur = A;
+    Csr cur = A, last_down;
+    D.release();
     int lev = 0;
     while (cur.n > kCoarseMax && lev < kMaxLevels) {
         std::vector<double> d = diagonal(cur);
@@ -492,7 +545,8 @@ int AmgPrecond::setup(int n, const int* rowptr, const int* colidx, const double*
             P.rp[i + 1] = (int)P.ci.size();
         }
         Csr R = transpose(P);
-        Csr Ac = spgemm(R, spgemm(cur, P));
+        const Csr AP = spgemm(cur, P);
+        Csr Ac = spgemm(R, AP);
         Level L;
         L.n = cur.n;
         // smoother weight: 1.3 x the prolongator's 4/(3 rho) (omega rho ~ 1.7 < 2,
@@ -510,13 +564,17 @@ int AmgPrecond::setup(int n, const int* rowptr, const int* colidx, const double*
             TM_CHECK(L.dinv.upload(di.data(), di.size(), s));
         }
         TM_CHECK(upload_csrv(P, L.P, s));
+        L.P.lpr = 4;  // rows of a few entries
         TM_CHECK(upload_csrv(R, L.R, s));
         L.nnz_a = cur.rp[cur.n];
         L.nnz_p = P.rp[P.n];
-        TM_CHECK(L.x.alloc(cur.n));
-        TM_CHECK(L.x2.alloc(cur.n));
-        TM_CHECK(L.r.alloc(cur.n));
-        TM_CHECK(L.b.alloc(na));
+        const Csr Q = smoothed(P, AP, d, L.omega);
+        last_down = transpose(Q);  // R (I - A w D^-1): A and D are symmetric
+        TM_CHECK(upload_csrv(last_down, L.down, s));
+        if (lev > 0 || up0_lpr > 0) TM_CHECK(upload_csrv(up_operator(cur, d, L.omega, Q), L.up, s));
+        else TM_CHECK(L.x.alloc(cur.n));
+        if (lev == 0 && up0_lpr > 0) L.up.lpr = up0_lpr;
+        if (lev > 0) TM_CHECK(L.bx.alloc((size_t)cur.n + na));
         levels.push_back(std::move(L));
         cur = std::move(Ac);
         excl.assign((size_t)cur.n, 0);
@@ -529,50 +587,78 @@ int AmgPrecond::setup(int n, const int* rowptr, const int* colidx, const double*
         for (int q = cur.rp[i]; q < cur.rp[i + 1]; ++q) dense[(size_t)i * nc + cur.ci[q]] = cur.v[q];
     if (!dense_inverse(dense, nc)) return TM_ERR_UNSUPPORTED;
     TM_CHECK(Cinv.upload(dense.data(), dense.size(), s));
-    TM_CHECK(xc.alloc(nc));
     TM_CHECK(bc.alloc(nc));
+    std::vector<double> dd;
+    if (!levels.empty() && (int64_t)nc * levels.back().n <= kDenseMax) {  // D = Cinv * down
+        const int m = levels.back().n;
+        dd.assign((size_t)nc * m, 0.0);
+        for (int i = 0; i < nc; ++i)
+            for (int k = 0; k < nc; ++k) {
+                const double c = dense[(size_t)i * nc + k];
+                for (int q = last_down.rp[k]; q < last_down.rp[k + 1]; ++q)
+                    dd[(size_t)i * m + last_down.ci[q]] += c * last_down.v[q];
+            }
+        TM_CHECK(D.upload(dd.data(), dd.size(), s));
+    }
     TM_HIP(hipStreamSynchronize(s));
     return TM_OK;
 }
 
-// z = M^-1 r (one V-cycle); writes the (r, z) partials of `grid` blocks to part.
-int AmgPrecond::apply(const double* r0, double* z, double* part, int grid, hipStream_t s, CgState* st,
-                      const double* rr_part) {
+AmgPrecond::First AmgPrecond::first() const {
+    if (levels.size() == 1 && D.p) return First{nc, nullptr, D.p, nullptr};
+    return First{levels[0].down.n, &levels[0].down, nullptr, levels.size() > 1 ? levels[1].bx.p : bc.p};
+}
+
+int AmgPrecond::apply(double* r, double* z, double* part, int grid, hipStream_t s, CgState* st, const double* rr_part,
+                      bool first_done) {
     const int L = (int)levels.size();
     if (L == 0) {
-        hipLaunchKernelGGL(k_amg_dense, dim3((nc + 3) / 4), dim3(kBlock), 0, s, st, nc, Cinv.p, r0, z);
-        hipLaunchKernelGGL(k_amg_dot, dim3(grid), dim3(kBlock), 0, s, st, nc, r0, z, part);
+        hipLaunchKernelGGL(k_amg_dense, dim3((nc + 3) / 4), dim3(kBlock), 0, s, st, nc, Cinv.p, (const double*)r, z);
+        hipLaunchKernelGGL(k_amg_dot, dim3(grid), dim3(kBlock), 0, s, st, nc, (const double*)r, z, part);
         TM_HIP(hipGetLastError());
         return TM_OK;
     }
-    const double* b = r0;
+    auto mv = [&](const CsrDev& M, const double* x, double* y) {
+        with_lanes(M.lpr, [&](auto lpr) {
+            constexpr int kL = decltype(lpr)::value;
+            hipLaunchKernelGGL(k_amg_mv<kL>, dim3((M.n + kBlock / kL - 1) / (kBlock / kL)), dim3(kBlock), 0, s, st,
+                               rr_part, grid, M.n, M.rp.p, M.ci.p, M.v.p, x, y);
+        });
+        rr_part = nullptr;  // tested once
+    };
+    auto dmv = [&](int rows, int m, const double* M, const double* x, double* y) {
+        hipLaunchKernelGGL(k_amg_dmv, dim3(rows), dim3(kBlock), 0, s, st, rr_part, grid, m, M, x, y);
+        rr_part = nullptr;
+    };
+    auto vec = [&](int l) { return l == 0 ? r : levels[l].bx.p; };  // [b | x_c] of level l
     for (int l = 0; l < L; ++l) {
         Level& V = levels[l];
-        if (l == 0) {
-            const SellPattern& A = *V.A_ext;
-            hipLaunchKernelGGL(k_amg_pre, dim3(grid), dim3(kBlock), 0, s, st, view(A), V.Aval_ext, V.dinv_ext, b, V.omega,
-                               V.x.p, V.r.p, rr_part, grid);
+        const bool have = l == 0 && first_done;
+        if (l + 1 < L) {
+            if (!have) mv(V.down, vec(l), vec(l + 1));
+        } else if (D.p) {
+            if (!have) dmv(nc, V.n, D.p, vec(l), vec(l) + V.n);
         } else {
-            csrv_launch<2>(st, V.A, nullptr, V.dinv.p, b, V.omega, V.x.p, V.r.p, s);
+            if (!have) mv(V.down, vec(l), bc.p);
+            dmv(nc, nc, Cinv.p, bc.p, vec(l) + V.n);
         }
-        csrv_launch<0>(st, V.R, V.r.p, nullptr, nullptr, 0.0, V.b.p, nullptr, s);  // b_{l+1} = P^T r
-        b = V.b.p;
     }
-    hipLaunchKernelGGL(k_amg_dense, dim3((nc + 3) / 4), dim3(kBlock), 0, s, st, nc, Cinv.p, levels[L - 1].b.p, xc.p);
-    const double* xcoarse = xc.p;
-    for (int l = L - 1; l >= 0; --l) {
-        Level& V = levels[l];
-        const double* bl = l == 0 ? r0 : levels[l - 1].b.p;
-        csrv_launch<1>(st, V.P, xcoarse, nullptr, nullptr, 0.0, V.x.p, nullptr, s);  // x += P x_c
-        if (l == 0) {
-            const SellPattern& A = *V.A_ext;
-            hipLaunchKernelGGL(k_amg_post, dim3(grid), dim3(kBlock), 0, s, st, view(A), V.Aval_ext, V.dinv_ext, bl,
-                               V.omega, V.x.p, z, part);
-            xcoarse = z;
-        } else {
-            csrv_launch<3>(st, V.A, V.x.p, V.dinv.p, bl, V.omega, nullptr, V.x2.p, s);
-            xcoarse = V.x2.p;
-        }
+    for (int l = L - 1; l > 0; --l) mv(levels[l].up, vec(l), vec(l - 1) + levels[l - 1].n);
+    Level& V = levels[0];
+    if (up0()) {
+        with_lanes(V.up.lpr, [&](auto lpr) {
+            hipLaunchKernelGGL(k_amg_up0<decltype(lpr)::value>, dim3(grid), dim3(kBlock), 0, s, st, rr_part, V.n,
+                               V.up.rp.p, V.up.ci.p, V.up.v.p, (const double*)r, z, part);
+        });
+    } else {
+        with_lanes(V.P.lpr, [&](auto lpr) {
+            constexpr int kL = decltype(lpr)::value;
+            hipLaunchKernelGGL(k_amg_prolong<kL>, dim3((V.n + kBlock / kL - 1) / (kBlock / kL)), dim3(kBlock), 0, s,
+                               (const CgState*)st, V.n, V.P.rp.p, V.P.ci.p, V.P.v.p, V.dinv_ext, (const double*)r,
+                               V.omega, (const double*)(r + V.n), V.x.p);
+        });
+        hipLaunchKernelGGL(k_amg_post, dim3(grid), dim3(kBlock), 0, s, (const CgState*)st, view(*V.A_ext),
+                           V.Aval_ext, V.dinv_ext, (const double*)r, V.omega, (const double*)V.x.p, z, part);
     }
     TM_HIP(hipGetLastError());
     return TM_OK;

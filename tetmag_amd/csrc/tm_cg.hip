@@ -10,16 +10,28 @@
 // reference's systems and returns the reference's solution (same gauge for
 // the Neumann problem).
 //
-// Each iteration is two kernels with no host round trip and no device-scope
+// Each iteration is two kernels, the second of which also forms the first
+// product of the next V-cycle, with no host round trip and no device-scope
 // fence:
-//   k_cg_spmv(k)   : gamma_k, (r,r) from the update's partials; beta; p = z +
-//                    beta p_old fused into the gathers; q = A p; partial (p,q)
-//   k_cg_update(k) : alpha = gamma_k / (p,q); x += alpha p; r -= alpha q;
-//                    z = D^-1 r; partials (r,z), (r,r)
-// Every block reduces the producer's partials itself (tm_internal.hpp), so all
-// blocks take the same convergence decision; block 0 publishes the scalars.
-// Grids are at most kMaxCgBlocks blocks (grid-stride), which keeps the
-// partial arrays short.  The host checks the state once per chunk.
+//   k_cg_spmv(k) : gamma_k, (r,r) from the partials; beta; q = A z + beta q
+//                  (= A p, the gathers read z only); p = z + beta p; partial (p,q)
+//   k_cg_step(k) : alpha = gamma_k / (p,q); x += alpha p; r' = r - alpha q;
+//                  partial (r',r'); and on further blocks F r' = F r - alpha F q
+//                  for the preconditioner's first product F
+// (k_cg_update is the step without that product.)  Every block reduces the
+// producer's partials itself (tm_internal.hpp), so all blocks take the same
+// convergence decision; block 0 publishes the scalars.  Grids are at most
+// kMaxCgBlocks blocks, which keeps the partial arrays short.  A solve of a
+// single right-hand side is bound by the number of its launches (each a few
+// microseconds, most of it latency), so every kernel starts with the loads of
+// its rows and reduces the scalars it needs while they are in flight.  The
+// host reads the state once per chunk of iterations.  With the V-cycle as one
+// product per level (tm_amg.hip) an iteration of a two-level solve is three
+// launches (of a four-level one eight), where separate smoothing, restriction,
+// prolongation and update kernels took eight (fifteen): a cold Neumann solve
+// of 71,825 nodes 1,178 -> 791 us, one FP64 evaluation at 29,760 nodes 710 ->
+// 352 us, at 282,897 nodes 3.49 -> 2.89 ms (2.05 ms of it the boundary
+// product).
 #include <algorithm>
 #include <cmath>
 
@@ -64,13 +76,20 @@ __device__ inline void block_partials(double* part, int stride, double v0, doubl
 // newest, least squares in the residual norm; the method is described with
 // kSolveWindow in tm_internal.hpp).  Slots are ordered newest first.
 
-// per-block partials wpart[q * G + block] of the kWinDots dots.  The new b
-// goes into the head slot as it is read: when the window is full that slot
-// holds the oldest pair, whose value this thread has already loaded.
+// per-block partials wpart[q * G + block] of the kWinDots dots and, as the
+// last row, of (b, b).  The new b goes into the head slot as it is read: when
+// the window is full that slot holds the oldest pair, whose value this thread
+// has already loaded.  Eight threads sum the block's values of a dot from LDS
+// (a shuffle tree per dot, 29 of them, took longer than the loads).
+constexpr int kWinRows = kWinDots + 1;
+constexpr int kWinBlocks = 256;  // at most, so that k_cg_win_combine has few partials to read
+static_assert(8 * kWinRows <= kBlock, "eight threads per sum");
+
 __global__ __launch_bounds__(kBlock) void k_cg_win_dots(int n, const CgWindow* w, double* __restrict__ Bw,
                                                         const double* __restrict__ b, double* wpart) {
     const int cnt = w->cnt, head = w->head;
     double acc[kWinDots] = {};
+    double bb = 0.0;
     const double* src[kSolveWindow];
 #pragma unroll
     for (int i = 0; i < kSolveWindow; ++i) src[i] = Bw + (size_t)win_slot(head, i) * n;
@@ -83,95 +102,73 @@ __global__ __launch_bounds__(kBlock) void k_cg_win_dots(int n, const CgWindow* w
         const double r = bi - v[0];
         win_differences(v, cnt);
         win_accumulate(acc, v, r);
+        bb += bi * bi;
         dst[e] = bi;
     }
-    __shared__ double sp[kWinDots][kBlock / kWave];
-    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+    __shared__ double sp[kWinRows][kBlock + 8];
 #pragma unroll
-    for (int q = 0; q < kWinDots; ++q) {
-        const double t = wave_sum(acc[q]);
-        if (lane == 0) sp[q][wid] = t;
-    }
+    for (int q = 0; q < kWinDots; ++q) sp[q][threadIdx.x] = acc[q];
+    sp[kWinDots][threadIdx.x] = bb;
     __syncthreads();
-    if (threadIdx.x < kWinDots) {
-        double a = 0.0;
-        for (int k = 0; k < kBlock / kWave; ++k) a += sp[threadIdx.x][k];
-        wpart[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = a;
-    }
+    const int q = threadIdx.x >> 3, sub = threadIdx.x & 7;
+    if (q >= kWinRows) return;
+    double t = 0.0;
+#pragma unroll 8
+    for (int k = sub; k < kBlock; k += 8) t += sp[q][k];
+    t = group_sum<8>(t);
+    if (sub == 0) wpart[(size_t)q * gridDim.x + blockIdx.x] = t;
 }
 
-// one block: the dots, then the coefficients (thread 0)
-// (one pass over all partials with every load independent; the solve on
-// register copies, so the unrolled factorisation makes no memory accesses)
-__global__ __launch_bounds__(kBlock) void k_cg_win_solve(int G, CgWindow* w, const double* wpart) {
-    double v[kWinDots] = {};
-    for (int g = threadIdx.x; g < G; g += kBlock)
+// x0 = sum_i a_i x_slot(i) (the caller's x when the window is empty), x = b on
+// the fixed rows, x = 0 when b = 0.  Every block sums the partials of the dots
+// and solves the small least-squares system itself.
+__global__ __launch_bounds__(kBlock) void k_cg_win_combine(int n, int G, const CgWindow* w, const double* wpart,
+                                                           const double* __restrict__ Xw,
+                                                           const unsigned char* __restrict__ fixed,
+                                                           const double* __restrict__ b, double* __restrict__ x) {
+    __shared__ double sd[kWinRows];
+    __shared__ double sa[kSolveWindow];
+    const int cnt = w->cnt, head = w->head;
+    const int q = threadIdx.x >> 3, sub = threadIdx.x & 7;
+    double t = 0.0;
+    if (q < kWinRows) {
+#pragma unroll 8
+        for (int g = sub; g < G; g += 8) t += wpart[(size_t)q * G + g];
+    }
+    t = group_sum<8>(t);
+    if (q < kWinRows && sub == 0) sd[q] = t;
+    __syncthreads();
+    if (threadIdx.x == 0 && cnt > 0) {
+        double d[kWinDots], a[kSolveWindow];
 #pragma unroll
-        for (int q = 0; q < kWinDots; ++q) v[q] += wpart[(size_t)q * G + g];
-    __shared__ double sr[kWinDots][kBlock / kWave];
-    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+        for (int k = 0; k < kWinDots; ++k) d[k] = sd[k];
+        win_coefficients(cnt, d, a);
 #pragma unroll
-    for (int q = 0; q < kWinDots; ++q) {
-        const double s = wave_sum(v[q]);
-        if (lane == 0) sr[q][wid] = s;
+        for (int i = 0; i < kSolveWindow; ++i) sa[i] = a[i];
     }
     __syncthreads();
-    const int cnt = w->cnt;
-    if (threadIdx.x != 0 || cnt == 0) return;
-    double t[kWinDots];
-#pragma unroll
-    for (int q = 0; q < kWinDots; ++q) {
-        double s = 0.0;
-#pragma unroll
-        for (int k = 0; k < kBlock / kWave; ++k) s += sr[q][k];
-        t[q] = s;
-    }
-    double a[kSolveWindow];
-    win_coefficients(cnt, t, a);
-#pragma unroll
-    for (int i = 0; i < kSolveWindow; ++i) w->a[i] = a[i];
-}
-
-// x0 = sum_i a_i x_slot(i) (nothing when the window is empty)
-__global__ __launch_bounds__(kBlock) void k_cg_win_combine(int n, const CgWindow* w, const double* __restrict__ Xw,
-                                                           double* __restrict__ x) {
-    const int cnt = w->cnt;
-    if (cnt == 0) return;
+    const bool zero = sd[kWinDots] == 0.0;
     double a[kSolveWindow];
     const double* src[kSolveWindow];
 #pragma unroll
     for (int i = 0; i < kSolveWindow; ++i) {
-        a[i] = w->a[i];
-        src[i] = Xw + (size_t)win_slot(w->head, i) * n;
+        a[i] = i < cnt ? sa[i] : 0.0;
+        src[i] = Xw + (size_t)win_slot(head, i) * n;
     }
     for (int e = blockIdx.x * kBlock + threadIdx.x; e < n; e += gridDim.x * kBlock) {
-        double acc = 0.0;
+        if (zero) x[e] = 0.0;
+        else if (fixed[e]) x[e] = b[e];
+        else if (cnt > 0) {
+            double acc = 0.0;
 #pragma unroll
-        for (int i = 0; i < kSolveWindow; ++i)
-            if (i < cnt) acc += a[i] * src[i][e];
-        x[e] = acc;
+            for (int i = 0; i < kSolveWindow; ++i)
+                if (i < cnt) acc += a[i] * src[i][e];
+            x[e] = acc;
+        }
     }
 }
 
-// the solution into the head slot (its b is there already)
-__global__ __launch_bounds__(kBlock) void k_cg_win_store(int n, const CgWindow* w, const double* __restrict__ x,
-                                                         double* __restrict__ Xw) {
-    const size_t off = (size_t)w->head * n;
-    for (int e = blockIdx.x * kBlock + threadIdx.x; e < n; e += gridDim.x * kBlock) Xw[off + e] = x[e];
-}
-
-// keep the pair and advance the head; a failed solve empties the window
-__global__ void k_cg_win_advance(CgWindow* w, const CgState* st) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    if (st->done != 1) {
-        w->cnt = 0;
-        w->head = 0;
-        return;
-    }
-    w->head = (w->head + 1) % kSolveWindow;
-    w->cnt = min(w->cnt + 1, kSolveWindow);
-}
-
+// ---- iterations ---------------------------------------------------------------
 // part layout: [0, G) bb | [G, 2G) rz | [2G, 3G) rr | [3G, 4G) pq
 __global__ __launch_bounds__(kBlock) void k_cg_init_fixed(int n, const unsigned char* __restrict__ fixed,
                                                           const double* __restrict__ b, double* __restrict__ x,
@@ -185,22 +182,30 @@ __global__ __launch_bounds__(kBlock) void k_cg_init_fixed(int n, const unsigned 
     block_partials(part, 0, v, 0.0, 1);
 }
 
+// the state of a new solve, from the Gb partials of (b, b); b = 0 has the
+// solution 0 (which k_cg_finish writes)
+__device__ inline void cg_begin(const double* bbpart, int Gb, double tol, CgState* st) {
+    double bb[1];
+    reduce_partials_all<1>(bbpart, Gb, Gb, bb);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->bb = bb[0];
+        st->tol2bb = tol * tol * bb[0];
+        st->iters = 0;
+        st->done = bb[0] == 0.0 ? 1 : 0;
+        st->rr = 0.0;
+    }
+}
+
+// r = b - A x, one lane per row (SELL)
 template <bool JAC>
 __global__ __launch_bounds__(kBlock) void k_cg_init_res(SellView A, const double* __restrict__ val,
                                                         const double* __restrict__ dinv,
                                                         const double* __restrict__ b, const double* __restrict__ x,
                                                         double* __restrict__ r, double* __restrict__ z,
-                                                        double* part, double tol, CgState* st) {
+                                                        const double* bbpart, int Gb, double* part, double tol,
+                                                        CgState* st) {
     const int G = gridDim.x;
-    double bb[1];
-    reduce_partials_all<1>(part, G, G, bb);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        st->bb = bb[0];
-        st->tol2bb = tol * tol * bb[0];
-        st->iters = 0;
-        st->done = 0;
-        st->rr = 0.0;
-    }
+    cg_begin(bbpart, Gb, tol, st);
     double vrz = 0.0, vrr = 0.0;
     CG_SLICE_LOOP(A) {
         double acc = 0.0;
@@ -221,19 +226,42 @@ __global__ __launch_bounds__(kBlock) void k_cg_init_res(SellView A, const double
     else block_partials(part + 2 * G, G, vrr, 0.0, 1);
 }
 
-__global__ __launch_bounds__(kBlock) void k_cg_spmv(SellView A, const double* __restrict__ val,
-                                                    const double* __restrict__ z, const double* __restrict__ p_old,
-                                                    double* __restrict__ p_new, double* __restrict__ q, int k,
-                                                    double* part, CgState* st) {
-    if (st->done) return;
+// r = b - A x, LPR lanes per row
+template <int LPR>
+__global__ __launch_bounds__(kBlock) void k_cg_init_res_l(int n, const int* __restrict__ rp,
+                                                          const int* __restrict__ ci, const double* __restrict__ v,
+                                                          const double* __restrict__ b, const double* __restrict__ x,
+                                                          double* __restrict__ r, const double* bbpart, int Gb,
+                                                          double* part, double tol, CgState* st) {
     const int G = gridDim.x;
+    const RowShare R = row_share<LPR>(n, xcd_block(), G);
+    const int sub = threadIdx.x & (LPR - 1);
+    int row = R.r0 + threadIdx.x / LPR;
+    double s[1] = {0.0};
+    if (row < R.r1) csr_row<LPR, 1>(rp, ci, v, {x}, row, sub, s);
+    cg_begin(bbpart, Gb, tol, st);
+    double vrr = 0.0;
+    while (row < R.r1) {
+        if (sub == 0) {
+            const double ri = b[row] - s[0];
+            r[row] = ri;
+            vrr += ri * ri;
+        }
+        row += kBlock / LPR;
+        if (row < R.r1) csr_row<LPR, 1>(rp, ci, v, {x}, row, sub, s);
+    }
+    block_partials(part + 2 * G, G, vrr, 0.0, 1);
+}
+
+// gamma_k, convergence on the last (r, r), beta_k; false when the solve stops
+__device__ inline bool cg_beta(int k, const double* part, int G, CgState* st, double& beta) {
     double t[2];
     reduce_partials_all<2>(part + G, G, G, t);  // (r,z), (r,r)
     const double gam = t[0], rr = t[1];
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     if (!isfinite(gam) || !isfinite(rr)) {
         if (lead) st->done = 2;
-        return;
+        return false;
     }
     if (rr <= st->tol2bb) {
         if (lead) {
@@ -241,27 +269,81 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv(SellView A, const double* __
             st->rr = rr;
             st->iters = k;
         }
-        return;
+        return false;
     }
-    const double beta = k > 0 ? gam / st->gam[(k - 1) & 1] : 0.0;
+    beta = k > 0 ? gam / st->gam[(k - 1) & 1] : 0.0;
     if (lead) {
         st->gam[k & 1] = gam;
         st->rr = rr;
     }
+    return true;
+}
+
+// p = z + beta p, q = A p = A z + beta q, partial (p, q); one lane per row (SELL)
+__global__ __launch_bounds__(kBlock) void k_cg_spmv(SellView A, const double* __restrict__ val,
+                                                    const double* __restrict__ z, double* __restrict__ p,
+                                                    double* __restrict__ q, int k, double* part, CgState* st) {
+    if (st->done) return;
+    const int G = gridDim.x;
+    double beta;
+    if (!cg_beta(k, part, G, st, beta)) return;
     double v = 0.0;
     CG_SLICE_LOOP(A) {
         double acc = 0.0;
-        if (k == 0) sell_row(A, s, lane, [&](int64_t e, int c) { acc += val[e] * z[c]; });
-        else sell_row(A, s, lane, [&](int64_t e, int c) { acc += val[e] * (z[c] + beta * p_old[c]); });
+        sell_row(A, s, lane, [&](int64_t e, int c) { acc += val[e] * z[c]; });
         const int row = s * kWave + lane;
         if (row < A.n) {
-            const double pi = k == 0 ? z[row] : z[row] + beta * p_old[row];
-            p_new[row] = pi;
-            q[row] = acc;
-            v += pi * acc;
+            const double pi = k == 0 ? z[row] : z[row] + beta * p[row];
+            const double qi = k == 0 ? acc : acc + beta * q[row];
+            p[row] = pi;
+            q[row] = qi;
+            v += pi * qi;
         }
     }
     block_partials(part + 3 * G, G, v, 0.0, 1);
+}
+
+// the same with LPR lanes per row
+template <int LPR>
+__global__ __launch_bounds__(kBlock) void k_cg_spmv_l(int n, const int* __restrict__ rp, const int* __restrict__ ci,
+                                                      const double* __restrict__ v, const double* __restrict__ z,
+                                                      double* __restrict__ p, double* __restrict__ q, int k,
+                                                      double* part, CgState* st) {
+    if (st->done) return;
+    const int G = gridDim.x;
+    const RowShare R = row_share<LPR>(n, xcd_block(), G);
+    const int sub = threadIdx.x & (LPR - 1);
+    int row = R.r0 + threadIdx.x / LPR;
+    double s[1] = {0.0};
+    if (row < R.r1) csr_row<LPR, 1>(rp, ci, v, {z}, row, sub, s);
+    double beta;
+    if (!cg_beta(k, part, G, st, beta)) return;
+    double dot = 0.0;
+    while (row < R.r1) {
+        if (sub == 0) {
+            const double pi = k == 0 ? z[row] : z[row] + beta * p[row];
+            const double qi = k == 0 ? s[0] : s[0] + beta * q[row];
+            p[row] = pi;
+            q[row] = qi;
+            dot += pi * qi;
+        }
+        row += kBlock / LPR;
+        if (row < R.r1) csr_row<LPR, 1>(rp, ci, v, {z}, row, sub, s);
+    }
+    block_partials(part + 3 * G, G, dot, 0.0, 1);
+}
+
+// alpha_k from the G partials of (p, q); false on breakdown
+__device__ inline bool cg_alpha(int k, const double* part, int G, CgState* st, double& alpha) {
+    double t[1];
+    reduce_partials_all<1>(part + 3 * G, G, G, t);
+    const double pq = t[0];
+    if (!(pq > 0.0) || !isfinite(pq)) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) st->done = 2;
+        return false;
+    }
+    alpha = st->gam[k & 1] / pq;
+    return true;
 }
 
 template <bool JAC>
@@ -271,15 +353,8 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(int n, const double* __res
                                                       double* __restrict__ z, int k, double* part, CgState* st) {
     if (st->done) return;
     const int G = gridDim.x;
-    double t[1];
-    reduce_partials_all<1>(part + 3 * G, G, G, t);
-    const double pq = t[0];
-    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-    if (!(pq > 0.0) || !isfinite(pq)) {
-        if (lead) st->done = 2;
-        return;
-    }
-    const double alpha = st->gam[k & 1] / pq;
+    double alpha;
+    if (!cg_alpha(k, part, G, st, alpha)) return;
     double vrz = 0.0, vrr = 0.0;
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += G * kBlock) {
         x[i] += alpha * p[i];
@@ -292,45 +367,120 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(int n, const double* __res
             vrz += ri * zi;
         }
     }
-    if (lead) st->iters = k + 1;
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->iters = k + 1;
     if (JAC) block_partials(part + G, G, vrz, vrr, 2);
     else block_partials(part + 2 * G, G, vrr, 0.0, 1);
 }
 
-// (r, r) after the last update when the loop stopped on maxit.
-__global__ __launch_bounds__(kBlock) void k_cg_final(int G, double* part, CgState* st) {
-    double t[2];
-    reduce_partials_all<2>(part + G, G, G, t);
-    if (threadIdx.x == 0 && st->done == 0) st->rr = t[1];
-}
-
-// Fixed-budget solves (CgSolver::enqueue): b = 0 gives x = 0 at once.
-__global__ __launch_bounds__(kBlock) void k_cg_trivial(int n, double* __restrict__ x, CgState* st) {
-    if (st->bb != 0.0) return;
-    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) x[i] = 0.0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        st->done = 1;
-        st->rr = 0.0;
-    }
-}
-
-// End of a fixed-budget solve: a residual that met the tolerance on the last
-// update counts as converged; anything else increments *fails.  *imax keeps
-// the largest iteration count seen.
-__global__ __launch_bounds__(kBlock) void k_cg_check(int G, int budget, const double* part, CgState* st,
-                                                     unsigned* fails, int* imax) {
-    double t[2];
-    reduce_partials_all<2>(part + G, G, G, t);
-    if (threadIdx.x != 0) return;
-    if (st->done == 0) {
-        st->rr = t[1];
-        if (t[1] <= st->tol2bb) {
-            st->done = 1;
-            st->iters = budget;
+// Blocks [0, G): x += alpha p, rn = r - alpha q, partial (rn, rn).  Further
+// blocks: out = F rn = F r - alpha F q for the preconditioner's first product
+// F, LPR lanes per row of a CSR matrix (LPR = 0: one block per row of a dense
+// rows x n matrix).  r is only read (rn is another vector), so the two parts
+// need no order.
+template <int LPR>
+__global__ __launch_bounds__(kBlock) void k_cg_step(int n, int G, const double* __restrict__ p,
+                                                    const double* __restrict__ q, double* __restrict__ x,
+                                                    const double* __restrict__ r, double* __restrict__ rn, int rows,
+                                                    const int* __restrict__ rp, const int* __restrict__ ci,
+                                                    const double* __restrict__ v, double* __restrict__ out, int k,
+                                                    double* part, CgState* st) {
+    if (st->done) return;
+    double alpha;
+    if ((int)blockIdx.x < G) {
+        if (!cg_alpha(k, part, G, st, alpha)) return;
+        double vrr = 0.0;
+        for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += G * kBlock) {
+            x[i] += alpha * p[i];
+            const double ri = r[i] - alpha * q[i];
+            rn[i] = ri;
+            vrr += ri * ri;
+        }
+        if (blockIdx.x == 0 && threadIdx.x == 0) st->iters = k + 1;
+        block_partials(part + 2 * G, G, vrr, 0.0, 1);
+    } else if constexpr (LPR > 0) {
+        const int row = ((blockIdx.x - G) * kBlock + threadIdx.x) / LPR, sub = threadIdx.x & (LPR - 1);
+        double s[2] = {0.0, 0.0};
+        if (row < rows) csr_row<LPR, 2>(rp, ci, v, {r, q}, row, sub, s);
+        if (!cg_alpha(k, part, G, st, alpha)) return;
+        if (row < rows && sub == 0) out[row] = s[0] - alpha * s[1];
+    } else {
+        __shared__ double sp[2][kBlock / kWave];
+        const int row = blockIdx.x - G;
+        const double* d = v + (size_t)row * n;
+        double sr = 0.0, sq = 0.0;
+        for (int j = threadIdx.x; j < n; j += kBlock) {
+            const double c = d[j];
+            sr += c * r[j];
+            sq += c * q[j];
+        }
+        if (!cg_alpha(k, part, G, st, alpha)) return;
+        sr = wave_sum(sr);
+        sq = wave_sum(sq);
+        if ((threadIdx.x & (kWave - 1)) == 0) {
+            sp[0][threadIdx.x / kWave] = sr;
+            sp[1][threadIdx.x / kWave] = sq;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double a = 0.0, c = 0.0;
+            for (int w = 0; w < kBlock / kWave; ++w) {
+                a += sp[0][w];
+                c += sp[1][w];
+            }
+            out[row] = a - alpha * c;
         }
     }
-    if (st->done != 1) fails[0] += 1u;
-    if (st->iters > imax[0]) imax[0] = st->iters;
+}
+
+// After a chunk of iterations: a residual that met the tolerance on the last
+// update counts as converged (the preconditioner that would test it has not
+// run).  When the solve has ended (converged, broken down, or `last`: no more
+// iterations follow): b = 0 gives x = 0; with a window (w) the solution goes
+// into its head slot, beside its b, and the head advances, or the window is
+// emptied after a failure; fails / imax (fixed budgets): solves that missed
+// the tolerance and the largest iteration count.  host: a copy of the state
+// in pinned memory.  The block that arrives last at the ticket changes the
+// window state, which every block has read by then.
+__global__ __launch_bounds__(kBlock) void k_cg_finish(int n, int G, int last, CgWindow* w, double* __restrict__ Xw,
+                                                      double* __restrict__ x, const double* part, CgState* st,
+                                                      unsigned* ticket, unsigned* fails, int* imax, CgState* host) {
+    double t[1];
+    reduce_partials_all<1>(part + 2 * G, G, G, t);
+    const int done = st->done;
+    const bool conv = done == 1 || (done == 0 && t[0] <= st->tol2bb);
+    const bool zero = st->bb == 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        CgState c = *st;
+        if (done == 0) {
+            c.rr = t[0];
+            c.done = conv ? 1 : 0;
+            *st = c;
+        }
+        if (host) *host = c;
+        if (fails && last) {
+            if (!conv) fails[0] += 1u;
+            if (c.iters > imax[0]) imax[0] = c.iters;
+        }
+    }
+    if (!conv && done == 0 && !last) return;
+    const int head = w ? w->head : 0;
+    if (zero || (w && conv))
+        for (int e = blockIdx.x * kBlock + threadIdx.x; e < n; e += gridDim.x * kBlock) {
+            const double xe = zero ? 0.0 : x[e];
+            if (zero) x[e] = xe;
+            if (w && conv) Xw[(size_t)head * n + e] = xe;
+        }
+    if (!w) return;
+    __syncthreads();  // every thread of the block has read the window state
+    if (threadIdx.x != 0 || atomicAdd(ticket, 1u) != gridDim.x - 1u) return;
+    *ticket = 0u;
+    if (conv) {
+        w->cnt = min(w->cnt + 1, kSolveWindow);
+        w->head = (head + 1) % kSolveWindow;
+    } else {
+        w->cnt = 0;
+        w->head = 0;
+    }
 }
 
 }  // namespace
@@ -447,97 +597,161 @@ int CgSolver::setup(int n_, const int* rowptr, const int* colidx, const double* 
     TM_CHECK(val.upload(sv.data(), sv.size(), s));
     TM_CHECK(dinv.upload(di.data(), di.size(), s));
     TM_CHECK(fixed.upload(fx.data(), fx.size(), s));
-    TM_CHECK(r.alloc(n));
     TM_CHECK(z.alloc(n));
     TM_CHECK(q.alloc(n));
-    TM_CHECK(p0.alloc(n));
-    TM_CHECK(p1.alloc(n));
-    grid = xcd_grid(std::min(kMaxCgBlocks, (pat.nslices + kBlock / kWave - 1) / (kBlock / kWave)));
+    TM_CHECK(p.alloc(n));
+    lanes = precond == TM_PRECOND_AMG && n <= kLaneRows;
+    if (lanes) {
+        // lanes per row: what fills the chip (1,024 blocks) once, at most 16
+        A.n = n;
+        A.lpr = 4;
+        while (A.lpr < 16 && (int64_t)2 * A.lpr * n <= (int64_t)1024 * kBlock) A.lpr *= 2;
+        TM_CHECK(A.rp.upload(rowptr, (size_t)n + 1, s));
+        TM_CHECK(A.ci.upload(colidx, (size_t)rowptr[n], s));
+        TM_CHECK(A.v.upload(vals, (size_t)rowptr[n], s));
+    }
+    grid = lanes ? grid_for((int64_t)n * A.lpr) : (pat.nslices + kBlock / kWave - 1) / (kBlock / kWave);
+    grid = xcd_grid(std::min(kMaxCgBlocks, grid));
     TM_CHECK(part.alloc((size_t)4 * grid));
     TM_CHECK(winX.alloc((size_t)kSolveWindow * n));
     TM_CHECK(winB.alloc((size_t)kSolveWindow * n));
-    TM_CHECK(wpart.alloc((size_t)kWinDots * grid));
+    TM_CHECK(wpart.alloc((size_t)kWinRows * kWinBlocks));
     TM_CHECK(win.alloc(1));
     TM_HIP(hipMemsetAsync(win.p, 0, sizeof(CgWindow), s));
+    TM_CHECK(ticket.alloc(1));
+    TM_HIP(hipMemsetAsync(ticket.p, 0, sizeof(unsigned), s));
     TM_CHECK(st.alloc(1));
     TM_HIP(hipMemsetAsync(st.p, 0, sizeof(CgState), s));
     if (!h_st) TM_HIP(hipHostMalloc((void**)&h_st, sizeof(CgState), hipHostMallocDefault));
     TM_HIP(hipStreamSynchronize(s));
-    if (precond == TM_PRECOND_AMG) TM_CHECK(amg.setup(n, rowptr, colidx, vals, fx, &pat, val.p, dinv.p, s));
-    last_iters = 0;
+    if (precond == TM_PRECOND_AMG) TM_CHECK(amg.setup(n, rowptr, colidx, vals, fx, &pat, val.p, dinv.p, lanes ? A.lpr : 0, s));
+    for (auto& v : rb) {
+        v.release();
+        TM_CHECK(v.alloc((size_t)n + (precond == TM_PRECOND_AMG ? amg.tail() : 0)));
+        if (!lanes) break;  // one residual vector, updated in place
+    }
+    last_iters[0] = last_iters[1] = -1;
     return TM_OK;
 }
 
-void CgSolver::win_project(const double* b, double* x, hipStream_t s) {
-    hipLaunchKernelGGL(k_cg_win_dots, dim3(grid), dim3(kBlock), 0, s, n, (const CgWindow*)win.p, winB.p, b, wpart.p);
-    hipLaunchKernelGGL(k_cg_win_solve, dim3(1), dim3(kBlock), 0, s, grid, win.p, (const double*)wpart.p);
-    hipLaunchKernelGGL(k_cg_win_combine, dim3(grid), dim3(kBlock), 0, s, n, (const CgWindow*)win.p,
-                       (const double*)winX.p, x);
+// Initial guess (project: from the window, b going into its head slot) and
+// residual; the convergence state.
+int CgSolver::start(Seq& sq, const double* b, double* x, double tol, hipStream_t s, bool project) {
+    const double* bbpart = part.p;
+    int Gb = grid;
+    if (project) {
+        Gb = std::min(kWinBlocks, grid_for(n));
+        hipLaunchKernelGGL(k_cg_win_dots, dim3(Gb), dim3(kBlock), 0, s, n, (const CgWindow*)win.p, winB.p, b, wpart.p);
+        hipLaunchKernelGGL(k_cg_win_combine, dim3(std::min(grid, grid_for(n))), dim3(kBlock), 0, s, n, Gb,
+                           (const CgWindow*)win.p, (const double*)wpart.p, (const double*)winX.p,
+                           (const unsigned char*)fixed.p, b, x);
+        bbpart = wpart.p + (size_t)kWinDots * Gb;
+    } else {
+        hipLaunchKernelGGL(k_cg_init_fixed, dim3(grid), dim3(kBlock), 0, s, n, fixed.p, b, x, part.p);
+    }
+    sq = Seq{rb[0].p, rb[1].p, false, true};
+    if (lanes)
+        with_lanes(A.lpr, [&](auto lpr) {
+            hipLaunchKernelGGL(k_cg_init_res_l<decltype(lpr)::value>, dim3(grid), dim3(kBlock), 0, s, n, A.rp.p,
+                               A.ci.p, A.v.p, b, (const double*)x, sq.rcur, bbpart, Gb, part.p, tol, st.p);
+        });
+    else if (precond == TM_PRECOND_JACOBI)
+        hipLaunchKernelGGL(k_cg_init_res<true>, dim3(grid), dim3(kBlock), 0, s, view(pat), val.p, dinv.p, b,
+                           (const double*)x, sq.rcur, z.p, bbpart, Gb, part.p, tol, st.p);
+    else
+        hipLaunchKernelGGL(k_cg_init_res<false>, dim3(grid), dim3(kBlock), 0, s, view(pat), val.p, dinv.p, b,
+                           (const double*)x, sq.rcur, z.p, bbpart, Gb, part.p, tol, st.p);
+    TM_HIP(hipGetLastError());
+    return TM_OK;
 }
 
-// after win_project with the same b: the head slot holds b already
-void CgSolver::win_record(const double* x, hipStream_t s) {
-    hipLaunchKernelGGL(k_cg_win_store, dim3(grid), dim3(kBlock), 0, s, n, (const CgWindow*)win.p, x, winX.p);
-    hipLaunchKernelGGL(k_cg_win_advance, dim3(1), dim3(1), 0, s, win.p, (const CgState*)st.p);
+int CgSolver::precondition(Seq& sq, hipStream_t s) {
+    if (precond == TM_PRECOND_JACOBI) return TM_OK;  // z = D^-1 r comes with the update
+    TM_CHECK(amg.apply(sq.rcur, z.p, part.p + grid, grid, s, st.p, sq.rr_new ? part.p + 2 * (size_t)grid : nullptr,
+                       sq.first_done));
+    sq.rr_new = false;
+    return TM_OK;
+}
+
+// another: the preconditioner runs on the new residual, and its first product
+// is formed along with the update
+int CgSolver::iteration(Seq& sq, double* x, int k, bool another, hipStream_t s) {
+    const int G = grid;
+    const bool jac = precond == TM_PRECOND_JACOBI;
+    if (lanes)
+        with_lanes(A.lpr, [&](auto lpr) {
+            hipLaunchKernelGGL(k_cg_spmv_l<decltype(lpr)::value>, dim3(G), dim3(kBlock), 0, s, n, A.rp.p, A.ci.p,
+                               A.v.p, (const double*)z.p, p.p, q.p, k, part.p, st.p);
+        });
+    else
+        hipLaunchKernelGGL(k_cg_spmv, dim3(G), dim3(kBlock), 0, s, view(pat), val.p, (const double*)z.p, p.p, q.p, k,
+                           part.p, st.p);
+    sq.first_done = lanes && another && !amg.levels.empty();
+    if (sq.first_done) {
+        const AmgPrecond::First F = amg.first();
+        double* out = F.out ? F.out : sq.rnext + n;
+        if (F.dense)
+            hipLaunchKernelGGL(k_cg_step<0>, dim3(G + F.rows), dim3(kBlock), 0, s, n, G, (const double*)p.p,
+                               (const double*)q.p, x, (const double*)sq.rcur, sq.rnext, F.rows, (const int*)nullptr,
+                               (const int*)nullptr, F.dense, out, k, part.p, st.p);
+        else
+            with_lanes(F.csr->lpr, [&](auto lpr) {
+                constexpr int kL = decltype(lpr)::value;
+                hipLaunchKernelGGL(k_cg_step<kL>, dim3(G + (F.rows + kBlock / kL - 1) / (kBlock / kL)), dim3(kBlock),
+                                   0, s, n, G, (const double*)p.p, (const double*)q.p, x, (const double*)sq.rcur,
+                                   sq.rnext, F.rows, F.csr->rp.p, F.csr->ci.p, F.csr->v.p, out, k, part.p, st.p);
+            });
+        std::swap(sq.rcur, sq.rnext);
+    } else if (jac) {
+        hipLaunchKernelGGL(k_cg_update<true>, dim3(G), dim3(kBlock), 0, s, n, dinv.p, p.p, q.p, x, sq.rcur, z.p, k,
+                           part.p, st.p);
+    } else {
+        hipLaunchKernelGGL(k_cg_update<false>, dim3(G), dim3(kBlock), 0, s, n, dinv.p, p.p, q.p, x, sq.rcur, z.p, k,
+                           part.p, st.p);
+    }
+    sq.rr_new = true;
+    TM_HIP(hipGetLastError());
+    return TM_OK;
+}
+
+int CgSolver::finish(const double* x, hipStream_t s, bool project, bool last, unsigned* fails, int* imax,
+                     CgState* out) {
+    // few blocks: each takes a ticket, one after the other
+    hipLaunchKernelGGL(k_cg_finish, dim3(std::min(64, grid_for(n, 4 * kBlock))), dim3(kBlock), 0, s, n, grid, last ? 1 : 0, project ? win.p : nullptr, winX.p,
+                       const_cast<double*>(x), (const double*)part.p, st.p, ticket.p, fails, imax, out);
+    TM_HIP(hipGetLastError());
+    return TM_OK;
 }
 
 int CgSolver::solve(const double* b, double* x, double tol, int maxit, hipStream_t s, int* iters, double* relres,
                     bool project) {
     if (n == 0) return TM_ERR_NOT_READY;
     if (!(tol > 0.0) || maxit < 1) return TM_ERR_BAD_ARG;
-    const int G = grid;
-    const SellView A = view(pat);
-    if (project) win_project(b, x, s);
-    hipLaunchKernelGGL(k_cg_init_fixed, dim3(G), dim3(kBlock), 0, s, n, fixed.p, b, x, part.p);
-    const bool jac = precond == TM_PRECOND_JACOBI;
-    if (jac)
-        hipLaunchKernelGGL(k_cg_init_res<true>, dim3(G), dim3(kBlock), 0, s, A, val.p, dinv.p, b, x, r.p, z.p, part.p,
-                           tol, st.p);
-    else
-        hipLaunchKernelGGL(k_cg_init_res<false>, dim3(G), dim3(kBlock), 0, s, A, val.p, dinv.p, b, x, r.p, z.p,
-                           part.p, tol, st.p);
-    TM_HIP(hipGetLastError());
-    if (!jac) TM_CHECK(amg.apply(r.p, z.p, part.p + G, G, s, st.p, part.p + 2 * G));
-    // First chunk sized from the previous solve (warm-started solves along a
-    // trajectory need similar counts), then small chunks.
+    Seq sq;
+    TM_CHECK(start(sq, b, x, tol, s, project));
+    // The first chunk is what the last such solve needed (solves along a
+    // trajectory need similar counts); no preconditioner runs after a chunk's last
+    // iteration before the host has seen that another one is needed.
+    int& known = last_iters[project ? 0 : 1];
     int enq = 0;
-    int chunk = std::max(4, std::min(maxit, last_iters > 8 ? last_iters - 2 : 8));
-    double* pcur = p0.p;
-    double* pold = p1.p;
-    for (;;) {
-        for (int c = 0; c < chunk && enq < maxit; ++c, ++enq) {
-            hipLaunchKernelGGL(k_cg_spmv, dim3(G), dim3(kBlock), 0, s, A, val.p, z.p, pold, pcur, q.p, enq, part.p,
-                               st.p);
-            if (jac) {
-                hipLaunchKernelGGL(k_cg_update<true>, dim3(G), dim3(kBlock), 0, s, n, dinv.p, pcur, q.p, x, r.p, z.p,
-                                   enq, part.p, st.p);
-            } else {
-                hipLaunchKernelGGL(k_cg_update<false>, dim3(G), dim3(kBlock), 0, s, n, dinv.p, pcur, q.p, x, r.p,
-                                   z.p, enq, part.p, st.p);
-                TM_CHECK(amg.apply(r.p, z.p, part.p + G, G, s, st.p, part.p + 2 * G));
-            }
-            std::swap(pcur, pold);
+    int chunk = known < 0 ? 8 : known;
+    for (int more = 2;; more = std::min(2 * more, 8)) {
+        const int end = std::min(maxit, enq + chunk);
+        for (; enq < end; ++enq) {
+            TM_CHECK(precondition(sq, s));
+            TM_CHECK(iteration(sq, x, enq, enq + 1 < end, s));
         }
-        TM_HIP(hipGetLastError());
-        TM_HIP(hipMemcpyAsync(h_st, st.p, sizeof(CgState), hipMemcpyDeviceToHost, s));
+        TM_CHECK(finish(x, s, project, enq >= maxit, nullptr, nullptr, h_st));
         TM_HIP(hipStreamSynchronize(s));
         if (h_st->done || enq >= maxit) break;
-        chunk = 4;
-    }
-    if (!h_st->done) {
-        // one more convergence test on the last residual
-        hipLaunchKernelGGL(k_cg_final, dim3(1), dim3(kBlock), 0, s, G, part.p, st.p);
-        TM_HIP(hipMemcpyAsync(h_st, st.p, sizeof(CgState), hipMemcpyDeviceToHost, s));
-        TM_HIP(hipStreamSynchronize(s));
+        chunk = more;
     }
     const CgState hs = *h_st;
-    if (hs.bb == 0.0) TM_HIP(hipMemsetAsync(x, 0, sizeof(double) * n, s));
-    if (project) win_record(x, s);
-    last_iters = hs.iters;
+    known = hs.iters;
     if (iters) *iters = hs.iters;
     if (relres) *relres = hs.bb > 0 ? std::sqrt(hs.rr / hs.bb) : 0.0;
     if (hs.done == 2) return TM_ERR_NONFINITE;
-    if (hs.done == 1 || hs.bb == 0.0 || hs.rr <= hs.tol2bb) return TM_OK;
+    if (hs.done == 1 || hs.bb == 0.0) return TM_OK;
     return TM_ERR_MAXITER;
 }
 
@@ -545,38 +759,13 @@ int CgSolver::enqueue(const double* b, double* x, double tol, int budget, hipStr
                       int* imax, bool project) {
     if (n == 0) return TM_ERR_NOT_READY;
     if (!(tol > 0.0) || budget < 1 || !fails || !imax) return TM_ERR_BAD_ARG;
-    const int G = grid;
-    const SellView A = view(pat);
-    const bool jac = precond == TM_PRECOND_JACOBI;
-    if (project) win_project(b, x, s);
-    hipLaunchKernelGGL(k_cg_init_fixed, dim3(G), dim3(kBlock), 0, s, n, fixed.p, b, x, part.p);
-    if (jac)
-        hipLaunchKernelGGL(k_cg_init_res<true>, dim3(G), dim3(kBlock), 0, s, A, val.p, dinv.p, b, x, r.p, z.p, part.p,
-                           tol, st.p);
-    else
-        hipLaunchKernelGGL(k_cg_init_res<false>, dim3(G), dim3(kBlock), 0, s, A, val.p, dinv.p, b, x, r.p, z.p,
-                           part.p, tol, st.p);
-    hipLaunchKernelGGL(k_cg_trivial, dim3(G), dim3(kBlock), 0, s, n, x, st.p);
-    if (!jac) TM_CHECK(amg.apply(r.p, z.p, part.p + G, G, s, st.p, part.p + 2 * G));
-    double* pcur = p0.p;
-    double* pold = p1.p;
+    Seq sq;
+    TM_CHECK(start(sq, b, x, tol, s, project));
     for (int k = 0; k < budget; ++k) {
-        hipLaunchKernelGGL(k_cg_spmv, dim3(G), dim3(kBlock), 0, s, A, val.p, z.p, pold, pcur, q.p, k, part.p, st.p);
-        if (jac) {
-            hipLaunchKernelGGL(k_cg_update<true>, dim3(G), dim3(kBlock), 0, s, n, dinv.p, pcur, q.p, x, r.p, z.p, k,
-                               part.p, st.p);
-        } else {
-            hipLaunchKernelGGL(k_cg_update<false>, dim3(G), dim3(kBlock), 0, s, n, dinv.p, pcur, q.p, x, r.p, z.p, k,
-                               part.p, st.p);
-            if (k + 1 < budget)  // the z of the last update would go unused
-                TM_CHECK(amg.apply(r.p, z.p, part.p + G, G, s, st.p, part.p + 2 * G));
-        }
-        std::swap(pcur, pold);
+        TM_CHECK(precondition(sq, s));
+        TM_CHECK(iteration(sq, x, k, k + 1 < budget, s));
     }
-    hipLaunchKernelGGL(k_cg_check, dim3(1), dim3(kBlock), 0, s, G, budget, (const double*)part.p, st.p, fails, imax);
-    if (project) win_record(x, s);
-    TM_HIP(hipGetLastError());
-    return TM_OK;
+    return finish(x, s, project, true, fails, imax, nullptr);
 }
 
 int CgSolver::solve_transposed(const double* w, double* y, double tol, int maxit, hipStream_t s, int* iters,

@@ -7,6 +7,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <type_traits>
 #include <vector>
 
 #include "tetmag_hip.h"
@@ -222,6 +223,74 @@ __device__ inline int xcd_block() {
     return (b % kXcd) * (G / kXcd) + b / kXcd;
 }
 
+// ---- rows of a CSR matrix shared by LPR lanes each -------------------------
+template <int LPR>
+__device__ inline double group_sum(double v) {
+#pragma unroll
+    for (int o = LPR / 2; o > 0; o >>= 1) v += __shfl_down(v, o, LPR);
+    return v;
+}
+
+// The row's sum of v * x[col] over NX vectors (complete on lane sub = 0).  A
+// lane takes entries sub, sub + LPR, ..., four at a time: their columns, then
+// their values and gathers, are in flight together (entries past the row's end
+// read its first entry with weight zero; an empty row reads nothing).
+template <int LPR, int NX>
+__device__ inline void csr_row(const int* __restrict__ rp, const int* __restrict__ ci, const double* __restrict__ v,
+                               const double* const (&x)[NX], int row, int sub, double (&out)[NX]) {
+    const int q0 = rp[row], q1 = rp[row + 1];
+    double acc[NX];
+#pragma unroll
+    for (int j = 0; j < NX; ++j) acc[j] = 0.0;
+    for (int q = q0 + sub; q < q1; q += 4 * LPR) {
+        int e[4], c[4];
+        double w[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) e[k] = q + k * LPR < q1 ? q + k * LPR : q;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            c[k] = ci[e[k]];
+            w[k] = v[e[k]];
+        }
+#pragma unroll
+        for (int j = 0; j < NX; ++j) {
+            double g[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) g[k] = x[j][c[k]];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc[j] += q + k * LPR < q1 ? w[k] * g[k] : 0.0;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NX; ++j) out[j] = group_sum<LPR>(acc[j]);
+}
+
+// Rows of this block's contiguous share of n rows (XCD-contiguous, so a row
+// meets the same L2 in every kernel of a solve), LPR lanes per row:
+// row = r0 + threadIdx.x / LPR, then + kBlock / LPR, while < r1.
+struct RowShare {
+    int r0, r1;
+};
+template <int LPR>
+__device__ inline RowShare row_share(int n, int block, int blocks) {
+    constexpr int kGroups = kBlock / LPR;
+    const int per = ((n + blocks - 1) / blocks + kGroups - 1) / kGroups * kGroups;
+    const int64_t r0 = (int64_t)block * per;
+    return RowShare{(int)(r0 < n ? r0 : n), (int)(r0 + per < n ? r0 + per : n)};
+}
+
+// calls f(std::integral_constant<int, LPR>) for the lane counts in use
+template <class F>
+inline void with_lanes(int lpr, F&& f) {
+    switch (lpr) {
+        case 4: f(std::integral_constant<int, 4>{}); break;
+        case 8: f(std::integral_constant<int, 8>{}); break;
+        case 16: f(std::integral_constant<int, 16>{}); break;
+        case 32: f(std::integral_constant<int, 32>{}); break;
+        default: f(std::integral_constant<int, 64>{}); break;
+    }
+}
+
 // Copies between a caller pointer (host or device) and a device buffer.
 int copy_in(double* dst_dev, const double* src, int where, size_t count, hipStream_t s);
 int copy_out(double* dst, int where, const double* src_dev, size_t count, hipStream_t s);
@@ -250,8 +319,7 @@ constexpr int kWinGram = kSolveWindow * (kSolveWindow + 1) / 2;
 constexpr int kWinDots = kWinGram + kSolveWindow + 1;
 
 struct CgWindow {
-    int head, cnt;             // slot the next pair goes to; pairs held
-    double a[kSolveWindow];    // x0 = sum_i a_i x_i (newest first), from the last projection
+    int head, cnt;  // slot the next pair goes to; pairs held
 };
 
 // slot of the i-th newest pair in a ring of kSolveWindow slots
@@ -384,6 +452,9 @@ struct CgState {
 struct AmgPrecond {
     static constexpr int kCoarseMax = 512;
     static constexpr int kMaxLevels = 8;
+    // entries up to which the coarsest level's restriction and inverse are
+    // kept as one dense matrix (8 MB)
+    static constexpr int64_t kDenseMax = (int64_t)1 << 20;
     // CSR on the device, processed with `lpr` lanes per row.
     struct CsrDev {
         int n = 0;
@@ -401,19 +472,41 @@ struct AmgPrecond {
         const double* dinv_ext = nullptr;
         CsrDev A, P, R;  // A used on levels >= 1
         DevBuf<double> dinv;
-        DevBuf<double> x, x2, r, b;  // b: restricted right-hand side of the next level
+        CsrDev down;        // R (I - A w D^-1): pre-smoothing from zero and restriction
+        CsrDev up;          // [2 w D^-1 - w D^-1 A w D^-1 | (I - w D^-1 A) P] on [b | x_c]
+        DevBuf<double> bx;  // levels >= 1: [b | x_c], the restricted right-hand side and the coarser correction
+        DevBuf<double> x;   // level 0 without `up`: w D^-1 b + P x_c
     };
     std::vector<Level> levels;
     int nc = 0;
-    DevBuf<double> Cinv, xc, bc;
+    DevBuf<double> Cinv, bc;
+    DevBuf<double> D;   // dense Cinv * down of the last level (nc x n), where it is small enough
+    // The level-0 vectors handed to apply() are [r | x_c] with tail() further
+    // entries for the coarse correction.
+    int tail() const { return levels.empty() ? 0 : (levels.size() > 1 ? levels[1].n : nc); }
+    // Level 0 goes up in one product (`up`) instead of prolongation and
+    // post-smoothing.
+    bool up0() const { return !levels.empty() && levels[0].up.n > 0; }
+    // up0_lpr: lanes per row of level 0's product upwards (0: in two steps)
     int setup(int n, const int* rowptr, const int* colidx, const double* vals, const std::vector<unsigned char>& fixed,
-              const SellPattern* A0, const double* A0val, const double* A0dinv, hipStream_t s);
-    // z = M^-1 r (one V-cycle); every kernel returns at once when st != NULL
-    // and st->done is set (the CG it serves has stopped).  With rr_part (the
-    // grid partials of (r, r) from the CG update) the first kernel ends the
-    // CG when ||r||^2 <= st->tol2bb, so a converged CG skips the V-cycle.
-    int apply(const double* r, double* z, double* part, int grid, hipStream_t s, CgState* st = nullptr,
-              const double* rr_part = nullptr);
+              const SellPattern* A0, const double* A0val, const double* A0dinv, int up0_lpr, hipStream_t s);
+    // z = M^-1 r (one V-cycle) for r = [r | x_c]; the (r, z) partials of `grid`
+    // blocks go to part.  Every kernel returns at once when st != NULL and
+    // st->done is set (the CG it serves has stopped).  With rr_part (the
+    // `grid` partials of (r, r) from the CG update) the first kernel ends
+    // the CG when ||r||^2 <= st->tol2bb, so a converged CG skips the V-cycle.
+    // first_done: the V-cycle's first product has been formed already (first()).
+    int apply(double* r, double* z, double* part, int grid, hipStream_t s, CgState* st, const double* rr_part,
+              bool first_done);
+    // The V-cycle's first product out = F r: `down` of level 0, or the dense
+    // matrix where there is one level only (out is then the tail of r).
+    struct First {
+        int rows;
+        const CsrDev* csr;    // or
+        const double* dense;  // rows x n
+        double* out;          // null: the tail of r
+    };
+    First first() const;
 };
 
 struct CgSolver {
@@ -426,17 +519,22 @@ struct CgSolver {
     std::vector<unsigned char> h_fixed;
     DevBuf<double> dinv;     // inverse diagonal (1 on fixed rows)
     DevBuf<unsigned char> fixed;  // 1 on identity rows
-    DevBuf<double> r, z, q, p0, p1;
+    // lanes: several lanes share a matrix row (CSR copy A); rb: [r | x_c],
+    // the two swapped by each fused update
+    bool lanes = false;
+    AmgPrecond::CsrDev A;
+    DevBuf<double> rb[2], z, q, p;
     DevBuf<double> part;     // partial sums: bb | rz | rr | pq, grid entries each
     DevBuf<CgState> st;
-    CgState* h_st = nullptr;  // pinned mirror for the convergence check
+    CgState* h_st = nullptr;  // pinned; written by the device at the end of a chunk of iterations
     // the last kSolveWindow solved pairs (x, b) and the initial-guess state
     DevBuf<double> winX, winB, wpart;
     DevBuf<CgWindow> win;
+    DevBuf<unsigned> ticket;  // blocks of the finishing kernel that have read the window state
     int precond = TM_PRECOND_JACOBI;
     AmgPrecond amg;
     int nfixed = 0;
-    int last_iters = 0;
+    int last_iters[2] = {-1, -1};  // of the last projected and the last other solve (-1: none yet)
     // Coupling of the identity rows to the free unknowns, for the transposed
     // solve: row r (node fix_idx[r]) holds A_ij over free rows i that have a
     // column j = fix_idx[r].
@@ -457,15 +555,32 @@ struct CgSolver {
     // if the tolerance was not met, and *imax keeps the largest count.
     int enqueue(const double* b, double* x, double tol, int budget, hipStream_t s, unsigned* fails, int* imax,
                 bool project = false);
-    void win_project(const double* b, double* x, hipStream_t s);
-    void win_record(const double* x, hipStream_t s);  // after win_project with the same b
     // Solves A^T y = w for the same matrix (identity rows on the fixed set F):
     // y_free = A_ff^-1 w_free (A_ff symmetric), y_F = w_F - A_{free,F}^T y_free.
     int solve_transposed(const double* w, double* y, double tol, int maxit, hipStream_t s, int* iters,
                          double* relres);
+
+private:
+    // One solve as a sequence of launches: start, then iterations 0, 1, ...,
+    // each preceded by precondition() (of the current residual), and finish.
+    struct Seq {
+        double* rcur;
+        double* rnext;
+        bool first_done;  // the V-cycle's first product of rcur is formed already
+        bool rr_new;      // the (r, r) partials of rcur have not been tested yet
+    };
+    int start(Seq& q, const double* b, double* x, double tol, hipStream_t s, bool project);
+    int precondition(Seq& q, hipStream_t s);
+    int iteration(Seq& q, double* x, int k, bool another, hipStream_t s);
+    int finish(const double* x, hipStream_t s, bool project, bool last, unsigned* fails, int* imax, CgState* out);
 };
 
-constexpr int kMaxCgBlocks = 512;
+constexpr int kMaxCgBlocks = 2048;
+// Rows up to which several lanes share a matrix row in the single-sample
+// solver's level-0 kernels (above, one lane per row in SELL order fills the
+// chip, and the fused step's two gathers per entry cost more than the launch
+// they save).
+constexpr int kLaneRows = 1 << 17;
 
 // Read-only view of a field context's device data (tm_field.hip), used by
 // the batched evaluator.
