@@ -81,6 +81,8 @@ int rk4_step(tm_ctx* c, double dt, double alpha, int variant, const int* budget,
         if (iters) {
             iters[0] = std::max(iters[0], es.iters_neumann);
             iters[1] = std::max(iters[1], es.iters_dirichlet);
+            iters[2] = es.iters_neumann;  // of the last stage
+            iters[3] = es.iters_dirichlet;
         }
     }
     hipLaunchKernelGGL(k_rk_final, dim3(grid_for(n)), dim3(kBlock), 0, c->stream, n, m,
@@ -90,7 +92,38 @@ int rk4_step(tm_ctx* c, double dt, double alpha, int variant, const int* budget,
     return st;
 }
 
+// Iteration budgets of a captured step.  An iteration past convergence costs
+// its launches (three to five of about 2 us), a solve that misses its budget
+// a whole host-polled step, so the budget is what the solves need now, from their
+// starts over the window of earlier solutions, and a margin of two.  A cold
+// solve's count (the first stages of a run) is no guide: 16 to 18 iterations
+// where the later ones take 3 to 5.
+int margin(int iters) { return iters + 2; }
+// after a miss: 1.25 x the largest count of the polled step
 int grow(int iters) { return (int)std::ceil(1.25 * iters) + 4; }
+// a graph is captured again with smaller budgets after this many replays in
+// which no solve needed more than half of them
+constexpr int kShrinkAfter = 8;
+
+// The largest counts seen by a graph since its capture.
+struct Replays {
+    int count = 0;
+    int imax[2] = {0, 0};
+    void add(const int* it) {
+        ++count;
+        imax[0] = std::max(imax[0], it[0]);
+        imax[1] = std::max(imax[1], it[1]);
+    }
+    bool loose(const int* budget) const {
+        return count >= kShrinkAfter && 2 * (margin(imax[0]) + margin(imax[1])) <= budget[0] + budget[1];
+    }
+    // budgets as the replays needed them (never larger); starts anew
+    void tighten(int* budget) {
+        if (count > 0)
+            for (int w = 0; w < 2; ++w) budget[w] = std::min(budget[w], margin(imax[w]));
+        *this = Replays();
+    }
+};
 
 }  // namespace
 
@@ -116,9 +149,10 @@ int tm_ctx_run_rk4(tm_ctx* c, double dtau, int nsteps, double alpha, int variant
     hipGraphExec_t exec = nullptr;
     int status = TM_OK;
     int* budget = c->rk_budget;
+    Replays seen;
     for (int step = 0; step < nsteps && status == TM_OK; ++step) {
         if (!use_graph || budget[0] == 0) {
-            int it[2] = {0, 0};
+            int it[4] = {0, 0, 0, 0};
             const int zero[2] = {0, 0};
             int r = rk4_step(c, dtau, alpha, variant, zero, it);
             if (r != TM_OK) {
@@ -128,9 +162,14 @@ int tm_ctx_run_rk4(tm_ctx* c, double dtau, int nsteps, double alpha, int variant
             S.sync_steps += 1;
             S.max_iters_neumann = std::max(S.max_iters_neumann, it[0]);
             S.max_iters_dirichlet = std::max(S.max_iters_dirichlet, it[1]);
-            budget[0] = std::max(budget[0], grow(it[0]));
-            budget[1] = std::max(budget[1], grow(it[1]));
+            budget[0] = std::max(budget[0], margin(it[2]));
+            budget[1] = std::max(budget[1], margin(it[3]));
             continue;
+        }
+        if (exec && seen.loose(budget)) {
+            seen.tighten(budget);
+            (void)hipGraphExecDestroy(exec);
+            exec = nullptr;
         }
         if (!exec) {
             hipGraph_t g = nullptr;
@@ -161,11 +200,13 @@ int tm_ctx_run_rk4(tm_ctx* c, double dtau, int nsteps, double alpha, int variant
         S.max_iters_dirichlet = std::max(S.max_iters_dirichlet, imax[1]);
         if (fail == 0) {
             S.graph_steps += 1;
+            seen.add(imax);
             continue;
         }
+        seen = Replays();
         // a solve missed the tolerance within its budget: redo the step
         TM_HIP(hipMemcpyAsync(c->m.p, c->rk_bak.p, n3 * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-        int it[2] = {0, 0};
+        int it[4] = {0, 0, 0, 0};
         const int zero[2] = {0, 0};
         const int r = rk4_step(c, dtau, alpha, variant, zero, it);
         if (r != TM_OK) {
@@ -180,6 +221,7 @@ int tm_ctx_run_rk4(tm_ctx* c, double dtau, int nsteps, double alpha, int variant
         (void)hipGraphExecDestroy(exec);
         exec = nullptr;
     }
+    seen.tighten(budget);  // for the next call
     if (exec) (void)hipGraphExecDestroy(exec);
     TM_HIP(hipEventRecord(e1, c->stream));
     TM_HIP(hipEventSynchronize(e1));
@@ -368,6 +410,8 @@ int dp_step(tm_ctx* c, OdeState* s, double alpha, int variant, const int* budget
         if (iters) {
             iters[0] = std::max(iters[0], es.iters_neumann);
             iters[1] = std::max(iters[1], es.iters_dirichlet);
+            iters[2] = es.iters_neumann;  // of the last stage
+            iters[3] = es.iters_dirichlet;
         }
     }
     // ode_y now holds the 5th-order solution y7 (a_7j = b_j)
@@ -460,12 +504,18 @@ int tm_ctx_integrate(tm_ctx* c, double tau_span, double rtol, double atol, doubl
     S.evaluations = 1;
     hipGraphExec_t exec = nullptr;
     int* budget = c->rk_budget;
+    Replays seen;
     OdeState hs = h;
     for (int step = 0; status == TM_OK && !hs.done && step < max_steps; ++step) {
         bool polled = !use_graph || budget[0] == 0;
         unsigned fail = 0;
         int imax[2] = {0, 0};
         if (!polled) {
+            if (exec && seen.loose(budget)) {
+                seen.tighten(budget);
+                (void)hipGraphExecDestroy(exec);
+                exec = nullptr;
+            }
             if (!exec) {
                 hipGraph_t g = nullptr;
                 TM_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
@@ -495,15 +545,17 @@ int tm_ctx_integrate(tm_ctx* c, double tau_span, double rtol, double atol, doubl
             S.max_iters_dirichlet = std::max(S.max_iters_dirichlet, imax[1]);
             if (fail == 0) {
                 S.graph_steps += 1;
+                seen.add(imax);
             } else {  // the commit was skipped: redo the step with host-polled solves
                 S.redone_steps += 1;
                 polled = true;
+                seen = Replays();
                 (void)hipGraphExecDestroy(exec);
                 exec = nullptr;
             }
         }
         if (polled) {
-            int it[2] = {0, 0};
+            int it[4] = {0, 0, 0, 0};
             const int zero[2] = {0, 0};
             const int r = dp_step(c, sd, alpha, variant, zero, it);
             if (r != TM_OK && r != TM_ERR_MAXITER) {
@@ -516,12 +568,13 @@ int tm_ctx_integrate(tm_ctx* c, double tau_span, double rtol, double atol, doubl
             S.sync_steps += 1;
             S.max_iters_neumann = std::max(S.max_iters_neumann, it[0]);
             S.max_iters_dirichlet = std::max(S.max_iters_dirichlet, it[1]);
-            budget[0] = std::max(budget[0] + (fail ? 4 : 0), grow(it[0]));
-            budget[1] = std::max(budget[1] + (fail ? 4 : 0), grow(it[1]));
+            budget[0] = std::max(budget[0] + (fail ? 4 : 0), fail ? grow(it[0]) : margin(it[2]));
+            budget[1] = std::max(budget[1] + (fail ? 4 : 0), fail ? grow(it[1]) : margin(it[3]));
         }
         if (hs.nonfinite && hs.h < 1e-300) status = TM_ERR_NONFINITE;
     }
     if (exec) (void)hipGraphExecDestroy(exec);
+    seen.tighten(budget);  // for the next call
     if (status == TM_OK && !hs.done) status = TM_ERR_MAXITER;  // max_steps reached before tau_span
     if (normalize && (status == TM_OK || status == TM_ERR_MAXITER))
         hipLaunchKernelGGL(k_ode_normalize, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, c->n, c->m.p);
