@@ -222,15 +222,30 @@ __global__ __launch_bounds__(kBlock) void k_bem_gemv_part(int b, int ld, const d
 }
 
 // y_r = sum_s part[s][r]; optionally also scattered to dst[sidx[r]]
-// (DemagField.cpp:195-199, boundary values of the Dirichlet problem).
+// (DemagField.cpp:195-199, boundary values of the Dirichlet problem).  A block
+// owns 16 rows (128 contiguous bytes of every split); its 16 groups of 16
+// lanes take every 16th split, so that the partials of a small matrix (many
+// splits, few rows) are read by enough wavefronts at once.
+constexpr int kFinishRows = 16;
+
 __global__ __launch_bounds__(kBlock) void k_bem_gemv_finish(int b, int ld, int splits,
                                                             const double* __restrict__ part,
                                                             double* __restrict__ y, const int* __restrict__ sidx,
                                                             double* __restrict__ dst) {
-    const int r = blockIdx.x * kBlock + threadIdx.x;
-    if (r >= b) return;
+    constexpr int kGroups = kBlock / kFinishRows;
+    __shared__ double sp[kGroups][kFinishRows + 1];
+    const int lr = threadIdx.x % kFinishRows, g = threadIdx.x / kFinishRows;
+    const int r = blockIdx.x * kFinishRows + lr;
     double s = 0.0;
-    for (int k = 0; k < splits; ++k) s += part[(size_t)k * ld + r];
+    if (r < b)
+#pragma unroll 4
+        for (int k = g; k < splits; k += kGroups) s += part[(size_t)k * ld + r];
+    sp[g][lr] = s;
+    __syncthreads();
+    if (g != 0 || r >= b) return;
+    s = 0.0;
+#pragma unroll
+    for (int k = 0; k < kGroups; ++k) s += sp[k][lr];
     if (y) y[r] = s;
     if (dst) dst[sidx[r]] = s;
 }
@@ -307,9 +322,11 @@ int bem_assemble(int b, int ld, int nbel, const double* bxyz, const int* faces, 
 
 int bem_gemv_splits(int b) {
     const int tiles = (b + kGemvTile - 1) / kGemvTile;
-    // aim for >= 1024 blocks so all 256 CUs have several to overlap
+    // >= 1024 blocks (four per CU, what its registers hold), down to 16
+    // columns a block: with 256 a small matrix left most of the chip idle
+    // (b = 1,122: 66 us on 4 blocks; b = 7,680: 98 us on 120)
     int splits = (1024 + tiles - 1) / tiles;
-    const int min_cols = 256;
+    const int min_cols = 16;
     splits = std::min(splits, std::max(1, b / min_cols));
     while ((b + splits - 1) / splits > kGemvMaxCols) ++splits;
     return std::max(1, splits);
@@ -324,7 +341,7 @@ int bem_gemv(int b, int ld, const double* B, const double* src, const int* gidx,
     const int splits = bem_gemv_splits(b);
     const int cps = (b + splits - 1) / splits;
     hipLaunchKernelGGL(k_bem_gemv_part, dim3(tiles, splits), dim3(kBlock), 0, s, b, ld, B, src, gidx, cps, part);
-    hipLaunchKernelGGL(k_bem_gemv_finish, dim3(grid_for(b)), dim3(kBlock), 0, s, b, ld, splits, part, y, sidx, dst);
+    hipLaunchKernelGGL(k_bem_gemv_finish, dim3(grid_for(b, kFinishRows)), dim3(kBlock), 0, s, b, ld, splits, part, y, sidx, dst);
     TM_HIP(hipGetLastError());
     return TM_OK;
 }
