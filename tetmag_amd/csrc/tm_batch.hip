@@ -440,9 +440,10 @@ __global__ __launch_bounds__(kBlock) void k_b_resid(SlotArgs A, int S, const dou
     b_partial(part_rr, S, vr);
 }
 
-// outer decision per sample; inner tolerance and initial inner state.
+// outer decision per sample; inner tolerance and initial inner state.  track:
+// keeps the largest iteration count of the refinement step that has ended.
 __global__ void k_b_outer_red(int G, int S, const double* part_bb, const double* part_rr, double tol, double itol,
-                              OState* os, BState* bs) {
+                              OState* os, BState* bs, int* track) {
     const int s = blockIdx.x;
     const double bb = b_total(part_bb, G);
     __syncthreads();
@@ -458,6 +459,7 @@ __global__ void k_b_outer_red(int G, int S, const double* part_bb, const double*
         const double i2 = itol * itol * rr;
         bs->itol2[s] = std::max(a2, i2);
         bs->rr[s] = rr;
+        if (track && bs->iters[s] > 0) atomicMax(track, bs->iters[s]);
         bs->active[s] = done ? 0 : 1;
         bs->iters[s] = 0;
         bs->beta[s] = 0.0;
@@ -1690,8 +1692,8 @@ __global__ void k_b_activate(int S, BState* bs) {
     }
 }
 
-__global__ void k_b_reset_fail(unsigned* fail) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) fail[0] = 0u;
+__global__ void k_b_reset_fail(int cnt, unsigned* fail) {
+    if ((int)threadIdx.x < cnt && blockIdx.x == 0) fail[threadIdx.x] = 0u;
 }
 
 __global__ __launch_bounds__(kBlock) void k_b_copy(size_t tot, const double* __restrict__ a, double* __restrict__ b) {
@@ -2423,7 +2425,8 @@ struct BatchSolver {
         int pend_step = 0;
         for (;;) {
             resid(b, x, pbb, prr, s);
-            hipLaunchKernelGGL(k_b_outer_red, dim3(S), dim3(kBlock), 0, s, G, S, pbb, prr, tol, itol, ost.p, bst.p);
+            hipLaunchKernelGGL(k_b_outer_red, dim3(S), dim3(kBlock), 0, s, G, S, pbb, prr, tol, itol, ost.p, bst.p,
+                               (int*)nullptr);
             if (!(outer == 0 && spec_ok && last_inner[0] > 0)) {
                 TM_HIP(hipMemcpyAsync(h_ost, ost.p, sizeof(OState), hipMemcpyDeviceToHost, s));
                 TM_HIP(hipStreamSynchronize(s));
@@ -2591,11 +2594,12 @@ struct BatchSolver {
     // steps and iterations past convergence cost only their launches, and
     // iterations a sample did not take carry alpha = beta = 0 into the
     // combination.  A final residual check adds the number of samples that
-    // missed the tolerance to *fail on the device.
+    // missed the tolerance to *fail on the device, and track[o] keeps the
+    // largest iteration count of refinement step o.
     int enqueue(const double* b, double* x, double tol, int nouter, const int* ninner, hipStream_t s,
-                unsigned* fail) {
+                unsigned* fail, int* track) {
         if (cg->precond != TM_PRECOND_AMG || cg->amg.levels.empty()) return TM_ERR_UNSUPPORTED;
-        if (nouter < 0 || nouter > kMaxOuter || !fail) return TM_ERR_BAD_ARG;
+        if (nouter < 0 || nouter > kMaxOuter || !fail || !track) return TM_ERR_BAD_ARG;
         const size_t NS = (size_t)n * S;
         double* pbb = part.p;
         double* prr = part.p + (size_t)S * G;
@@ -2606,7 +2610,8 @@ struct BatchSolver {
         else hipLaunchKernelGGL(k_b_fix, dim3(elem_grid(NS)), dim3(kBlock), 0, s, n, S, fixed.p, b, x);
         for (int o = 0;; ++o) {
             resid(b, x, pbb, prr, s);
-            hipLaunchKernelGGL(k_b_outer_red, dim3(S), dim3(kBlock), 0, s, G, S, pbb, prr, tol, itol, ost.p, bst.p);
+            hipLaunchKernelGGL(k_b_outer_red, dim3(S), dim3(kBlock), 0, s, G, S, pbb, prr, tol, itol, ost.p, bst.p,
+                               o > 0 ? track + (o - 1) : (int*)nullptr);
             if (o == nouter) break;
             TM_CHECK(precond(rT.p, ring.p, prz, s));
             hipLaunchKernelGGL(k_b_red_rz, dim3(S), dim3(kBlock), 0, s, G, S, prz, -1, bst.p, bhist.p);
@@ -2670,13 +2675,42 @@ struct tm_batch {
     float i8ms = 0.0f, i8ms_first = 0.0f;
     DevBuf<double> rk_k[4], rk_base;   // RK4 stages and the step's start state
     // graph-replayed RK4 steps: samples whose fixed-budget solve missed the
-    // tolerance (device counter), and the budgets learnt from host-polled
-    // solves: refinement steps and inner iterations per step of the
-    // Neumann (0) and Dirichlet (1) solves
-    DevBuf<unsigned> rk_fail;
+    // tolerance and the iterations that each refinement step of the two
+    // solves took (device counters), and the budgets: refinement
+    // steps and inner iterations per step of the Neumann (0) and Dirichlet (1)
+    // solves
+    static constexpr int kMaxBud = 8;
+    DevBuf<unsigned> rk_fail;  // 1 + 2 kMaxBud
     bool bud_set = false;
     int bud_outer[2] = {0, 0};
-    int bud_inner[2][8] = {};
+    int bud_inner[2][kMaxBud] = {};
+    // The captured step is kept for the next call with the same arguments
+    // (capturing and instantiating its few hundred nodes takes as long as two
+    // replays); the key holds everything the graph has by value that can
+    // change after the batch's creation, the magnetisation's buffer and the
+    // context's per-node field among it.
+    struct StepKey {
+        double dtau = 0.0, alpha = 0.0;
+        int variant = -1;
+        const double* m = nullptr;
+        const double* hfield = nullptr;
+        int outer[2] = {0, 0};
+        int inner[2][kMaxBud] = {};
+        bool operator==(const StepKey& o) const {
+            bool e = dtau == o.dtau && alpha == o.alpha && variant == o.variant && m == o.m && hfield == o.hfield;
+            for (int w = 0; w < 2; ++w) {
+                e = e && outer[w] == o.outer[w];
+                for (int k = 0; k < outer[w] && e; ++k) e = inner[w][k] == o.inner[w][k];
+            }
+            return e;
+        }
+    };
+    StepKey step_key;
+    hipGraphExec_t step_exec = nullptr;
+    void drop_step() {
+        if (step_exec) (void)hipGraphExecDestroy(step_exec);
+        step_exec = nullptr;
+    }
     int gemm_sol = 0;                  // tuned rocBLAS solution index (0: library default)
     bool gemm_own = false;             // the MFMA kernel k_b_gemm64 won the tuning
     int gemm_shape = 0, gemm_ks = 1;   // its tile shape and K split
@@ -3176,17 +3210,20 @@ int eval_enqueue(tm_batch* bt, double alpha, int variant, double* dmdt) {
     const size_t NS = (size_t)n * S;
     hipStream_t s = bt->stream;
     const CtxView& v = bt->cv;
+    constexpr int kMaxBud = tm_batch::kMaxBud;
+    unsigned* fail = bt->rk_fail.p;
+    int* track = reinterpret_cast<int*>(fail + 1);
     launch_div(bt);
     TM_HIP(hipGetLastError());
     if (bt->prec == TM_PREC_FP64)
-        TM_CHECK(bt->sN64.enqueue(bt->rhsN.p, bt->u1.p, v.tol, bt->bud_outer[0], bt->bud_inner[0], s, bt->rk_fail.p));
+        TM_CHECK(bt->sN64.enqueue(bt->rhsN.p, bt->u1.p, v.tol, bt->bud_outer[0], bt->bud_inner[0], s, fail, track));
     else
-        TM_CHECK(bt->sN32.enqueue(bt->rhsN.p, bt->u1.p, v.tol, bt->bud_outer[0], bt->bud_inner[0], s, bt->rk_fail.p));
+        TM_CHECK(bt->sN32.enqueue(bt->rhsN.p, bt->u1.p, v.tol, bt->bud_outer[0], bt->bud_inner[0], s, fail, track));
     TM_CHECK(boundary_product(bt, v.bnodes, bt->u1.p, bt->rhsD.p));
     if (bt->prec == TM_PREC_FP64)
-        TM_CHECK(bt->sD64.enqueue(bt->rhsD.p, bt->u2.p, v.tol, bt->bud_outer[1], bt->bud_inner[1], s, bt->rk_fail.p));
+        TM_CHECK(bt->sD64.enqueue(bt->rhsD.p, bt->u2.p, v.tol, bt->bud_outer[1], bt->bud_inner[1], s, fail, track + kMaxBud));
     else
-        TM_CHECK(bt->sD32.enqueue(bt->rhsD.p, bt->u2.p, v.tol, bt->bud_outer[1], bt->bud_inner[1], s, bt->rk_fail.p));
+        TM_CHECK(bt->sD32.enqueue(bt->rhsD.p, bt->u2.p, v.tol, bt->bud_outer[1], bt->bud_inner[1], s, fail, track + kMaxBud));
     hipLaunchKernelGGL(k_b_sum2, dim3(elem_grid(NS)), dim3(kBlock), 0, s, NS, (const double*)bt->u1.p,
                        (const double*)bt->u2.p, bt->usum.p);
     return launch_fields(bt, alpha, variant, dmdt, nullptr, false);
@@ -3320,6 +3357,7 @@ int tm_batch_create(tm_ctx* c, int nsamples, int precision, tm_batch** out) {
 int tm_batch_destroy(tm_batch* bt) {
     if (!bt) return TM_OK;
     if (bt->stream) (void)hipStreamSynchronize(bt->stream);
+    bt->drop_step();
     if (bt->blas) rocblas_destroy_handle(bt->blas);
     for (auto& e : bt->ev)
         if (e) (void)hipEventDestroy(e);
@@ -3488,7 +3526,8 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
     const size_t NS = (size_t)bt->n * bt->S, N3 = 3 * NS;
     for (auto& k : bt->rk_k) TM_CHECK(k.alloc(N3));
     TM_CHECK(bt->rk_base.alloc(N3));
-    TM_CHECK(bt->rk_fail.alloc(1));
+    constexpr int kMaxBud = tm_batch::kMaxBud, kCount = 1 + 2 * kMaxBud;
+    TM_CHECK(bt->rk_fail.alloc(kCount));
     hipStream_t s = bt->stream;
     const dim3 g(elem_grid(N3));
     const double cst[4] = {0.0, 0.5 * dtau, 0.5 * dtau, dtau};
@@ -3501,24 +3540,45 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
     TM_HIP(hipEventCreate(&e0));
     TM_HIP(hipEventCreate(&e1));
     TM_HIP(hipEventRecord(e0, s));
-    auto learn = [bt, &R]() {  // budgets from the last host-polled solves
-        const int on = bt->prec == TM_PREC_FP64 ? bt->sN64.last_outer : bt->sN32.last_outer;
-        const int od = bt->prec == TM_PREC_FP64 ? bt->sD64.last_outer : bt->sD32.last_outer;
-        const int* inN = bt->prec == TM_PREC_FP64 ? bt->sN64.last_inner : bt->sN32.last_inner;
-        const int* inD = bt->prec == TM_PREC_FP64 ? bt->sD64.last_inner : bt->sD32.last_inner;
-        const int o[2] = {on, od};
-        const int* in[2] = {inN, inD};
+    // Budgets from the last host-polled solves, one iteration per refinement
+    // step more than they took.  Only a step's last stage sets them: the first
+    // solves of a run start cold and take several times the iterations of
+    // the later ones, and a queued iteration past convergence costs its dozen
+    // launches.  After a miss (grow) every stage counts, and no budget shrinks.
+    auto learn = [bt](bool grow) {
+        constexpr int kMaxBud = tm_batch::kMaxBud;
+        const bool f64 = bt->prec == TM_PREC_FP64;
+        const int o[2] = {f64 ? bt->sN64.last_outer : bt->sN32.last_outer,
+                          f64 ? bt->sD64.last_outer : bt->sD32.last_outer};
+        const int* in[2] = {f64 ? bt->sN64.last_inner : bt->sN32.last_inner,
+                            f64 ? bt->sD64.last_inner : bt->sD32.last_inner};
         for (int w = 0; w < 2; ++w) {
-            bt->bud_outer[w] = std::min(8, std::max(bt->bud_outer[w], o[w]));
-            for (int k = 0; k < o[w] && k < 8; ++k) bt->bud_inner[w][k] = std::max(bt->bud_inner[w][k], in[w][k] + 2);
-            int tot = 0;
-            for (int k = 0; k < bt->bud_outer[w]; ++k) tot += bt->bud_inner[w][k];
-            if (w == 0) R.budget_neumann = tot;
-            else R.budget_dirichlet = tot;
+            const int had = grow ? bt->bud_outer[w] : 0;
+            bt->bud_outer[w] = std::min(kMaxBud, std::max(std::max(1, o[w]), had));
+            for (int k = 0; k < bt->bud_outer[w]; ++k) {
+                const int now = k < o[w] ? in[w][k] + (grow ? 2 : 1) : 1;
+                bt->bud_inner[w][k] = k < had ? std::max(bt->bud_inner[w][k], now) : now;
+            }
         }
         bt->bud_set = true;
     };
-    auto polled_step = [&](bool final_step) -> int {
+    // What the replays needed since the last tightening: the budgets shrink to
+    // it, plus one, at the end of a call and after eight replays.
+    int seen[2 * kMaxBud] = {}, replays = 0;
+    auto tighten = [&]() {
+        constexpr int kMaxBud = tm_batch::kMaxBud;
+        for (int w = 0; w < 2 && replays > 0; ++w) {
+            int used = 0;
+            for (int k = 0; k < bt->bud_outer[w]; ++k) {
+                if (seen[w * kMaxBud + k] > 0) used = k + 1;
+                bt->bud_inner[w][k] = std::min(bt->bud_inner[w][k], seen[w * kMaxBud + k] + 1);
+            }
+            bt->bud_outer[w] = std::max(1, used);
+        }
+        replays = 0;
+        std::fill(seen, seen + 2 * kMaxBud, 0);
+    };
+    auto polled_step = [&](bool final_step, bool missed) -> int {
         int st = TM_OK;
         hipLaunchKernelGGL(k_b_copy, g, dim3(kBlock), 0, s, N3, (const double*)bt->m.p, bt->rk_base.p);
         for (int k = 0; k < 4; ++k) {
@@ -3534,7 +3594,7 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
             R.max_iters_neumann = std::max(R.max_iters_neumann, es.inner_neumann);
             R.max_iters_dirichlet = std::max(R.max_iters_dirichlet, es.inner_dirichlet);
             if (fin && last) *last = es;
-            learn();
+            if (missed || k == 3) learn(missed);
         }
         hipLaunchKernelGGL(k_b_rk_final, dim3(elem_grid(NS)), dim3(kBlock), 0, s, NS, (const double*)bt->rk_base.p,
                            (const double*)bt->rk_k[0].p, (const double*)bt->rk_k[1].p, (const double*)bt->rk_k[2].p,
@@ -3544,12 +3604,24 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
         return st;
     };
     int status = TM_OK;
-    hipGraphExec_t exec = nullptr;
     if (last) *last = tm_batch_stats{};
     for (int step = 0; step < nsteps; ++step) {
         const bool fin = step == nsteps - 1;
+        bool missed = false;
         if (graph_ok && bt->bud_set) {
-            if (!exec) {
+            if (replays >= 8) tighten();
+            tm_batch::StepKey key;
+            key.dtau = dtau;
+            key.alpha = alpha;
+            key.variant = variant;
+            key.m = bt->m.p;
+            key.hfield = ctx_hext_field(bt->ctx);
+            for (int w = 0; w < 2; ++w) {
+                key.outer[w] = bt->bud_outer[w];
+                for (int k = 0; k < kMaxBud; ++k) key.inner[w][k] = bt->bud_inner[w][k];
+            }
+            if (!bt->step_exec || !(key == bt->step_key)) {
+                bt->drop_step();
                 hipGraph_t gr = nullptr;
                 // the captured boundary products use the fastest verified own kernel
                 const bool k_own = bt->gemm_own;
@@ -3559,7 +3631,7 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
                 bt->gemm_ks = bt->own_ks;
                 TM_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
                 int r = TM_OK;
-                hipLaunchKernelGGL(k_b_reset_fail, dim3(1), dim3(64), 0, s, bt->rk_fail.p);
+                hipLaunchKernelGGL(k_b_reset_fail, dim3(1), dim3(64), 0, s, kCount, bt->rk_fail.p);
                 hipLaunchKernelGGL(k_b_copy, g, dim3(kBlock), 0, s, N3, (const double*)bt->m.p, bt->rk_base.p);
                 for (int k = 0; k < 4 && r == TM_OK; ++k) {
                     if (k > 0)
@@ -3580,23 +3652,34 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
                     status = r != TM_OK ? r : TM_ERR_HIP;
                     break;
                 }
-                const hipError_t ei = hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0);
+                const hipError_t ei = hipGraphInstantiate(&bt->step_exec, gr, nullptr, nullptr, 0);
                 (void)hipGraphDestroy(gr);
                 if (ei != hipSuccess) {
-                    exec = nullptr;
+                    bt->step_exec = nullptr;
                     status = TM_ERR_HIP;
                     break;
                 }
+                bt->step_key = key;
                 R.captures += 1;
             }
-            unsigned fail = 0;
-            if (hipGraphLaunch(exec, s) != hipSuccess ||
-                hipMemcpyAsync(&fail, bt->rk_fail.p, sizeof(unsigned), hipMemcpyDeviceToHost, s) != hipSuccess ||
+            unsigned counts[kCount] = {};
+            if (hipGraphLaunch(bt->step_exec, s) != hipSuccess ||
+                hipMemcpyAsync(counts, bt->rk_fail.p, sizeof(counts), hipMemcpyDeviceToHost, s) != hipSuccess ||
                 hipStreamSynchronize(s) != hipSuccess) {
                 status = TM_ERR_HIP;
                 break;
             }
-            if (fail == 0) {
+            for (int w = 0; w < 2; ++w) {
+                const int* took = reinterpret_cast<const int*>(counts) + 1 + w * kMaxBud;
+                int sum = 0;
+                for (int k = 0; k < kMaxBud; ++k) sum += took[k];
+                (w == 0 ? R.max_iters_neumann : R.max_iters_dirichlet) =
+                    std::max(w == 0 ? R.max_iters_neumann : R.max_iters_dirichlet, sum);
+                for (int k = 0; k < kMaxBud; ++k)
+                    seen[w * kMaxBud + k] = std::max(seen[w * kMaxBud + k], took[k]);
+            }
+            ++replays;
+            if (counts[0] == 0) {
                 R.graph_steps += 1;
                 if (fin && last) last->nsamples = bt->S;
                 continue;
@@ -3605,19 +3688,23 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
             // the step's start state and redo it with host-polled solves
             hipLaunchKernelGGL(k_b_copy, g, dim3(kBlock), 0, s, N3, (const double*)bt->rk_base.p, bt->m.p);
             R.redone_steps += 1;
-            for (int w = 0; w < 2; ++w)
-                for (int k = 0; k < bt->bud_outer[w]; ++k) bt->bud_inner[w][k] += 2;
-            (void)hipGraphExecDestroy(exec);
-            exec = nullptr;
+            missed = true;
+            replays = 0;
+            std::fill(seen, seen + 2 * kMaxBud, 0);
         }
-        const int r = polled_step(fin);
+        const int r = polled_step(fin, missed);
         if (r != TM_OK && r != TM_ERR_MAXITER) {
             status = r;
             break;
         }
         if (r == TM_ERR_MAXITER) status = r;
     }
-    if (exec) (void)hipGraphExecDestroy(exec);
+    tighten();
+    for (int w = 0; w < 2; ++w) {
+        int tot = 0;
+        for (int k = 0; k < bt->bud_outer[w]; ++k) tot += bt->bud_inner[w][k];
+        (w == 0 ? R.budget_neumann : R.budget_dirichlet) = tot;
+    }
     TM_HIP(hipEventRecord(e1, s));
     TM_HIP(hipEventSynchronize(e1));
     float ms = 0.0f;
