@@ -1,0 +1,42 @@
+"""Batched kernels that gather from tiles in LDS (divergence, fields, outer
+residual): sample counts at and off the edges of the 16-sample chunks, with
+and without each field term, against the single-sample path."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("S, dmi, ku, field", [(64, False, True, False), (64, True, False, True), (63, True, True, False),
+                                               (33, False, False, False), (18, True, True, True), (17, False, True, True)])
+def test_tiles_match_single_sample(gpu_available, S, dmi, ku, field):
+    """17,424 nodes: 545 tiles or more, more units than the kernels have
+    blocks.  Both sides solve to 1e-13, so the fields agree to a few thousand
+    times that (the systems' condition), 1e-9; the torque likewise."""
+    from tetmag_amd import _native as N
+    from tetmag_amd import problem as P
+    from tetmag_amd.batch import BatchContext, from_batch, to_batch
+    from tetmag_amd.context import FieldContext
+    mat = P.Material(Ku=4e4 if ku else 0.0, ku_axis=(0.6, 0.0, 0.8), D=1e-3 if dmi else 0.0, B_ext=(0.01, 0.02, -0.03))
+    prob = P.cuboid_problem("tiles", 32, 32, 15, 3.0, 0.1, 3, mat)
+    assert prob.n * ((S + 15) // 16) >= 1024 * 32
+    ctx = FieldContext(prob, tol=1e-13)
+    try:
+        if field:
+            ctx.set_hext(prob.hext, 1e4 * np.random.default_rng(1).standard_normal(3 * prob.n))
+        bc = BatchContext(ctx, S, N.TM_PREC_FP64)
+        ms = P.smooth_random_fields(prob.mesh, S, seed=S)
+        for rep in range(2):  # warm solves too
+            dm, H, st = bc.eval_rhs_host(to_batch(ms))
+            for s in (0, S // 2, S - 1):
+                d1, h1, st1 = ctx.eval_rhs_host(ms[s])
+                eh, ed = rel_l2(from_batch(H, s), h1), rel_l2(from_batch(dm, s), d1)
+                print("S", S, "rep", rep, "sample", s, "Heff", eh, "dm/dt", ed, flush=True)
+                assert eh < 1e-9 and ed < 1e-9
+                assert abs(st["max_torque"][s] - st1["max_torque"]) <= 1e-9 * st1["max_torque"]
+            ms = [m + 1e-3 * np.roll(m, 1) for m in ms]
+        bc.close()
+    finally:
+        ctx.close()

@@ -26,6 +26,8 @@
 #include <algorithm>
 #include <cstddef>
 #include <cmath>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "tm_internal.hpp"
@@ -939,6 +941,223 @@ __device__ inline double pair_sum(d2v s) {
     return (l & 1) ? vy : vx;
 }
 
+// ---- FP64 gathers from tiles in LDS -----------------------------------------
+// The kernels that gather FP64 rows (divergence, fields, outer residual) moved
+// every neighbour's samples from L2 once per entry of the operator, about 15
+// times per node, at the rate of the L2 (11 to 12 TB/s of gathered lines at
+// 282,897 nodes).  Here a block takes a unit: a tile of up to 32 rows (chosen to
+// share neighbours, see TileOp) and 16 samples.  It stages the distinct nodes
+// that the rows refer to, about four per row, in LDS and gathers from there.
+// Lane j of a 16-lane group holds sample 16 c + j of its group's row; the
+// row's slots (place in the tile, weights) are one coalesced load, lane j
+// holding slot j, and slot k is handed to the group by a DPP row broadcast.
+// Sixteen samples keep a gathered row one 128-byte line and leave room for
+// tiles of 32 rows at two blocks per CU.  A block walks several units and is
+// pipelined over them: while it computes one, the nodes of the next are on
+// their way into registers, and the next's slots and the node list of the one
+// after that are being read (one unit at a time, without this, every unit waits for
+// four dependent loads, and the kernels were no faster than the gathers
+// from L2).  64 samples at 282,897 nodes, against the gathers from L2: fields
+// 1,006 -> 606 us, divergence 513 -> 293, FP64 residual 216 -> 143; 24 samples
+// at 38,025 nodes 102 -> 41, 55 -> 24 and 25 -> 14.  A third of the lanes' time
+// goes into vector instructions, a third into LDS; two (fields, divergence) and
+// four (residual) blocks per CU were the fastest.
+constexpr int kTileThreads = 512;
+constexpr int kTileRows = kTileThreads / 16;
+constexpr int kTileS = 16;       // samples of a unit
+constexpr int kTileNodes = 128;  // nodes of a tile: 64 KB of LDS with four components
+
+struct TileRow {
+    int row, q0;  // its first slot
+    int more;     // chunks of kSlot slots << 16 | its own place in the tile
+};
+
+struct TileArgs {
+    int nt;               // tiles
+    int S, nch;           // samples, chunks of kTileS of them
+    const int* row0;      // nt + 1: entries of `rows` of a tile
+    const TileRow* rows;
+    const int* node0;     // nt + 1: its entries of `nodes`
+    const int* nodes;
+    const unsigned short* loc;  // per slot: the gathered node's place in the tile (padding: the row's own)
+};
+
+// blocks of a tile kernel with `percu` of them per CU: each XCD's blocks a
+// multiple of the chunks, so that a block keeps to one chunk
+inline int tile_blocks(int nch, int percu) { return kXcd * (32 * percu / nch * nch); }
+
+// A unit of work.  k counts the units of a block: XCD-contiguous tiles, the
+// chunks of a tile in neighbouring blocks (they share the slots), neighbouring
+// tiles next to them.  Past the end: valid = false, with the data of the last
+// tile (loads need no conditions).
+struct TileUnit {
+    bool valid;
+    int r0, nr, n0, nn;
+};
+__device__ inline int tile_chunk(const TileArgs& t) { return (int)(blockIdx.x / kXcd) % t.nch * kTileS; }
+__device__ inline TileUnit tile_unit(const TileArgs& t, int k) {
+    const int x = blockIdx.x % kXcd, bx = gridDim.x / kXcd / t.nch;
+    const int per = (t.nt + kXcd - 1) / kXcd, in = (int)(blockIdx.x / kXcd) / t.nch + k * bx;
+    const int tile = min(x * per + in, t.nt - 1);
+    const cint_p r = (cint_p)t.row0, c = (cint_p)t.node0;
+    const int r0 = r[tile], r1 = r[tile + 1], n0 = c[tile], n1 = c[tile + 1];
+    return TileUnit{in < per && x * per + in < t.nt, r0, r1 - r0, n0, n1 - n0};
+}
+
+// the value that lane K of the 16-lane group holds
+template <int K>
+__device__ inline int bcast16(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x150 + K, 0xf, 0xf, true);  // row_newbcast
+}
+template <int K>
+__device__ inline double bcast16(double v) {
+    return __builtin_amdgcn_update_dpp(0.0, v, 0x150 + K, 0xf, 0xf, true);
+}
+template <class F, int... K>
+__device__ inline void each16(F&& f, std::integer_sequence<int, K...>) {
+    (f(std::integral_constant<int, K>{}), ...);
+}
+
+// 16 slots of this group's row: lane j's place and NW weights of slot q + j
+template <int NW>
+struct TileSlots {
+    int loc;
+    double w[NW];
+    __device__ void load(const TileArgs& t, int q, const double* const (&src)[NW]) {
+        q += threadIdx.x & 15;
+        loc = t.loc[q];
+#pragma unroll
+        for (int i = 0; i < NW; ++i) w[i] = src[i][q];
+    }
+    // f(components gathered by slot k, its weights) for k = 0 .. 15
+    template <int NC, class F>
+    __device__ void each(const double* lds, F&& f) const {
+        const int at = loc * (NC * kTileS);
+        const double* mine = lds + (threadIdx.x & 15);
+        each16(
+            [&](auto kk) {
+                constexpr int K = decltype(kk)::value;
+                const double* g = mine + bcast16<K>(at);
+                double v[NC], ww[NW];
+#pragma unroll
+                for (int c = 0; c < NC; ++c) v[c] = g[c * kTileS];
+#pragma unroll
+                for (int i = 0; i < NW; ++i) ww[i] = bcast16<K>(w[i]);
+                f(v, ww);
+            },
+            std::make_integer_sequence<int, kSlot>{});
+    }
+};
+
+// A unit on its way through the pipeline: first its tile's bounds, node list
+// and this group's row, then the nodes (in the walk's registers) and the
+// row's first slots.
+template <int NC, int NW, bool EVEN>
+struct TileStep {
+    static constexpr int kLanes = EVEN ? 8 : 16;  // lanes per row of samples, 16 or 8 bytes each
+    static constexpr int kGroups = kTileThreads / kLanes;
+    static constexpr int kRounds = kTileNodes / kGroups;
+    TileUnit u;
+    int id[kRounds];
+    TileRow row;
+    TileSlots<NW> slots;
+    __device__ void lists(const TileArgs& t, int k) {
+        u = tile_unit(t, k);
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r)
+            id[r] = t.nodes[u.n0 + min((int)threadIdx.x / kLanes + r * kGroups, u.nn - 1)];
+        row = t.rows[u.r0 + min((int)threadIdx.x / 16, u.nr - 1)];
+    }
+};
+
+// The units of this block, pipelined.  NC components of a tile's nodes in
+// place [node][component][16] in LDS, component c < NC - 1 from m + c cs and the
+// last from `last`.  EVEN (S even): rows of samples are 16-byte aligned.  Lanes
+// past the last sample load the last one's data; groups without a row (nr <
+// kTileRows) compute the tile's last row once more; neither stores.  Per unit:
+// begin(row) loads the row's own data, add(v, w) per entry, end(row, lds, on)
+// when the row is summed (on: this group's row and this lane's sample exist).
+template <int NC, int NW, bool EVEN, class Begin, class Add, class End>
+__device__ inline void tile_walk(const TileArgs& t, const double* m, size_t cs, const double* last,
+                                 const double* const (&w)[NW], double* lds, Begin&& begin, Add&& add, End&& end) {
+    using Step = TileStep<NC, NW, EVEN>;
+    using V = std::conditional_t<EVEN, d2v, double>;
+    constexpr int kLanes = Step::kLanes, kGroups = Step::kGroups, kRounds = Step::kRounds, kPer = 16 / kLanes;
+    V v[kRounds][NC];
+    const int s0 = tile_chunk(t), S = t.S;
+    const bool lane_on = s0 + (int)(threadIdx.x & 15) < S;
+    const int ks = min(s0 + (int)(threadIdx.x % kLanes) * kPer, S - kPer);
+    auto load = [&](const Step& p) {
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r) {
+            const size_t e = (size_t)p.id[r] * S + ks;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) v[r][c] = *(const V*)((c == NC - 1 ? last : m + c * cs) + e);
+        }
+    };
+    auto store = [&]() {  // places past the tile's last node are not read
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r)
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                *(V*)(lds + ((threadIdx.x / kLanes + r * kGroups) * NC + c) * kTileS +
+                      (threadIdx.x % kLanes) * kPer) = v[r][c];
+    };
+    Step p[3];
+    p[0].lists(t, 0);
+    if (!p[0].u.valid) return;  // the whole block
+    load(p[0]);
+    p[0].slots.load(t, p[0].row.q0, w);
+    p[1].lists(t, 1);
+    store();
+    __syncthreads();
+    int k = 2;
+    // computes unit c while c1's data are loaded and c2's lists are read; false at the end
+    auto step = [&](Step& c, Step& c1, Step& c2) {
+        begin(c.row);
+        load(c1);
+        c1.slots.load(t, c1.row.q0, w);
+        c2.lists(t, k++);
+        c.slots.template each<NC>(lds, add);
+        for (int i = 1; i < c.row.more >> 16; ++i) {
+            c.slots.load(t, c.row.q0 + i * kSlot, w);
+            c.slots.template each<NC>(lds, add);
+        }
+        end(c.row, lds, lane_on && (int)threadIdx.x / 16 < c.u.nr);
+        if (!c1.u.valid) return false;
+        __syncthreads();
+        store();
+        __syncthreads();
+        return true;
+    };
+    while (step(p[0], p[1], p[2]) && step(p[1], p[2], p[0]) && step(p[2], p[0], p[1])) {
+    }
+}
+
+// b = sum_d tGrad_d (Js m_d) / mu0, as k_b_div
+constexpr int kDivPerCu = 2;
+template <bool EVEN>
+__global__ __launch_bounds__(kTileThreads, 2 * kDivPerCu) void k_b_div_t(TileArgs t, const double* __restrict__ wx,
+                                                                        const double* __restrict__ wy,
+                                                                        const double* __restrict__ wz, int n,
+                                                                        const double* __restrict__ m,
+                                                                        double* __restrict__ out) {
+    __shared__ double lds[kTileNodes * 3 * kTileS];
+    const size_t NS = (size_t)n * t.S;
+    const int s = tile_chunk(t) + (threadIdx.x & 15);
+    double sx = 0.0, sy = 0.0, sz = 0.0;
+    tile_walk<3, 3, EVEN>(
+        t, m, NS, m + 2 * NS, {wx, wy, wz}, lds, [&](const TileRow&) { sx = sy = sz = 0.0; },
+        [&](const double (&v)[3], const double (&w)[3]) {
+            sx += w[0] * v[0];
+            sy += w[1] * v[1];
+            sz += w[2] * v[2];
+        },
+        [&](const TileRow& r, const double*, bool on) {
+            if (on) out[(size_t)r.row * t.S + s] = sx + sy + sz;
+        });
+}
+
 struct BEvalArgs {
     SlotArgs P;                        // union pattern in slots, w = exchange weights (may be null)
     const double* gx; const double* gy; const double* gz;
@@ -1196,6 +1415,144 @@ __global__ __launch_bounds__(kBlock) void k_b_eval_w(BEvalArgs a) {
         for (int k = 1; k < kRowsPerBlock; ++k) t = fmax(t, st[k][lane]);
         atomic_max_nonneg(a.torque + lane, t);
     }
+}
+
+// k_b_eval from tiles in LDS (xw: the exchange weights, zeros without exchange)
+constexpr int kEvalPerCu = 2;
+template <bool DMI, bool EVEN>
+__global__ __launch_bounds__(kTileThreads, DMI && !EVEN ? 2 : 2 * kEvalPerCu) void k_b_eval_t(BEvalArgs a, const double* xw, TileArgs t) {
+    __shared__ double lds[kTileNodes * 4 * kTileS];
+    constexpr int NW = DMI ? 7 : 4;
+    const int S = t.S, n = a.n;
+    const size_t NS = (size_t)n * S;
+    const int j = threadIdx.x & 15, s = tile_chunk(t) + j, sc = min(s, S - 1);
+    const double* w[NW];
+    w[0] = xw;
+    w[1] = a.gx;
+    w[2] = a.gy;
+    w[3] = a.gz;
+    if constexpr (DMI) {
+        w[4] = a.cx;
+        w[5] = a.cy;
+        w[6] = a.cz;
+    }
+    __shared__ double hs[3][kTileS];
+    if (threadIdx.x < 3 * kTileS) hs[threadIdx.x / kTileS][j] = a.hext[(threadIdx.x / kTileS) * S + sc];
+    // no branch around a load of the pipeline: without anisotropy the
+    // constants are any values, left out by `end`
+    const double* kup = a.ku ? a.ku : a.invjs;
+    const double* kap = a.ku ? a.kaxis : a.m;
+    double ex, ey, ez, dx, dy, dz, cxs, cys, czs;
+    double ku, kx, ky, kz, ij, sx, sy, sz, fd;
+    double tmax = 0.0;
+    tile_walk<4, NW, EVEN>(
+        t, a.m, NS, a.u, w, lds,
+        [&](const TileRow& r) {
+            ex = ey = ez = dx = dy = dz = cxs = cys = czs = 0.0;
+            ku = kup[r.row];
+            kx = kap[r.row];
+            ky = kap[n + r.row];
+            kz = kap[2 * n + r.row];
+            ij = a.invjs[r.row];
+            if constexpr (DMI) {
+                sx = a.nvs[r.row];
+                sy = a.nvs[n + r.row];
+                sz = a.nvs[2 * n + r.row];
+                fd = a.dmi_fac[r.row];
+            }
+        },
+        [&](const double (&v)[4], const double (&ww)[NW]) {
+            ex += ww[0] * v[0];
+            ey += ww[0] * v[1];
+            ez += ww[0] * v[2];
+            dx += ww[1] * v[3];
+            dy += ww[2] * v[3];
+            dz += ww[3] * v[3];
+            if constexpr (DMI) {
+                cxs += ww[5] * v[2] - ww[6] * v[1];
+                cys += ww[6] * v[0] - ww[4] * v[2];
+                czs += ww[4] * v[1] - ww[5] * v[0];
+            }
+        },
+        [&](const TileRow& r, const double* tile, bool on) {
+            if (!on) return;
+            const int row = r.row;
+            const size_t e = (size_t)row * S + s;
+            const double* own = tile + (r.more & 0xffff) * (4 * kTileS) + j;
+            const double mx = own[0], my = own[kTileS], mz = own[2 * kTileS];
+            double hx = ex, hy = ey, hz = ez;
+            if (a.ku) {
+                const double f = 2.0 * ku * (kx * mx + ky * my + kz * mz);
+                hx += f * kx;
+                hy += f * ky;
+                hz += f * kz;
+            }
+            if constexpr (DMI) {
+                hx += ((my * sz - mz * sy) - 2.0 * cxs) * fd;
+                hy += ((mz * sx - mx * sz) - 2.0 * cys) * fd;
+                hz += ((mx * sy - my * sx) - 2.0 * czs) * fd;
+            }
+            hx = hx * ij + hs[0][j] - dx;
+            hy = hy * ij + hs[1][j] - dy;
+            hz = hz * ij + hs[2][j] - dz;
+            if (a.hfield) {
+                hx += a.hfield[row];
+                hy += a.hfield[n + row];
+                hz += a.hfield[2 * n + row];
+            }
+            if (a.heff) {
+                a.heff[e] = hx;
+                a.heff[NS + e] = hy;
+                a.heff[2 * NS + e] = hz;
+            }
+            const double tx = my * hz - mz * hy, ty = mz * hx - mx * hz, tz = mx * hy - my * hx;
+            const double bx = my * tz - mz * ty, by = mz * tx - mx * tz, bz = mx * ty - my * tx;
+            // -tx - alpha bx (TM_LLG_CLASSIC) or -alpha bx (TM_LLG_NOPREC)
+            const bool prec = a.variant != TM_LLG_NOPREC;
+            b_store_llg(a, e, NS, mx, my, mz, (prec ? -tx : 0.0) - a.alpha * bx, (prec ? -ty : 0.0) - a.alpha * by,
+                        (prec ? -tz : 0.0) - a.alpha * bz);
+            tmax = fmax(tmax, sqrt(tx * tx + ty * ty + tz * tz));
+        });
+    if (a.torque && s < S) atomic_max_nonneg(a.torque + s, tmax);
+}
+
+// k_b_resid from tiles in LDS: the block's partials as b_partial lays them out
+// (zero for the samples of the other chunks)
+constexpr int kResidPerCu = 4;
+template <typename T, bool EVEN>
+__global__ __launch_bounds__(kTileThreads, 2 * kResidPerCu) void k_b_resid_t(TileArgs t, const double* __restrict__ w,
+                                                                            const double* __restrict__ b,
+                                                                            const double* __restrict__ x,
+                                                                            T* __restrict__ rT, double* part_bb,
+                                                                            double* part_rr) {
+    __shared__ double lds[kTileNodes * kTileS];
+    const int j = threadIdx.x & 15, g = threadIdx.x / 16, s = tile_chunk(t) + j, sc = min(s, t.S - 1);
+    double bi = 0.0, acc = 0.0, vb = 0.0, vr = 0.0;
+    tile_walk<1, 1, EVEN>(
+        t, x, 0, x, {w}, lds,
+        [&](const TileRow& r) {
+            acc = 0.0;
+            bi = b[(size_t)r.row * t.S + sc];
+        },
+        [&](const double (&v)[1], const double (&ww)[1]) { acc += ww[0] * v[0]; },
+        [&](const TileRow& r, const double*, bool on) {
+            if (!on) return;
+            const double ri = bi - acc;
+            rT[(size_t)r.row * t.S + s] = (T)ri;
+            vb += bi * bi;
+            vr += ri * ri;
+        });
+    __syncthreads();
+    static_assert(kTileNodes >= 2 * kTileRows, "the tile's LDS holds the partial sums");
+    lds[(2 * g) * kTileS + j] = vb;
+    lds[(2 * g + 1) * kTileS + j] = vr;
+    __syncthreads();
+    const int q = threadIdx.x / kMaxS, sm = threadIdx.x % kMaxS;
+    if (q >= 2 || sm >= t.S) return;
+    double v = 0.0;
+    if (sm >= s - j && sm < s - j + kTileS)
+        for (int k = 0; k < kTileRows; ++k) v += lds[(2 * k + q) * kTileS + (sm - (s - j))];
+    (q == 0 ? part_bb : part_rr)[(size_t)sm * gridDim.x + blockIdx.x] = v;
 }
 
 // U[j][s] = u[bn[j]][s]  (S x b column-major, ld S)
@@ -1859,6 +2216,112 @@ struct SlotOp {
     }
 };
 
+// Tiles of a SlotOp's rows (see TileArgs): a tile starts at the first row that
+// no tile has and takes, as long as they fit, the row that adds the fewest nodes,
+// among the rows that are nodes of the tile already: 4.1 nodes per row on the
+// 282,897-node cuboid, where 32 consecutive rows of its Z-order
+// numbering need 5.  None (nt = 0) when a row alone refers to too many
+// nodes, or when there are fewer than 1,024 units, two for each block (the
+// smaller problems sit in L2, where a gather's latency is all it costs).
+struct TileOp {
+    int nt = 0;
+    DevBuf<int> row0, node0, nodes;
+    DevBuf<TileRow> rows;
+    DevBuf<unsigned short> loc;
+
+    int build(const SlotOp& op, hipStream_t s) {
+        nt = 0;
+        const int n = op.n, nch = (op.S + kTileS - 1) / kTileS;
+        if (n != op.ncols || (int64_t)n * nch < (int64_t)1024 * kTileRows) return TM_OK;
+        std::vector<int> hr{0}, hn{0}, hnode, order, place((size_t)n, -1), deg((size_t)n, 0), have((size_t)n, 0), cand;
+        std::vector<char> taken((size_t)n, 0);
+        for (int i = 0; i < n; ++i) {  // a row's nodes: its columns and itself
+            bool self = false;
+            for (int q = op.h_rp[i]; q < op.h_rp[i + 1]; ++q) self = self || op.h_ci[q] == i;
+            deg[i] = op.h_rp[i + 1] - op.h_rp[i] + (self ? 0 : 1);
+            if (deg[i] > kTileNodes) return TM_OK;
+        }
+        // rows by column: the rows that refer to a node
+        std::vector<int> tp((size_t)n + 1, 0), tr(op.h_ci.size());
+        for (int c : op.h_ci) ++tp[c + 1];
+        for (int i = 0; i < n; ++i) tp[i + 1] += tp[i];
+        {
+            std::vector<int> fill(tp.begin(), tp.end() - 1);
+            for (int i = 0; i < n; ++i)
+                for (int q = op.h_rp[i]; q < op.h_rp[i + 1]; ++q) tr[fill[op.h_ci[q]]++] = i;
+        }
+        std::vector<unsigned short> hl((size_t)op.h_sp[n], 0);
+        std::vector<TileRow> hrow((size_t)n);
+        int first = 0;
+        while ((int)order.size() < n) {
+            while (taken[first]) ++first;
+            const size_t base = hnode.size(), rbase = order.size();
+            cand.clear();
+            auto add_node = [&](int c) {  // counts for the rows that refer to it (have: nodes of theirs in the tile)
+                if (place[c] >= 0) return;
+                place[c] = (int)(hnode.size() - base);
+                hnode.push_back(c);
+                bool self = false;
+                for (int q = tp[c]; q < tp[c + 1]; ++q) {
+                    ++have[tr[q]];
+                    self = self || tr[q] == c;
+                }
+                if (!self) ++have[c];
+                if (!taken[c]) cand.push_back(c);
+            };
+            for (int row = first; row >= 0;) {
+                taken[row] = 1;
+                order.push_back(row);
+                add_node(row);
+                for (int q = op.h_rp[row]; q < op.h_rp[row + 1]; ++q) add_node(op.h_ci[q]);
+                row = -1;
+                if ((int)(order.size() - rbase) == kTileRows) break;
+                const int room = kTileNodes - (int)(hnode.size() - base);
+                int best = 0;
+                size_t kept = 0;
+                for (size_t k = 0; k < cand.size(); ++k) {
+                    const int c = cand[k];
+                    if (taken[c]) continue;
+                    cand[kept++] = c;
+                    const int more = deg[c] - have[c];
+                    if (more <= room && (row < 0 || more < best || (more == best && c < row))) {
+                        row = c;
+                        best = more;
+                    }
+                }
+                cand.resize(kept);
+            }
+            for (size_t k = rbase; k < order.size(); ++k) {
+                const int i = order[k];
+                hrow[k] = TileRow{i, op.h_sp[i], (op.h_sp[i + 1] - op.h_sp[i]) / kSlot << 16 | place[i]};
+                size_t e = (size_t)op.h_sp[i];
+                for (int q = op.h_rp[i]; q < op.h_rp[i + 1]; ++q)
+                    if (op.kept(i, q)) hl[e++] = (unsigned short)place[op.h_ci[q]];
+                for (; e < (size_t)op.h_sp[i + 1]; ++e) hl[e] = (unsigned short)place[i];
+            }
+            for (size_t k = base; k < hnode.size(); ++k) {  // clean up for the next tile
+                const int c = hnode[k];
+                place[c] = -1;
+                have[c] = 0;
+                for (int q = tp[c]; q < tp[c + 1]; ++q) have[tr[q]] = 0;
+            }
+            hr.push_back((int)order.size());
+            hn.push_back((int)hnode.size());
+        }
+        TM_CHECK(row0.upload(hr.data(), hr.size(), s));
+        TM_CHECK(node0.upload(hn.data(), hn.size(), s));
+        TM_CHECK(nodes.upload(hnode.data(), hnode.size(), s));
+        TM_CHECK(rows.upload(hrow.data(), hrow.size(), s));
+        TM_CHECK(loc.upload(hl.data(), hl.size(), s));
+        TM_HIP(hipStreamSynchronize(s));
+        nt = (int)hr.size() - 1;
+        return TM_OK;
+    }
+    TileArgs args(const SlotOp& op) const {
+        return TileArgs{nt, op.S, (op.S + kTileS - 1) / kTileS, row0.p, rows.p, node0.p, nodes.p, loc.p};
+    }
+};
+
 // C = R (I - A w D^-1): the level-0 pre-smoother from zero followed by the
 // restriction, as one operator (rows of R, columns of A).  R: nr x n CSR;
 // A: n x n CSR (rp, ci, v); dinv: A's inverse diagonal.
@@ -2101,6 +2564,8 @@ struct BatchSolver {
     DevBuf<T> wIDA0;              // on sl0: I - w D^-1 A (level-0 post-smoother, wide form)
     bool post1 = false;           // wIDA0 is set (every level-0 row fits one chunk with its diagonal)
     DevBuf<double> wA64;          // A in FP64 (outer residual)
+    TileOp t0;                    // tiles of sl0 for the outer residual
+    int Gr = 0;                   // partials per sample of the outer residual
     struct LvOps {
         SlotOp A, R, P;           // level l >= 1: A; every level: restriction, prolongation
         DevBuf<T> wA, wR, wP;
@@ -2151,6 +2616,8 @@ struct BatchSolver {
         TM_CHECK(sl0.build(n, n, solver.pat.h_rowptr.data(), solver.pat.h_csrcol.data(), S, s));
         TM_CHECK(sl0.values(solver.h_val, wA0, s));
         TM_CHECK(sl0.values(solver.h_val, wA64, s));
+        TM_CHECK(t0.build(sl0, s));
+        Gr = t0.nt > 0 ? tile_blocks((S + kTileS - 1) / kTileS, kResidPerCu) : G;
         if (wide() && L > 0) {
             const int* cc = solver.pat.h_csrcol.data();
             TM_CHECK(sl0w.build(n, n, solver.pat.h_rowptr.data(), cc, S, s, true));
@@ -2221,7 +2688,7 @@ struct BatchSolver {
             TM_CHECK(lv[l].b.alloc((size_t)L.R.n * S));
         }
         TM_CHECK(xc.alloc((size_t)std::max(1, solver.amg.nc) * S));
-        TM_CHECK(part.alloc((size_t)std::max(4, kWinDots) * S * G + (size_t)kWinDots * kWinChunks * S));
+        TM_CHECK(part.alloc((size_t)std::max(4, kWinDots) * S * std::max(G, Gr) + (size_t)kWinDots * kWinChunks * S));
         TM_CHECK(winX.alloc((size_t)kSolveWindow * NS));
         TM_CHECK(winB.alloc((size_t)kSolveWindow * NS));
         TM_CHECK(win.alloc(1));
@@ -2382,8 +2849,18 @@ struct BatchSolver {
 
     // r = b - A x in FP64 (b, x: [n][S]), rT = (T) r, partials (b, b), (r, r)
     void resid(const double* b, const double* x, double* pbb, double* prr, hipStream_t s) {
-        hipLaunchKernelGGL((k_b_resid<T>), dim3(G), dim3(kBlock), 0, s, sl0.args(8, wA64.p), S, b, x, rT.p, pbb,
-                           prr);
+        if (t0.nt > 0) {
+            const TileArgs t = t0.args(sl0);
+            if (S % 2 == 0)
+                hipLaunchKernelGGL((k_b_resid_t<T, true>), dim3(Gr), dim3(kTileThreads), 0, s, t,
+                                   (const double*)wA64.p, b, x, rT.p, pbb, prr);
+            else
+                hipLaunchKernelGGL((k_b_resid_t<T, false>), dim3(Gr), dim3(kTileThreads), 0, s, t,
+                                   (const double*)wA64.p, b, x, rT.p, pbb, prr);
+        } else {
+            hipLaunchKernelGGL((k_b_resid<T>), dim3(G), dim3(kBlock), 0, s, sl0.args(8, wA64.p), S, b, x, rT.p, pbb,
+                               prr);
+        }
     }
 
     // iteration k: q = A p_k = A z_k + beta q, partial (z_k, q)
@@ -2404,9 +2881,9 @@ struct BatchSolver {
         if (cg->precond != TM_PRECOND_AMG || cg->amg.levels.empty()) return TM_ERR_UNSUPPORTED;
         const size_t NS = (size_t)n * S;
         double* pbb = part.p;
-        double* prr = part.p + (size_t)S * G;
-        double* prz = part.p + (size_t)2 * S * G;
-        double* pzq = part.p + (size_t)3 * S * G;
+        double* prr = part.p + (size_t)S * std::max(G, Gr);
+        double* prz = part.p + (size_t)2 * S * std::max(G, Gr);
+        double* pzq = part.p + (size_t)3 * S * std::max(G, Gr);
         const double itol = sizeof(T) == 4 ? 1e-5 : 0.0;  // FP32 inner target per refinement step
         int outer = 0, inner_total = 0;
         if (use_window) win_project(b, x, s);  // (sets the fixed rows too)
@@ -2425,7 +2902,7 @@ struct BatchSolver {
         int pend_step = 0;
         for (;;) {
             resid(b, x, pbb, prr, s);
-            hipLaunchKernelGGL(k_b_outer_red, dim3(S), dim3(kBlock), 0, s, G, S, pbb, prr, tol, itol, ost.p, bst.p,
+            hipLaunchKernelGGL(k_b_outer_red, dim3(S), dim3(kBlock), 0, s, Gr, S, pbb, prr, tol, itol, ost.p, bst.p,
                                (int*)nullptr);
             if (!(outer == 0 && spec_ok && last_inner[0] > 0)) {
                 TM_HIP(hipMemcpyAsync(h_ost, ost.p, sizeof(OState), hipMemcpyDeviceToHost, s));
@@ -2534,8 +3011,8 @@ struct BatchSolver {
         if (cg->amg.levels.empty()) return TM_ERR_UNSUPPORTED;
         const int e = (int)sizeof(T);
         const double nS = (double)n * S;
-        double* pzq = part.p + (size_t)3 * S * G;
-        double* prz = part.p + (size_t)2 * S * G;
+        double* pzq = part.p + (size_t)3 * S * std::max(G, Gr);
+        double* prz = part.p + (size_t)2 * S * std::max(G, Gr);
         auto add = [&out](const char* nm, double ms, double bytes) {
             tm_batch_kernel_time k = {};
             std::snprintf(k.name, sizeof(k.name), "%s", nm);
@@ -2549,7 +3026,7 @@ struct BatchSolver {
         add(wide() ? "k_b_cg_spmv_w" : "k_b_cg_spmv", timeit([&] { cg_spmv(ring.p, 0, pzq, s); }),
             slots(A0) * (4 + e) + (wide() ? (double)n * e : 0.0) + 3.0 * nS * e);
         add(sizeof(T) == 4 ? "k_b_cg_update<float>" : "k_b_cg_update<double>",
-            timeit([&] { cg_update(part.p + (size_t)S * G, s); }), 3.0 * nS * e);
+            timeit([&] { cg_update(part.p + (size_t)S * std::max(G, Gr), s); }), 3.0 * nS * e);
         const LvOps& O = lo[0];
         const int n1 = cg->amg.levels[0].R.n;
         add(O.RA.long_rows() ? "k_b_spmm_w<long> (R(I-AwD^-1), level 0)" : "k_b_spmm (R(I-AwD^-1), level 0)",
@@ -2576,7 +3053,7 @@ struct BatchSolver {
             }
         }
         double* pbb = part.p;
-        double* prr = part.p + (size_t)S * G;
+        double* prr = part.p + (size_t)S * std::max(G, Gr);
         add(sizeof(T) == 4 ? "k_b_resid<float>" : "k_b_resid<double>", timeit([&] {
                 resid(lv0_b64(), lv0_x64(), pbb, prr, s);
             }),
@@ -2602,15 +3079,15 @@ struct BatchSolver {
         if (nouter < 0 || nouter > kMaxOuter || !fail || !track) return TM_ERR_BAD_ARG;
         const size_t NS = (size_t)n * S;
         double* pbb = part.p;
-        double* prr = part.p + (size_t)S * G;
-        double* prz = part.p + (size_t)2 * S * G;
-        double* pzq = part.p + (size_t)3 * S * G;
+        double* prr = part.p + (size_t)S * std::max(G, Gr);
+        double* prz = part.p + (size_t)2 * S * std::max(G, Gr);
+        double* pzq = part.p + (size_t)3 * S * std::max(G, Gr);
         const double itol = sizeof(T) == 4 ? 1e-5 : 0.0;
         if (use_window) win_project(b, x, s);  // (sets the fixed rows too)
         else hipLaunchKernelGGL(k_b_fix, dim3(elem_grid(NS)), dim3(kBlock), 0, s, n, S, fixed.p, b, x);
         for (int o = 0;; ++o) {
             resid(b, x, pbb, prr, s);
-            hipLaunchKernelGGL(k_b_outer_red, dim3(S), dim3(kBlock), 0, s, G, S, pbb, prr, tol, itol, ost.p, bst.p,
+            hipLaunchKernelGGL(k_b_outer_red, dim3(S), dim3(kBlock), 0, s, Gr, S, pbb, prr, tol, itol, ost.p, bst.p,
                                o > 0 ? track + (o - 1) : (int*)nullptr);
             if (o == nouter) break;
             TM_CHECK(precond(rT.p, ring.p, prz, s));
@@ -2659,6 +3136,7 @@ struct tm_batch {
     rocblas_handle blas = nullptr;
     CtxView cv{};
     SlotOp eo;                         // union pattern of the per-node operators, in row slots
+    TileOp et;                         // its tiles
     DevBuf<double> xw, gx, gy, gz, tx, ty, tz, cx, cy, cz;  // slot weights: exchange, grad, tGrad, curl
     bool exch = false, dmi = false;
     DevBuf<double> m, dmdt, heff, u1, u2, usum, rhsN, rhsD, U, Gm, hext, torque;
@@ -3147,6 +3625,18 @@ int boundary_product(tm_batch* bt, const int* bn, const double* u, double* out) 
 // b = div(Js m) of every sample into the Neumann right-hand side
 void launch_div(tm_batch* bt) {
     const int n = bt->n, S = bt->S;
+    if (bt->et.nt > 0) {
+        const TileArgs t = bt->et.args(bt->eo);
+        if (S % 2 == 0)
+            hipLaunchKernelGGL(k_b_div_t<true>, dim3(tile_blocks(t.nch, kDivPerCu)), dim3(kTileThreads), 0, bt->stream, t,
+                               (const double*)bt->tx.p, (const double*)bt->ty.p, (const double*)bt->tz.p, n,
+                               (const double*)bt->m.p, bt->rhsN.p);
+        else
+            hipLaunchKernelGGL(k_b_div_t<false>, dim3(tile_blocks(t.nch, kDivPerCu)), dim3(kTileThreads), 0, bt->stream, t,
+                               (const double*)bt->tx.p, (const double*)bt->ty.p, (const double*)bt->tz.p, n,
+                               (const double*)bt->m.p, bt->rhsN.p);
+        return;
+    }
     hipLaunchKernelGGL(k_b_div, dim3(row_grid(n)), dim3(kBlock), 0, bt->stream, bt->eo.args(8, bt->tx.p),
                        (const double*)bt->ty.p, (const double*)bt->tz.p, S, (const double*)bt->m.p, bt->rhsN.p);
 }
@@ -3189,7 +3679,17 @@ int launch_fields(tm_batch* bt, double alpha, int variant, double* dmdt, double*
     a.dt = dt;
     if (torque) hipLaunchKernelGGL(k_b_zero_small, dim3(1), dim3(kMaxS), 0, s, S, bt->torque.p);
     const dim3 g(row_grid(n));
-    if (S == kMaxS) {
+    if (bt->et.nt > 0) {
+        const TileArgs t = bt->et.args(bt->eo);
+        const dim3 tg(tile_blocks(t.nch, kEvalPerCu)), tb(kTileThreads);
+        if (S % 2 == 0) {
+            if (bt->dmi) hipLaunchKernelGGL((k_b_eval_t<true, true>), tg, tb, 0, s, a, (const double*)bt->xw.p, t);
+            else hipLaunchKernelGGL((k_b_eval_t<false, true>), tg, tb, 0, s, a, (const double*)bt->xw.p, t);
+        } else {
+            if (bt->dmi) hipLaunchKernelGGL((k_b_eval_t<true, false>), tg, tb, 0, s, a, (const double*)bt->xw.p, t);
+            else hipLaunchKernelGGL((k_b_eval_t<false, false>), tg, tb, 0, s, a, (const double*)bt->xw.p, t);
+        }
+    } else if (S == kMaxS) {
         if (bt->dmi) hipLaunchKernelGGL(k_b_eval_w<true>, g, dim3(kBlock), 0, s, a);
         else hipLaunchKernelGGL(k_b_eval_w<false>, g, dim3(kBlock), 0, s, a);
     } else if (bt->dmi) {
@@ -3272,9 +3772,16 @@ int tm_batch_create(tm_ctx* c, int nsamples, int precision, tm_batch** out) {
     if ((int64_t)3 * P.n * nsamples * 8 > (int64_t)INT32_MAX) return fail(TM_ERR_UNSUPPORTED);
     if ((st = bt->eo.build(P.n, P.n, P.h_rowptr.data(), P.h_csrcol.data(), nsamples, bt->stream)) != TM_OK)
         return fail(st);
+    if ((st = bt->et.build(bt->eo, bt->stream)) != TM_OK) return fail(st);
     bt->exch = v.hop_set[TM_OP_EXCHANGE];
     int ops_ok = TM_OK;
-    if (bt->exch) ops_ok |= upload_op(bt, TM_OP_EXCHANGE, bt->xw);
+    if (bt->exch) {
+        ops_ok |= upload_op(bt, TM_OP_EXCHANGE, bt->xw);
+    } else if (bt->et.nt > 0) {
+        const std::vector<double> zeros((size_t)bt->eo.h_sp[P.n], 0.0);
+        ops_ok |= bt->xw.upload(zeros.data(), zeros.size(), bt->stream);
+        if (hipStreamSynchronize(bt->stream) != hipSuccess) return fail(TM_ERR_HIP);
+    }
     ops_ok |= upload_op(bt, TM_OP_GRAD_X, bt->gx);
     ops_ok |= upload_op(bt, TM_OP_GRAD_Y, bt->gy);
     ops_ok |= upload_op(bt, TM_OP_GRAD_Z, bt->gz);
