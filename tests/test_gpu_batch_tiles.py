@@ -40,3 +40,35 @@ def test_tiles_match_single_sample(gpu_available, S, dmi, ku, field):
         bc.close()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("ny", [16, 15])
+def test_inner_solve_tiles_match_fp64(gpu_available, ny):
+    """64 FP32-preconditioned samples at and just under the size from which the
+    inner solve's level-0 products come from tiles: 8,192 rows and 7,680.
+    Both precisions solve to 1e-12; the demag potentials then agree to the
+    systems' condition times that, 1e-8 (the bound of the solver's other tests)."""
+    from tetmag_amd import _native as N
+    from tetmag_amd import problem as P
+    from tetmag_amd.batch import BatchContext, to_batch
+    from tetmag_amd.context import FieldContext
+    prob = P.cuboid_problem("inner tiles", 31, ny - 1, 15, 3.0, 0.1, 3, P.Material())
+    assert (4 * prob.n >= 1024 * 32) == (ny == 16)
+    ctx = FieldContext(prob, tol=1e-12)
+    try:
+        ms = to_batch(P.smooth_random_fields(prob.mesh, 64, seed=4))
+        ms2 = ms + 1e-3 * np.roll(ms, 1, axis=1)
+        u = {}
+        for prec in (N.TM_PREC_FP64, N.TM_PREC_MIXED):
+            bc = BatchContext(ctx, 64, prec)
+            u[prec] = []
+            for m in (ms, ms2):  # a cold and a warm solve
+                bc.eval_rhs_host(m)
+                u[prec] += list(bc.potentials())
+            bc.close()
+        for k, (a, b) in enumerate(zip(u[N.TM_PREC_MIXED], u[N.TM_PREC_FP64])):
+            worst = max(rel_l2(a[:, s], b[:, s]) for s in range(64))
+            print("ny", ny, "potential", k, worst, flush=True)
+            assert worst < 1e-8
+    finally:
+        ctx.close()

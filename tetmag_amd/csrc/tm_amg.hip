@@ -557,23 +557,19 @@ int AmgPrecond::setup(int n, const int* rowptr, const int* colidx, const double*
             L.A_ext = A0;
             L.Aval_ext = A0val;
             L.dinv_ext = A0dinv;
-        } else {
-            TM_CHECK(upload_csrv(cur, L.A, s));
-            std::vector<double> di((size_t)cur.n);
-            for (int i = 0; i < cur.n; ++i) di[i] = d[i] != 0.0 ? 1.0 / d[i] : 0.0;
-            TM_CHECK(L.dinv.upload(di.data(), di.size(), s));
         }
-        TM_CHECK(upload_csrv(P, L.P, s));
-        L.P.lpr = 4;  // rows of a few entries
-        TM_CHECK(upload_csrv(R, L.R, s));
         L.nnz_a = cur.rp[cur.n];
         L.nnz_p = P.rp[P.n];
         const Csr Q = smoothed(P, AP, d, L.omega);
         last_down = transpose(Q);  // R (I - A w D^-1): A and D are symmetric
         TM_CHECK(upload_csrv(last_down, L.down, s));
         if (lev > 0 || up0_lpr > 0) TM_CHECK(upload_csrv(up_operator(cur, d, L.omega, Q), L.up, s));
-        else TM_CHECK(L.x.alloc(cur.n));
         if (lev == 0 && up0_lpr > 0) L.up.lpr = up0_lpr;
+        if (lev == 0 && up0_lpr == 0) {
+            TM_CHECK(upload_csrv(P, L.P, s));
+            L.P.lpr = 4;  // rows of a few entries
+            TM_CHECK(L.x.alloc(cur.n));
+        }
         if (lev > 0) TM_CHECK(L.bx.alloc((size_t)cur.n + na));
         levels.push_back(std::move(L));
         cur = std::move(Ac);

@@ -267,9 +267,9 @@ __device__ inline f4 shfl_xor4(f4 v, int m) {
 // epilogue's operands for samples 4j .. 4j+3; epi(row, j, acc, ld) runs on
 // every lane of a group whose row exists (BLK = false), on lanes 0-15 of
 // wavefront 0 (BLK = true).
-template <bool BLK, int CH = kSlot, typename LDF, typename EPIF>
+template <bool BLK, typename LDF, typename EPIF>
 __device__ inline void wide_walk(const SlotArgs& M, const void* x, LDF&& ld, EPIF&& epi) {
-    static_assert(CH == 16 || CH == 8, "chunks of 16 or 8 slots");
+    constexpr int CH = kSlot;
     const int n = M.n;
     const int lane = threadIdx.x & (kWave - 1), g = lane >> 4, j = lane & 15;
     const int wv = threadIdx.x / kWave;
@@ -323,7 +323,6 @@ __device__ inline void wide_walk(const SlotArgs& M, const void* x, LDF&& ld, EPI
             if (has) epi(row, j, acc, lv);
         }
     } else {
-        static_assert(!BLK || CH == 16, "long rows in chunks of 16");
         auto chunk = [&](int q, f4 acc) {  // lane group g: slots q+4g .. q+4g+3
             const i4 o = of[(q >> 2) + g];
             const f4 ww = w[(q >> 2) + g];
@@ -602,9 +601,8 @@ __global__ __launch_bounds__(kBlock) void k_b_cg_spmv(SlotArgs A, int S, const T
 }
 
 // k_b_cg_spmv for 64 FP32 samples, wide gathers
-__global__ __launch_bounds__(kBlock) void k_b_cg_spmv_w(SlotArgs A, const float* __restrict__ dg,
-                                                        const float* __restrict__ z, float* __restrict__ q, int k,
-                                                        const BState* bs, double* part) {
+__global__ __launch_bounds__(kBlock) void k_b_cg_spmv_w(SlotArgs A, const float* __restrict__ z, float* __restrict__ q,
+                                                        int k, const BState* bs, double* part) {
     if (!any_active(A.gate, A.gate_n)) return;
     const int j = threadIdx.x & 15;
     const f4 beta = k > 0 ? f4{(float)bs->beta[4 * j], (float)bs->beta[4 * j + 1], (float)bs->beta[4 * j + 2],
@@ -619,7 +617,6 @@ __global__ __launch_bounds__(kBlock) void k_b_cg_spmv_w(SlotArgs A, const float*
         return ZQ{*(const f4*)(z + e), k > 0 ? *(const f4*)(q + e) : f4{0.f, 0.f, 0.f, 0.f}};
     };
     auto epi = [&](int row, int jj, f4 acc, const ZQ& o) {
-        acc += dg[row] * o.z;  // diagonal kept out of the slots
         const f4 qi = acc + beta * o.q;
         *(f4*)(q + (size_t)row * 64 + 4 * jj) = qi;
         v[0] += (double)o.z.x * (double)qi.x;
@@ -709,123 +706,55 @@ __global__ __launch_bounds__(kBlock) void k_b_spmm(SlotArgs M, int S, const T* _
     slot_walk<T, T, kRowsPerStep<T>>(M, x, lc, ld, epi);
 }
 
-// x = w dinv b + P xc: the pre-smoothed iterate plus the coarse correction
-// (the pre-smoother from zero is folded into the restriction operator)
+// Level 0 upwards: z = U [r | x_c] (r's tail holds the coarse correction), and
+// the partial (r, z).  One product with U = [2 w D^-1 - w D^-1 A w D^-1 | Q] in
+// place of the prolongation (x = w D^-1 r + P x_c, written and gathered again) and
+// the post-smoothing; the levels below use the same form, so a level costs two
+// launches instead of three.  Bound by the gathers from L2 and, on small meshes,
+// by the launch: 24 FP64 samples at 38,025 nodes 1.54 -> 1.49 ms per evaluation.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_b_prolong(SlotArgs P, int S, const double* __restrict__ dinv,
-                                                      const T* __restrict__ b, double w, const T* __restrict__ xc,
-                                                      T* __restrict__ x) {
-    if (!any_active(P.gate, P.gate_n)) return;
-    const int lane = threadIdx.x & (kWave - 1);
-    const bool on = lane < S;
-    const int lc = min(lane, S - 1);
-    auto ld = [&](int row) { return b[(size_t)row * S + lc]; };
-    auto epi = [&](int row, T acc, T bi) {
-        if (on) x[(size_t)row * S + lane] = (T)(w * dinv[row]) * bi + acc;
-    };
-    slot_walk<T, T, kRowsPerStep<T>>(P, xc, lc, ld, epi);
-}
-
-// xo = x + w dinv (b - A x); optional partial (b, xo)
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_b_post(SlotArgs A, int S, const double* __restrict__ dinv,
-                                                   const T* __restrict__ b, double w, const T* __restrict__ x,
-                                                   T* __restrict__ xo, double* part) {
-    if (!any_active(A.gate, A.gate_n)) return;
+__global__ __launch_bounds__(kBlock) void k_b_up(SlotArgs U, int S, const T* __restrict__ r, T* __restrict__ z,
+                                                 double* part) {
+    if (!any_active(U.gate, U.gate_n)) return;
     const int lane = threadIdx.x & (kWave - 1);
     const bool on = lane < S;
     const int lc = min(lane, S - 1);
     double v = 0.0;
-    struct BX {
-        T b, x;
-    };
-    auto ld = [&](int row) {
-        const size_t er = (size_t)row * S + lc;
-        return BX{b[er], x[er]};
-    };
-    auto epi = [&](int row, T acc, const BX& bx) {
+    auto ld = [&](int row) { return r[(size_t)row * S + lc]; };
+    auto epi = [&](int row, T acc, T ri) {
         if (on) {
-            const T zi = bx.x + (T)(w * dinv[row]) * (bx.b - acc);
-            xo[(size_t)row * S + lane] = zi;
-            v += (double)bx.b * (double)zi;
+            z[(size_t)row * S + lane] = acc;
+            v += (double)ri * (double)acc;
         }
     };
-    slot_walk<T, T, kRowsPerStep<T>>(A, x, lc, ld, epi);
-    if (part) b_partial(part, S, v);
+    slot_walk<T, T, kRowsPerStep<T>>(U, r, lc, ld, epi);
+    b_partial(part, S, v);
 }
 
-// Wide-gather forms (FP32, S = 64) of the transfer products and the
-// post-smoothers (the pre-smoother from zero is folded into the restriction
-// operator R (I - A w D^-1)).
-// x = w dinv b + P xc: the pre-smoothed iterate (not stored by the restriction pass)
-// plus the coarse correction, in one pass (P in chunks of CH slots)
-template <bool BLK, int CH>
-__global__ __launch_bounds__(kBlock) void k_b_prolong_w(SlotArgs P, const double* __restrict__ dinv,
-                                                        const float* __restrict__ b, double w,
-                                                        const float* __restrict__ xc, float* __restrict__ x) {
-    if (!any_active(P.gate, P.gate_n)) return;
-    auto ld = [&](int row, int j) { return *(const f4*)(b + (size_t)row * 64 + 4 * j); };
-    auto epi = [&](int row, int j, f4 acc, f4 bi) {
-        *(f4*)(x + (size_t)row * 64 + 4 * j) = (float)(w * dinv[row]) * bi + acc;
+// k_b_up for 64 FP32 samples, wide gathers
+__global__ __launch_bounds__(kBlock) void k_b_up_w(SlotArgs U, const float* __restrict__ r, float* __restrict__ z,
+                                                   double* part) {
+    if (!any_active(U.gate, U.gate_n)) return;
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    auto ld = [&](int row, int j) { return *(const f4*)(r + (size_t)row * 64 + 4 * j); };
+    auto epi = [&](int row, int j, f4 acc, f4 ri) {
+        *(f4*)(z + (size_t)row * 64 + 4 * j) = acc;
+        v[0] += (double)ri.x * (double)acc.x;
+        v[1] += (double)ri.y * (double)acc.y;
+        v[2] += (double)ri.z * (double)acc.z;
+        v[3] += (double)ri.w * (double)acc.w;
     };
-    wide_walk<BLK, CH>(P, xc, ld, epi);
+    wide_walk<false>(U, r, ld, epi);
+    b_partial4(part, v);
 }
 
-// y = M x (the restriction operators)
+// y = M x for 64 FP32 samples
 template <bool BLK>
 __global__ __launch_bounds__(kBlock) void k_b_spmm_w(SlotArgs M, const float* __restrict__ x, float* __restrict__ y) {
     if (!any_active(M.gate, M.gate_n)) return;
     auto ld = [&](int, int) { return 0; };
     auto epi = [&](int row, int j, f4 acc, int) { *(f4*)(y + (size_t)row * 64 + 4 * j) = acc; };
     wide_walk<BLK>(M, x, ld, epi);
-}
-
-template <bool BLK>
-__global__ __launch_bounds__(kBlock) void k_b_post_w(SlotArgs A, const float* __restrict__ dg,
-                                                     const double* __restrict__ dinv, const float* __restrict__ b,
-                                                     double w, const float* __restrict__ x, float* __restrict__ xo,
-                                                     double* part) {
-    if (!any_active(A.gate, A.gate_n)) return;
-    double v[4] = {0.0, 0.0, 0.0, 0.0};
-    struct BX {
-        f4 b, x;
-    };
-    auto ld = [&](int row, int j) {
-        const size_t e = (size_t)row * 64 + 4 * j;
-        return BX{*(const f4*)(b + e), *(const f4*)(x + e)};
-    };
-    auto epi = [&](int row, int j, f4 acc, const BX& bx) {
-        if (dg) acc += dg[row] * bx.x;  // diagonal kept out of the slots
-        const f4 zi = bx.x + (float)(w * dinv[row]) * (bx.b - acc);
-        *(f4*)(xo + (size_t)row * 64 + 4 * j) = zi;
-        v[0] += (double)bx.b.x * (double)zi.x;
-        v[1] += (double)bx.b.y * (double)zi.y;
-        v[2] += (double)bx.b.z * (double)zi.z;
-        v[3] += (double)bx.b.w * (double)zi.w;
-    };
-    wide_walk<BLK>(A, x, ld, epi);
-    if (part) b_partial4(part, v);
-}
-
-// The level-0 post-smoother with the diagonal in the slots: z = M x + w dinv b
-// with M = I - w D^-1 A (only b is read per row); partial (b, z)
-__global__ __launch_bounds__(kBlock) void k_b_post1_w(SlotArgs M, const double* __restrict__ dinv,
-                                                      const float* __restrict__ b, double w,
-                                                      const float* __restrict__ x, float* __restrict__ z,
-                                                      double* part) {
-    if (!any_active(M.gate, M.gate_n)) return;
-    double v[4] = {0.0, 0.0, 0.0, 0.0};
-    auto ld = [&](int row, int j) { return *(const f4*)(b + (size_t)row * 64 + 4 * j); };
-    auto epi = [&](int row, int j, f4 acc, f4 bi) {
-        const f4 zi = acc + (float)(w * dinv[row]) * bi;
-        *(f4*)(z + (size_t)row * 64 + 4 * j) = zi;
-        v[0] += (double)bi.x * (double)zi.x;
-        v[1] += (double)bi.y * (double)zi.y;
-        v[2] += (double)bi.z * (double)zi.z;
-        v[3] += (double)bi.w * (double)zi.w;
-    };
-    wide_walk<false>(M, x, ld, epi);
-    b_partial4(part, v);
 }
 
 // x = C b for the dense coarse inverse (row-major nc x nc): one row per block,
@@ -994,7 +923,9 @@ struct TileUnit {
     bool valid;
     int r0, nr, n0, nn;
 };
-__device__ inline int tile_chunk(const TileArgs& t) { return (int)(blockIdx.x / kXcd) % t.nch * kTileS; }
+__device__ inline int tile_chunk(const TileArgs& t, int samples = kTileS) {
+    return (int)(blockIdx.x / kXcd) % t.nch * samples;
+}
 __device__ inline TileUnit tile_unit(const TileArgs& t, int k) {
     const int x = blockIdx.x % kXcd, bx = gridDim.x / kXcd / t.nch;
     const int per = (t.nt + kXcd - 1) / kXcd, in = (int)(blockIdx.x / kXcd) / t.nch + k * bx;
@@ -1013,17 +944,41 @@ template <int K>
 __device__ inline double bcast16(double v) {
     return __builtin_amdgcn_update_dpp(0.0, v, 0x150 + K, 0xf, 0xf, true);
 }
+template <int K>
+__device__ inline float bcast16(float v) {
+    return __builtin_bit_cast(float, bcast16<K>(__builtin_bit_cast(int, v)));
+}
 template <class F, int... K>
 __device__ inline void each16(F&& f, std::integer_sequence<int, K...>) {
     (f(std::integral_constant<int, K>{}), ...);
 }
 
-// 16 slots of this group's row: lane j's place and NW weights of slot q + j
-template <int NW>
-struct TileSlots {
+// The element and lane layout of a walk: T, VEC samples per lane (a unit has
+// 16 VEC samples: 128 bytes of a node in FP64, 256 in FP32), and whether rows of
+// samples are 16-byte aligned.
+template <typename T_, int VEC_, bool ALIGNED_>
+struct TileType {
+    using T = T_;
+    static constexpr int VEC = VEC_;
+    static constexpr int kSamples = 16 * VEC;
+    typedef T Vec __attribute__((ext_vector_type(VEC)));
+    using Lane = std::conditional_t<VEC == 1, T, Vec>;  // a lane's samples
+    static constexpr int kPer = ALIGNED_ ? 16 / (int)sizeof(T) : 1;  // elements per staging load
+    typedef T StageVec __attribute__((ext_vector_type(16 / sizeof(T))));
+    using Stage = std::conditional_t<ALIGNED_, StageVec, T>;
+    static constexpr int kLanes = kSamples / kPer;  // lanes per staged row of samples
+    static constexpr int kGroups = kTileThreads / kLanes;
+    static constexpr int kRounds = kTileNodes / kGroups;
+};
+
+// The first NP chunks of 16 slots of this group's row: lane j's place and NW
+// weights of the chunk's slot j
+template <class TT, int NW>
+struct TileChunk {
+    using T = typename TT::T;
     int loc;
-    double w[NW];
-    __device__ void load(const TileArgs& t, int q, const double* const (&src)[NW]) {
+    T w[NW];
+    __device__ void load(const TileArgs& t, int q, const T* const (&src)[NW]) {
         q += threadIdx.x & 15;
         loc = t.loc[q];
 #pragma unroll
@@ -1031,16 +986,17 @@ struct TileSlots {
     }
     // f(components gathered by slot k, its weights) for k = 0 .. 15
     template <int NC, class F>
-    __device__ void each(const double* lds, F&& f) const {
-        const int at = loc * (NC * kTileS);
-        const double* mine = lds + (threadIdx.x & 15);
+    __device__ void each(const T* lds, F&& f) const {
+        const int at = loc * (NC * TT::kSamples);
+        const T* mine = lds + (threadIdx.x & 15) * TT::VEC;
         each16(
             [&](auto kk) {
                 constexpr int K = decltype(kk)::value;
-                const double* g = mine + bcast16<K>(at);
-                double v[NC], ww[NW];
+                const T* g = mine + bcast16<K>(at);
+                typename TT::Lane v[NC];
+                T ww[NW];
 #pragma unroll
-                for (int c = 0; c < NC; ++c) v[c] = g[c * kTileS];
+                for (int c = 0; c < NC; ++c) v[c] = *(const typename TT::Lane*)(g + c * TT::kSamples);
 #pragma unroll
                 for (int i = 0; i < NW; ++i) ww[i] = bcast16<K>(w[i]);
                 f(v, ww);
@@ -1051,41 +1007,43 @@ struct TileSlots {
 
 // A unit on its way through the pipeline: first its tile's bounds, node list
 // and this group's row, then the nodes (in the walk's registers) and the
-// row's first slots.
-template <int NC, int NW, bool EVEN>
+// row's first slots (NP chunks).
+template <class TT, int NW, int NP>
 struct TileStep {
-    static constexpr int kLanes = EVEN ? 8 : 16;  // lanes per row of samples, 16 or 8 bytes each
-    static constexpr int kGroups = kTileThreads / kLanes;
-    static constexpr int kRounds = kTileNodes / kGroups;
     TileUnit u;
-    int id[kRounds];
+    int id[TT::kRounds];
     TileRow row;
-    TileSlots<NW> slots;
+    TileChunk<TT, NW> chunk[NP];
+    __device__ void slots(const TileArgs& t, const typename TT::T* const (&w)[NW]) {
+#pragma unroll
+        for (int i = 0; i < NP; ++i) chunk[i].load(t, row.q0 + (i < row.more >> 16 ? i * kSlot : 0), w);
+    }
     __device__ void lists(const TileArgs& t, int k) {
         u = tile_unit(t, k);
 #pragma unroll
-        for (int r = 0; r < kRounds; ++r)
-            id[r] = t.nodes[u.n0 + min((int)threadIdx.x / kLanes + r * kGroups, u.nn - 1)];
+        for (int r = 0; r < TT::kRounds; ++r)
+            id[r] = t.nodes[u.n0 + min((int)threadIdx.x / TT::kLanes + r * TT::kGroups, u.nn - 1)];
         row = t.rows[u.r0 + min((int)threadIdx.x / 16, u.nr - 1)];
     }
 };
 
 // The units of this block, pipelined.  NC components of a tile's nodes in
-// place [node][component][16] in LDS, component c < NC - 1 from m + c cs and the
-// last from `last`.  EVEN (S even): rows of samples are 16-byte aligned.  Lanes
-// past the last sample load the last one's data; groups without a row (nr <
-// kTileRows) compute the tile's last row once more; neither stores.  Per unit:
-// begin(row) loads the row's own data, add(v, w) per entry, end(row, lds, on)
-// when the row is summed (on: this group's row and this lane's sample exist).
-template <int NC, int NW, bool EVEN, class Begin, class Add, class End>
-__device__ inline void tile_walk(const TileArgs& t, const double* m, size_t cs, const double* last,
-                                 const double* const (&w)[NW], double* lds, Begin&& begin, Add&& add, End&& end) {
-    using Step = TileStep<NC, NW, EVEN>;
-    using V = std::conditional_t<EVEN, d2v, double>;
-    constexpr int kLanes = Step::kLanes, kGroups = Step::kGroups, kRounds = Step::kRounds, kPer = 16 / kLanes;
+// place [node][component][16 VEC] in LDS, component c < NC - 1 from m + c cs and
+// the last from `last`.  Lanes past the last sample load the last one's data;
+// groups without a row (nr < kTileRows) compute the tile's last row once more;
+// neither stores.  Per unit: begin(row) loads the row's own data, add(v, w) per
+// entry, end(row, lds, on) when the row is summed (on: this group's row and
+// this lane's samples exist).
+template <class TT, int NC, int NW, int NP = 1, class Begin, class Add, class End>
+__device__ inline void tile_walk(const TileArgs& t, const typename TT::T* m, size_t cs, const typename TT::T* last,
+                                 const typename TT::T* const (&w)[NW], typename TT::T* lds, Begin&& begin, Add&& add,
+                                 End&& end) {
+    using Step = TileStep<TT, NW, NP>;
+    using V = typename TT::Stage;
+    constexpr int kLanes = TT::kLanes, kGroups = TT::kGroups, kRounds = TT::kRounds, kPer = TT::kPer;
     V v[kRounds][NC];
-    const int s0 = tile_chunk(t), S = t.S;
-    const bool lane_on = s0 + (int)(threadIdx.x & 15) < S;
+    const int s0 = tile_chunk(t, TT::kSamples), S = t.S;
+    const bool lane_on = s0 + (int)(threadIdx.x & 15) * TT::VEC < S;
     const int ks = min(s0 + (int)(threadIdx.x % kLanes) * kPer, S - kPer);
     auto load = [&](const Step& p) {
 #pragma unroll
@@ -1100,14 +1058,14 @@ __device__ inline void tile_walk(const TileArgs& t, const double* m, size_t cs, 
         for (int r = 0; r < kRounds; ++r)
 #pragma unroll
             for (int c = 0; c < NC; ++c)
-                *(V*)(lds + ((threadIdx.x / kLanes + r * kGroups) * NC + c) * kTileS +
+                *(V*)(lds + ((threadIdx.x / kLanes + r * kGroups) * NC + c) * TT::kSamples +
                       (threadIdx.x % kLanes) * kPer) = v[r][c];
     };
     Step p[3];
     p[0].lists(t, 0);
     if (!p[0].u.valid) return;  // the whole block
     load(p[0]);
-    p[0].slots.load(t, p[0].row.q0, w);
+    p[0].slots(t, w);
     p[1].lists(t, 1);
     store();
     __syncthreads();
@@ -1116,12 +1074,15 @@ __device__ inline void tile_walk(const TileArgs& t, const double* m, size_t cs, 
     auto step = [&](Step& c, Step& c1, Step& c2) {
         begin(c.row);
         load(c1);
-        c1.slots.load(t, c1.row.q0, w);
+        c1.slots(t, w);
         c2.lists(t, k++);
-        c.slots.template each<NC>(lds, add);
-        for (int i = 1; i < c.row.more >> 16; ++i) {
-            c.slots.load(t, c.row.q0 + i * kSlot, w);
-            c.slots.template each<NC>(lds, add);
+        c.chunk[0].template each<NC>(lds, add);
+#pragma unroll
+        for (int i = 1; i < NP; ++i)
+            if (i < c.row.more >> 16) c.chunk[i].template each<NC>(lds, add);
+        for (int i = NP; i < c.row.more >> 16; ++i) {
+            c.chunk[0].load(t, c.row.q0 + i * kSlot, w);
+            c.chunk[0].template each<NC>(lds, add);
         }
         end(c.row, lds, lane_on && (int)threadIdx.x / 16 < c.u.nr);
         if (!c1.u.valid) return false;
@@ -1132,6 +1093,29 @@ __device__ inline void tile_walk(const TileArgs& t, const double* m, size_t cs, 
     };
     while (step(p[0], p[1], p[2]) && step(p[1], p[2], p[0]) && step(p[2], p[0], p[1])) {
     }
+}
+
+// 64 FP32 samples: the block's sums v (four samples per lane) to
+// part[s * gridDim.x + block], through the walk's LDS
+using TileF64 = TileType<float, 4, true>;
+constexpr int kTileFloats = kTileNodes * 64;
+__device__ inline void tile_partial4(float* lds, double* part, const double (&v)[4]) {
+    double* red = reinterpret_cast<double*>(lds);  // [kTileRows / 2][64]
+    static_assert(kTileFloats * 4 >= kTileRows / 2 * 64 * 8, "the partial sums of two groups at a time");
+    const int g = threadIdx.x / 16, j = threadIdx.x & 15;
+    __syncthreads();
+    double u[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) u[c] = v[c] + __shfl_xor(v[c], 16);
+    if ((g & 1) == 0)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) red[(g / 2) * 64 + 4 * j + c] = u[c];
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < kTileRows / 2; ++k) s += red[k * 64 + threadIdx.x];
+    part[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = s;
 }
 
 // b = sum_d tGrad_d (Js m_d) / mu0, as k_b_div
@@ -1146,7 +1130,7 @@ __global__ __launch_bounds__(kTileThreads, 2 * kDivPerCu) void k_b_div_t(TileArg
     const size_t NS = (size_t)n * t.S;
     const int s = tile_chunk(t) + (threadIdx.x & 15);
     double sx = 0.0, sy = 0.0, sz = 0.0;
-    tile_walk<3, 3, EVEN>(
+    tile_walk<TileType<double, 1, EVEN>, 3, 3>(
         t, m, NS, m + 2 * NS, {wx, wy, wz}, lds, [&](const TileRow&) { sx = sy = sz = 0.0; },
         [&](const double (&v)[3], const double (&w)[3]) {
             sx += w[0] * v[0];
@@ -1445,7 +1429,7 @@ __global__ __launch_bounds__(kTileThreads, DMI && !EVEN ? 2 : 2 * kEvalPerCu) vo
     double ex, ey, ez, dx, dy, dz, cxs, cys, czs;
     double ku, kx, ky, kz, ij, sx, sy, sz, fd;
     double tmax = 0.0;
-    tile_walk<4, NW, EVEN>(
+    tile_walk<TileType<double, 1, EVEN>, 4, NW>(
         t, a.m, NS, a.u, w, lds,
         [&](const TileRow& r) {
             ex = ey = ez = dx = dy = dz = cxs = cys = czs = 0.0;
@@ -1518,7 +1502,7 @@ __global__ __launch_bounds__(kTileThreads, DMI && !EVEN ? 2 : 2 * kEvalPerCu) vo
 
 // k_b_resid from tiles in LDS: the block's partials as b_partial lays them out
 // (zero for the samples of the other chunks)
-constexpr int kResidPerCu = 4;
+constexpr int kResidPerCu = 3;
 template <typename T, bool EVEN>
 __global__ __launch_bounds__(kTileThreads, 2 * kResidPerCu) void k_b_resid_t(TileArgs t, const double* __restrict__ w,
                                                                             const double* __restrict__ b,
@@ -1528,7 +1512,7 @@ __global__ __launch_bounds__(kTileThreads, 2 * kResidPerCu) void k_b_resid_t(Til
     __shared__ double lds[kTileNodes * kTileS];
     const int j = threadIdx.x & 15, g = threadIdx.x / 16, s = tile_chunk(t) + j, sc = min(s, t.S - 1);
     double bi = 0.0, acc = 0.0, vb = 0.0, vr = 0.0;
-    tile_walk<1, 1, EVEN>(
+    tile_walk<TileType<double, 1, EVEN>, 1, 1>(
         t, x, 0, x, {w}, lds,
         [&](const TileRow& r) {
             acc = 0.0;
@@ -1553,6 +1537,69 @@ __global__ __launch_bounds__(kTileThreads, 2 * kResidPerCu) void k_b_resid_t(Til
     if (sm >= s - j && sm < s - j + kTileS)
         for (int k = 0; k < kTileRows; ++k) v += lds[(2 * k + q) * kTileS + (sm - (s - j))];
     (q == 0 ? part_bb : part_rr)[(size_t)sm * gridDim.x + blockIdx.x] = v;
+}
+
+// k_b_cg_spmv_w from tiles in LDS: 64 samples per unit, a float4 per lane.
+// Gathers from L2 are bound by the texture unit's four lanes per cycle, these by
+// LDS and the nodes' staging: at 282,897 nodes 93 -> 54 us, at 26,325 nodes
+// 11.1 -> 9.3 (also with fewer units than two per block).  Two blocks per
+// CU; at four the pipeline's registers spill (123 us).
+constexpr int kSolvePerCu = 2;
+__global__ __launch_bounds__(kTileThreads, 2 * kSolvePerCu) void k_b_cg_spmv_t(TileArgs t, const float* __restrict__ w,
+                                                                              const float* __restrict__ z,
+                                                                              float* __restrict__ q, int k,
+                                                                              const BState* bs, double* part) {
+    __shared__ float lds[kTileFloats];
+    if (!any_active(bs->active, kMaxS)) return;
+    const int j = threadIdx.x & 15;
+    const f4 beta = k > 0 ? f4{(float)bs->beta[4 * j], (float)bs->beta[4 * j + 1], (float)bs->beta[4 * j + 2],
+                               (float)bs->beta[4 * j + 3]}
+                          : f4{0.f, 0.f, 0.f, 0.f};
+    // k = 0: q has no earlier value; z is read in its place, times zero
+    const float* qo = k > 0 ? q : z;
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    f4 acc, old;
+    tile_walk<TileF64, 1, 1>(
+        t, z, 0, z, {w}, lds,
+        [&](const TileRow& r) {
+            acc = f4{0.f, 0.f, 0.f, 0.f};
+            old = *(const f4*)(qo + (size_t)r.row * 64 + 4 * j);
+        },
+        [&](const f4 (&x)[1], const float (&ww)[1]) { acc += ww[0] * x[0]; },
+        [&](const TileRow& r, const float* tile, bool on) {
+            if (!on) return;
+            const f4 zi = *(const f4*)(tile + (r.more & 0xffff) * 64 + 4 * j);
+            const f4 qi = k > 0 ? acc + beta * old : acc;
+            *(f4*)(q + (size_t)r.row * 64 + 4 * j) = qi;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] += (double)zi[c] * (double)qi[c];
+        });
+    tile_partial4(lds, part, v);
+}
+
+// k_b_up_w from tiles in LDS (rows of about 27 entries: two chunks of slots):
+// 101 us at 282,897 nodes and 64 samples, where prolongation and post-smoothing
+// took 49 + 88 from L2; 12.3 -> 9.9 against k_b_up_w at 26,325 nodes
+__global__ __launch_bounds__(kTileThreads, 2 * kSolvePerCu) void k_b_up_t(TileArgs t, const float* __restrict__ w,
+                                                                         const float* __restrict__ r,
+                                                                         float* __restrict__ z, const int* gate,
+                                                                         double* part) {
+    __shared__ float lds[kTileFloats];
+    if (!any_active(gate, kMaxS)) return;
+    const int j = threadIdx.x & 15;
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    f4 acc;
+    tile_walk<TileF64, 1, 1, 2>(
+        t, r, 0, r, {w}, lds, [&](const TileRow&) { acc = f4{0.f, 0.f, 0.f, 0.f}; },
+        [&](const f4 (&g)[1], const float (&ww)[1]) { acc += ww[0] * g[0]; },
+        [&](const TileRow& row, const float* tile, bool on) {
+            if (!on) return;
+            const f4 ri = *(const f4*)(tile + (row.more & 0xffff) * 64 + 4 * j);
+            *(f4*)(z + (size_t)row.row * 64 + 4 * j) = acc;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] += (double)ri[c] * (double)acc[c];
+        });
+    tile_partial4(lds, part, v);
 }
 
 // U[j][s] = u[bn[j]][s]  (S x b column-major, ld S)
@@ -2122,39 +2169,29 @@ int fetch_csr(const AmgPrecond::CsrDev& M, HostCsr& h, hipStream_t s) {
 // offsets for gathered elements of 4 and of 8 bytes.
 struct SlotOp {
     int n = 0, ncols = 0, S = 0;
-    int chunk = kSlot;            // rows padded to a multiple of this (16; 8 for the wide kernels' short rows)
-    bool nodiag = false;          // diagonal entries left out (applied by the kernel's epilogue)
     std::vector<int> h_rp, h_ci, h_sp;
     DevBuf<int> sp, off4, off8;
 
-    bool kept(int i, int q) const { return !(nodiag && h_ci[q] == i); }
-
-    int build(int rows, int cols, const int* rp, const int* ci, int S_, hipStream_t s, bool drop_diag = false,
-              int chunk_ = kSlot) {
+    int build(int rows, int cols, const int* rp, const int* ci, int S_, hipStream_t s) {
         n = rows;
         ncols = cols;
         S = S_;
-        nodiag = drop_diag;
-        chunk = chunk_;
         if ((int64_t)cols * S * 8 > (int64_t)INT32_MAX) return TM_ERR_UNSUPPORTED;  // 32-bit byte offsets
         h_rp.assign(rp, rp + rows + 1);
         h_ci.assign(ci, ci + rp[rows]);
         h_sp.assign((size_t)rows + 1, 0);
         for (int i = 0; i < rows; ++i) {
-            int len = 0;
-            for (int q = rp[i]; q < rp[i + 1]; ++q) len += kept(i, q);
-            h_sp[i + 1] = h_sp[i] + std::max(1, (len + chunk - 1) / chunk) * chunk;
+            const int len = rp[i + 1] - rp[i];
+            h_sp[i + 1] = h_sp[i] + std::max(1, (len + kSlot - 1) / kSlot) * kSlot;
         }
         const size_t ns = (size_t)h_sp[rows];
         std::vector<int> o4(ns, 0), o8(ns, 0);
         for (int i = 0; i < rows; ++i) {
             size_t k = (size_t)h_sp[i];
-            for (int q = rp[i]; q < rp[i + 1]; ++q)
-                if (kept(i, q)) {
-                    o4[k] = ci[q] * S * 4;
-                    o8[k] = ci[q] * S * 8;
-                    ++k;
-                }
+            for (int q = rp[i]; q < rp[i + 1]; ++q, ++k) {
+                o4[k] = ci[q] * S * 4;
+                o8[k] = ci[q] * S * 8;
+            }
         }
         TM_CHECK(sp.upload(h_sp.data(), h_sp.size(), s));
         TM_CHECK(off4.upload(o4.data(), ns, s));
@@ -2165,52 +2202,21 @@ struct SlotOp {
 
     // per-slot weights from CSR values v (optionally scaled by colscale[col] * w0)
     template <typename W>
-    int values(const std::vector<double>& v, DevBuf<W>& out, hipStream_t s, const int* ci = nullptr,
-               const double* colscale = nullptr, double w0 = 1.0) const {
+    int values(const std::vector<double>& v, DevBuf<W>& out, hipStream_t s, const double* colscale = nullptr,
+               double w0 = 1.0) const {
         std::vector<W> h((size_t)h_sp[n], (W)0);
         for (int i = 0; i < n; ++i) {
             size_t k = (size_t)h_sp[i];
             for (int q = h_rp[i]; q < h_rp[i + 1]; ++q)
-                if (kept(i, q)) h[k++] = (W)(colscale ? v[q] * w0 * colscale[ci[q]] : v[q]);
+                h[k++] = (W)(colscale ? v[q] * w0 * colscale[h_ci[q]] : v[q]);
         }
         TM_CHECK(out.upload(h.data(), h.size(), s));
         TM_HIP(hipStreamSynchronize(s));
         return TM_OK;
     }
 
-    // the diagonal (summed if repeated) of CSR values v, optionally scaled as in values()
-    template <typename W>
-    int diagonal(const std::vector<double>& v, DevBuf<W>& out, hipStream_t s, const double* colscale = nullptr,
-                 double w0 = 1.0) const {
-        std::vector<W> h((size_t)n, (W)0);
-        for (int i = 0; i < n; ++i) {
-            double d = 0.0;
-            for (int q = h_rp[i]; q < h_rp[i + 1]; ++q)
-                if (h_ci[q] == i) d += colscale ? v[q] * w0 * colscale[i] : v[q];
-            h[i] = (W)d;
-        }
-        TM_CHECK(out.upload(h.data(), h.size(), s));
-        TM_HIP(hipStreamSynchronize(s));
-        return TM_OK;
-    }
-
-    // Chunk size for the wide kernels: 8 where it cuts the padded slots by a
-    // quarter or more (the prolongators' rows, a few coarse columns each).
-    // A padding slot costs a gather instruction's lanes like a real entry
-    // (its load is dropped by the range check, not skipped).
-    static int wide_chunk(int rows, const int* rp) {
-        int64_t s16 = 0, s8 = 0;
-        for (int i = 0; i < rows; ++i) {
-            const int len = rp[i + 1] - rp[i];
-            s16 += std::max(1, (len + 15) / 16) * 16;
-            s8 += std::max(1, (len + 7) / 8) * 8;
-        }
-        return 4 * s8 <= 3 * s16 ? 8 : kSlot;
-    }
     // long rows: more than 6 chunks of 16 on average (one block per row pays off there)
     bool long_rows() const { return n > 0 && (int64_t)h_sp[n] > (int64_t)kSlot * n * 6; }
-    // every row one chunk (rows have at least one)
-    bool one_chunk() const { return n > 0 && (int64_t)h_sp[n] == (int64_t)chunk * n; }
     SlotArgs args(int ebytes, const void* w) const {
         return SlotArgs{n, ncols * S * ebytes, sp.p, ebytes == 4 ? off4.p : off8.p, w};
     }
@@ -2231,9 +2237,9 @@ struct TileOp {
 
     int build(const SlotOp& op, hipStream_t s) {
         nt = 0;
-        const int n = op.n, nch = (op.S + kTileS - 1) / kTileS;
-        if (n != op.ncols || (int64_t)n * nch < (int64_t)1024 * kTileRows) return TM_OK;
-        std::vector<int> hr{0}, hn{0}, hnode, order, place((size_t)n, -1), deg((size_t)n, 0), have((size_t)n, 0), cand;
+        const int n = op.n, nc = op.ncols, nch = (op.S + kTileS - 1) / kTileS;
+        if (n > nc || (int64_t)n * nch < (int64_t)1024 * kTileRows) return TM_OK;
+        std::vector<int> hr{0}, hn{0}, hnode, order, place((size_t)nc, -1), deg((size_t)n, 0), have((size_t)n, 0), cand;
         std::vector<char> taken((size_t)n, 0);
         for (int i = 0; i < n; ++i) {  // a row's nodes: its columns and itself
             bool self = false;
@@ -2242,9 +2248,9 @@ struct TileOp {
             if (deg[i] > kTileNodes) return TM_OK;
         }
         // rows by column: the rows that refer to a node
-        std::vector<int> tp((size_t)n + 1, 0), tr(op.h_ci.size());
+        std::vector<int> tp((size_t)nc + 1, 0), tr(op.h_ci.size());
         for (int c : op.h_ci) ++tp[c + 1];
-        for (int i = 0; i < n; ++i) tp[i + 1] += tp[i];
+        for (int i = 0; i < nc; ++i) tp[i + 1] += tp[i];
         {
             std::vector<int> fill(tp.begin(), tp.end() - 1);
             for (int i = 0; i < n; ++i)
@@ -2261,13 +2267,13 @@ struct TileOp {
                 if (place[c] >= 0) return;
                 place[c] = (int)(hnode.size() - base);
                 hnode.push_back(c);
-                bool self = false;
+                bool self = c >= n;
                 for (int q = tp[c]; q < tp[c + 1]; ++q) {
                     ++have[tr[q]];
                     self = self || tr[q] == c;
                 }
                 if (!self) ++have[c];
-                if (!taken[c]) cand.push_back(c);
+                if (c < n && !taken[c]) cand.push_back(c);
             };
             for (int row = first; row >= 0;) {
                 taken[row] = 1;
@@ -2296,13 +2302,13 @@ struct TileOp {
                 hrow[k] = TileRow{i, op.h_sp[i], (op.h_sp[i + 1] - op.h_sp[i]) / kSlot << 16 | place[i]};
                 size_t e = (size_t)op.h_sp[i];
                 for (int q = op.h_rp[i]; q < op.h_rp[i + 1]; ++q)
-                    if (op.kept(i, q)) hl[e++] = (unsigned short)place[op.h_ci[q]];
+                    hl[e++] = (unsigned short)place[op.h_ci[q]];
                 for (; e < (size_t)op.h_sp[i + 1]; ++e) hl[e] = (unsigned short)place[i];
             }
             for (size_t k = base; k < hnode.size(); ++k) {  // clean up for the next tile
                 const int c = hnode[k];
                 place[c] = -1;
-                have[c] = 0;
+                if (c < n) have[c] = 0;
                 for (int q = tp[c]; q < tp[c + 1]; ++q) have[tr[q]] = 0;
             }
             hr.push_back((int)order.size());
@@ -2317,45 +2323,41 @@ struct TileOp {
         nt = (int)hr.size() - 1;
         return TM_OK;
     }
-    TileArgs args(const SlotOp& op) const {
-        return TileArgs{nt, op.S, (op.S + kTileS - 1) / kTileS, row0.p, rows.p, node0.p, nodes.p, loc.p};
+    TileArgs args(const SlotOp& op, int samples = kTileS) const {
+        return TileArgs{nt, op.S, (op.S + samples - 1) / samples, row0.p, rows.p, node0.p, nodes.p, loc.p};
     }
 };
 
-// C = R (I - A w D^-1): the level-0 pre-smoother from zero followed by the
-// restriction, as one operator (rows of R, columns of A).  R: nr x n CSR;
-// A: n x n CSR (rp, ci, v); dinv: A's inverse diagonal.
-void restrict_presmoothed(const HostCsr& R, int n, const int* arp, const int* aci, const std::vector<double>& av,
-                          const double* dinv, double w, HostCsr& C) {
-    const int nr = (int)R.rp.size() - 1;
-    C.n = nr;
-    C.rp.assign((size_t)nr + 1, 0);
-    C.ci.clear();
-    C.v.clear();
-    std::vector<double> acc((size_t)n, 0.0);
-    std::vector<int> mark((size_t)n, -1), touched;
-    for (int c = 0; c < nr; ++c) {
-        touched.clear();
-        for (int q = R.rp[c]; q < R.rp[c + 1]; ++q) {
-            const int i = R.ci[q];
-            const double r = R.v[q];
-            for (int t = arp[i]; t < arp[i + 1]; ++t) {
-                const int j = aci[t];
-                if (mark[j] != c) {
-                    mark[j] = c;
-                    acc[j] = 0.0;
-                    touched.push_back(j);
-                }
-                acc[j] += r * ((j == i ? 1.0 : 0.0) - av[t] * w * dinv[j]);
-            }
+// The V-cycle's way up on one level, [2 w D^-1 - w D^-1 A w D^-1 | Q] on [b | x_c],
+// from A (n rows) and down = R (I - A w D^-1), the transpose of Q = (I - w D^-1 A) P.
+// Fixed rows of A (identity, no part of the hierarchy) have columns of the
+// whole matrix; b is zero there.
+void up_operator(int n, const int* arp, const int* aci, const std::vector<double>& av, const double* dinv, double w,
+                 const HostCsr& down, HostCsr& U) {
+    const int nc = (int)down.rp.size() - 1;
+    std::vector<int> qp((size_t)n + 1, 0);
+    for (int c : down.ci) ++qp[c + 1];
+    U.n = n;
+    U.rp.assign((size_t)n + 1, 0);
+    for (int i = 0; i < n; ++i) U.rp[i + 1] = U.rp[i] + (arp[i + 1] - arp[i]) + qp[i + 1];
+    U.ci.resize((size_t)U.rp[n]);
+    U.v.resize((size_t)U.rp[n]);
+    std::vector<int> fill((size_t)n);
+    for (int i = 0; i < n; ++i) {
+        int k = U.rp[i];
+        for (int q = arp[i]; q < arp[i + 1]; ++q, ++k) {
+            const int j = aci[q];
+            U.ci[k] = j;
+            U.v[k] = (j == i ? 2.0 * w * dinv[i] : 0.0) - w * dinv[i] * av[q] * w * dinv[j];
         }
-        std::sort(touched.begin(), touched.end());
-        for (int j : touched) {
-            C.ci.push_back(j);
-            C.v.push_back(acc[j]);
-        }
-        C.rp[c + 1] = (int)C.ci.size();
+        fill[i] = k;
     }
+    for (int c = 0; c < nc; ++c)
+        for (int q = down.rp[c]; q < down.rp[c + 1]; ++q) {
+            const int k = fill[down.ci[q]]++;
+            U.ci[k] = n + c;
+            U.v[k] = down.v[q];
+        }
 }
 
 // ---- initial guesses from earlier solves (successive right-hand sides) ----
@@ -2559,32 +2561,29 @@ struct BatchSolver {
     int n = 0, S = 0, G = 0;
     SlotOp sl0;                   // level-0 operator in slots
     DevBuf<T> wA0;                // its weights
-    SlotOp sl0w;                  // the same without the diagonal, for the wide kernels
-    DevBuf<T> wA0w, dA0;          // its weights and the diagonal
-    DevBuf<T> wIDA0;              // on sl0: I - w D^-1 A (level-0 post-smoother, wide form)
-    bool post1 = false;           // wIDA0 is set (every level-0 row fits one chunk with its diagonal)
     DevBuf<double> wA64;          // A in FP64 (outer residual)
     TileOp t0;                    // tiles of sl0 for the outer residual
     int Gr = 0;                   // partials per sample of the outer residual
+    int Gq = 0, Gz = 0;           // of (z, q) and of (r, z)
+    int gmax() const { return std::max(std::max(G, Gr), std::max(Gq, Gz)); }
+    // the level-0 products of the inner solve from tiles (64 FP32 samples)
+    bool tiled() const { return wide() && t0.nt > 0 && tu.nt > 0; }
+    TileOp tu;                    // tiles of level 0's way up
     struct LvOps {
-        SlotOp A, R, P;           // level l >= 1: A; every level: restriction, prolongation
-        DevBuf<T> wA, wR, wP;
         SlotOp RA;                // R (I - A w D^-1): pre-smoothing from zero + restriction
         DevBuf<T> wRA;
+        SlotOp U;                 // on [b | x_c]: prolongation + post-smoothing
+        DevBuf<T> wU;
     };
     std::vector<LvOps> lo;
-    DevBuf<double> dinv;
     DevBuf<unsigned char> fixed;
-    DevBuf<T> rT, q;
+    DevBuf<T> rT, q;              // rT: [r | x_c]
     static constexpr int kRing = 40;  // iterations per inner solve (a longer one is cut there; the outer loop goes on)
     DevBuf<T> ring;                   // (kRing + 1) x [n][S]: the preconditioned residuals z_k
     DevBuf<double> ahist, bhist;      // (kRing + 1) x kMaxS: alpha_k, beta_k
     DevBuf<double> chist;             // kRing x kMaxS: the combination coefficients c_i
-    struct Lv {
-        DevBuf<T> x, x2, b;
-    };
-    std::vector<Lv> lv;
-    DevBuf<T> xc;
+    std::vector<DevBuf<T>> bx;    // levels >= 1: [b | x_c]
+    DevBuf<T> bc;                 // the coarsest right-hand side
     DevBuf<double> part;          // 4 slots x S x G
     DevBuf<OState> ost;
     DevBuf<BState> bst;
@@ -2618,77 +2617,40 @@ struct BatchSolver {
         TM_CHECK(sl0.values(solver.h_val, wA64, s));
         TM_CHECK(t0.build(sl0, s));
         Gr = t0.nt > 0 ? tile_blocks((S + kTileS - 1) / kTileS, kResidPerCu) : G;
-        if (wide() && L > 0) {
-            const int* cc = solver.pat.h_csrcol.data();
-            TM_CHECK(sl0w.build(n, n, solver.pat.h_rowptr.data(), cc, S, s, true));
-            TM_CHECK(sl0w.values(solver.h_val, wA0w, s));
-            TM_CHECK(sl0w.diagonal(solver.h_val, dA0, s));
-            // the level-0 post-smoother's operator I - w D^-1 A with the
-            // diagonal in the slots (rows of up to 16 entries: one chunk)
-            if (sl0.one_chunk()) {
-                const int* rp = solver.pat.h_rowptr.data();
-                const double w = M.levels[0].omega;
-                const std::vector<double>& dv = solver.h_dinv;
-                std::vector<double> v2(solver.h_val.size());
-                for (int i = 0; i < n; ++i)
-                    for (int q = rp[i]; q < rp[i + 1]; ++q)
-                        v2[q] = (cc[q] == i ? 1.0 : 0.0) - solver.h_val[q] * w * dv[i];
-                TM_CHECK(sl0.values(v2, wIDA0, s));
-                post1 = true;
-            }
-        }
         lo.clear();
         lo.resize((size_t)L);
         for (int l = 0; l < L; ++l) {
             const auto& V = M.levels[l];
             const int nnext = l + 1 < L ? M.levels[l + 1].n : M.nc;
-            HostCsr h, ha;
-            std::vector<double> dv;
-            if (l > 0) {
-                TM_CHECK(fetch_csr(V.A, ha, s));
-                dv.resize((size_t)V.n);
-                TM_HIP(hipMemcpyAsync(dv.data(), V.dinv.p, dv.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-                TM_HIP(hipStreamSynchronize(s));
-                TM_CHECK(lo[l].A.build(V.n, V.n, ha.rp.data(), ha.ci.data(), S, s));
-                TM_CHECK(lo[l].A.values(ha.v, lo[l].wA, s));
+            HostCsr down, up;
+            TM_CHECK(fetch_csr(V.down, down, s));
+            TM_CHECK(lo[l].RA.build(nnext, V.n, down.rp.data(), down.ci.data(), S, s));
+            TM_CHECK(lo[l].RA.values(down.v, lo[l].wRA, s));
+            if (l == 0) {
+                up_operator(n, solver.pat.h_rowptr.data(), solver.pat.h_csrcol.data(), solver.h_val,
+                            solver.h_dinv.data(), V.omega, down, up);
+            } else {
+                TM_CHECK(fetch_csr(V.up, up, s));
             }
-            TM_CHECK(fetch_csr(V.R, h, s));
-            TM_CHECK(lo[l].R.build(V.R.n, V.n, h.rp.data(), h.ci.data(), S, s));
-            TM_CHECK(lo[l].R.values(h.v, lo[l].wR, s));
-            {  // pre-smoothing from zero and restriction in one pass: R (I - A w D^-1)
-                HostCsr c;
-                if (l == 0)
-                    restrict_presmoothed(h, n, solver.pat.h_rowptr.data(), solver.pat.h_csrcol.data(), solver.h_val,
-                                         solver.h_dinv.data(), V.omega, c);
-                else
-                    restrict_presmoothed(h, V.n, ha.rp.data(), ha.ci.data(), ha.v, dv.data(), V.omega, c);
-                TM_CHECK(lo[l].RA.build(V.R.n, V.n, c.rp.data(), c.ci.data(), S, s));
-                TM_CHECK(lo[l].RA.values(c.v, lo[l].wRA, s));
-            }
-            TM_CHECK(fetch_csr(V.P, h, s));
-            TM_CHECK(lo[l].P.build(V.P.n, nnext, h.rp.data(), h.ci.data(), S, s, false,
-                                   wide() ? SlotOp::wide_chunk(V.P.n, h.rp.data()) : kSlot));
-            TM_CHECK(lo[l].P.values(h.v, lo[l].wP, s));
+            TM_CHECK(lo[l].U.build(V.n, V.n + nnext, up.rp.data(), up.ci.data(), S, s));
+            TM_CHECK(lo[l].U.values(up.v, lo[l].wU, s));
+            if (l == 0 && wide()) TM_CHECK(tu.build(lo[0].U, s));
         }
-        TM_CHECK(dinv.upload(solver.h_dinv.data(), n, s));
+        Gq = Gz = tiled() ? tile_blocks(1, kSolvePerCu) : G;
         TM_CHECK(fixed.upload(solver.h_fixed.data(), n, s));
         const size_t NS = (size_t)n * S;
-        TM_CHECK(rT.alloc(NS));
+        TM_CHECK(rT.alloc(NS + (size_t)M.tail() * S));
         TM_CHECK(ring.alloc((size_t)(kRing + 1) * NS));
         TM_CHECK(ahist.alloc((size_t)(kRing + 1) * kMaxS));
         TM_CHECK(bhist.alloc((size_t)(kRing + 1) * kMaxS));
         TM_CHECK(chist.alloc((size_t)(kRing + 1) * kMaxS));
         TM_CHECK(q.alloc(NS));
-        lv.clear();
-        lv.resize(solver.amg.levels.size());
-        for (size_t l = 0; l < solver.amg.levels.size(); ++l) {
-            const auto& L = solver.amg.levels[l];
-            TM_CHECK(lv[l].x.alloc((size_t)L.n * S));
-            TM_CHECK(lv[l].x2.alloc((size_t)L.n * S));
-            TM_CHECK(lv[l].b.alloc((size_t)L.R.n * S));
-        }
-        TM_CHECK(xc.alloc((size_t)std::max(1, solver.amg.nc) * S));
-        TM_CHECK(part.alloc((size_t)std::max(4, kWinDots) * S * std::max(G, Gr) + (size_t)kWinDots * kWinChunks * S));
+        bx.clear();
+        bx.resize((size_t)L);
+        for (int l = 1; l < L; ++l)
+            TM_CHECK(bx[l].alloc((size_t)(M.levels[l].n + (l + 1 < L ? M.levels[l + 1].n : M.nc)) * S));
+        TM_CHECK(bc.alloc((size_t)std::max(1, M.nc) * S));
+        TM_CHECK(part.alloc((size_t)std::max(4, kWinDots) * S * gmax() + (size_t)kWinDots * kWinChunks * S));
         TM_CHECK(winX.alloc((size_t)kSolveWindow * NS));
         TM_CHECK(winB.alloc((size_t)kSolveWindow * NS));
         TM_CHECK(win.alloc(1));
@@ -2702,55 +2664,42 @@ struct BatchSolver {
         return TM_OK;
     }
 
-    // z = M r (AMG V-cycle, batched), partial (r, z) into prz
-    int precond(const T* r, T* zout, double* prz, hipStream_t s) {
+    // z = M r (AMG V-cycle, batched) for r = [r | x_c], partial (r, z) into prz:
+    // one product per level in each direction, as the single-sample solver's
+    int precond(T* r, T* zout, double* prz, hipStream_t s) {
         const AmgPrecond& M = cg->amg;
         const int L = (int)M.levels.size();
         if (L == 0) return TM_ERR_UNSUPPORTED;  // the batched solve needs at least one AMG level
-        const int e = (int)sizeof(T);
-        const T* b = r;
+        auto vec = [&](int l) { return l == 0 ? r : bx[l].p; };  // [b | x_c] of level l
+        auto tail = [&](int l) { return vec(l) + (size_t)M.levels[l].n * S; };
         for (int l = 0; l < L; ++l) {
-            const auto& V = M.levels[l];
             const LvOps& O = lo[l];
-            // b_{l+1} = R (I - A w D^-1) b: pre-smoothing from zero and
-            // restriction in one pass over the coarse rows (the pre-smoothed
-            // iterate w D^-1 b is formed by the prolongation pass)
-            spmm(O.RA.long_rows(), dim3(row_grid(V.R.n)), O.RA.args(e, O.wRA.p), b, lv[l].b.p, s);
-            b = lv[l].b.p;
+            spmm(O.RA, O.wRA.p, vec(l), l + 1 < L ? vec(l + 1) : bc.p, s);
         }
         hipLaunchKernelGGL((k_b_dense<T>), dim3(std::max(1, std::min(M.nc, 4096))), dim3(kBlock), 0, s, M.nc, S,
-                           M.Cinv.p, b, xc.p, gate());
-        const T* xcoarse = xc.p;
-        for (int l = L - 1; l >= 0; --l) {
-            const auto& V = M.levels[l];
-            const LvOps& O = lo[l];
-            const T* bl = l == 0 ? r : lv[l - 1].b.p;
-            if (wide())
-                prolong(O.P.long_rows(), O.P.chunk, dim3(row_grid(V.P.n)), O.P.args(e, O.wP.p),
-                        l == 0 ? dinv.p : V.dinv.p, bl, V.omega, xcoarse, lv[l].x.p, s);
-            else
-                hipLaunchKernelGGL((k_b_prolong<T>), dim3(row_grid(V.P.n)), dim3(kBlock), 0, s,
-                                   gated(O.P.args(e, O.wP.p)), S, l == 0 ? dinv.p : V.dinv.p, bl, V.omega, xcoarse,
-                                   lv[l].x.p);
-            if (l == 0) {
-                if (wide() && post1) {  // z = (I - w D^-1 A) x + w D^-1 b
-                    if constexpr (kWideT)
-                        hipLaunchKernelGGL(k_b_post1_w, dim3(G), dim3(kBlock), 0, s, gated(sl0.args(e, wIDA0.p)),
-                                           dinv.p, (const float*)bl, V.omega, (const float*)lv[0].x.p, (float*)zout,
-                                           prz);
-                } else if (wide())
-                    post(false, dim3(G), sl0w.args(e, wA0w.p), dinv.p, bl, V.omega, lv[0].x.p, zout, prz, s, dA0.p);
-                else
-                    post(sl0.long_rows(), dim3(G), sl0.args(e, wA0.p), dinv.p, bl, V.omega, lv[0].x.p, zout, prz, s);
-                xcoarse = zout;
-            } else {
-                post(O.A.long_rows(), dim3(row_grid(V.n)), O.A.args(e, O.wA.p), V.dinv.p, bl, V.omega, lv[l].x.p,
-                     lv[l].x2.p, nullptr, s);
-                xcoarse = lv[l].x2.p;
-            }
-        }
+                           M.Cinv.p, (const T*)bc.p, tail(L - 1), gate());
+        for (int l = L - 1; l > 0; --l) spmm(lo[l].U, lo[l].wU.p, vec(l), tail(l - 1), s);
+        up0(r, zout, prz, s);
         TM_HIP(hipGetLastError());
         return TM_OK;
+    }
+
+    // level 0 upwards: z = U [r | x_c], partial (r, z)
+    void up0(const T* r, T* z, double* prz, hipStream_t s) {
+        if constexpr (kWideT) {
+            if (tiled()) {
+                hipLaunchKernelGGL(k_b_up_t, dim3(Gz), dim3(kTileThreads), 0, s, tu.args(lo[0].U, 64),
+                                   (const float*)lo[0].wU.p, (const float*)r, (float*)z, gate(), prz);
+                return;
+            }
+            if (wide()) {
+                hipLaunchKernelGGL(k_b_up_w, dim3(G), dim3(kBlock), 0, s, gated(lo[0].U.args(4, lo[0].wU.p)),
+                                   (const float*)r, (float*)z, prz);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((k_b_up<T>), dim3(G), dim3(kBlock), 0, s, gated(lo[0].U.args((int)sizeof(T), lo[0].wU.p)),
+                           S, r, z, prz);
     }
 
     // the per-sample active flags of the inner solve (device address)
@@ -2768,50 +2717,18 @@ struct BatchSolver {
     bool wide() const { return kWideT && S == kMaxS; }
     // one block per row for long-row operators (grid: a multiple of the XCD count)
     static dim3 blk_grid(int rows) { return dim3(xcd_grid(std::min(4096, std::max(rows, 1)))); }
-    // y = M x; lg: one block per row (long rows, wide form)
-    void spmm(bool lg, dim3 g, SlotArgs a, const T* x, T* y, hipStream_t s) {
-        a = gated(a);
+    // y = M x (one block per row for long rows in the wide form)
+    void spmm(const SlotOp& M, const T* w, const T* x, T* y, hipStream_t s) {
+        const SlotArgs a = gated(M.args((int)sizeof(T), w));
         if constexpr (kWideT)
             if (wide()) {
                 const float* xf = (const float*)x;
                 float* yf = (float*)y;
-                if (lg) hipLaunchKernelGGL(k_b_spmm_w<true>, blk_grid(a.n), dim3(kBlock), 0, s, a, xf, yf);
-                else hipLaunchKernelGGL(k_b_spmm_w<false>, g, dim3(kBlock), 0, s, a, xf, yf);
+                if (M.long_rows()) hipLaunchKernelGGL(k_b_spmm_w<true>, blk_grid(a.n), dim3(kBlock), 0, s, a, xf, yf);
+                else hipLaunchKernelGGL(k_b_spmm_w<false>, dim3(row_grid(a.n)), dim3(kBlock), 0, s, a, xf, yf);
                 return;
             }
-        hipLaunchKernelGGL((k_b_spmm<T>), g, dim3(kBlock), 0, s, a, S, x, y);
-    }
-    // x = w dinv b + P xc (wide form only); ch: P's chunk size
-    void prolong(bool lg, int ch, dim3 g, SlotArgs a, const double* di, const T* bb, double w, const T* xc, T* x,
-                 hipStream_t s) {
-        a = gated(a);
-        if constexpr (kWideT) {
-            const float* bf = (const float*)bb;
-            const float* xf = (const float*)xc;
-            if (ch == 8)
-                hipLaunchKernelGGL((k_b_prolong_w<false, 8>), g, dim3(kBlock), 0, s, a, di, bf, w, xf, (float*)x);
-            else if (lg)
-                hipLaunchKernelGGL((k_b_prolong_w<true, kSlot>), blk_grid(a.n), dim3(kBlock), 0, s, a, di, bf, w, xf,
-                                   (float*)x);
-            else
-                hipLaunchKernelGGL((k_b_prolong_w<false, kSlot>), g, dim3(kBlock), 0, s, a, di, bf, w, xf, (float*)x);
-        }
-    }
-    void post(bool lg, dim3 g, SlotArgs a, const double* di, const T* bb, double w, const T* x, T* xo, double* part,
-              hipStream_t s, const T* dg = nullptr) {
-        a = gated(a);
-        if constexpr (kWideT)
-            if (wide()) {
-                const float* df = (const float*)dg;
-                if (lg && !part)  // partial sums are laid out per block of the row grid g
-                    hipLaunchKernelGGL(k_b_post_w<true>, blk_grid(a.n), dim3(kBlock), 0, s, a, df, di,
-                                       (const float*)bb, w, (const float*)x, (float*)xo, part);
-                else
-                    hipLaunchKernelGGL(k_b_post_w<false>, g, dim3(kBlock), 0, s, a, df, di, (const float*)bb, w,
-                                       (const float*)x, (float*)xo, part);
-                return;
-            }
-        hipLaunchKernelGGL((k_b_post<T>), g, dim3(kBlock), 0, s, a, S, di, bb, w, x, xo, part);
+        hipLaunchKernelGGL((k_b_spmm<T>), dim3(row_grid(a.n)), dim3(kBlock), 0, s, a, S, x, y);
     }
 
     // initial guess of the solve of A x = b from the window of solved pairs;
@@ -2866,9 +2783,15 @@ struct BatchSolver {
     // iteration k: q = A p_k = A z_k + beta q, partial (z_k, q)
     void cg_spmv(const T* zk, int k, double* pzq, hipStream_t s) {
         if constexpr (kWideT)
+            if (tiled()) {
+                hipLaunchKernelGGL(k_b_cg_spmv_t, dim3(Gq), dim3(kTileThreads), 0, s, t0.args(sl0, 64),
+                                   (const float*)wA0.p, (const float*)zk, (float*)q.p, k, (const BState*)bst.p, pzq);
+                return;
+            }
+        if constexpr (kWideT)
             if (wide()) {
-                hipLaunchKernelGGL(k_b_cg_spmv_w, dim3(G), dim3(kBlock), 0, s, gated(sl0w.args(4, wA0w.p)),
-                                   (const float*)dA0.p, (const float*)zk, (float*)q.p, k, (const BState*)bst.p, pzq);
+                hipLaunchKernelGGL(k_b_cg_spmv_w, dim3(G), dim3(kBlock), 0, s, gated(sl0.args(4, wA0.p)),
+                                   (const float*)zk, (float*)q.p, k, (const BState*)bst.p, pzq);
                 return;
             }
         hipLaunchKernelGGL((k_b_cg_spmv<T>), dim3(G), dim3(kBlock), 0, s, gated(sl0.args((int)sizeof(T), wA0.p)), S,
@@ -2881,9 +2804,9 @@ struct BatchSolver {
         if (cg->precond != TM_PRECOND_AMG || cg->amg.levels.empty()) return TM_ERR_UNSUPPORTED;
         const size_t NS = (size_t)n * S;
         double* pbb = part.p;
-        double* prr = part.p + (size_t)S * std::max(G, Gr);
-        double* prz = part.p + (size_t)2 * S * std::max(G, Gr);
-        double* pzq = part.p + (size_t)3 * S * std::max(G, Gr);
+        double* prr = part.p + (size_t)S * gmax();
+        double* prz = part.p + (size_t)2 * S * gmax();
+        double* pzq = part.p + (size_t)3 * S * gmax();
         const double itol = sizeof(T) == 4 ? 1e-5 : 0.0;  // FP32 inner target per refinement step
         int outer = 0, inner_total = 0;
         if (use_window) win_project(b, x, s);  // (sets the fixed rows too)
@@ -2934,7 +2857,7 @@ struct BatchSolver {
             ++outer;
             // inner solve A d = rT from d = 0; x += d at the end
             TM_CHECK(precond(rT.p, ring.p, prz, s));
-            hipLaunchKernelGGL(k_b_red_rz, dim3(S), dim3(kBlock), 0, s, G, S, prz, -1, bst.p, bhist.p);
+            hipLaunchKernelGGL(k_b_red_rz, dim3(S), dim3(kBlock), 0, s, Gz, S, prz, -1, bst.p, bhist.p);
             int enq = 0;
             const int kmax = std::min(kRing, maxit);
             // iterations enqueued before the first check: what this refinement
@@ -2949,7 +2872,7 @@ struct BatchSolver {
                 for (int c = 0; c < chunk && enq < kmax; ++c, ++enq) {
                     T* zk = ring.p + (size_t)enq * NS;
                     cg_spmv(zk, enq, pzq, s);
-                    hipLaunchKernelGGL(k_b_red_pq, dim3(S), dim3(kBlock), 0, s, G, S, pzq, bst.p,
+                    hipLaunchKernelGGL(k_b_red_pq, dim3(S), dim3(kBlock), 0, s, Gq, S, pzq, bst.p,
                                        ahist.p + (size_t)enq * kMaxS);
                     cg_update(prr, s);
                     conv_check(prr, s);
@@ -2957,7 +2880,7 @@ struct BatchSolver {
                     // (or of the ring): its z would go unused
                     if ((spec && c + 1 == chunk) || enq + 1 == kmax) continue;
                     TM_CHECK(precond(rT.p, zk + NS, prz, s));
-                    hipLaunchKernelGGL(k_b_red_rz, dim3(S), dim3(kBlock), 0, s, G, S, prz, enq, bst.p,
+                    hipLaunchKernelGGL(k_b_red_rz, dim3(S), dim3(kBlock), 0, s, Gz, S, prz, enq, bst.p,
                                        bhist.p + (size_t)(enq + 1) * kMaxS);
                 }
                 TM_HIP(hipGetLastError());
@@ -3011,8 +2934,8 @@ struct BatchSolver {
         if (cg->amg.levels.empty()) return TM_ERR_UNSUPPORTED;
         const int e = (int)sizeof(T);
         const double nS = (double)n * S;
-        double* pzq = part.p + (size_t)3 * S * std::max(G, Gr);
-        double* prz = part.p + (size_t)2 * S * std::max(G, Gr);
+        double* pzq = part.p + (size_t)3 * S * gmax();
+        double* prz = part.p + (size_t)2 * S * gmax();
         auto add = [&out](const char* nm, double ms, double bytes) {
             tm_batch_kernel_time k = {};
             std::snprintf(k.name, sizeof(k.name), "%s", nm);
@@ -3022,38 +2945,19 @@ struct BatchSolver {
         };
         auto slots = [](const SlotOp& o) { return (double)o.h_sp[o.n]; };
         hipLaunchKernelGGL(k_b_activate, dim3(1), dim3(kMaxS), 0, s, S, bst.p);
-        const SlotOp& A0 = wide() ? sl0w : sl0;
-        add(wide() ? "k_b_cg_spmv_w" : "k_b_cg_spmv", timeit([&] { cg_spmv(ring.p, 0, pzq, s); }),
-            slots(A0) * (4 + e) + (wide() ? (double)n * e : 0.0) + 3.0 * nS * e);
+        add(tiled() ? "k_b_cg_spmv_t" : wide() ? "k_b_cg_spmv_w" : "k_b_cg_spmv",
+            timeit([&] { cg_spmv(ring.p, 0, pzq, s); }), slots(sl0) * (4 + e) + 3.0 * nS * e);
         add(sizeof(T) == 4 ? "k_b_cg_update<float>" : "k_b_cg_update<double>",
-            timeit([&] { cg_update(part.p + (size_t)S * std::max(G, Gr), s); }), 3.0 * nS * e);
+            timeit([&] { cg_update(part.p + (size_t)S * gmax(), s); }), 3.0 * nS * e);
         const LvOps& O = lo[0];
-        const int n1 = cg->amg.levels[0].R.n;
-        add(O.RA.long_rows() ? "k_b_spmm_w<long> (R(I-AwD^-1), level 0)" : "k_b_spmm (R(I-AwD^-1), level 0)",
-            timeit([&] { spmm(O.RA.long_rows(), dim3(row_grid(n1)), O.RA.args(e, O.wRA.p), rT.p, lv[0].b.p, s); }),
-            slots(O.RA) * (4 + e) + nS * e + (double)n1 * S * e);
-        const auto& V0 = cg->amg.levels[0];
-        add(wide() ? "k_b_prolong_w (level 0)" : "k_b_prolong (level 0)", timeit([&] {
-                if (wide())
-                    prolong(O.P.long_rows(), O.P.chunk, dim3(row_grid(V0.P.n)), O.P.args(e, O.wP.p), dinv.p, rT.p,
-                            V0.omega, lv[0].b.p, lv[0].x.p, s);
-                else
-                    hipLaunchKernelGGL((k_b_prolong<T>), dim3(row_grid(V0.P.n)), dim3(kBlock), 0, s,
-                                       gated(O.P.args(e, O.wP.p)), S, dinv.p, rT.p, V0.omega, lv[0].b.p, lv[0].x.p);
-            }),
-            slots(O.P) * (4 + e) + 8.0 * n + 2.0 * nS * e + (double)n1 * S * e);
-        if constexpr (kWideT) {
-            if (wide() && post1) {
-                add("k_b_post1_w (level 0)", timeit([&] {
-                        hipLaunchKernelGGL(k_b_post1_w, dim3(G), dim3(kBlock), 0, s, gated(sl0.args(e, wIDA0.p)),
-                                           dinv.p, (const float*)rT.p, V0.omega, (const float*)lv[0].x.p,
-                                           (float*)ring.p, prz);
-                    }),
-                    slots(sl0) * (4 + e) + 8.0 * n + 3.0 * nS * e);
-            }
-        }
+        const double n1 = O.RA.n;
+        T* y1 = cg->amg.levels.size() > 1 ? bx[1].p : bc.p;
+        add(O.RA.long_rows() && wide() ? "k_b_spmm_w<long> (R(I-AwD^-1), level 0)" : "k_b_spmm (R(I-AwD^-1), level 0)",
+            timeit([&] { spmm(O.RA, O.wRA.p, rT.p, y1, s); }), slots(O.RA) * (4 + e) + nS * e + n1 * S * e);
+        add(tiled() ? "k_b_up_t (level 0)" : wide() ? "k_b_up_w (level 0)" : "k_b_up (level 0)",
+            timeit([&] { up0(rT.p, ring.p, prz, s); }), slots(O.U) * (4 + e) + 2.0 * nS * e + n1 * S * e);
         double* pbb = part.p;
-        double* prr = part.p + (size_t)S * std::max(G, Gr);
+        double* prr = part.p + (size_t)S * gmax();
         add(sizeof(T) == 4 ? "k_b_resid<float>" : "k_b_resid<double>", timeit([&] {
                 resid(lv0_b64(), lv0_x64(), pbb, prr, s);
             }),
@@ -3079,9 +2983,9 @@ struct BatchSolver {
         if (nouter < 0 || nouter > kMaxOuter || !fail || !track) return TM_ERR_BAD_ARG;
         const size_t NS = (size_t)n * S;
         double* pbb = part.p;
-        double* prr = part.p + (size_t)S * std::max(G, Gr);
-        double* prz = part.p + (size_t)2 * S * std::max(G, Gr);
-        double* pzq = part.p + (size_t)3 * S * std::max(G, Gr);
+        double* prr = part.p + (size_t)S * gmax();
+        double* prz = part.p + (size_t)2 * S * gmax();
+        double* pzq = part.p + (size_t)3 * S * gmax();
         const double itol = sizeof(T) == 4 ? 1e-5 : 0.0;
         if (use_window) win_project(b, x, s);  // (sets the fixed rows too)
         else hipLaunchKernelGGL(k_b_fix, dim3(elem_grid(NS)), dim3(kBlock), 0, s, n, S, fixed.p, b, x);
@@ -3091,18 +2995,18 @@ struct BatchSolver {
                                o > 0 ? track + (o - 1) : (int*)nullptr);
             if (o == nouter) break;
             TM_CHECK(precond(rT.p, ring.p, prz, s));
-            hipLaunchKernelGGL(k_b_red_rz, dim3(S), dim3(kBlock), 0, s, G, S, prz, -1, bst.p, bhist.p);
+            hipLaunchKernelGGL(k_b_red_rz, dim3(S), dim3(kBlock), 0, s, Gz, S, prz, -1, bst.p, bhist.p);
             const int K = std::max(1, std::min(kRing, ninner[o]));
             for (int k = 0; k < K; ++k) {
                 T* zk = ring.p + (size_t)k * NS;
                 cg_spmv(zk, k, pzq, s);
-                hipLaunchKernelGGL(k_b_red_pq, dim3(S), dim3(kBlock), 0, s, G, S, pzq, bst.p,
+                hipLaunchKernelGGL(k_b_red_pq, dim3(S), dim3(kBlock), 0, s, Gq, S, pzq, bst.p,
                                    ahist.p + (size_t)k * kMaxS);
                 cg_update(prr, s);
                 conv_check(prr, s);
                 if (k + 1 == K) break;  // the last z would go unused
                 TM_CHECK(precond(rT.p, zk + NS, prz, s));
-                hipLaunchKernelGGL(k_b_red_rz, dim3(S), dim3(kBlock), 0, s, G, S, prz, k, bst.p,
+                hipLaunchKernelGGL(k_b_red_rz, dim3(S), dim3(kBlock), 0, s, Gz, S, prz, k, bst.p,
                                    bhist.p + (size_t)(k + 1) * kMaxS);
             }
             if (S == kMaxS && K <= kCombineK) {
@@ -3239,7 +3143,7 @@ int csr_on_pattern(const SellPattern& P, const std::vector<int>& rp, const std::
 int upload_op(tm_batch* bt, int op, DevBuf<double>& dst, const double* colscale = nullptr, double w0 = 1.0) {
     std::vector<double> v;
     TM_CHECK(csr_on_pattern(*bt->cv.pat, *bt->cv.hop_rp[op], *bt->cv.hop_col[op], *bt->cv.hop_val[op], v));
-    return bt->eo.values(v, dst, bt->stream, bt->cv.pat->h_csrcol.data(), colscale, w0);
+    return bt->eo.values(v, dst, bt->stream, colscale, w0);
 }
 
 }  // namespace

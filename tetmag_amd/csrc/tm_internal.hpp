@@ -470,12 +470,11 @@ struct AmgPrecond {
         const SellPattern* A_ext = nullptr;
         const double* Aval_ext = nullptr;
         const double* dinv_ext = nullptr;
-        CsrDev A, P, R;  // A used on levels >= 1
-        DevBuf<double> dinv;
         CsrDev down;        // R (I - A w D^-1): pre-smoothing from zero and restriction
         CsrDev up;          // [2 w D^-1 - w D^-1 A w D^-1 | (I - w D^-1 A) P] on [b | x_c]
         DevBuf<double> bx;  // levels >= 1: [b | x_c], the restricted right-hand side and the coarser correction
-        DevBuf<double> x;   // level 0 without `up`: w D^-1 b + P x_c
+        CsrDev P;           // level 0 without `up`: the prolongator, and
+        DevBuf<double> x;   // w D^-1 b + P x_c
     };
     std::vector<Level> levels;
     int nc = 0;
