@@ -1942,96 +1942,102 @@ __global__ __launch_bounds__(kBlock) void k_b_i8_uslice(int b, int S, int nC, co
 }
 
 // P[ks][row][col] (row-major, 64 columns) = sum_d 2^-7d acc_d over the K
-// chunks [ks cper, (ks+1) cper) of the slices.  Block: 4 wavefronts x MT
-// row tiles of 16 rows; the chunk's U digits (24 KB) are staged in LDS and
-// shared by the four wavefronts, double-buffered: while the MFMAs of chunk
-// c run, the B digits of chunk c+1 are in flight into registers and its U
-// digits into registers, stored to the other buffer afterwards.
+// chunks [ks cper, (ks+1) cper) of the slices.  Block: NW wavefronts of 16 rows
+// each; the chunk's U digits (24 KB) are staged in LDS and shared by the
+// wavefronts, double-buffered: while the MFMAs of chunk c run, U's digits of
+// chunk c + 1 are in flight into registers, stored to the other buffer
+// afterwards, and B's digits of chunks c + 1 and c + 2 into a rotation of three
+// register sets: 8 wavefronts then keep 80 KB per CU in flight, with one chunk
+// ahead (40 KB) every wavefront waited for memory.  Bound by HBM and the
+// matrix cores alike: 40,930 boundary nodes and 64 samples 1,700 -> 1,440 us, B's
+// 8.4 GB of digits at 5.8 TB/s (the 131 M products alone: 1.5 ms at the 2.86
+// POPS that the instruction sustains over long runs, 0.86 at its peak).
 // v_mfma_i32_16x16x64_i8: A lane l = row l % 16, B lane l = column l % 16,
 // both the 16 k of block l / 16; D lane l register r = C[4 (l / 16) + r][l % 16].
-template <int MT>
-__global__ __launch_bounds__(kBlock) void k_b_gemm_i8(int b, int nT, int nC, int cper,
-                                                      const i32x4* __restrict__ Bq, const i32x4* __restrict__ Uq,
-                                                      double* __restrict__ P) {
-    constexpr int UPT = kI8DigitsU * 4 * kI8Op / kBlock;  // U operands per thread per chunk (6)
+template <int NW>
+__global__ __launch_bounds__(64 * NW, 2) void k_b_gemm_i8(int b, int nT, int nC, int cper,
+                                                          const i32x4* __restrict__ Bq,
+                                                          const i32x4* __restrict__ Uq, double* __restrict__ P) {
+    constexpr int UPT = kI8DigitsU * 4 * kI8Op / (64 * NW);  // U operands per thread per chunk
     __shared__ i32x4 us[2][kI8DigitsU * 4 * kI8Op];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int T0 = (blockIdx.x * (kBlock / 64) + wv) * MT;
-    const int cb = blockIdx.y * cper, ce = min(nC, cb + cper);
-    const int ncc = ce > cb ? ce - cb : 0;  // uniform over the block
-    i32x4 acc[kI8MaxD + 1][MT][4];
+    const int lane = threadIdx.x & 63;
+    const int T = blockIdx.x * NW + (int)(threadIdx.x >> 6);
+    const int cb = blockIdx.y * cper, ce = min(nC, cb + cper);  // (empty: cb >= nC)
+    i32x4 acc[kI8MaxD + 1][4];
 #pragma unroll
     for (int d = 0; d <= kI8MaxD; ++d)
 #pragma unroll
-        for (int t = 0; t < MT; ++t)
+        for (int u = 0; u < 4; ++u) acc[d][u] = i32x4{0, 0, 0, 0};
+    // tiles and chunks past the last load the last one (the tile is not stored,
+    // the chunk is multiplied with zero): no load depends on a condition
+    const i32x4* src = Bq + (size_t)min(T, nT - 1) * nC * (kI8Digits * kI8Op) + lane;
+    i32x4 ur[UPT];
+    typedef i32x4 Ops[kI8Digits];
+    auto load_a = [&](int c, Ops& dst) {
+        const i32x4* s = src + (size_t)min(c, nC - 1) * (kI8Digits * kI8Op);
 #pragma unroll
-            for (int u = 0; u < 4; ++u) acc[d][t][u] = i32x4{0, 0, 0, 0};
-    bool tin[MT];
-#pragma unroll
-    for (int t = 0; t < MT; ++t) tin[t] = T0 + t < nT;
-    i32x4 a[MT][kI8Digits], an[MT][kI8Digits], ur[UPT];
-    auto load_a = [&](int c, i32x4 (&dst)[MT][kI8Digits]) {
-#pragma unroll
-        for (int t = 0; t < MT; ++t)
-#pragma unroll
-            for (int p = 0; p < kI8Digits; ++p)
-                dst[t][p] = tin[t] ? Bq[(((size_t)(T0 + t) * nC + c) * kI8Digits + p) * kI8Op + lane]
-                                   : i32x4{0, 0, 0, 0};
+        for (int p = 0; p < kI8Digits; ++p) dst[p] = __builtin_nontemporal_load(s + p * kI8Op);
     };
     auto load_u = [&](int c) {
+        const i32x4* s = Uq + (size_t)min(c, nC - 1) * (kI8DigitsU * 4 * kI8Op) + threadIdx.x;
 #pragma unroll
-        for (int i = 0; i < UPT; ++i) ur[i] = Uq[(size_t)c * (kI8DigitsU * 4 * kI8Op) + threadIdx.x + i * kBlock];
+        for (int i = 0; i < UPT; ++i) ur[i] = s[i * 64 * NW];
     };
-    auto store_u = [&](int buf) {
+    auto store_u = [&](int c) {
 #pragma unroll
-        for (int i = 0; i < UPT; ++i) us[buf][threadIdx.x + i * kBlock] = ur[i];
+        for (int i = 0; i < UPT; ++i)
+            us[(c - cb) & 1][threadIdx.x + i * 64 * NW] = c < ce ? ur[i] : i32x4{0, 0, 0, 0};
     };
-    auto mfmas = [&](const i32x4 (&av)[MT][kI8Digits], int buf) {
+    // U's operand of step (u, q) is read two steps ahead; the scheduling barriers keep
+    // the compiler from reading all 24 at once, which spills
+    auto mfmas = [&](const Ops& av, int buf) {
+        const i32x4* ul = us[buf] + lane;
+        auto at = [&](int i) { return ul[((i % kI8DigitsU) * 4 + i / kI8DigitsU) * kI8Op]; };
+        constexpr int kSteps = 4 * kI8DigitsU;
+        i32x4 bq[3];
+        bq[0] = at(0);
+        bq[1] = at(1);
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+        for (int i = 0; i < kSteps; ++i) {
+            if (i + 2 < kSteps) bq[(i + 2) % 3] = at(i + 2);
+            const int u = i / kI8DigitsU, q = i % kI8DigitsU;
 #pragma unroll
-            for (int q = 0; q < kI8DigitsU; ++q) {
-                const i32x4 bq = us[buf][(q * 4 + u) * kI8Op + lane];
-#pragma unroll
-                for (int t = 0; t < MT; ++t)
-#pragma unroll
-                    for (int p = 0; p < kI8Digits && p + q <= kI8MaxD; ++p)
-                        acc[p + q][t][u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[t][p], bq, acc[p + q][t][u], 0, 0, 0);
-            }
-    };
-    if (ncc > 0) {
-        load_u(cb);
-        load_a(cb, an);
-        store_u(0);
-    }
-    __syncthreads();
-    for (int c = 0; c < ncc; ++c) {
-#pragma unroll
-        for (int t = 0; t < MT; ++t)
-#pragma unroll
-            for (int p = 0; p < kI8Digits; ++p) a[t][p] = an[t][p];
-        const bool more = c + 1 < ncc;
-        if (more) {
-            load_u(cb + c + 1);
-            load_a(cb + c + 1, an);
+            for (int p = 0; p < kI8Digits && p + q <= kI8MaxD; ++p)
+                acc[p + q][u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[p], bq[i % 3], acc[p + q][u], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        mfmas(a, c & 1);
-        if (more) store_u((c + 1) & 1);  // that buffer was last read in chunk c-1
+    };
+    Ops a[3];
+    load_u(cb);
+    load_a(cb, a[0]);
+    load_a(cb + 1, a[1]);
+    store_u(cb);
+    __syncthreads();
+    // chunk c from `now`, chunk c + 2 on its way into `next2`
+    auto step = [&](int c, const Ops& now, Ops& next2) {
+        load_u(c + 1);
+        load_a(c + 2, next2);
+        mfmas(now, (c - cb) & 1);
+        store_u(c + 1);  // that buffer was last read in chunk c - 1
         __syncthreads();
+    };
+    for (int c = cb; c < ce; c += 3) {  // chunks past ce add nothing (zero digits of U)
+        step(c, a[0], a[2]);
+        step(c + 1, a[1], a[0]);
+        step(c + 2, a[2], a[1]);
     }
+    if (T >= nT) return;
     double* out = P + (size_t)blockIdx.y * b * 64;
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+        for (int r = 0; r < 4; ++r) {
+            const int row = T * 16 + 4 * (lane >> 4) + r;
+            double v = 0.0;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = (T0 + t) * 16 + 4 * (lane >> 4) + r;
-                double v = 0.0;
-#pragma unroll
-                for (int d = kI8MaxD; d >= 0; --d) v = v * (1.0 / 128.0) + (double)acc[d][t][u][r];
-                if (tin[t] && row < b) out[(size_t)row * 64 + u * 16 + (lane & 15)] = v;
-            }
+            for (int d = kI8MaxD; d >= 0; --d) v = v * (1.0 / 128.0) + (double)acc[d][u][r];
+            if (row < b) out[(size_t)row * 64 + u * 16 + (lane & 15)] = v;
+        }
 }
 
 // out[bn[j]][s] = sigma_j tau_s 2^-12 sum_ks P[ks][j][s] (s < S); without bn: out[j][s]
@@ -2048,12 +2054,12 @@ __global__ __launch_bounds__(kBlock) void k_b_i8_finish(int b, int S, int nks, c
     }
 }
 
-void launch_gemm_i8(int mt, dim3 g, hipStream_t s, int b, int nT, int nC, int cper, const i32x4* Bq,
+void launch_gemm_i8(int nw, dim3 g, hipStream_t s, int b, int nT, int nC, int cper, const i32x4* Bq,
                     const i32x4* Uq, double* P) {
-    if (mt == 2)
-        hipLaunchKernelGGL(k_b_gemm_i8<2>, g, dim3(kBlock), 0, s, b, nT, nC, cper, Bq, Uq, P);
+    if (nw == 8)
+        hipLaunchKernelGGL(k_b_gemm_i8<8>, g, dim3(512), 0, s, b, nT, nC, cper, Bq, Uq, P);
     else
-        hipLaunchKernelGGL(k_b_gemm_i8<1>, g, dim3(kBlock), 0, s, b, nT, nC, cper, Bq, Uq, P);
+        hipLaunchKernelGGL(k_b_gemm_i8<4>, g, dim3(256), 0, s, b, nT, nC, cper, Bq, Uq, P);
 }
 
 __global__ __launch_bounds__(kBlock) void k_b_to_float(size_t tot, const double* __restrict__ a,
@@ -3053,7 +3059,7 @@ struct tm_batch {
     // maxima, the split-K partials, and the tuned tile rows / K split
     DevBuf<int> Bq, Uq;
     DevBuf<double> i8rmax, i8umax, i8P;
-    int i8nT = 0, i8nC = 0, i8mt = 1, i8ks = 1, i8candidates = 0;
+    int i8nT = 0, i8nC = 0, i8nw = 8, i8ks = 1, i8candidates = 0;
     float i8ms = 0.0f, i8ms_first = 0.0f;
     DevBuf<double> rk_k[4], rk_base;   // RK4 stages and the step's start state
     // graph-replayed RK4 steps: samples whose fixed-budget solve missed the
@@ -3371,10 +3377,13 @@ int tune_gemm(tm_batch* bt) {
 // ---- int8 digit-slice boundary product: set-up, tuning, one product --------
 inline const i32x4* i8ops(const DevBuf<int>& q) { return reinterpret_cast<const i32x4*>(q.p); }
 
-int i8_gemm(tm_batch* bt, int mt, int ks) {
-    const int cper = (bt->i8nC + ks - 1) / ks;
-    const dim3 g((bt->i8nT + 4 * mt - 1) / (4 * mt), ks);
-    launch_gemm_i8(mt, g, bt->stream, bt->cv.bnx, bt->i8nT, bt->i8nC, cper, i8ops(bt->Bq), i8ops(bt->Uq), bt->i8P.p);
+// chunks per K range: a multiple of the kernel's three register sets
+inline int i8_range(int nC, int ks) { return ((nC + ks - 1) / ks + 2) / 3 * 3; }
+
+int i8_gemm(tm_batch* bt, int nw, int ks) {
+    const int cper = i8_range(bt->i8nC, ks);
+    const dim3 g((bt->i8nT + nw - 1) / nw, ks);
+    launch_gemm_i8(nw, g, bt->stream, bt->cv.bnx, bt->i8nT, bt->i8nC, cper, i8ops(bt->Bq), i8ops(bt->Uq), bt->i8P.p);
     TM_HIP(hipGetLastError());
     return TM_OK;
 }
@@ -3395,7 +3404,7 @@ int i8_uslice(tm_batch* bt, const int* bn, const double* u) {
 int i8_product(tm_batch* bt, const int* bn, const double* u, double* out) {
     TM_CHECK(i8_uslice(bt, bn, u));
     bt->live_mark(0);
-    TM_CHECK(i8_gemm(bt, bt->i8mt, bt->i8ks));
+    TM_CHECK(i8_gemm(bt, bt->i8nw, bt->i8ks));
     bt->live_mark(1);
     hipLaunchKernelGGL(k_b_i8_finish, dim3(elem_grid((size_t)bt->cv.bnx * 64)), dim3(kBlock), 0, bt->stream,
                        bt->cv.bnx, bt->S, bt->i8ks, bn, (const double*)bt->i8P.p, (const double*)bt->i8rmax.p,
@@ -3404,11 +3413,10 @@ int i8_product(tm_batch* bt, const int* bn, const double* u, double* out) {
     return TM_OK;
 }
 
-constexpr int kI8Splits[] = {1, 2, 3, 4, 6, 8};
+constexpr int kI8Splits[] = {1, 2, 3, 4, 5, 6, 7, 8};
 constexpr int kI8MaxSplit = 8;
 
-// B's digits (once per batch), then the tile rows (1 or 2 tiles of 16 per
-// wavefront) and K split by timing each candidate on the digits of a
+// B's digits (once per batch), then the block size (4 or 8 wavefronts of 16 rows) and K split by timing each candidate on the digits of a
 // non-zero U
 int i8_setup(tm_batch* bt) {
     const CtxView& v = bt->cv;
@@ -3440,23 +3448,23 @@ int i8_setup(tm_batch* bt) {
     // rounds in which the clock has settled under the MFMA load; a single
     // launch's time varies by a few per cent
     struct Cand {
-        int mt, ks;
+        int nw, ks;
         float ms;
         std::vector<float> t;
     };
     std::vector<Cand> cands;
-    for (int mt = 1; mt <= 2; ++mt)
+    for (int nw = 4; nw <= 8; nw += 4)
         for (int ks : kI8Splits) {
-            const int cper = (bt->i8nC + ks - 1) / ks;
+            const int cper = i8_range(bt->i8nC, ks);
             if (ks > bt->i8nC || (size_t)cper * 64 > (size_t)kI8MaxK) continue;  // int32 bound per K range
-            cands.push_back({mt, ks, 1e30f, {}});
+            cands.push_back({nw, ks, 1e30f, {}});
         }
     const int cand = (int)cands.size();
     for (int round = 0; round < 2; ++round)
         for (Cand& c : cands)
             for (int r = 0; r < 5; ++r) {
                 (void)hipEventRecord(e0, s);
-                if (i8_gemm(bt, c.mt, c.ks) != TM_OK) break;
+                if (i8_gemm(bt, c.nw, c.ks) != TM_OK) break;
                 (void)hipEventRecord(e1, s);
                 if (hipEventSynchronize(e1) != hipSuccess) break;
                 float ms = 0.0f;
@@ -3473,7 +3481,7 @@ int i8_setup(tm_batch* bt) {
     for (const Cand& c : cands)
         if (c.ms < best) {
             best = c.ms;
-            bt->i8mt = c.mt;
+            bt->i8nw = c.nw;
             bt->i8ks = c.ks;
         }
     if (cand > 0) bt->i8ms_first = cands[0].ms;
@@ -4130,8 +4138,8 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
 int tm_batch_gemm_info(tm_batch* bt, int* solution, int* own_kernel, int* candidates, double* ms_default,
                        double* ms_tuned, int* ksplit) {
     if (!bt) return TM_ERR_BAD_ARG;
-    if (bt->prec == TM_PREC_MIXED_BEMI8) {  // k_b_gemm_i8: solution = row tiles per wavefront
-        if (solution) *solution = bt->i8mt;
+    if (bt->prec == TM_PREC_MIXED_BEMI8) {  // k_b_gemm_i8: solution = wavefronts per block
+        if (solution) *solution = bt->i8nw;
         if (own_kernel) *own_kernel = 1;
         if (candidates) *candidates = bt->i8candidates;
         if (ksplit) *ksplit = bt->i8ks;
@@ -4192,7 +4200,7 @@ int tm_batch_time_kernels(tm_batch* bt, int reps, tm_batch_kernel_time* out, int
         // B's digit slices once, U's digits and the FP64 partials
         const double bytes = (double)bt->i8nT * bt->i8nC * kI8Digits * 1024.0 +
                              (double)bt->i8nC * kI8DigitsU * 4 * 1024.0 + 8.0 * bt->i8ks * bt->cv.bnx * 64.0;
-        add("boundary GEMM (k_b_gemm_i8, int8 digits, tuned)", timeit([&] { (void)i8_gemm(bt, bt->i8mt, bt->i8ks); }),
+        add("boundary GEMM (k_b_gemm_i8, int8 digits, tuned)", timeit([&] { (void)i8_gemm(bt, bt->i8nw, bt->i8ks); }),
             bytes);
     } else if (bt->prec != TM_PREC_MIXED_BEM32) {
         const double bb = (double)bt->cv.bnx;
