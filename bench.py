@@ -536,8 +536,8 @@ def main():
             ops = 20 * flops  # digit products with p + q <= 5 (5 digits of B, 6 of U)
             result["roofline"] = {"bound": "hbm",
                                   "kernel": "k_b_gemm_i8 (int8 digit slices of B and U, 20 digit products, "
-                                            "%d row tile(s) of 16 per wavefront, K split %d)"
-                                            % (gt.get("solution", 1), gt.get("ksplit", 1)),
+                                            "%d wavefronts of 16 rows per block, K split %d)"
+                                            % (gt.get("solution", 8), gt.get("ksplit", 1)),
                                   "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
                                   "traffic": measured_i8_traffic(prob.name, b),
                                   "algorithmic_bytes": alg, "kernel_ms": ms_k,

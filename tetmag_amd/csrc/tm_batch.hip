@@ -1627,21 +1627,23 @@ __global__ __launch_bounds__(kBlock) void k_b_scatter(int b, int S, const int* _
 // of the split; U^T chunks of KGK rows are staged in LDS.
 // v_mfma_f64_16x16x4f64 operand layout (measured): A lane l = A[l%16][l/16],
 // B lane l = B[l/16][l%16], D lane l register r = C[4r + l/16][l%16].
-// PIPE = false: per chunk, stage U^T, then load the chunk's B values and run
-// its MFMAs.  PIPE = true: software-pipelined; while the MFMAs of chunk c
-// run, the B values of chunk c+1 are in flight into registers and its U^T
-// rows into registers, stored to the other of two LDS buffers afterwards
-// (one barrier per chunk).
+// Software-pipelined: while the MFMAs of chunk c run, its successor's U^T rows
+// are in flight into registers, stored to the other of two LDS buffers
+// afterwards (one barrier per chunk), and the B values of chunks c + 1 and c + 2
+// into a rotation of three register sets.  No load depends on a condition: rows
+// and columns past the last load the last one, U^T past the range's end is zero.
+// Bound by the FP64 matrix cores under their power limit (54 TFLOP/s is what
+// the library's best kernel sustains at 40,962 boundary nodes): 64 samples, 10,242
+// boundary nodes 0.258 -> 0.245 ms, 9,602 0.226 -> 0.220 against masked loads one chunk ahead.
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 
-template <int KGK, int MT, bool PIPE>
+template <int KGK, int MT>
 __global__ __launch_bounds__(kBlock) void k_b_gemm64(int b, int ld, const double* __restrict__ B,
                                                      const double* __restrict__ U, int kper,
                                                      double* __restrict__ P) {
-    constexpr int NB = PIPE ? 2 : 1;
     constexpr int UPT = KGK * 64 / kBlock;  // U^T values per thread per chunk
     static_assert(KGK % 4 == 0 && (KGK * 64) % kBlock == 0, "chunk shape");
-    __shared__ double us[NB][KGK * 64];  // U^T chunk: us[buf][k * 64 + j]
+    __shared__ double us[2][KGK * 64];  // U^T chunk: us[buf][k * 64 + j]
     const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     const int m0 = (blockIdx.x * (kBlock / kWave) + wv) * 16 * MT;  // this wavefront's rows
     const int ks = blockIdx.y;
@@ -1654,35 +1656,34 @@ __global__ __launch_bounds__(kBlock) void k_b_gemm64(int b, int ld, const double
 #pragma unroll
         for (int u = 0; u < 4; ++u) acc[t][u] = dbl4{0.0, 0.0, 0.0, 0.0};
     int rr[MT];
-    bool ok[MT];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        rr[t] = m0 + 16 * t + li;  // the A row of this lane in tile t
-        ok[t] = rr[t] < b;
-    }
-    double a[MT][KGK / 4], an[MT][KGK / 4], ur[UPT];
-    auto load_b = [&](int k0, double (&dst)[MT][KGK / 4]) {
+    for (int t = 0; t < MT; ++t) rr[t] = min(m0 + 16 * t + li, b - 1);  // the A row of this lane in tile t
+    typedef double Vals[MT][KGK / 4];
+    double ur[UPT];
+    auto load_b = [&](int c, Vals& dst) {
+        const int k0 = kb + c * KGK;
 #pragma unroll
         for (int q = 0; q < KGK / 4; ++q) {
-            const int kc = k0 + 4 * q + lk;  // this lane's K column
-            const bool kin = kc < ke;
+            const double* col = B + (size_t)min(k0 + 4 * q + lk, b - 1) * ld;  // this lane's K column
 #pragma unroll
-            for (int t = 0; t < MT; ++t) dst[t][q] = (ok[t] && kin) ? B[(size_t)kc * ld + rr[t]] : 0.0;
+            for (int t = 0; t < MT; ++t) dst[t][q] = col[rr[t]];
         }
     };
-    auto load_u = [&](int k0) {
+    auto load_u = [&](int c) {
 #pragma unroll
         for (int i = 0; i < UPT; ++i) {
             const int t = threadIdx.x + i * kBlock;
-            const int kk = k0 + t / 64;
-            ur[i] = kk < ke ? U[(size_t)kk * 64 + (t & 63)] : 0.0;
+            ur[i] = U[(size_t)min(kb + c * KGK + t / 64, b - 1) * 64 + (t & 63)];
         }
     };
-    auto store_u = [&](int buf) {
+    auto store_u = [&](int c) {
 #pragma unroll
-        for (int i = 0; i < UPT; ++i) us[buf][threadIdx.x + i * kBlock] = ur[i];
+        for (int i = 0; i < UPT; ++i) {
+            const int t = threadIdx.x + i * kBlock;
+            us[c & 1][t] = kb + c * KGK + t / 64 < ke ? ur[i] : 0.0;
+        }
     };
-    auto mfmas = [&](const double (&av)[MT][KGK / 4], int buf) {
+    auto mfmas = [&](const Vals& av, int buf) {
 #pragma unroll
         for (int q = 0; q < KGK / 4; ++q) {
 #pragma unroll
@@ -1694,37 +1695,24 @@ __global__ __launch_bounds__(kBlock) void k_b_gemm64(int b, int ld, const double
             }
         }
     };
-    if constexpr (PIPE) {
-        if (nc > 0) {
-            load_u(kb);
-            load_b(kb, an);
-            store_u(0);
-        }
+    Vals a[3];
+    load_u(0);
+    load_b(0, a[0]);
+    load_b(1, a[1]);
+    store_u(0);
+    __syncthreads();
+    // chunk c from `now`, chunk c + 2 on its way into `next2`
+    auto step = [&](int c, const Vals& now, Vals& next2) {
+        load_u(c + 1);
+        load_b(c + 2, next2);
+        mfmas(now, c & 1);
+        store_u(c + 1);  // that buffer was last read in chunk c - 1
         __syncthreads();
-        for (int c = 0; c < nc; ++c) {
-#pragma unroll
-            for (int t = 0; t < MT; ++t)
-#pragma unroll
-                for (int q = 0; q < KGK / 4; ++q) a[t][q] = an[t][q];
-            const bool more = c + 1 < nc;
-            if (more) {  // next chunk's loads in flight during this chunk's MFMAs
-                load_u(kb + (c + 1) * KGK);
-                load_b(kb + (c + 1) * KGK, an);
-            }
-            mfmas(a, c & 1);
-            if (more) store_u((c + 1) & 1);  // that buffer was last read in chunk c-1
-            __syncthreads();
-        }
-    } else {
-        for (int c = 0; c < nc; ++c) {
-            const int k0 = kb + c * KGK;
-            __syncthreads();  // the previous chunk has been consumed
-            load_u(k0);
-            store_u(0);
-            __syncthreads();
-            load_b(k0, a);  // all of the chunk's B loads in flight before its MFMAs
-            mfmas(a, 0);
-        }
+    };
+    for (int c = 0; c < nc; c += 3) {  // chunks past the last add nothing
+        step(c, a[0], a[2]);
+        step(c + 1, a[1], a[0]);
+        step(c + 2, a[2], a[1]);
     }
     double* out = P + (size_t)ks * b * 64;
 #pragma unroll
@@ -1740,11 +1728,8 @@ __global__ __launch_bounds__(kBlock) void k_b_gemm64(int b, int ld, const double
 
 struct GemmShape {
     int kgk, mt;
-    bool pipe;
 };
-constexpr GemmShape kGemmShapes[] = {{32, 2, false}, {64, 2, false}, {32, 2, true}, {16, 2, true},
-                                     {16, 4, true},  {32, 4, true},  {8, 2, true},  {8, 4, true},
-                                     {16, 1, true},  {32, 1, true}};
+constexpr GemmShape kGemmShapes[] = {{16, 2}, {32, 2}, {8, 2}, {16, 4}, {8, 4}, {16, 1}, {32, 1}};
 constexpr int kNumGemmShapes = sizeof(kGemmShapes) / sizeof(kGemmShapes[0]);
 
 inline int gemm_rows_per_block(int shape) { return (kBlock / kWave) * 16 * kGemmShapes[shape].mt; }
@@ -1752,16 +1737,13 @@ inline int gemm_rows_per_block(int shape) { return (kBlock / kWave) * 16 * kGemm
 template <class F>
 void gemm_dispatch(int shape, F&& f) {
     switch (shape) {
-        case 0: f(k_b_gemm64<32, 2, false>); break;
-        case 1: f(k_b_gemm64<64, 2, false>); break;
-        case 2: f(k_b_gemm64<32, 2, true>); break;
-        case 3: f(k_b_gemm64<16, 2, true>); break;
-        case 4: f(k_b_gemm64<16, 4, true>); break;
-        case 5: f(k_b_gemm64<32, 4, true>); break;
-        case 6: f(k_b_gemm64<8, 2, true>); break;
-        case 7: f(k_b_gemm64<8, 4, true>); break;
-        case 8: f(k_b_gemm64<16, 1, true>); break;
-        default: f(k_b_gemm64<32, 1, true>); break;
+        case 0: f(k_b_gemm64<16, 2>); break;
+        case 1: f(k_b_gemm64<32, 2>); break;
+        case 2: f(k_b_gemm64<8, 2>); break;
+        case 3: f(k_b_gemm64<16, 4>); break;
+        case 4: f(k_b_gemm64<8, 4>); break;
+        case 5: f(k_b_gemm64<16, 1>); break;
+        default: f(k_b_gemm64<32, 1>); break;
     }
 }
 
