@@ -72,3 +72,31 @@ def test_inner_solve_tiles_match_fp64(gpu_available, ny):
             assert worst < 1e-8
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("prec", ["FP64", "MIXED"])
+@pytest.mark.parametrize("S, nx, ny, nz", [(1, 13, 11, 5), (16, 20, 20, 4), (17, 20, 20, 4), (63, 13, 11, 5), (40, 40, 30, 9)])
+def test_coarsest_level_product(gpu_available, S, nx, ny, nz, prec):
+    """Sample counts at and off the 16 of a block, coarsest levels reached from
+    the first and from the second level.  Solves to 1e-13 on both sides: fields
+    within a few thousand times that in FP64, 1e-9; 1e-8 for the mixed form
+    (the bound of its other tests)."""
+    from tetmag_amd import _native as N
+    from tetmag_amd import problem as P
+    from tetmag_amd.batch import BatchContext, from_batch, to_batch
+    from tetmag_amd.context import FieldContext
+    prob = P.cuboid_problem("coarse", nx, ny, nz, 3.0, 0.1, 3, P.Material())
+    ctx = FieldContext(prob, tol=1e-13)
+    try:
+        print("n", prob.n, "levels", ctx.amg_levels(0), ctx.amg_levels(1), flush=True)
+        bc = BatchContext(ctx, S, getattr(N, "TM_PREC_" + prec))
+        ms = P.smooth_random_fields(prob.mesh, S, seed=S)
+        dm, H, st = bc.eval_rhs_host(to_batch(ms))
+        for s in sorted({0, S // 2, S - 1}):
+            d1, h1, _ = ctx.eval_rhs_host(ms[s])
+            eh, ed = rel_l2(from_batch(H, s), h1), rel_l2(from_batch(dm, s), d1)
+            print("S", S, prec, "sample", s, eh, ed, flush=True)
+            assert max(eh, ed) < (1e-9 if prec == "FP64" else 1e-8)
+        bc.close()
+    finally:
+        ctx.close()

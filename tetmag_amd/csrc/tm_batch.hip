@@ -757,43 +757,6 @@ __global__ __launch_bounds__(kBlock) void k_b_spmm_w(SlotArgs M, const float* __
     wide_walk<BLK>(M, x, ld, epi);
 }
 
-// x = C b for the dense coarse inverse (row-major nc x nc): one row per block,
-// its columns dealt to the 4 wavefronts in 16-column chunks (C's entries are
-// wavefront-uniform scalar loads), the wavefronts' sums added in LDS.
-constexpr int kDenseCh = 16;
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_b_dense(int nc, int S, const double* __restrict__ C,
-                                                    const T* __restrict__ b, T* __restrict__ x,
-                                                    const int* gate) {
-    if (!any_active(gate, S)) return;
-    const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
-    const int lc = min(lane, S - 1);
-    const cw_p<double> Cc = (cw_p<double>)C;
-    __shared__ double red[kRowsPerBlock][kWave];
-    for (int row = blockIdx.x; row < nc; row += gridDim.x) {  // block-uniform
-        double acc = 0.0;
-        for (int k0 = kDenseCh * wv; k0 < nc; k0 += kDenseCh * kRowsPerBlock) {
-            double cv[kDenseCh], bv[kDenseCh];
-#pragma unroll
-            for (int k = 0; k < kDenseCh; ++k) {
-                const int kk = min(k0 + k, nc - 1);
-                cv[k] = Cc[(size_t)row * nc + kk];
-                bv[k] = (double)b[(size_t)kk * S + lc];
-            }
-#pragma unroll
-            for (int k = 0; k < kDenseCh; ++k) acc = k0 + k < nc ? acc + cv[k] * bv[k] : acc;
-        }
-        red[wv][lane] = acc;
-        __syncthreads();
-        if (wv == 0 && lane < S) {
-            double t = red[0][lane];
-            for (int k = 1; k < kRowsPerBlock; ++k) t += red[k][lane];
-            x[(size_t)row * S + lane] = (T)t;
-        }
-        __syncthreads();
-    }
-}
-
 // ------------------------------------------------------ fields and LLG --
 // The per-node operators (exchange, grad, tGrad, curl) share the union
 // pattern, stored in row slots (SlotArgs) with FP64-row offsets; the slot
@@ -1600,6 +1563,78 @@ __global__ __launch_bounds__(kTileThreads, 2 * kSolvePerCu) void k_b_up_t(TileAr
             for (int c = 0; c < 4; ++c) v[c] += (double)ri[c] * (double)acc[c];
         });
     tile_partial4(lds, part, v);
+}
+
+// y = M x for a dense M (row-major, m columns; the V-cycle's coarsest level),
+// R rows and 16 VEC samples per block: the columns are dealt in chunks of 16 to
+// the block's 32 groups of 16 lanes, lane j holds M's entries of column j and
+// passes them on by DPP, so that a chunk costs its 16 rows of x and one load per
+// row of M; the groups' sums are added across lanes and in LDS.  Bound by the
+// texture unit (17 loads per chunk) where a block per CU covers the rows, so a
+// second row per block is free beyond that (R = 2 for more than 256 blocks).
+// With M = C^-1 R (I - A w D^-1) (the single-sample solver's, up to 2^20 entries) it
+// takes the place of the last restriction and of the product with C^-1: 24 FP64
+// samples at 38,025 nodes 1.49 -> 1.36 ms per evaluation, 7 samples at 2,205
+// nodes 11.1 -> 5.5 us per V-cycle.  64 FP32 samples keep the two products: the
+// FP64 sums over the restriction's columns cost more there (152 x 2,216: 15.3 us)
+// than the restriction in FP32 and C^-1 (10.4).
+constexpr int kDmvThreads = 512;
+template <typename T, int VEC, int R>
+__global__ __launch_bounds__(kDmvThreads) void k_b_dmv(int rows, int m, int S, const double* __restrict__ M,
+                                                       const T* __restrict__ x, T* __restrict__ y, const int* gate) {
+    if (!any_active(gate, S)) return;
+    typedef T Vec __attribute__((ext_vector_type(VEC)));
+    using Lane = std::conditional_t<VEC == 1, T, Vec>;
+    constexpr int kWaves = kDmvThreads / kWave;
+    __shared__ double red[kWaves][R][16 * VEC];
+    const int j = threadIdx.x & 15, g = threadIdx.x / 16;
+    const int r0 = blockIdx.x * R, s = (blockIdx.y * 16 + j) * VEC, sc = min(s, S - VEC);
+    double acc[R][VEC];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) acc[r][v] = 0.0;
+    for (int k0 = g * 16; k0 < m; k0 += kDmvThreads) {
+        double w[R];
+        Lane xv[16];
+#pragma unroll
+        for (int r = 0; r < R; ++r) w[r] = M[(size_t)min(r0 + r, rows - 1) * m + min(k0 + j, m - 1)];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) xv[k] = *(const Lane*)(x + (size_t)min(k0 + k, m - 1) * S + sc);
+        if (k0 + j >= m)
+#pragma unroll
+            for (int r = 0; r < R; ++r) w[r] = 0.0;
+        each16(
+            [&](auto kk) {
+                constexpr int K = decltype(kk)::value;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const double ww = bcast16<K>(w[r]);
+                    if constexpr (VEC == 1) acc[r][0] += ww * (double)xv[K];
+                    else
+#pragma unroll
+                        for (int v = 0; v < VEC; ++v) acc[r][v] += ww * (double)xv[K][v];
+                }
+            },
+            std::make_integer_sequence<int, 16>{});
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) {
+            double a = acc[r][v];
+            a += __shfl_xor(a, 16);
+            a += __shfl_xor(a, 32);
+            if ((threadIdx.x & (kWave - 1)) < 16) red[threadIdx.x / kWave][r][j * VEC + v] = a;
+        }
+    __syncthreads();
+    for (int e = threadIdx.x; e < R * 16 * VEC; e += kDmvThreads) {
+        const int r = e / (16 * VEC), q = e % (16 * VEC), sq = (int)blockIdx.y * 16 * VEC + q;
+        double a = 0.0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) a += red[w][r][q];
+        if (r0 + r < rows && sq < S) y[(size_t)(r0 + r) * S + sq] = (T)a;
+    }
 }
 
 // U[j][s] = u[bn[j]][s]  (S x b column-major, ld S)
@@ -2612,8 +2647,10 @@ struct BatchSolver {
             const int nnext = l + 1 < L ? M.levels[l + 1].n : M.nc;
             HostCsr down, up;
             TM_CHECK(fetch_csr(V.down, down, s));
-            TM_CHECK(lo[l].RA.build(nnext, V.n, down.rp.data(), down.ci.data(), S, s));
-            TM_CHECK(lo[l].RA.values(down.v, lo[l].wRA, s));
+            if (l + 1 < L || !fold()) {
+                TM_CHECK(lo[l].RA.build(nnext, V.n, down.rp.data(), down.ci.data(), S, s));
+                TM_CHECK(lo[l].RA.values(down.v, lo[l].wRA, s));
+            }
             if (l == 0) {
                 up_operator(n, solver.pat.h_rowptr.data(), solver.pat.h_csrcol.data(), solver.h_val,
                             solver.h_dinv.data(), V.omega, down, up);
@@ -2660,16 +2697,34 @@ struct BatchSolver {
         if (L == 0) return TM_ERR_UNSUPPORTED;  // the batched solve needs at least one AMG level
         auto vec = [&](int l) { return l == 0 ? r : bx[l].p; };  // [b | x_c] of level l
         auto tail = [&](int l) { return vec(l) + (size_t)M.levels[l].n * S; };
-        for (int l = 0; l < L; ++l) {
-            const LvOps& O = lo[l];
-            spmm(O.RA, O.wRA.p, vec(l), l + 1 < L ? vec(l + 1) : bc.p, s);
-        }
-        hipLaunchKernelGGL((k_b_dense<T>), dim3(std::max(1, std::min(M.nc, 4096))), dim3(kBlock), 0, s, M.nc, S,
-                           M.Cinv.p, (const T*)bc.p, tail(L - 1), gate());
+        const bool dense = fold();
+        for (int l = 0; l < (dense ? L - 1 : L); ++l)
+            spmm(lo[l].RA, lo[l].wRA.p, vec(l), l + 1 < L ? vec(l + 1) : bc.p, s);
+        if (dense) dmv(M.nc, M.levels[L - 1].n, M.D.p, vec(L - 1), tail(L - 1), s);
+        else dmv(M.nc, M.nc, M.Cinv.p, bc.p, tail(L - 1), s);
         for (int l = L - 1; l > 0; --l) spmm(lo[l].U, lo[l].wU.p, vec(l), tail(l - 1), s);
         up0(r, zout, prz, s);
         TM_HIP(hipGetLastError());
         return TM_OK;
+    }
+
+    // C^-1 folded into the last restriction (see k_b_dmv for the line)
+    bool fold() const { return cg->amg.D.p != nullptr && !wide(); }
+    // y = D x, dense
+    void dmv(int rows, int m, const double* D, const T* x, T* y, hipStream_t s) {
+        auto run = [&](auto vec) {
+            constexpr int VEC = decltype(vec)::value;
+            const int nch = (S + 16 * VEC - 1) / (16 * VEC);
+            if (rows * nch <= 256)
+                hipLaunchKernelGGL((k_b_dmv<T, VEC, 1>), dim3(rows, nch), dim3(kDmvThreads), 0, s, rows, m, S, D, x, y,
+                                   gate());
+            else
+                hipLaunchKernelGGL((k_b_dmv<T, VEC, 2>), dim3((rows + 1) / 2, nch), dim3(kDmvThreads), 0, s, rows, m,
+                                   S, D, x, y, gate());
+        };
+        if constexpr (kWideT)
+            if (wide()) return run(std::integral_constant<int, 4>{});
+        run(std::integral_constant<int, 1>{});
     }
 
     // level 0 upwards: z = U [r | x_c], partial (r, z)
@@ -2938,10 +2993,18 @@ struct BatchSolver {
         add(sizeof(T) == 4 ? "k_b_cg_update<float>" : "k_b_cg_update<double>",
             timeit([&] { cg_update(part.p + (size_t)S * gmax(), s); }), 3.0 * nS * e);
         const LvOps& O = lo[0];
-        const double n1 = O.RA.n;
-        T* y1 = cg->amg.levels.size() > 1 ? bx[1].p : bc.p;
-        add(O.RA.long_rows() && wide() ? "k_b_spmm_w<long> (R(I-AwD^-1), level 0)" : "k_b_spmm (R(I-AwD^-1), level 0)",
-            timeit([&] { spmm(O.RA, O.wRA.p, rT.p, y1, s); }), slots(O.RA) * (4 + e) + nS * e + n1 * S * e);
+        const AmgPrecond& M = cg->amg;
+        const double n1 = M.levels.size() > 1 ? M.levels[1].n : M.nc;
+        if (O.RA.n > 0) {
+            T* y1 = M.levels.size() > 1 ? bx[1].p : bc.p;
+            add(O.RA.long_rows() && wide() ? "k_b_spmm_w<long> (R(I-AwD^-1), level 0)"
+                                           : "k_b_spmm (R(I-AwD^-1), level 0)",
+                timeit([&] { spmm(O.RA, O.wRA.p, rT.p, y1, s); }), slots(O.RA) * (4 + e) + nS * e + n1 * S * e);
+        } else {
+            add("k_b_dmv (C^-1 R(I-AwD^-1), level 0)",
+                timeit([&] { dmv(M.nc, n, M.D.p, rT.p, rT.p + (size_t)n * S, s); }),
+                8.0 * M.nc * n + nS * e + n1 * S * e);
+        }
         add(tiled() ? "k_b_up_t (level 0)" : wide() ? "k_b_up_w (level 0)" : "k_b_up (level 0)",
             timeit([&] { up0(rT.p, ring.p, prz, s); }), slots(O.U) * (4 + e) + 2.0 * nS * e + n1 * S * e);
         double* pbb = part.p;
