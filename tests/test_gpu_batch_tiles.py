@@ -75,7 +75,7 @@ def test_inner_solve_tiles_match_fp64(gpu_available, ny):
 
 
 @pytest.mark.parametrize("prec", ["FP64", "MIXED"])
-@pytest.mark.parametrize("S, nx, ny, nz", [(1, 13, 11, 5), (16, 20, 20, 4), (17, 20, 20, 4), (63, 13, 11, 5), (40, 40, 30, 9)])
+@pytest.mark.parametrize("S, nx, ny, nz", [(1, 13, 11, 5), (16, 20, 20, 4), (17, 20, 20, 4), (63, 13, 11, 5), (40, 40, 30, 9), (33, 40, 30, 9)])
 def test_coarsest_level_product(gpu_available, S, nx, ny, nz, prec):
     """Sample counts at and off the 16 of a block, coarsest levels reached from
     the first and from the second level.  Solves to 1e-13 on both sides: fields

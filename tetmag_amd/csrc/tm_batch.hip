@@ -692,20 +692,6 @@ __global__ void k_b_red_rz(int G, int S, const double* part_rz, int k, BState* b
 }
 
 // --------------------------------------------------------- AMG V-cycle --
-// y = M x
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_b_spmm(SlotArgs M, int S, const T* __restrict__ x, T* __restrict__ y) {
-    if (!any_active(M.gate, M.gate_n)) return;
-    const int lane = threadIdx.x & (kWave - 1);
-    const bool on = lane < S;
-    const int lc = min(lane, S - 1);
-    auto ld = [&](int) { return (T)0; };
-    auto epi = [&](int row, T acc, T) {
-        if (on) y[(size_t)row * S + lane] = acc;
-    };
-    slot_walk<T, T, kRowsPerStep<T>>(M, x, lc, ld, epi);
-}
-
 // Level 0 upwards: z = U [r | x_c] (r's tail holds the coarse correction), and
 // the partial (r, z).  One product with U = [2 w D^-1 - w D^-1 A w D^-1 | Q] in
 // place of the prolongation (x = w D^-1 r + P x_c, written and gathered again) and
@@ -1058,27 +1044,39 @@ __device__ inline void tile_walk(const TileArgs& t, const typename TT::T* m, siz
     }
 }
 
-// 64 FP32 samples: the block's sums v (four samples per lane) to
-// part[s * gridDim.x + block], through the walk's LDS
-using TileF64 = TileType<float, 4, true>;
-constexpr int kTileFloats = kTileNodes * 64;
-__device__ inline void tile_partial4(float* lds, double* part, const double (&v)[4]) {
-    double* red = reinterpret_cast<double*>(lds);  // [kTileRows / 2][64]
-    static_assert(kTileFloats * 4 >= kTileRows / 2 * 64 * 8, "the partial sums of two groups at a time");
+// the c-th of a lane's samples
+template <class TT>
+__device__ inline typename TT::T lane_at(const typename TT::Lane& v, int c) {
+    if constexpr (TT::VEC == 1) return v;
+    else return v[c];
+}
+
+// The block's sums v (a lane's samples) to part[s * gridDim.x + block], zero for
+// the samples of other chunks, through the walk's LDS
+template <class TT>
+constexpr int kTileElems = kTileNodes * TT::kSamples;
+template <class TT>
+__device__ inline void tile_partial(typename TT::T* lds, double* part, int S, const double (&v)[TT::VEC], int s0) {
+    constexpr int kPerRow = TT::kSamples;
+    double* red = reinterpret_cast<double*>(lds);  // [kTileRows / 2][16 VEC]
+    static_assert(kTileElems<TT> * sizeof(typename TT::T) >= kTileRows / 2 * kPerRow * sizeof(double),
+                  "the partial sums of two groups at a time");
     const int g = threadIdx.x / 16, j = threadIdx.x & 15;
     __syncthreads();
-    double u[4];
+    double u[TT::VEC];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) u[c] = v[c] + __shfl_xor(v[c], 16);
+    for (int c = 0; c < TT::VEC; ++c) u[c] = v[c] + __shfl_xor(v[c], 16);
     if ((g & 1) == 0)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) red[(g / 2) * 64 + 4 * j + c] = u[c];
+        for (int c = 0; c < TT::VEC; ++c) red[(g / 2) * kPerRow + TT::VEC * j + c] = u[c];
     __syncthreads();
-    if (threadIdx.x >= 64) return;
+    const int sm = threadIdx.x, q = sm - s0;
+    if (sm >= S) return;
     double s = 0.0;
+    if (q >= 0 && q < kPerRow)
 #pragma unroll
-    for (int k = 0; k < kTileRows / 2; ++k) s += red[k * 64 + threadIdx.x];
-    part[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = s;
+        for (int k = 0; k < kTileRows / 2; ++k) s += red[k * kPerRow + q];
+    part[(size_t)sm * gridDim.x + blockIdx.x] = s;
 }
 
 // b = sum_d tGrad_d (Js m_d) / mu0, as k_b_div
@@ -1502,67 +1500,130 @@ __global__ __launch_bounds__(kTileThreads, 2 * kResidPerCu) void k_b_resid_t(Til
     (q == 0 ? part_bb : part_rr)[(size_t)sm * gridDim.x + blockIdx.x] = v;
 }
 
-// k_b_cg_spmv_w from tiles in LDS: 64 samples per unit, a float4 per lane.
-// Gathers from L2 are bound by the texture unit's four lanes per cycle, these by
-// LDS and the nodes' staging: at 282,897 nodes 93 -> 54 us, at 26,325 nodes
-// 11.1 -> 9.3 (also with fewer units than two per block).  Two blocks per
-// CU; at four the pipeline's registers spill (123 us).
-constexpr int kSolvePerCu = 2;
-__global__ __launch_bounds__(kTileThreads, 2 * kSolvePerCu) void k_b_cg_spmv_t(TileArgs t, const float* __restrict__ w,
-                                                                              const float* __restrict__ z,
-                                                                              float* __restrict__ q, int k,
-                                                                              const BState* bs, double* part) {
-    __shared__ float lds[kTileFloats];
+// k_b_cg_spmv and k_b_cg_spmv_w from tiles in LDS: 64 samples per unit, a float4
+// per lane, for 64 FP32 samples; 16 per unit otherwise.  Gathers from L2 are bound
+// by the texture unit's four lanes per cycle, these by LDS and the nodes' staging:
+// 64 FP32 samples at 282,897 nodes 93 -> 54 us, at 26,325 nodes 11.1 -> 9.3 (also
+// with fewer units than two per block); 24 FP64 samples at 38,025 nodes
+// 24.2 -> 12.8.  Two (float4) and three blocks per CU; at four the float4 form's
+// registers spill (123 us).
+template <class TT>
+constexpr int kSolvePerCu = TT::VEC == 1 ? 3 : 2;
+template <class TT>
+__global__ __launch_bounds__(kTileThreads, 2 * kSolvePerCu<TT>) void k_b_cg_spmv_t(
+    TileArgs t, const typename TT::T* __restrict__ w, const typename TT::T* __restrict__ z, typename TT::T* __restrict__ q,
+    int k, const BState* bs, double* part) {
+    using T = typename TT::T;
+    using Lane = typename TT::Lane;
+    constexpr int VEC = TT::VEC;
+    __shared__ T lds[kTileElems<TT>];
     if (!any_active(bs->active, kMaxS)) return;
-    const int j = threadIdx.x & 15;
-    const f4 beta = k > 0 ? f4{(float)bs->beta[4 * j], (float)bs->beta[4 * j + 1], (float)bs->beta[4 * j + 2],
-                               (float)bs->beta[4 * j + 3]}
-                          : f4{0.f, 0.f, 0.f, 0.f};
-    // k = 0: q has no earlier value; z is read in its place, times zero
-    const float* qo = k > 0 ? q : z;
-    double v[4] = {0.0, 0.0, 0.0, 0.0};
-    f4 acc, old;
-    tile_walk<TileF64, 1, 1>(
+    const int s0 = tile_chunk(t, TT::kSamples), sc = min(s0 + VEC * (int)(threadIdx.x & 15), t.S - VEC);
+    Lane beta, acc = {}, old = {};
+    if constexpr (VEC == 1) {
+        beta = k > 0 ? (T)bs->beta[sc] : (T)0;
+    } else {
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) beta[c] = k > 0 ? (T)bs->beta[sc + c] : (T)0;
+    }
+    // k = 0: q has no earlier value; z is read in its place and left out
+    const T* qo = k > 0 ? q : z;
+    double v[VEC] = {};
+    tile_walk<TT, 1, 1>(
         t, z, 0, z, {w}, lds,
         [&](const TileRow& r) {
-            acc = f4{0.f, 0.f, 0.f, 0.f};
-            old = *(const f4*)(qo + (size_t)r.row * 64 + 4 * j);
+            acc = Lane{};
+            old = *(const Lane*)(qo + (size_t)r.row * t.S + sc);
         },
-        [&](const f4 (&x)[1], const float (&ww)[1]) { acc += ww[0] * x[0]; },
-        [&](const TileRow& r, const float* tile, bool on) {
+        [&](const Lane (&x)[1], const T (&ww)[1]) { acc += ww[0] * x[0]; },
+        [&](const TileRow& r, const T* tile, bool on) {
             if (!on) return;
-            const f4 zi = *(const f4*)(tile + (r.more & 0xffff) * 64 + 4 * j);
-            const f4 qi = k > 0 ? acc + beta * old : acc;
-            *(f4*)(q + (size_t)r.row * 64 + 4 * j) = qi;
+            const Lane zi = *(const Lane*)(tile + (r.more & 0xffff) * TT::kSamples + VEC * (int)(threadIdx.x & 15));
+            const Lane qi = k > 0 ? acc + beta * old : acc;
+            *(Lane*)(q + (size_t)r.row * t.S + sc) = qi;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) v[c] += (double)zi[c] * (double)qi[c];
+            for (int c = 0; c < VEC; ++c) v[c] += (double)lane_at<TT>(zi, c) * (double)lane_at<TT>(qi, c);
         });
-    tile_partial4(lds, part, v);
+    tile_partial<TT>(lds, part, t.S, v, s0);
 }
 
-// k_b_up_w from tiles in LDS (rows of about 27 entries: two chunks of slots):
-// 101 us at 282,897 nodes and 64 samples, where prolongation and post-smoothing
-// took 49 + 88 from L2; 12.3 -> 9.9 against k_b_up_w at 26,325 nodes
-__global__ __launch_bounds__(kTileThreads, 2 * kSolvePerCu) void k_b_up_t(TileArgs t, const float* __restrict__ w,
-                                                                         const float* __restrict__ r,
-                                                                         float* __restrict__ z, const int* gate,
-                                                                         double* part) {
-    __shared__ float lds[kTileFloats];
+// k_b_up and k_b_up_w from tiles in LDS (rows of about 27 entries: two chunks of
+// slots): 64 FP32 samples at 282,897 nodes 101 us, where prolongation and
+// post-smoothing took 49 + 88 from L2; 12.3 -> 9.9 against k_b_up_w at 26,325
+// nodes; 24 FP64 samples at 38,025 nodes 41 -> 21
+template <class TT>
+__global__ __launch_bounds__(kTileThreads, 4) void k_b_up_t(TileArgs t, const typename TT::T* __restrict__ w,
+                                                            const typename TT::T* __restrict__ r,
+                                                            typename TT::T* __restrict__ z, const int* gate,
+                                                            double* part) {
+    using T = typename TT::T;
+    using Lane = typename TT::Lane;
+    constexpr int VEC = TT::VEC;
+    __shared__ T lds[kTileElems<TT>];
     if (!any_active(gate, kMaxS)) return;
-    const int j = threadIdx.x & 15;
-    double v[4] = {0.0, 0.0, 0.0, 0.0};
-    f4 acc;
-    tile_walk<TileF64, 1, 1, 2>(
-        t, r, 0, r, {w}, lds, [&](const TileRow&) { acc = f4{0.f, 0.f, 0.f, 0.f}; },
-        [&](const f4 (&g)[1], const float (&ww)[1]) { acc += ww[0] * g[0]; },
-        [&](const TileRow& row, const float* tile, bool on) {
+    const int s0 = tile_chunk(t, TT::kSamples), sc = min(s0 + VEC * (int)(threadIdx.x & 15), t.S - VEC);
+    double v[VEC] = {};
+    Lane acc = {};
+    tile_walk<TT, 1, 1, 2>(
+        t, r, 0, r, {w}, lds, [&](const TileRow&) { acc = Lane{}; },
+        [&](const Lane (&g)[1], const T (&ww)[1]) { acc += ww[0] * g[0]; },
+        [&](const TileRow& row, const T* tile, bool on) {
             if (!on) return;
-            const f4 ri = *(const f4*)(tile + (row.more & 0xffff) * 64 + 4 * j);
-            *(f4*)(z + (size_t)row.row * 64 + 4 * j) = acc;
+            const Lane ri = *(const Lane*)(tile + (row.more & 0xffff) * TT::kSamples + VEC * (int)(threadIdx.x & 15));
+            *(Lane*)(z + (size_t)row.row * t.S + sc) = acc;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) v[c] += (double)ri[c] * (double)acc[c];
+            for (int c = 0; c < VEC; ++c) v[c] += (double)lane_at<TT>(ri, c) * (double)lane_at<TT>(acc, c);
         });
-    tile_partial4(lds, part, v);
+    tile_partial<TT>(lds, part, t.S, v, s0);
+}
+constexpr int kUpPerCu = 2;
+
+// y = M x (the V-cycle's restrictions and its way up below level 0; any sample count
+// but 64 in FP32).  A row and 16 samples per wavefront, or per block of four
+// (BLK, where there are too few rows to fill the chip): its 16-slot chunks are
+// dealt to the 16-lane groups, lane j reads slot j's offset and weight and
+// passes them on by DPP.  The rows are long (60 to 180 entries) and few, so this is
+// bound by latency: with one wavefront per row and a lane per sample a row was
+// a chain of 4 to 12 chunks, and at 24 samples 40 lanes were idle.  24 FP64
+// samples at 38,025 nodes: 19.5 -> 11.2 us (1,520 rows from 38,025), 20.5 -> 5.5
+// (96 from 1,520), 12.3 -> 8.5 (up).
+template <typename T, bool BLK>
+__global__ __launch_bounds__(kBlock) void k_b_spmm(SlotArgs M, int S, const T* __restrict__ x, T* __restrict__ y) {
+    if (!any_active(M.gate, M.gate_n)) return;
+    constexpr int kGroups = BLK ? kBlock / 16 : kWave / 16;
+    const int j = threadIdx.x & 15, g = threadIdx.x / 16 % kGroups;
+    const int row = __builtin_amdgcn_readfirstlane(
+        BLK ? xcd_block() : xcd_block() * kRowsPerBlock + (int)(threadIdx.x / kWave));
+    const int s = blockIdx.y * 16 + j;
+    if (row >= M.n) return;  // (a whole block if BLK)
+    const cint_p sp = (cint_p)M.sp;
+    const int a0 = sp[row], a1 = sp[row + 1];
+    const char* xs = (const char*)(x + min(s, S - 1));
+    const T* w = (const T*)M.w;
+    T acc = 0;
+    for (int q = a0 + kSlot * g; q < a1; q += kSlot * kGroups) {
+        const int off = M.off[q + j];
+        const T ww = w[q + j];
+        T v[kSlot];
+        each16([&](auto kk) { v[decltype(kk)::value] = *(const T*)(xs + bcast16<decltype(kk)::value>(off)); },
+               std::make_integer_sequence<int, kSlot>{});
+        each16([&](auto kk) { acc += bcast16<decltype(kk)::value>(ww) * v[decltype(kk)::value]; },
+               std::make_integer_sequence<int, kSlot>{});
+    }
+    acc += __shfl_xor(acc, 16);
+    acc += __shfl_xor(acc, 32);
+    if constexpr (BLK) {
+        __shared__ T red[kRowsPerBlock][16];
+        if ((threadIdx.x & (kWave - 1)) < 16) red[threadIdx.x / kWave][j] = acc;
+        __syncthreads();
+        if (threadIdx.x >= 16) return;
+        acc = red[0][j];
+#pragma unroll
+        for (int k = 1; k < kRowsPerBlock; ++k) acc += red[k][j];
+    } else if (g != 0) {
+        return;
+    }
+    if (s < S) y[(size_t)row * S + s] = acc;
 }
 
 // y = M x for a dense M (row-major, m columns; the V-cycle's coarsest level),
@@ -2589,8 +2650,17 @@ struct BatchSolver {
     int Gr = 0;                   // partials per sample of the outer residual
     int Gq = 0, Gz = 0;           // of (z, q) and of (r, z)
     int gmax() const { return std::max(std::max(G, Gr), std::max(Gq, Gz)); }
-    // the level-0 products of the inner solve from tiles (64 FP32 samples)
-    bool tiled() const { return wide() && t0.nt > 0 && tu.nt > 0; }
+    // the level-0 products of the inner solve from tiles
+    bool tiled() const { return t0.nt > 0 && tu.nt > 0; }
+    // f(tile type) for this batch: a float4 per lane for 64 FP32 samples
+    template <class F>
+    void with_tile_type(F&& f) const {
+        if constexpr (sizeof(T) == 4) {
+            if (S == kMaxS) return f(TileType<T, 4, true>{});
+        }
+        if (S % (16 / (int)sizeof(T)) == 0) f(TileType<T, 1, true>{});
+        else f(TileType<T, 1, false>{});
+    }
     TileOp tu;                    // tiles of level 0's way up
     struct LvOps {
         SlotOp RA;                // R (I - A w D^-1): pre-smoothing from zero + restriction
@@ -2659,9 +2729,16 @@ struct BatchSolver {
             }
             TM_CHECK(lo[l].U.build(V.n, V.n + nnext, up.rp.data(), up.ci.data(), S, s));
             TM_CHECK(lo[l].U.values(up.v, lo[l].wU, s));
-            if (l == 0 && wide()) TM_CHECK(tu.build(lo[0].U, s));
+            if (l == 0) TM_CHECK(tu.build(lo[0].U, s));
         }
-        Gq = Gz = tiled() ? tile_blocks(1, kSolvePerCu) : G;
+        Gq = Gz = G;
+        if (tiled())
+            with_tile_type([&](auto tt) {
+                using TT = decltype(tt);
+                const int nch = (S + TT::kSamples - 1) / TT::kSamples;
+                Gq = tile_blocks(nch, kSolvePerCu<TT>);
+                Gz = tile_blocks(nch, kUpPerCu);
+            });
         TM_CHECK(fixed.upload(solver.h_fixed.data(), n, s));
         const size_t NS = (size_t)n * S;
         TM_CHECK(rT.alloc(NS + (size_t)M.tail() * S));
@@ -2729,12 +2806,15 @@ struct BatchSolver {
 
     // level 0 upwards: z = U [r | x_c], partial (r, z)
     void up0(const T* r, T* z, double* prz, hipStream_t s) {
+        if (tiled()) {
+            with_tile_type([&](auto tt) {
+                using TT = decltype(tt);
+                hipLaunchKernelGGL(k_b_up_t<TT>, dim3(Gz), dim3(kTileThreads), 0, s, tu.args(lo[0].U, TT::kSamples),
+                                   (const T*)lo[0].wU.p, r, z, gate(), prz);
+            });
+            return;
+        }
         if constexpr (kWideT) {
-            if (tiled()) {
-                hipLaunchKernelGGL(k_b_up_t, dim3(Gz), dim3(kTileThreads), 0, s, tu.args(lo[0].U, 64),
-                                   (const float*)lo[0].wU.p, (const float*)r, (float*)z, gate(), prz);
-                return;
-            }
             if (wide()) {
                 hipLaunchKernelGGL(k_b_up_w, dim3(G), dim3(kBlock), 0, s, gated(lo[0].U.args(4, lo[0].wU.p)),
                                    (const float*)r, (float*)z, prz);
@@ -2771,7 +2851,12 @@ struct BatchSolver {
                 else hipLaunchKernelGGL(k_b_spmm_w<false>, dim3(row_grid(a.n)), dim3(kBlock), 0, s, a, xf, yf);
                 return;
             }
-        hipLaunchKernelGGL((k_b_spmm<T>), dim3(row_grid(a.n)), dim3(kBlock), 0, s, a, S, x, y);
+        const int nch = (S + 15) / 16;
+        if ((int64_t)a.n * nch < 2048)
+            hipLaunchKernelGGL((k_b_spmm<T, true>), dim3(xcd_grid(a.n), nch), dim3(kBlock), 0, s, a, S, x, y);
+        else
+            hipLaunchKernelGGL((k_b_spmm<T, false>), dim3(xcd_grid((a.n + kRowsPerBlock - 1) / kRowsPerBlock), nch),
+                               dim3(kBlock), 0, s, a, S, x, y);
     }
 
     // initial guess of the solve of A x = b from the window of solved pairs;
@@ -2825,12 +2910,14 @@ struct BatchSolver {
 
     // iteration k: q = A p_k = A z_k + beta q, partial (z_k, q)
     void cg_spmv(const T* zk, int k, double* pzq, hipStream_t s) {
-        if constexpr (kWideT)
-            if (tiled()) {
-                hipLaunchKernelGGL(k_b_cg_spmv_t, dim3(Gq), dim3(kTileThreads), 0, s, t0.args(sl0, 64),
-                                   (const float*)wA0.p, (const float*)zk, (float*)q.p, k, (const BState*)bst.p, pzq);
-                return;
-            }
+        if (tiled()) {
+            with_tile_type([&](auto tt) {
+                using TT = decltype(tt);
+                hipLaunchKernelGGL(k_b_cg_spmv_t<TT>, dim3(Gq), dim3(kTileThreads), 0, s, t0.args(sl0, TT::kSamples),
+                                   (const T*)wA0.p, zk, q.p, k, (const BState*)bst.p, pzq);
+            });
+            return;
+        }
         if constexpr (kWideT)
             if (wide()) {
                 hipLaunchKernelGGL(k_b_cg_spmv_w, dim3(G), dim3(kBlock), 0, s, gated(sl0.args(4, wA0.p)),
