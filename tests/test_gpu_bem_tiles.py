@@ -1,5 +1,5 @@
 """The batched boundary products at the edges of their tiles.  From int8
-digits: 16-row tiles, 8 or 4 per block; 64-column chunks.  FP64 (64 samples):
+digits: 16-row tiles, 8 or 4 per block; 64-column chunks.  FP64 (16 to 64 columns):
 64 to 256 rows per block; 8- to 32-column chunks.  Both take three chunks per
 pass of the loop and split the columns over several ranges."""
 import numpy as np
@@ -10,7 +10,8 @@ from conftest import rel_l2
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("prec, S, tol", [("MIXED_BEMI8", 64, 2e-7), ("MIXED_BEMI8", 5, 2e-7), ("FP64", 64, 1e-13)])
+@pytest.mark.parametrize("prec, S, tol", [("MIXED_BEMI8", 64, 2e-7), ("MIXED_BEMI8", 5, 2e-7), ("FP64", 64, 1e-13), ("FP64", 1, 1e-13),
+                                          ("FP64", 16, 1e-13), ("FP64", 17, 1e-13), ("FP64", 48, 1e-13), ("FP64", 49, 1e-13)])
 @pytest.mark.parametrize("nx, ny, nz", [(2, 2, 1), (5, 3, 2), (7, 3, 2), (6, 5, 4), (13, 8, 1), (12, 12, 3), (23, 11, 4)])
 def test_product_at_tile_edges(gpu_available, nx, ny, nz, prec, S, tol):
     """Against the dense FP64 product on the host.  Five digits of B and six of

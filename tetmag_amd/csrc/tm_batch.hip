@@ -1718,9 +1718,10 @@ __global__ __launch_bounds__(kBlock) void k_b_scatter(int b, int S, const int* _
 
 // ---- FP64 MFMA GEMM for the boundary product ---------------------------
 // P[ks] (b x S, row-major: P[ks][row][j]) = B[:, K_ks] (b x |K_ks|,
-// column-major, ld) * U^T[K_ks, :] with U S x b column-major (ld S), S = 64
-// columns.  Block: 4 wavefronts x 16 MT rows, all 64 columns, one K range ks
-// of the split; U^T chunks of KGK rows are staged in LDS.
+// column-major, ld) * U^T[K_ks, :] with U S x b column-major (ld S), S <= 16 NT
+// columns.  Block: 4 wavefronts x 16 MT rows, all columns (those past S compute
+// the last one and are not stored), one K range ks of the split; U^T chunks of KGK
+// rows are staged in LDS.
 // v_mfma_f64_16x16x4f64 operand layout (measured): A lane l = A[l%16][l/16],
 // B lane l = B[l/16][l%16], D lane l register r = C[4r + l/16][l%16].
 // Software-pipelined: while the MFMAs of chunk c run, its successor's U^T rows
@@ -1731,26 +1732,30 @@ __global__ __launch_bounds__(kBlock) void k_b_scatter(int b, int S, const int* _
 // Bound by the FP64 matrix cores under their power limit (54 TFLOP/s is what
 // the library's best kernel sustains at 40,962 boundary nodes): 64 samples, 10,242
 // boundary nodes 0.258 -> 0.245 ms, 9,602 0.226 -> 0.220 against masked loads one chunk ahead.
+// Fewer samples take as many column tiles as they need and are bound by reading
+// B: 24 samples, 10,242 boundary nodes 204 us (the library's fastest) -> 163 (5.1
+// TB/s), 7 samples, 1,122 boundary nodes 21.7 -> 5.2 + 3 for the partials' sum.
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 
-template <int KGK, int MT>
-__global__ __launch_bounds__(kBlock) void k_b_gemm64(int b, int ld, const double* __restrict__ B,
+template <int KGK, int MT, int NT>
+__global__ __launch_bounds__(kBlock) void k_b_gemm64(int b, int ld, int S, const double* __restrict__ B,
                                                      const double* __restrict__ U, int kper,
                                                      double* __restrict__ P) {
-    constexpr int UPT = KGK * 64 / kBlock;  // U^T values per thread per chunk
-    static_assert(KGK % 4 == 0 && (KGK * 64) % kBlock == 0, "chunk shape");
-    __shared__ double us[2][KGK * 64];  // U^T chunk: us[buf][k * 64 + j]
+    constexpr int kCols = 16 * NT;
+    constexpr int UPT = KGK * kCols / kBlock;  // U^T values per thread per chunk
+    static_assert(KGK % 4 == 0 && UPT * kBlock == KGK * kCols, "chunk shape");
+    __shared__ double us[2][KGK * kCols];  // U^T chunk: us[buf][k * kCols + j]
     const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     const int m0 = (blockIdx.x * (kBlock / kWave) + wv) * 16 * MT;  // this wavefront's rows
     const int ks = blockIdx.y;
     const int kb = ks * kper, ke = min(b, kb + kper);
     const int nc = ke > kb ? (ke - kb + KGK - 1) / KGK : 0;  // chunks, uniform over the block
     const int li = lane & 15, lk = lane >> 4;
-    dbl4 acc[MT][4];
+    dbl4 acc[MT][NT];
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) acc[t][u] = dbl4{0.0, 0.0, 0.0, 0.0};
+        for (int u = 0; u < NT; ++u) acc[t][u] = dbl4{0.0, 0.0, 0.0, 0.0};
     int rr[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) rr[t] = min(m0 + 16 * t + li, b - 1);  // the A row of this lane in tile t
@@ -1769,22 +1774,22 @@ __global__ __launch_bounds__(kBlock) void k_b_gemm64(int b, int ld, const double
 #pragma unroll
         for (int i = 0; i < UPT; ++i) {
             const int t = threadIdx.x + i * kBlock;
-            ur[i] = U[(size_t)min(kb + c * KGK + t / 64, b - 1) * 64 + (t & 63)];
+            ur[i] = U[(size_t)min(kb + c * KGK + t / kCols, b - 1) * S + min(t % kCols, S - 1)];
         }
     };
     auto store_u = [&](int c) {
 #pragma unroll
         for (int i = 0; i < UPT; ++i) {
             const int t = threadIdx.x + i * kBlock;
-            us[c & 1][t] = kb + c * KGK + t / 64 < ke ? ur[i] : 0.0;
+            us[c & 1][t] = kb + c * KGK + t / kCols < ke ? ur[i] : 0.0;
         }
     };
     auto mfmas = [&](const Vals& av, int buf) {
 #pragma unroll
         for (int q = 0; q < KGK / 4; ++q) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const double bu = us[buf][(4 * q + lk) * 64 + u * 16 + li];
+            for (int u = 0; u < NT; ++u) {
+                const double bu = us[buf][(4 * q + lk) * kCols + u * 16 + li];
 #pragma unroll
                 for (int t = 0; t < MT; ++t)
                     acc[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[t][q], bu, acc[t][u], 0, 0, 0);
@@ -1810,48 +1815,57 @@ __global__ __launch_bounds__(kBlock) void k_b_gemm64(int b, int ld, const double
         step(c + 1, a[1], a[0]);
         step(c + 2, a[2], a[1]);
     }
-    double* out = P + (size_t)ks * b * 64;
+    double* out = P + (size_t)ks * b * S;
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+        for (int u = 0; u < NT; ++u)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int row = m0 + t * 16 + 4 * r + lk;
-                if (row < b) out[(size_t)row * 64 + u * 16 + li] = acc[t][u][r];
+                const int row = m0 + t * 16 + 4 * r + lk, col = u * 16 + li;
+                if (row < b && col < S) out[(size_t)row * S + col] = acc[t][u][r];
             }
 }
 
 struct GemmShape {
     int kgk, mt;
 };
-constexpr GemmShape kGemmShapes[] = {{16, 2}, {32, 2}, {8, 2}, {16, 4}, {8, 4}, {16, 1}, {32, 1}};
+constexpr GemmShape kGemmShapes[] = {{16, 2}, {32, 2}, {16, 1}, {32, 1}, {8, 2}, {16, 4}, {8, 4}};
 constexpr int kNumGemmShapes = sizeof(kGemmShapes) / sizeof(kGemmShapes[0]);
+// the last three for four column tiles only
+inline int gemm_shapes(int S) { return S > 48 ? kNumGemmShapes : 4; }
 
 inline int gemm_rows_per_block(int shape) { return (kBlock / kWave) * 16 * kGemmShapes[shape].mt; }
 
 template <class F>
-void gemm_dispatch(int shape, F&& f) {
-    switch (shape) {
-        case 0: f(k_b_gemm64<16, 2>); break;
-        case 1: f(k_b_gemm64<32, 2>); break;
-        case 2: f(k_b_gemm64<8, 2>); break;
-        case 3: f(k_b_gemm64<16, 4>); break;
-        case 4: f(k_b_gemm64<8, 4>); break;
-        case 5: f(k_b_gemm64<16, 1>); break;
-        default: f(k_b_gemm64<32, 1>); break;
-    }
+void gemm_dispatch(int shape, int S, F&& f) {
+    auto first4 = [&](auto nt) {
+        constexpr int NT = decltype(nt)::value;
+        switch (shape) {
+            case 0: f(k_b_gemm64<16, 2, NT>); break;
+            case 1: f(k_b_gemm64<32, 2, NT>); break;
+            case 2: f(k_b_gemm64<16, 1, NT>); break;
+            default: f(k_b_gemm64<32, 1, NT>); break;
+        }
+    };
+    if (S <= 16) first4(std::integral_constant<int, 1>{});
+    else if (S <= 32) first4(std::integral_constant<int, 2>{});
+    else if (S <= 48) first4(std::integral_constant<int, 3>{});
+    else if (shape < 4) first4(std::integral_constant<int, 4>{});
+    else if (shape == 4) f(k_b_gemm64<8, 2, 4>);
+    else if (shape == 5) f(k_b_gemm64<16, 4, 4>);
+    else f(k_b_gemm64<8, 4, 4>);
 }
 
-void launch_gemm64(int shape, dim3 g, hipStream_t s, int b, int ld, const double* B, const double* U, int kper,
+void launch_gemm64(int shape, dim3 g, hipStream_t s, int b, int ld, int S, const double* B, const double* U, int kper,
                    double* P) {
-    gemm_dispatch(shape, [&](auto k) { hipLaunchKernelGGL(k, g, dim3(kBlock), 0, s, b, ld, B, U, kper, P); });
+    gemm_dispatch(shape, S, [&](auto k) { hipLaunchKernelGGL(k, g, dim3(kBlock), 0, s, b, ld, S, B, U, kper, P); });
 }
 
 // resident blocks per CU of a tile shape (0 if the runtime cannot say)
-int gemm_blocks_per_cu(int shape) {
+int gemm_blocks_per_cu(int shape, int S) {
     int nb = 0;
-    gemm_dispatch(shape, [&](auto k) {
+    gemm_dispatch(shape, S, [&](auto k) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k, kBlock, 0) != hipSuccess) nb = 0;
     });
     return nb;
@@ -3342,11 +3356,11 @@ __global__ __launch_bounds__(kBlock) void k_b_fill_pattern(size_t n, double* __r
 // and those that fill j = 1..6 rounds of the resident block slots (all
 // blocks carry the same work, so a last round that is only partly filled
 // leaves CUs idle).  At most 16 partial products.
-std::vector<int> gemm_ks_candidates(int b, int shape, int ncu) {
+std::vector<int> gemm_ks_candidates(int b, int shape, int S, int ncu) {
     const int rows = gemm_rows_per_block(shape);
     const int grid_m = (b + rows - 1) / rows;
     std::vector<int> ks = {std::max(1, std::min(16, (1024 + grid_m - 1) / grid_m))};
-    const int slots = ncu * gemm_blocks_per_cu(shape);
+    const int slots = ncu * gemm_blocks_per_cu(shape, S);
     for (int j = 1; j <= 6 && slots > 0; ++j) {
         const int k = std::max(1, std::min(16, j * slots / grid_m));
         if (std::find(ks.begin(), ks.end(), k) == ks.end()) ks.push_back(k);
@@ -3359,8 +3373,8 @@ int gemm_own_run(tm_batch* bt, double* G) {
     const int b = v.bnx;
     const int rows = gemm_rows_per_block(bt->gemm_shape);
     const int kper = (b + bt->gemm_ks - 1) / bt->gemm_ks;
-    launch_gemm64(bt->gemm_shape, dim3((b + rows - 1) / rows, bt->gemm_ks), bt->stream, b, v.bld, v.B,
-                  (const double*)bt->U.p, kper, bt->Pd.p);
+    launch_gemm64(bt->gemm_shape, dim3((b + rows - 1) / rows, bt->gemm_ks), bt->stream, b, v.bld,
+                  bt->S, v.B, (const double*)bt->U.p, kper, bt->Pd.p);
     TM_HIP(hipGetLastError());
     if (G) {  // sum the partials into G (b x S, row-major) without scatter
         hipLaunchKernelGGL(k_b_ksum_scatter, dim3(elem_grid((size_t)b * bt->S)), dim3(kBlock), 0, bt->stream, b,
@@ -3430,15 +3444,15 @@ int tune_gemm(tm_batch* bt) {
     bt->gemm_candidates = cap;
     // the MFMA kernel, each tile shape and K split: checked against the
     // library on a non-zero U, then timed
-    if (!f32 && S == 64) {
+    if (!f32) {
         int dev = 0, ncu = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
             ncu = 0;
         std::vector<std::pair<int, int>> cand;  // (shape, ks)
         int ksmax = 1;
-        for (int sh = 0; sh < kNumGemmShapes; ++sh)
-            for (int k : gemm_ks_candidates(b, sh, ncu)) {
+        for (int sh = 0; sh < gemm_shapes(S); ++sh)
+            for (int k : gemm_ks_candidates(b, sh, S, ncu)) {
                 cand.push_back({sh, k});
                 ksmax = std::max(ksmax, k);
             }
@@ -3480,7 +3494,7 @@ int tune_gemm(tm_batch* bt) {
                         best_shape = bt->gemm_shape;
                         best_ks = bt->gemm_ks;
                     }
-                    if (!bt->own_ok || ms < bt->own_ms) {  // the fastest verified own kernel, for graphs
+                    if (S == 64 && (!bt->own_ok || ms < bt->own_ms)) {  // the fastest verified own kernel, for graphs
                         bt->own_ok = true;
                         bt->own_ms = ms;
                         bt->own_shape = bt->gemm_shape;
