@@ -360,6 +360,8 @@ __host__ __device__ inline void win_coefficients(int cnt, const double* t, doubl
     // every loop runs to the compile-time window size with the count as a
     // condition, so the small arrays stay in registers
     double sc[kSolveWindow], c[kSolveWindow], y[kSolveWindow];
+    // L's diagonal as its reciprocal: one thread runs this between two kernels'
+    // work, and a chain of 27 divisions was most of its time
     double L[kSolveWindow][kSolveWindow];
     bool keep[kSolveWindow];
     bool fin = true;
@@ -385,10 +387,10 @@ __host__ __device__ inline void win_coefficients(int cnt, const double* t, doubl
                 for (int k = 0; k < j; ++k)
                     if (keep[k]) v -= L[i][k] * L[j][k];
                 if (j < i) {
-                    L[i][j] = v / L[j][j];
+                    L[i][j] = v * L[j][j];
                 } else {
                     keep[i] = sc[i] > 0.0 && v > 1e-12;
-                    L[i][i] = keep[i] ? sqrt(v) : 1.0;
+                    L[i][i] = keep[i] ? 1.0 / sqrt(v) : 1.0;
                 }
             }
         }
@@ -399,7 +401,7 @@ __host__ __device__ inline void win_coefficients(int cnt, const double* t, doubl
 #pragma unroll
             for (int k = 0; k < i; ++k)
                 if (keep[k]) v -= L[i][k] * y[k];
-            y[i] = v / L[i][i];
+            y[i] = v * L[i][i];
         }
 #pragma unroll
         for (int i = kSolveWindow - 1; i >= 0; --i) {
@@ -408,7 +410,7 @@ __host__ __device__ inline void win_coefficients(int cnt, const double* t, doubl
 #pragma unroll
             for (int k = i + 1; k < kSolveWindow; ++k)
                 if (keep[k]) v -= L[k][i] * c[k];
-            c[i] = v / L[i][i];
+            c[i] = v * L[i][i];
         }
         double est = t[kWinDots - 1];
 #pragma unroll
