@@ -66,3 +66,59 @@ def test_boundary_product_splits(gpu_available, b):
     torch.cuda.synchronize()
     M = B[:, :b].T.contiguous()
     assert bool(((y - M @ x).abs() <= 2 * b * 2.3e-16 * (M.abs() @ x.abs())).all())
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1000, 8192, 8193, 20000])
+def test_sparse_product_lanes(gpu_available, n):
+    """16 lanes to a row up to 8,192 rows, 4 above; rows of 0 to 70 entries.  The
+    sums differ from scipy's by at most (entries + 1) eps |A| |x|; an infinite x
+    gives the infinity of the plain sum."""
+    import scipy.sparse as sp
+    import torch
+    from tetmag_amd.gpu import SpMatCUDA
+    rng = np.random.default_rng(n)
+    lens = rng.integers(0, min(n, 30) + 1, n)
+    lens[n // 2] = min(n, 70)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    ci = np.concatenate([np.sort(rng.choice(n, k, replace=False)) for k in lens]).astype(np.int32)
+    A = sp.csr_matrix((rng.standard_normal(len(ci)), ci, rp), shape=(n, n))
+    x = rng.standard_normal(n)
+    y = SpMatCUDA(A).mvp(torch.from_numpy(x).cuda()).cpu().numpy()
+    bound = (lens + 1) * 2.3e-16 * (abs(A) @ abs(x))
+    print("n", n, "worst error / bound", np.max(np.abs(y - A @ x) / np.maximum(bound, 1e-300)), flush=True)
+    assert np.all(np.abs(y - A @ x) <= bound)
+    if n > 1:
+        B = abs(A)
+        x = abs(x)
+        x[n // 3] = np.inf
+        y = SpMatCUDA(B).mvp(torch.from_numpy(x).cuda()).cpu().numpy()
+        hit = np.asarray((B[:, [n // 3]] != 0).todense()).ravel()
+        assert np.all(np.isposinf(y[hit])) and hit.any()
+
+
+@pytest.mark.parametrize("cells", [(31, 15, 15), (32, 15, 15), (13, 11, 5)])
+@pytest.mark.parametrize("dmi", [False, True])
+def test_field_lanes(gpu_available, cells, dmi):
+    """Divergence and fields with 16 lanes to a row (8,192 nodes and fewer) and with
+    4, against the batched kernels.  Both sides solve to 1e-13: fields within a
+    few thousand times that, 1e-9."""
+    from conftest import rel_l2
+    from tetmag_amd import _native as N
+    from tetmag_amd import problem as P
+    from tetmag_amd.batch import BatchContext, from_batch, to_batch
+    from tetmag_amd.context import FieldContext
+    mat = P.Material(Ku=4e4, ku_axis=(0.6, 0.0, 0.8), D=1e-3 if dmi else 0.0, B_ext=(0.01, 0.02, -0.03))
+    prob = P.cuboid_problem("lanes", *cells, 3.0, 0.1, 3, mat)
+    ctx = FieldContext(prob, tol=1e-13)
+    try:
+        bc = BatchContext(ctx, 2, N.TM_PREC_FP64)
+        ms = P.smooth_random_fields(prob.mesh, 2, seed=4)
+        dm, H, _ = bc.eval_rhs_host(to_batch(ms))
+        for s in range(2):
+            d1, h1, _ = ctx.eval_rhs_host(ms[s])
+            e = max(rel_l2(h1, from_batch(H, s)), rel_l2(d1, from_batch(dm, s)))
+            print(cells, prob.n, "dmi", dmi, "sample", s, e, flush=True)
+            assert e < 1e-9
+        bc.close()
+    finally:
+        ctx.close()

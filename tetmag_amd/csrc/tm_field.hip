@@ -194,22 +194,34 @@ __global__ __launch_bounds__(kBlock) void k_stt_uterm(SellView A, const double* 
 }
 
 // GpuPotential::calcDivM (GpuPotential.cu:86-106): sum_d tGrad_d (Js m_d), times `scale`.
+template <int LPR>
 __global__ __launch_bounds__(kBlock) void k_div(SellView A, const double* __restrict__ tx,
                                                 const double* __restrict__ ty, const double* __restrict__ tz,
                                                 const double* __restrict__ js, const double* __restrict__ m,
                                                 double scale, double* __restrict__ out) {
-    SELL_ROW_PROLOGUE
     const int n = A.n;
+    const SellLanes<LPR> L;
+    if (L.s >= (n + kWave - 1) / kWave) return;
+    double v[1] = {};
     double sx = 0, sy = 0, sz = 0;
-    (void)base;
-    (void)w;
-    sell_row(A, s, lane, [&](int64_t q, int cc) {
+    L.each(A, [&](int64_t q, int cc, bool on) {
         const double j = js[cc];
-        sx += tx[q] * (m[cc] * j);
-        sy += ty[q] * (m[n + cc] * j);
-        sz += tz[q] * (m[2 * n + cc] * j);
+        const double x = tx[q] * (m[cc] * j), y = ty[q] * (m[n + cc] * j), z = tz[q] * (m[2 * n + cc] * j);
+        sx += on ? x : 0.0;
+        sy += on ? y : 0.0;
+        sz += on ? z : 0.0;
     });
-    if (row < n) out[row] = (sx + sy + sz) * scale;
+    v[0] = sx + sy + sz;
+    L.sum(v);
+    if (L.row < n && L.sub == 0) out[L.row] = v[0] * scale;
+}
+
+template <class... Args>
+void launch_div(hipStream_t s, const SellView& A, Args... args) {
+    with_row_lanes(A.n, [&](auto lpr) {
+        constexpr int kL = decltype(lpr)::value;
+        hipLaunchKernelGGL(k_div<kL>, dim3(row_lanes_grid<kL>(A.n)), dim3(kBlock), 0, s, A, args...);
+    });
 }
 
 // GpuPotential::calcGradientField (GpuPotential.cu:109-122): H = -grad(u1 [+ u2]).
@@ -364,9 +376,13 @@ struct EvalArgs {
 //   H_z = -D (grad_x m_x + grad_y m_y) + (tGrad_x (D m_x) + tGrad_y (D m_y)) / V.
 // ia: grad_x m_z, grad_y m_z, grad_x m_x + grad_y m_y, tGrad_x(D m_z),
 //     tGrad_y(D m_z), tGrad_x(D m_x) + tGrad_y(D m_y)
-__device__ inline void idmi_accumulate(const EvalArgs& a, int64_t q, int cc, double mx, double my, double mz,
+__device__ inline void idmi_accumulate(const EvalArgs& a, int64_t q, int cc, double mx, double my, double mz, bool on,
                                        double (&ia)[8]) {
-    const double gx = a.igx[q], gy = a.igy[q], tx = a.itx[q], ty = a.ity[q];
+    double gx = a.igx[q], gy = a.igy[q], tx = a.itx[q], ty = a.ity[q];
+    gx = on ? gx : 0.0;
+    gy = on ? gy : 0.0;
+    tx = on ? tx : 0.0;
+    ty = on ? ty : 0.0;
     const double Dc = a.idmi[cc];
     ia[0] += gx * mz;
     ia[1] += gy * mz;
@@ -388,47 +404,58 @@ __device__ inline void idmi_field(const EvalArgs& a, int row, const double (&ia)
 // one pass over the shared pattern computes exchange, demag gradient and DMI
 // curl for the row, then the pointwise terms, the LLG right-hand side and the
 // torque maximum.
-template <bool EXCH, bool DEMAG, bool DMI>
+template <bool EXCH, bool DEMAG, bool DMI, int LPR>
 __global__ __launch_bounds__(kBlock) void k_eval(EvalArgs a) {
     __shared__ double smem[kBlock / kWave];
     const SellView A = a.A;
     const int n = A.n;
-    const int row = xcd_block() * kBlock + threadIdx.x;
-    const int s = row / kWave, lane = row & (kWave - 1);
+    const SellLanes<LPR> L;
+    const int row = L.row;
     double t = 0.0;
-    if (s < (n + kWave - 1) / kWave) {
+    if (L.s < (n + kWave - 1) / kWave) {
         const double* __restrict__ m = a.m;
-        double ex = 0, ey = 0, ez = 0, dx = 0, dy = 0, dz = 0, cx = 0, cy = 0, cz = 0;
+        double ve[3] = {}, vd[3] = {}, vc[3] = {};
         double ia[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // interfacial DMI row sums
         const bool idmi = a.idmi != nullptr;
-        sell_row(A, s, lane, [&](int64_t q, int cc) {
+        L.each(A, [&](int64_t q, int cc, bool on) {
             double mx = 0, my = 0, mz = 0;
             if (EXCH || DMI || idmi) {
                 mx = m[cc];
                 my = m[n + cc];
                 mz = m[2 * n + cc];
             }
-            if (idmi) idmi_accumulate(a, q, cc, mx, my, mz, ia);
+            if (idmi) idmi_accumulate(a, q, cc, mx, my, mz, on, ia);
             if (EXCH) {
-                const double e = a.xc[q];
-                ex += e * mx;
-                ey += e * my;
-                ez += e * mz;
+                double e = a.xc[q];
+                e = on ? e : 0.0;
+                ve[0] += e * mx;
+                ve[1] += e * my;
+                ve[2] += e * mz;
             }
             if (DEMAG) {
-                const double u = a.u1[cc] + a.u2[cc];
-                dx += a.gx[q] * u;
-                dy += a.gy[q] * u;
-                dz += a.gz[q] * u;
+                double u = a.u1[cc] + a.u2[cc];
+                const double X = a.gx[q], Y = a.gy[q], Z = a.gz[q];
+                vd[0] += (on ? X : 0.0) * u;
+                vd[1] += (on ? Y : 0.0) * u;
+                vd[2] += (on ? Z : 0.0) * u;
             }
             if (DMI) {
-                const double X = a.cx[q], Y = a.cy[q], Z = a.cz[q];
-                cx += Y * mz - Z * my;
-                cy += Z * mx - X * mz;
-                cz += X * my - Y * mx;
+                double X = a.cx[q], Y = a.cy[q], Z = a.cz[q];
+                X = on ? X : 0.0;
+                Y = on ? Y : 0.0;
+                Z = on ? Z : 0.0;
+                vc[0] += Y * mz - Z * my;
+                vc[1] += Z * mx - X * mz;
+                vc[2] += X * my - Y * mx;
             }
         });
-        if (row < n) {
+        if (EXCH) L.sum(ve);
+        if (DEMAG) L.sum(vd);
+        if (DMI) L.sum(vc);
+        if (idmi) L.sum(ia);
+        const double ex = ve[0], ey = ve[1], ez = ve[2], dx = vd[0], dy = vd[1], dz = vd[2];
+        const double cx = vc[0], cy = vc[1], cz = vc[2];
+        if (row < n && L.sub == 0) {
             const double mx = m[row], my = m[n + row], mz = m[2 * n + row];
             double hx = ex, hy = ey, hz = ez;  // J/m^3 terms
             if (a.ku) {
@@ -494,21 +521,24 @@ __global__ __launch_bounds__(kBlock) void k_eval(EvalArgs a) {
 }
 
 template <bool E, bool D, bool M>
-void launch_eval(const EvalArgs& a, int grid, hipStream_t s) {
-    hipLaunchKernelGGL((k_eval<E, D, M>), dim3(grid), dim3(kBlock), 0, s, a);
+void launch_eval(const EvalArgs& a, hipStream_t s) {
+    with_row_lanes(a.A.n, [&](auto lpr) {
+        constexpr int kL = decltype(lpr)::value;
+        hipLaunchKernelGGL((k_eval<E, D, M, kL>), dim3(row_lanes_grid<kL>(a.A.n)), dim3(kBlock), 0, s, a);
+    });
 }
 
-int eval_dispatch(const EvalArgs& a, bool e, bool d, bool m, int grid, hipStream_t s) {
+int eval_dispatch(const EvalArgs& a, bool e, bool d, bool m, hipStream_t s) {
     const int key = (e ? 4 : 0) | (d ? 2 : 0) | (m ? 1 : 0);
     switch (key) {
-        case 0: launch_eval<false, false, false>(a, grid, s); break;
-        case 1: launch_eval<false, false, true>(a, grid, s); break;
-        case 2: launch_eval<false, true, false>(a, grid, s); break;
-        case 3: launch_eval<false, true, true>(a, grid, s); break;
-        case 4: launch_eval<true, false, false>(a, grid, s); break;
-        case 5: launch_eval<true, false, true>(a, grid, s); break;
-        case 6: launch_eval<true, true, false>(a, grid, s); break;
-        default: launch_eval<true, true, true>(a, grid, s); break;
+        case 0: launch_eval<false, false, false>(a, s); break;
+        case 1: launch_eval<false, false, true>(a, s); break;
+        case 2: launch_eval<false, true, false>(a, s); break;
+        case 3: launch_eval<false, true, true>(a, s); break;
+        case 4: launch_eval<true, false, false>(a, s); break;
+        case 5: launch_eval<true, false, true>(a, s); break;
+        case 6: launch_eval<true, true, false>(a, s); break;
+        default: launch_eval<true, true, true>(a, s); break;
     }
     TM_HIP(hipGetLastError());
     return TM_OK;
@@ -548,7 +578,7 @@ __global__ __launch_bounds__(kBlock) void k_energy(EvalArgs a, const double* __r
                 my = m[n + cc];
                 mz = m[2 * n + cc];
             }
-            if (idmi) idmi_accumulate(a, q, cc, mx, my, mz, ia);
+            if (idmi) idmi_accumulate(a, q, cc, mx, my, mz, true, ia);
             if (EXCH) {
                 const double v = a.xc[q];
                 ex += v * mx;
@@ -962,8 +992,8 @@ int tm_div_m(tm_ctx* c, const double* m3n, int mwhere, double* b, int bwhere) {
     const double* md = nullptr;
     TM_CHECK(stage_in(c, m3n, mwhere, (size_t)3 * c->n, c->w3b, &md));
     double* o = bwhere == TM_DEVICE ? b : c->wn.p;
-    hipLaunchKernelGGL(k_div, dim3(sell_grid(c)), dim3(kBlock), 0, c->stream, view(c->pat), c->opv[TM_OP_TGRAD_X].p,
-                       c->opv[TM_OP_TGRAD_Y].p, c->opv[TM_OP_TGRAD_Z].p, c->js.p, md, 1.0, o);
+    launch_div(c->stream, view(c->pat), c->opv[TM_OP_TGRAD_X].p, c->opv[TM_OP_TGRAD_Y].p,
+               c->opv[TM_OP_TGRAD_Z].p, c->js.p, md, 1.0, o);
     TM_HIP(hipGetLastError());
     return finish_out(c, b, bwhere, o, (size_t)c->n);
 }
@@ -1107,8 +1137,8 @@ int demag_potential_dev(tm_ctx* c, const double* md, tm_eval_stats* stats) {
     if (!c->has_op[TM_OP_TGRAD_X] || !c->has_op[TM_OP_TGRAD_Y] || !c->has_op[TM_OP_TGRAD_Z]) return TM_ERR_NOT_READY;
     if (c->timers) TM_HIP(hipEventRecord(c->ev[0], c->stream));
     // rhsPoisson (DemagField.cpp:124-136): divM / mu0
-    hipLaunchKernelGGL(k_div, dim3(sell_grid(c)), dim3(kBlock), 0, c->stream, view(c->pat), c->opv[TM_OP_TGRAD_X].p,
-                       c->opv[TM_OP_TGRAD_Y].p, c->opv[TM_OP_TGRAD_Z].p, c->js.p, md, 1.0 / kMu0, c->rhsN.p);
+    launch_div(c->stream, view(c->pat), c->opv[TM_OP_TGRAD_X].p, c->opv[TM_OP_TGRAD_Y].p,
+               c->opv[TM_OP_TGRAD_Z].p, c->js.p, md, 1.0 / kMu0, c->rhsN.p);
     TM_HIP(hipGetLastError());
     int itN = 0, itD = 0;
     double rN = 0, rD = 0;
@@ -1165,9 +1195,8 @@ int eval_device(tm_ctx* c, const double* md, double* dmdt, double alpha, int var
         if (budgetN > 0) {
             if (!c->has_js || !c->has_op[TM_OP_TGRAD_X] || !c->has_op[TM_OP_TGRAD_Y] || !c->has_op[TM_OP_TGRAD_Z])
                 return TM_ERR_NOT_READY;
-            hipLaunchKernelGGL(k_div, dim3(sell_grid(c)), dim3(kBlock), 0, c->stream, view(c->pat),
-                               c->opv[TM_OP_TGRAD_X].p, c->opv[TM_OP_TGRAD_Y].p, c->opv[TM_OP_TGRAD_Z].p, c->js.p, md,
-                               1.0 / kMu0, c->rhsN.p);
+            launch_div(c->stream, view(c->pat), c->opv[TM_OP_TGRAD_X].p, c->opv[TM_OP_TGRAD_Y].p,
+                       c->opv[TM_OP_TGRAD_Z].p, c->js.p, md, 1.0 / kMu0, c->rhsN.p);
             TM_HIP(hipGetLastError());
             TM_CHECK(c->cgN.enqueue(c->rhsN.p, c->u1.p, c->tol, budgetN, c->stream, fails, imax2, true));
             TM_CHECK(bem_gemv(c->bnx, c->bld, c->B.p, c->u1.p, c->bnodes.p, c->bpart.p, nullptr, c->bnodes.p,
@@ -1210,7 +1239,7 @@ int eval_device(tm_ctx* c, const double* md, double* dmdt, double alpha, int var
     a.alpha = alpha;
     a.variant = variant;
     a.dmdt = dmdt;
-    TM_CHECK(eval_dispatch(a, exch, demag, dmi, sell_grid(c), c->stream));
+    TM_CHECK(eval_dispatch(a, exch, demag, dmi, c->stream));
     return st;
 }
 }  // namespace tmh
@@ -1310,7 +1339,7 @@ int tm_eval_rhs(tm_ctx* c, const double* m3n, int mwhere, double alpha, int vari
     a.heff = Heff ? (hwhere == TM_DEVICE ? Heff : c->w3b.p) : nullptr;
     a.torque = stats ? c->scal.p : nullptr;
     if (stats) hipLaunchKernelGGL(k_zero1, dim3(1), dim3(1), 0, c->stream, c->scal.p);
-    TM_CHECK(eval_dispatch(a, exch, demag, dmi, sell_grid(c), c->stream));
+    TM_CHECK(eval_dispatch(a, exch, demag, dmi, c->stream));
     if (c->timers && solve) {
         TM_HIP(hipEventRecord(c->ev[5], c->stream));
         TM_HIP(hipEventSynchronize(c->ev[5]));
@@ -1364,7 +1393,7 @@ int tm_idmi_field(tm_ctx* c, double* out, int where) {
     a.m = c->m.p;
     double* o = out_target(c, out, where);
     a.heff = o;
-    TM_CHECK(eval_dispatch(a, false, false, false, sell_grid(c), c->stream));
+    TM_CHECK(eval_dispatch(a, false, false, false, c->stream));
     return finish_out(c, out, where, o, (size_t)3 * c->n);
 }
 

@@ -223,6 +223,65 @@ __device__ inline int xcd_block() {
     return (b % kXcd) * (G / kXcd) + b / kXcd;
 }
 
+// sell_row with LPR lanes to a row: lane `sub` takes entries sub, sub + LPR, ...,
+// four (one with 16 lanes) in flight.  f(entry, column, on): `on` is false past
+// the row's end, where the last entry is loaded and its weights have to be
+// taken as zero (no load depends on a condition).  Lanes 64 / LPR apart share a
+// row, so a load still reads LPR runs of 64 / LPR neighbouring entries.
+template <int LPR>
+struct SellLanes {
+    static constexpr int kRows = kWave / LPR;  // rows of a wavefront
+    int row, s, l, sub;
+    __device__ SellLanes() {
+        const int lane = threadIdx.x & (kWave - 1);
+        row = (xcd_block() * (kBlock / kWave) + (int)(threadIdx.x / kWave)) * kRows + lane % kRows;
+        sub = lane / kRows;
+        s = row / kWave;
+        l = row & (kWave - 1);
+    }
+    template <class F>
+    __device__ __forceinline__ void each(const SellView& A, F&& f) const {
+        constexpr int kUnroll = LPR >= 16 ? 1 : 4;
+        const int64_t base = A.off[s] + l;
+        const int w = A.w[s];
+        for (int k = sub; k < w + sub; k += kUnroll * LPR) {  // (the same count on every lane)
+            int64_t e[kUnroll];
+            int c[kUnroll];
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) {
+                e[u] = base + (int64_t)min(k + u * LPR, w - 1) * kWave;
+                c[u] = A.col[e[u]];
+            }
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) f(e[u], c[u], k + u * LPR < w);
+        }
+    }
+    // the row's sum on each of its lanes
+    template <int NV>
+    __device__ void sum(double (&v)[NV]) const {
+#pragma unroll
+        for (int o = kRows; o < kWave; o <<= 1)
+#pragma unroll
+            for (int q = 0; q < NV; ++q) v[q] += __shfl_xor(v[q], o);
+    }
+};
+
+// Lanes to a row for SellLanes.  A row is a chain of loads (column, weights
+// and gathers of up to 16 entries); one lane per row leaves most of the chip
+// idle on small meshes and too few loads in flight on large ones.  Fields /
+// divergence in us with 1, 4 and 16 lanes (8 at 29,760 nodes): 2,205 nodes 8.0 / 7.6,
+// 5.1 / 4.1, 4.3 / 3.2; 29,760 nodes (DMI) 13.4 / 9.9, 9.5 / 5.7, 14.8 / 7.8;
+// 282,897 nodes 68 / 48 and 56 / 35.
+template <class F>
+void with_row_lanes(int n, F&& f) {
+    if (n <= 8192) f(std::integral_constant<int, 16>{});
+    else f(std::integral_constant<int, 4>{});
+}
+template <int LPR>
+int row_lanes_grid(int n) {
+    return xcd_grid((int)(((int64_t)(n + kWave - 1) / kWave * kWave * LPR + kBlock - 1) / kBlock));
+}
+
 // ---- rows of a CSR matrix shared by LPR lanes each -------------------------
 template <int LPR>
 __device__ inline double group_sum(double v) {

@@ -100,26 +100,27 @@ int copy_out(double* dst, int where, const double* src_dev, size_t count, hipStr
     return TM_OK;
 }
 
-// y = A x, one row per lane.
+// y = A x.  One lane per row had one entry in flight per wavefront's row: SPMV_FIG
+template <int LPR>
 __global__ __launch_bounds__(kBlock) void k_sell_spmv(SellView A, const double* __restrict__ val,
                                                       const double* __restrict__ x, double* __restrict__ y) {
-    const int row = xcd_block() * kBlock + threadIdx.x;
-    const int s = row / kWave, lane = row & (kWave - 1);
-    if (s >= (A.n + kWave - 1) / kWave) return;
-    const int64_t base = A.off[s] + lane;
-    const int w = A.w[s];
-    double acc = 0.0;
-    for (int k = 0; k < w; ++k) {
-        const int64_t q = base + (int64_t)k * kWave;
-        acc += val[q] * x[A.col[q]];
-    }
-    if (row < A.n) y[row] = acc;
+    const SellLanes<LPR> L;
+    if (L.s >= (A.n + kWave - 1) / kWave) return;
+    double v[1] = {};
+    L.each(A, [&](int64_t e, int c, bool on) {
+        const double p = val[e] * x[c];
+        v[0] += on ? p : 0.0;
+    });
+    L.sum(v);
+    if (L.row < A.n && L.sub == 0) y[L.row] = v[0];
 }
 
 int spmv(const SellPattern& P, const double* val, const double* x, double* y, hipStream_t s) {
     if (P.n == 0) return TM_OK;
-    hipLaunchKernelGGL(k_sell_spmv, dim3(xcd_grid(grid_for((int64_t)P.nslices * kWave))), dim3(kBlock), 0, s, view(P),
-                       val, x, y);
+    with_row_lanes(P.n, [&](auto lpr) {
+        constexpr int kL = decltype(lpr)::value;
+        hipLaunchKernelGGL(k_sell_spmv<kL>, dim3(row_lanes_grid<kL>(P.n)), dim3(kBlock), 0, s, view(P), val, x, y);
+    });
     TM_HIP(hipGetLastError());
     return TM_OK;
 }
