@@ -836,8 +836,8 @@ __device__ inline double pair_sum(d2v s) {
 // after that are being read (one unit at a time, without this, every unit waits for
 // four dependent loads, and the kernels were no faster than the gathers
 // from L2).  64 samples at 282,897 nodes, against the gathers from L2: fields
-// 1,006 -> 606 us, divergence 513 -> 293, FP64 residual 216 -> 143; 24 samples
-// at 38,025 nodes 102 -> 41, 55 -> 24 and 25 -> 14.  A third of the lanes' time
+// 1,006 -> 591 us, divergence 513 -> 282, FP64 residual 216 -> 134; 24 samples
+// at 38,025 nodes 102 -> 39, 55 -> 20 and 25 -> 12.  A third of the lanes' time
 // goes into vector instructions, a third into LDS; two (fields, divergence) and
 // four (residual) blocks per CU were the fastest.
 constexpr int kTileThreads = 512;
@@ -905,7 +905,7 @@ __device__ inline void each16(F&& f, std::integer_sequence<int, K...>) {
 // The element and lane layout of a walk: T, VEC samples per lane (a unit has
 // 16 VEC samples: 128 bytes of a node in FP64, 256 in FP32), and whether rows of
 // samples are 16-byte aligned.
-template <typename T_, int VEC_, bool ALIGNED_>
+template <typename T_, int VEC_, bool ALIGNED_, int NODES = kTileNodes>
 struct TileType {
     using T = T_;
     static constexpr int VEC = VEC_;
@@ -917,7 +917,8 @@ struct TileType {
     using Stage = std::conditional_t<ALIGNED_, StageVec, T>;
     static constexpr int kLanes = kSamples / kPer;  // lanes per staged row of samples
     static constexpr int kGroups = kTileThreads / kLanes;
-    static constexpr int kRounds = kTileNodes / kGroups;
+    static constexpr int kRounds = (NODES + kGroups - 1) / kGroups;
+    static constexpr int kStaged = kRounds * kGroups;  // node places of a tile in LDS
 };
 
 // The first NP chunks of 16 slots of this group's row: lane j's place and NW
@@ -1054,7 +1055,7 @@ __device__ inline typename TT::T lane_at(const typename TT::Lane& v, int c) {
 // The block's sums v (a lane's samples) to part[s * gridDim.x + block], zero for
 // the samples of other chunks, through the walk's LDS
 template <class TT>
-constexpr int kTileElems = kTileNodes * TT::kSamples;
+constexpr int kTileElems = TT::kStaged * TT::kSamples;
 template <class TT>
 __device__ inline void tile_partial(typename TT::T* lds, double* part, int S, const double (&v)[TT::VEC], int s0) {
     constexpr int kPerRow = TT::kSamples;
@@ -1503,9 +1504,9 @@ __global__ __launch_bounds__(kTileThreads, 2 * kResidPerCu) void k_b_resid_t(Til
 // k_b_cg_spmv and k_b_cg_spmv_w from tiles in LDS: 64 samples per unit, a float4
 // per lane, for 64 FP32 samples; 16 per unit otherwise.  Gathers from L2 are bound
 // by the texture unit's four lanes per cycle, these by LDS and the nodes' staging:
-// 64 FP32 samples at 282,897 nodes 93 -> 54 us, at 26,325 nodes 11.1 -> 9.3 (also
+// 64 FP32 samples at 282,897 nodes 93 -> 45 us, at 25,785 nodes 11.1 -> 9.0 (also
 // with fewer units than two per block); 24 FP64 samples at 38,025 nodes
-// 24.2 -> 12.8.  Two (float4) and three blocks per CU; at four the float4 form's
+// 24.2 -> 11.9.  Two (float4) and three blocks per CU; at four the float4 form's
 // registers spill (123 us).
 template <class TT>
 constexpr int kSolvePerCu = TT::VEC == 1 ? 3 : 2;
@@ -1548,9 +1549,11 @@ __global__ __launch_bounds__(kTileThreads, 2 * kSolvePerCu<TT>) void k_b_cg_spmv
 }
 
 // k_b_up and k_b_up_w from tiles in LDS (rows of about 27 entries: two chunks of
-// slots): 64 FP32 samples at 282,897 nodes 101 us, where prolongation and
-// post-smoothing took 49 + 88 from L2; 12.3 -> 9.9 against k_b_up_w at 26,325
-// nodes; 24 FP64 samples at 38,025 nodes 41 -> 21
+// slots; tiles of up to 192 nodes, since 128 with the coarse ones among them hold
+// 26 rows and leave lanes idle): 64 FP32 samples at 282,897 nodes 62 us, where
+// prolongation and post-smoothing took 49 + 88 from L2 (with 128, 160 and 224 nodes
+// 81, 64 and 64); 12.3 -> 9.4 against k_b_up_w at 25,785 nodes; 24 FP64 samples at
+// 38,025 nodes 41 -> 17
 template <class TT>
 __global__ __launch_bounds__(kTileThreads, 4) void k_b_up_t(TileArgs t, const typename TT::T* __restrict__ w,
                                                             const typename TT::T* __restrict__ r,
@@ -1577,6 +1580,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void k_b_up_t(TileArgs t, const ty
     tile_partial<TT>(lds, part, t.S, v, s0);
 }
 constexpr int kUpPerCu = 2;
+constexpr int kUpNodes = 192;
 
 // y = M x (the V-cycle's restrictions and its way up below level 0; any sample count
 // but 64 in FP32).  A row and 16 samples per wavefront, or per block of four
@@ -2321,19 +2325,21 @@ struct SlotOp {
 };
 
 // Tiles of a SlotOp's rows (see TileArgs): a tile starts at the first row that
-// no tile has and takes, as long as they fit, the row that adds the fewest nodes,
-// among the rows that are nodes of the tile already: 4.1 nodes per row on the
-// 282,897-node cuboid, where 32 consecutive rows of its Z-order
-// numbering need 5.  None (nt = 0) when a row alone refers to too many
-// nodes, or when there are fewer than 1,024 units, two for each block (the
-// smaller problems sit in L2, where a gather's latency is all it costs).
+// no tile has and takes, as long as they fit, the row that adds the fewest nodes
+// among the rows that are nodes of the tile already, and the next row of the
+// numbering when none of those fits: 31.7 of 32 rows per tile on the 282,897-node
+// cuboid (28 without the next row, and the kernels 5 to 30 per cent slower), 4
+// nodes per row where 32 consecutive rows of its Z-order numbering need 5.
+// None (nt = 0) when a row alone refers to too many nodes, or when there are fewer
+// than 1,024 units, two for each block (the smaller problems sit in L2, where a
+// gather's latency is all it costs).
 struct TileOp {
     int nt = 0;
     DevBuf<int> row0, node0, nodes;
     DevBuf<TileRow> rows;
     DevBuf<unsigned short> loc;
 
-    int build(const SlotOp& op, hipStream_t s) {
+    int build(const SlotOp& op, hipStream_t s, int max_nodes = kTileNodes) {
         nt = 0;
         const int n = op.n, nc = op.ncols, nch = (op.S + kTileS - 1) / kTileS;
         if (n > nc || (int64_t)n * nch < (int64_t)1024 * kTileRows) return TM_OK;
@@ -2343,7 +2349,7 @@ struct TileOp {
             bool self = false;
             for (int q = op.h_rp[i]; q < op.h_rp[i + 1]; ++q) self = self || op.h_ci[q] == i;
             deg[i] = op.h_rp[i + 1] - op.h_rp[i] + (self ? 0 : 1);
-            if (deg[i] > kTileNodes) return TM_OK;
+            if (deg[i] > max_nodes) return TM_OK;
         }
         // rows by column: the rows that refer to a node
         std::vector<int> tp((size_t)nc + 1, 0), tr(op.h_ci.size());
@@ -2380,7 +2386,7 @@ struct TileOp {
                 for (int q = op.h_rp[row]; q < op.h_rp[row + 1]; ++q) add_node(op.h_ci[q]);
                 row = -1;
                 if ((int)(order.size() - rbase) == kTileRows) break;
-                const int room = kTileNodes - (int)(hnode.size() - base);
+                const int room = max_nodes - (int)(hnode.size() - base);
                 int best = 0;
                 size_t kept = 0;
                 for (size_t k = 0; k < cand.size(); ++k) {
@@ -2394,6 +2400,9 @@ struct TileOp {
                     }
                 }
                 cand.resize(kept);
+                if (row >= 0) continue;
+                while (first < n && taken[first]) ++first;
+                if (first < n && deg[first] <= room) row = first;  // no neighbour fits: the next row
             }
             for (size_t k = rbase; k < order.size(); ++k) {
                 const int i = order[k];
@@ -2667,13 +2676,13 @@ struct BatchSolver {
     // the level-0 products of the inner solve from tiles
     bool tiled() const { return t0.nt > 0 && tu.nt > 0; }
     // f(tile type) for this batch: a float4 per lane for 64 FP32 samples
-    template <class F>
+    template <int NODES, class F>
     void with_tile_type(F&& f) const {
         if constexpr (sizeof(T) == 4) {
-            if (S == kMaxS) return f(TileType<T, 4, true>{});
+            if (S == kMaxS) return f(TileType<T, 4, true, NODES>{});
         }
-        if (S % (16 / (int)sizeof(T)) == 0) f(TileType<T, 1, true>{});
-        else f(TileType<T, 1, false>{});
+        if (S % (16 / (int)sizeof(T)) == 0) f(TileType<T, 1, true, NODES>{});
+        else f(TileType<T, 1, false, NODES>{});
     }
     TileOp tu;                    // tiles of level 0's way up
     struct LvOps {
@@ -2743,11 +2752,11 @@ struct BatchSolver {
             }
             TM_CHECK(lo[l].U.build(V.n, V.n + nnext, up.rp.data(), up.ci.data(), S, s));
             TM_CHECK(lo[l].U.values(up.v, lo[l].wU, s));
-            if (l == 0) TM_CHECK(tu.build(lo[0].U, s));
+            if (l == 0) TM_CHECK(tu.build(lo[0].U, s, kUpNodes));
         }
         Gq = Gz = G;
         if (tiled())
-            with_tile_type([&](auto tt) {
+            with_tile_type<kTileNodes>([&](auto tt) {
                 using TT = decltype(tt);
                 const int nch = (S + TT::kSamples - 1) / TT::kSamples;
                 Gq = tile_blocks(nch, kSolvePerCu<TT>);
@@ -2821,7 +2830,7 @@ struct BatchSolver {
     // level 0 upwards: z = U [r | x_c], partial (r, z)
     void up0(const T* r, T* z, double* prz, hipStream_t s) {
         if (tiled()) {
-            with_tile_type([&](auto tt) {
+            with_tile_type<kUpNodes>([&](auto tt) {
                 using TT = decltype(tt);
                 hipLaunchKernelGGL(k_b_up_t<TT>, dim3(Gz), dim3(kTileThreads), 0, s, tu.args(lo[0].U, TT::kSamples),
                                    (const T*)lo[0].wU.p, r, z, gate(), prz);
@@ -2925,7 +2934,7 @@ struct BatchSolver {
     // iteration k: q = A p_k = A z_k + beta q, partial (z_k, q)
     void cg_spmv(const T* zk, int k, double* pzq, hipStream_t s) {
         if (tiled()) {
-            with_tile_type([&](auto tt) {
+            with_tile_type<kTileNodes>([&](auto tt) {
                 using TT = decltype(tt);
                 hipLaunchKernelGGL(k_b_cg_spmv_t<TT>, dim3(Gq), dim3(kTileThreads), 0, s, t0.args(sl0, TT::kSamples),
                                    (const T*)wA0.p, zk, q.p, k, (const BState*)bst.p, pzq);
