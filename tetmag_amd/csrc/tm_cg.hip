@@ -30,8 +30,8 @@
 // launches (of a four-level one eight), where separate smoothing, restriction,
 // prolongation and update kernels took eight (fifteen): a cold Neumann solve
 // of 71,825 nodes 1,178 -> 791 us, one FP64 evaluation at 29,760 nodes 710 ->
-// 352 us, at 282,897 nodes 3.49 -> 2.89 ms (2.05 ms of it the boundary
-// product).
+// 303 us, at 282,897 nodes 3.43 -> 2.79 ms (2.06 ms of it the boundary
+// product), the other kernels' changes included.
 #include <algorithm>
 #include <cmath>
 
