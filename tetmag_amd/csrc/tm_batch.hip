@@ -1504,9 +1504,9 @@ __global__ __launch_bounds__(kTileThreads, 2 * kResidPerCu) void k_b_resid_t(Til
 // k_b_cg_spmv and k_b_cg_spmv_w from tiles in LDS: 64 samples per unit, a float4
 // per lane, for 64 FP32 samples; 16 per unit otherwise.  Gathers from L2 are bound
 // by the texture unit's four lanes per cycle, these by LDS and the nodes' staging:
-// 64 FP32 samples at 282,897 nodes 93 -> 45 us, at 25,785 nodes 11.1 -> 9.0 (also
+// 64 FP32 samples at 282,897 nodes 96 -> 55 us, at 25,785 nodes a sixth less (also
 // with fewer units than two per block); 24 FP64 samples at 38,025 nodes
-// 24.2 -> 11.9.  Two (float4) and three blocks per CU; at four the float4 form's
+// 24.2 -> 12.8.  Two (float4) and three blocks per CU; at four the float4 form's
 // registers spill (123 us).
 template <class TT>
 constexpr int kSolvePerCu = TT::VEC == 1 ? 3 : 2;
@@ -1550,10 +1550,10 @@ __global__ __launch_bounds__(kTileThreads, 2 * kSolvePerCu<TT>) void k_b_cg_spmv
 
 // k_b_up and k_b_up_w from tiles in LDS (rows of about 27 entries: two chunks of
 // slots; tiles of up to 192 nodes, since 128 with the coarse ones among them hold
-// 26 rows and leave lanes idle): 64 FP32 samples at 282,897 nodes 62 us, where
-// prolongation and post-smoothing took 49 + 88 from L2 (with 128, 160 and 224 nodes
-// 81, 64 and 64); 12.3 -> 9.4 against k_b_up_w at 25,785 nodes; 24 FP64 samples at
-// 38,025 nodes 41 -> 17
+// 26 rows and leave lanes idle): 64 FP32 samples at 282,897 nodes 83 us, where
+// prolongation and post-smoothing took 58 + 91 from L2 (160 and 224 nodes: 3 per
+// cent slower); at 25,785 nodes a quarter less than k_b_up_w; 24 FP64 samples at
+// 38,025 nodes 41 -> 18
 template <class TT>
 __global__ __launch_bounds__(kTileThreads, 4) void k_b_up_t(TileArgs t, const typename TT::T* __restrict__ w,
                                                             const typename TT::T* __restrict__ r,
@@ -2045,7 +2045,7 @@ __global__ __launch_bounds__(kBlock) void k_b_i8_uslice(int b, int S, int nC, co
 // afterwards, and B's digits of chunks c + 1 and c + 2 into a rotation of three
 // register sets: 8 wavefronts then keep 80 KB per CU in flight, with one chunk
 // ahead (40 KB) every wavefront waited for memory.  Bound by HBM and the
-// matrix cores alike: 40,930 boundary nodes and 64 samples 1,700 -> 1,440 us, B's
+// matrix cores alike: 40,962 boundary nodes and 64 samples 1,700 -> 1,440 us, B's
 // 8.4 GB of digits at 5.8 TB/s (the 131 M products alone: 1.5 ms at the 2.86
 // POPS that the instruction sustains over long runs, 0.86 at its peak).
 // v_mfma_i32_16x16x64_i8: A lane l = row l % 16, B lane l = column l % 16,
