@@ -2045,8 +2045,8 @@ __global__ __launch_bounds__(kBlock) void k_b_i8_uslice(int b, int S, int nC, co
 // afterwards, and B's digits of chunks c + 1 and c + 2 into a rotation of three
 // register sets: 8 wavefronts then keep 80 KB per CU in flight, with one chunk
 // ahead (40 KB) every wavefront waited for memory.  Bound by HBM and the
-// matrix cores alike: 40,962 boundary nodes and 64 samples 1,700 -> 1,440 us, B's
-// 8.4 GB of digits at 5.8 TB/s (the 131 M products alone: 1.5 ms at the 2.86
+// matrix cores alike: 40,962 boundary nodes and 64 samples 1,700 -> 1,440 us (up
+// to 1,530 from box to box), B's 8.4 GB of digits at 5.8 TB/s (the 131 M products alone: 1.5 ms at the 2.86
 // POPS that the instruction sustains over long runs, 0.86 at its peak).
 // v_mfma_i32_16x16x64_i8: A lane l = row l % 16, B lane l = column l % 16,
 // both the 16 k of block l / 16; D lane l register r = C[4 (l / 16) + r][l % 16].
