@@ -228,8 +228,11 @@ int tm_bem_apply(tm_ctx* c, const double* ub, int uwhere, double* gb, int gwhere
  * products of the column splits live in a static device array of 32 MiB
  * (4,194,304 doubles) that every GPU the library runs on holds until the
  * process ends; sizes whose partials do not fit (bnx above about 92,000)
- * return TM_ERR_BAD_ARG before any device work.  Same kernels and results
- * as tm_bem_apply.  Calls that overlap on one GPU share that array and race.
+ * return TM_ERR_BAD_ARG before any device work.  Partials have the stride ld:
+ * a block of a larger matrix uses fewer splits where its ld leaves room for
+ * fewer (bnx <= 511 up to ld = 4,194,304; bnx = 4,111 up to 262,144; 8,192 up to
+ * 131,072).  Same kernels as tm_bem_apply, and the same results up to the
+ * order of the splits' sums.  Calls that overlap on one GPU share that array and race.
  * The array's address on a GPU is looked up when tm_set_device selects it,
  * else on the first call there (call tm_set_device before a capture). */
 int tm_bem_apply_noalloc(int bnx, int ld, const double* B, const double* x, double* y, void* stream);

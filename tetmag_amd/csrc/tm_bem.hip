@@ -320,30 +320,44 @@ int bem_assemble(int b, int ld, int nbel, const double* bxyz, const int* faces, 
     return TM_OK;
 }
 
-int bem_gemv_splits(int b) {
+// column splits of the product, each of at least min_cols columns
+static int gemv_splits(int b, int min_cols) {
     const int tiles = (b + kGemvTile - 1) / kGemvTile;
-    // >= 1024 blocks (four per CU, what its registers hold), down to 16
-    // columns a block: with 256 a small matrix left most of the chip idle
-    // (b = 1,122: 66 us on 4 blocks; b = 7,680: 98 us on 120)
     int splits = (1024 + tiles - 1) / tiles;
-    const int min_cols = 16;
     splits = std::min(splits, std::max(1, b / min_cols));
     while ((b + splits - 1) / splits > kGemvMaxCols) ++splits;
     return std::max(1, splits);
 }
 
+// >= 1024 blocks (four per CU, what its registers hold), down to 16
+// columns a block: with 256 a small matrix left most of the chip idle
+// (b = 1,122: 66 us on 4 blocks; b = 7,680: 98 us on 120)
+int bem_gemv_splits(int b) { return gemv_splits(b, 16); }
+
 // y = B x with x optionally gathered through gidx, y optionally scattered to
 // dst via sidx.  part needs splits * ld doubles.
-int bem_gemv(int b, int ld, const double* B, const double* src, const int* gidx, double* part, double* y,
-             const int* sidx, double* dst, hipStream_t s) {
+int bem_gemv_split(int b, int ld, int splits, const double* B, const double* src, const int* gidx, double* part,
+                   double* y, const int* sidx, double* dst, hipStream_t s) {
     if (ld % 2 != 0) return TM_ERR_BAD_ARG;
     const int tiles = (b + kGemvTile - 1) / kGemvTile;
-    const int splits = bem_gemv_splits(b);
     const int cps = (b + splits - 1) / splits;
     hipLaunchKernelGGL(k_bem_gemv_part, dim3(tiles, splits), dim3(kBlock), 0, s, b, ld, B, src, gidx, cps, part);
     hipLaunchKernelGGL(k_bem_gemv_finish, dim3(grid_for(b, kFinishRows)), dim3(kBlock), 0, s, b, ld, splits, part, y, sidx, dst);
     TM_HIP(hipGetLastError());
     return TM_OK;
+}
+
+int bem_gemv(int b, int ld, const double* B, const double* src, const int* gidx, double* part, double* y,
+             const int* sidx, double* dst, hipStream_t s) {
+    return bem_gemv_split(b, ld, bem_gemv_splits(b), B, src, gidx, part, y, sidx, dst, s);
+}
+
+// Splits for a caller with room for `room` doubles of partials: fewer where not
+// all fit (a small block of a matrix with a large ld), down to 256 columns each; 0
+// when those do not fit either.
+int bem_gemv_splits_within(int b, int ld, size_t room) {
+    const size_t fit = room / (size_t)ld;
+    return (size_t)gemv_splits(b, 256) <= fit ? (int)std::min((size_t)bem_gemv_splits(b), fit) : 0;
 }
 
 // y = B^T x with x optionally gathered through gidx (into xbuf, b doubles),
@@ -408,10 +422,12 @@ extern "C" {
 int tm_bem_apply_noalloc(int bnx, int ld, const double* B, const double* x, double* y, void* stream) {
     if (bnx <= 0 || ld < bnx || ld % 2 != 0 || !B || !x || !y) return TM_ERR_BAD_ARG;
     if (reinterpret_cast<uintptr_t>(B) % 16 != 0) return TM_ERR_BAD_ARG;  // 16-byte loads of column pairs
-    if ((size_t)tmh::bem_gemv_splits(bnx) * (size_t)ld > kNoallocScratchDoubles) return TM_ERR_BAD_ARG;
+    const int splits = tmh::bem_gemv_splits_within(bnx, ld, kNoallocScratchDoubles);
+    if (splits == 0) return TM_ERR_BAD_ARG;
     double* part = nullptr;
     TM_CHECK(noalloc_scratch(&part));
-    return tmh::bem_gemv(bnx, ld, B, x, nullptr, part, y, nullptr, nullptr, static_cast<hipStream_t>(stream));
+    return tmh::bem_gemv_split(bnx, ld, splits, B, x, nullptr, part, y, nullptr, nullptr,
+                               static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"
