@@ -51,3 +51,25 @@ def test_product_of_a_block(gpu_available, b, ld):
     torch.cuda.synchronize()
     M = B[:, :b].T.contiguous()
     assert bool(((y - M @ x).abs() <= 2 * b * 2.3e-16 * (M.abs() @ x.abs())).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b, ld, i0", [(64, 1000, 936), (1121, 5000, 3878), (2050, 6000, 3950), (4110, 4200, 90)])
+def test_block_at_the_end_of_its_matrix(gpu_available, b, ld, i0):
+    """The last rows and columns of a matrix, whose memory ends with the block's
+    last column: only rows of the block are read (an odd b shares its last pair
+    with the row after it), and what surrounds it (NaN here) has no part in the sums."""
+    import torch
+    N, f = _noalloc()
+    assert i0 % 2 == 0 and b <= ld - i0 <= b + 1
+    g = torch.Generator(device="cuda").manual_seed(b)
+    A = torch.full((b, ld), float("nan"), dtype=torch.float64, device="cuda")  # column j at A[j]
+    A[:, i0:i0 + b] = torch.randn((b, b), generator=g, dtype=torch.float64, device="cuda")
+    x = torch.randn(b, generator=g, dtype=torch.float64, device="cuda")
+    y = torch.full((b,), float("nan"), dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    print("b", b, "ld", ld, "first row", i0, flush=True)
+    assert f(b, ld, A.data_ptr() + 8 * i0, x.data_ptr(), y.data_ptr(), None) == N.TM_OK
+    torch.cuda.synchronize()
+    M = A[:, i0:i0 + b].T.contiguous()
+    assert bool(((y - M @ x).abs() <= 2 * b * 2.3e-16 * (M.abs() @ x.abs())).all())

@@ -167,7 +167,7 @@ __global__ __launch_bounds__(kBlock) void k_bem_gemv_part(int b, int ld, const d
     for (int k = 0; k < 4; ++k) acc[k] = dbl2{0.0, 0.0};
     bool valid[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) valid[k] = (r0 + 512 * k) < ld;  // rows in [b, ld) are padding (zero)
+    for (int k = 0; k < 4; ++k) valid[k] = (r0 + 512 * k) < b;  // (not < ld: memory may end after the last column's b rows)
     int c = c0;
     // four columns per step: 16 loads of 16 bytes in flight per thread
     for (; c + 3 < c1; c += 4) {
