@@ -475,11 +475,9 @@ __global__ __launch_bounds__(kBlock) void k_b_sum2(size_t tot, const double* __r
         c[e] = a[e] + b[e];
 }
 
-// x += sum_k alpha_k p_k of an inner solve of K iterations, from the kept
-// preconditioned residuals z_i (ring of [n][S] vectors): p_k = z_k +
-// beta_k p_{k-1} gives sum_k alpha_k p_k = sum_i c_i z_i with c_{K-1} =
-// alpha_{K-1}, c_i = alpha_i + beta_{i+1} c_{i+1} (alpha_i in ah[i * kMaxS +
-// s], beta_i in bh[i * kMaxS + s]).  Iterations a sample did not take have
+// x += sum_k alpha_k p_k = sum_i c_i z_i of an inner solve of K iterations, from
+// the kept preconditioned residuals z_i (ring of [n][S] vectors) and the
+// alpha_i, beta_i of every sample (ah, bh: [i][kMaxS]).  Iterations a sample did not take have
 // alpha 0 (and beta 0 after them), so c_i = 0 selects their z_i (whose
 // contents may be stale) out of the sum.
 template <typename T>
@@ -488,12 +486,11 @@ __global__ __launch_bounds__(kBlock) void k_b_combine(size_t NS, int S, int K, c
                                                       double* __restrict__ x) {
     for (size_t e = (size_t)blockIdx.x * kBlock + threadIdx.x; e < NS; e += (size_t)gridDim.x * kBlock) {
         const int sm = (int)(e % S);
-        double acc = 0.0, c = 0.0;
-        for (int i = K - 1; i >= 0; --i) {
-            c = ah[i * kMaxS + sm] + bh[(i + 1) * kMaxS + sm] * c;
+        double acc = 0.0;
+        combination_coefficients(K, ah + sm, bh + sm, kMaxS, [&](int i, double c) {
             const T v = ring[(size_t)i * NS + e];
             acc += c != 0.0 ? c * (double)v : 0.0;
-        }
+        });
         x[e] += acc;
     }
 }
@@ -503,11 +500,7 @@ __global__ void k_b_coef(int S, int K, const double* __restrict__ ah, const doub
                          double* __restrict__ ch) {
     const int sm = threadIdx.x;
     if (sm >= S) return;
-    double c = 0.0;
-    for (int i = K - 1; i >= 0; --i) {
-        c = ah[i * kMaxS + sm] + bh[(i + 1) * kMaxS + sm] * c;
-        ch[i * kMaxS + sm] = c;
-    }
+    combination_coefficients(K, ah + sm, bh + sm, kMaxS, [&](int i, double c) { ch[i * kMaxS + sm] = c; });
 }
 
 // k_b_combine for S = 64 with the c_i from k_b_coef (staged in LDS, K <=

@@ -500,6 +500,22 @@ __host__ __device__ inline void win_coefficients(int cnt, const double* t, doubl
     }
 }
 
+// f(i, c_i) for i = K - 1 .. 0: the coefficients of sum_k alpha_k p_k over the
+// preconditioned residuals z_i of K >= 1 CG iterations (p_k = z_k + beta_k p_{k-1}):
+// c_{K-1} = alpha_{K-1}, c_i = alpha_i + beta_{i+1} c_{i+1}.  alpha_i in
+// ah[i * stride], beta_i in bh[i * stride].  beta_K is not read: it belongs to the
+// iteration that was not taken, and nothing has written it when the V-cycle
+// after the last iteration was left out.
+template <class F>
+__host__ __device__ inline void combination_coefficients(int K, const double* ah, const double* bh, int stride,
+                                                         F&& f) {
+    double c = 0.0;
+    for (int i = K - 1; i >= 0; --i) {
+        c = ah[(size_t)i * stride] + (i + 1 < K ? bh[(size_t)(i + 1) * stride] * c : 0.0);
+        f(i, c);
+    }
+}
+
 struct CgState {
     double gam[2];   // (r, z) of iterations k (slot k & 1)
     double bb;       // (b, b)
