@@ -447,7 +447,10 @@ int tm_batch_set_zeeman(tm_batch* b, const double* h3s);
 int tm_batch_set_mag(tm_batch* b, const double* m, int where);
 int tm_batch_get_mag(tm_batch* b, double* m, int where);
 /* One Heff + LLG RHS evaluation of every sample (demag recomputed; solves
- * warm-started per sample).  m == NULL uses the batch magnetisation. */
+ * warm-started per sample).  m == NULL uses the batch magnetisation.  Every
+ * output is written also when the call returns TM_ERR_MAXITER or
+ * TM_ERR_NONFINITE: in some sample a solve missed the tolerance, or met NaN or
+ * Inf (that sample's values are then not finite, the others as without it). */
 int tm_batch_eval_rhs(tm_batch* b, const double* m, int mwhere, double alpha, int variant, double* dmdt, int dwhere,
                       double* heff, int hwhere, tm_batch_stats* stats);
 int tm_batch_get_potentials(tm_batch* b, double* u1, double* u2, int where);

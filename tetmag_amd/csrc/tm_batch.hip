@@ -55,7 +55,7 @@ struct BState {
 struct OState {
     double bb[kMaxS];
     double rr[kMaxS];
-    int done[kMaxS];
+    int done[kMaxS];  // 0 going on, 1 at the tolerance, 2 given up: the residual is not finite
 };
 
 // Wavefront w of block b walks rows b*4 + w, then + 4*G, ...  (A contiguous
@@ -453,7 +453,7 @@ __global__ void k_b_outer_red(int G, int S, const double* part_bb, const double*
         os->bb[s] = bb;
         os->rr[s] = rr;
         const bool done = !(rr > tol * tol * bb) || !std::isfinite(rr);
-        os->done[s] = done ? 1 : 0;
+        os->done[s] = !std::isfinite(rr) || !std::isfinite(bb) ? 2 : done ? 1 : 0;
         // inner target: the final tolerance, or a relative itol for the
         // refinement steps, whichever is looser
         const double a2 = tol * tol * bb;
@@ -2175,9 +2175,10 @@ __global__ void k_b_zero_small(int cnt, double* p) {
 }
 
 // *fail += number of samples whose outer residual missed the tolerance
-__global__ void k_b_count_undone(int S, const OState* os, unsigned* fail) {
+// *fail, *bad: the samples that missed the tolerance, and those that are not finite
+__global__ void k_b_count_undone(int S, const OState* os, unsigned* fail, unsigned* bad) {
     const int s = threadIdx.x;
-    if (s < S && !os->done[s]) atomicAdd(fail, 1u);
+    if (s < S && os->done[s] != 1) atomicAdd(os->done[s] == 0 ? fail : bad, 1u);
 }
 
 // every sample active with finite CG scalars (kernel timing only)
@@ -2586,8 +2587,9 @@ __global__ __launch_bounds__(kWave) void k_b_win_solve(int S, WinState* ws, cons
     for (int i = 0; i < kSolveWindow; ++i) ws->a[i][s] = a[i];
 }
 
-// x0 = sum_i a_i x_slot(i) (nothing when the window is empty), lane = sample
-// and the fixed rows' values x = b (also with an empty window)
+// x0 = sum_i a_i x_slot(i) (the caller's x when the window is empty), lane = sample,
+// and the fixed rows' values x = b.  A start that is not finite is zero: an
+// earlier right-hand side of that sample was not, and its solution is kept.
 __global__ __launch_bounds__(kBlock) void k_b_win_combine(int n, int S, const WinState* ws,
                                                           const double* __restrict__ Xw,
                                                           const unsigned char* __restrict__ fixed,
@@ -2618,12 +2620,12 @@ __global__ __launch_bounds__(kBlock) void k_b_win_combine(int n, int S, const Wi
                     acc1 += a[i] * src[i][e1];
                     acc2 += a[i] * src[i][e2];
                 }
-            if (fixed[row]) x[e1] = b[e1];
-            else if (cnt > 0) x[e1] = acc1;
-            if (two) {
-                if (fixed[row2]) x[e2] = b[e2];
-                else if (cnt > 0) x[e2] = acc2;
+            if (cnt == 0) {
+                acc1 = x[e1];
+                acc2 = x[e2];
             }
+            x[e1] = fixed[row] ? b[e1] : std::isfinite(acc1) ? acc1 : 0.0;
+            if (two) x[e2] = fixed[row2] ? b[e2] : std::isfinite(acc2) ? acc2 : 0.0;
         }
     }
 }
@@ -2991,12 +2993,14 @@ struct BatchSolver {
                         short_seen = true;
                     }
                 }
-                bool all = true;
+                bool all = true, finite = true;
                 double worst = 0.0;
                 for (int k = 0; k < S; ++k) {
                     all = all && h_ost->done[k];
+                    finite = finite && h_ost->done[k] != 2;
                     if (h_ost->bb[k] > 0) worst = std::max(worst, std::sqrt(h_ost->rr[k] / h_ost->bb[k]));
                 }
+                if (!finite) worst = NAN;
                 if (maxrel) *maxrel = worst;
                 if (all || outer >= 8 || inner_total >= maxit) break;
             }
@@ -3063,9 +3067,12 @@ struct BatchSolver {
         last_outer = outer;
         spec_next = outer == 1 && !short_seen;
         TM_HIP(hipGetLastError());
-        bool all = true;
-        for (int k = 0; k < S; ++k) all = all && h_ost->done[k];
-        return all ? TM_OK : TM_ERR_MAXITER;
+        int st = TM_OK;
+        for (int k = 0; k < S; ++k) {
+            if (h_ost->done[k] == 2) return TM_ERR_NONFINITE;
+            if (h_ost->done[k] == 0) st = TM_ERR_MAXITER;
+        }
+        return st;
     }
 
     int last_outer = 0;  // refinement steps of the last host-polled solve
@@ -3129,12 +3136,13 @@ struct BatchSolver {
     // steps and iterations past convergence cost only their launches, and
     // iterations a sample did not take carry alpha = beta = 0 into the
     // combination.  A final residual check adds the number of samples that
-    // missed the tolerance to *fail on the device, and track[o] keeps the
-    // largest iteration count of refinement step o.
+    // missed the tolerance to *fail on the device, the number of those that are
+    // not finite to *bad, and track[o] keeps the largest iteration count of
+    // refinement step o.
     int enqueue(const double* b, double* x, double tol, int nouter, const int* ninner, hipStream_t s,
-                unsigned* fail, int* track) {
+                unsigned* fail, unsigned* bad, int* track) {
         if (cg->precond != TM_PRECOND_AMG || cg->amg.levels.empty()) return TM_ERR_UNSUPPORTED;
-        if (nouter < 0 || nouter > kMaxOuter || !fail || !track) return TM_ERR_BAD_ARG;
+        if (nouter < 0 || nouter > kMaxOuter || !fail || !bad || !track) return TM_ERR_BAD_ARG;
         const size_t NS = (size_t)n * S;
         double* pbb = part.p;
         double* prr = part.p + (size_t)S * gmax();
@@ -3172,7 +3180,7 @@ struct BatchSolver {
                 hipLaunchKernelGGL((k_b_combine<T>), dim3(elem_grid(NS)), dim3(kBlock), 0, s, NS, S, K,
                                    (const T*)ring.p, (const double*)ahist.p, (const double*)bhist.p, x);
         }
-        hipLaunchKernelGGL(k_b_count_undone, dim3(1), dim3(kMaxS), 0, s, S, (const OState*)ost.p, fail);
+        hipLaunchKernelGGL(k_b_count_undone, dim3(1), dim3(kMaxS), 0, s, S, (const OState*)ost.p, fail, bad);
         if (use_window) win_record(x, s);
         TM_HIP(hipGetLastError());
         return TM_OK;
@@ -3211,12 +3219,13 @@ struct tm_batch {
     float i8ms = 0.0f, i8ms_first = 0.0f;
     DevBuf<double> rk_k[4], rk_base;   // RK4 stages and the step's start state
     // graph-replayed RK4 steps: samples whose fixed-budget solve missed the
-    // tolerance and the iterations that each refinement step of the two
-    // solves took (device counters), and the budgets: refinement
+    // tolerance, those that were not finite, and the iterations that each
+    // refinement step of the two solves took (device counters), and the budgets: refinement
     // steps and inner iterations per step of the Neumann (0) and Dirichlet (1)
     // solves
     static constexpr int kMaxBud = 8;
-    DevBuf<unsigned> rk_fail;  // 1 + 2 kMaxBud
+    static constexpr int kCounts = 2 + 2 * kMaxBud;  // missed, not finite, iterations
+    DevBuf<unsigned> rk_fail;
     bool bud_set = false;
     int bud_outer[2] = {0, 0};
     int bud_inner[2][kMaxBud] = {};
@@ -3771,19 +3780,21 @@ int eval_enqueue(tm_batch* bt, double alpha, int variant, double* dmdt) {
     hipStream_t s = bt->stream;
     const CtxView& v = bt->cv;
     constexpr int kMaxBud = tm_batch::kMaxBud;
-    unsigned* fail = bt->rk_fail.p;
-    int* track = reinterpret_cast<int*>(fail + 1);
+    unsigned *fail = bt->rk_fail.p, *bad = fail + 1;
+    int* track = reinterpret_cast<int*>(fail + 2);
     launch_div(bt);
     TM_HIP(hipGetLastError());
     if (bt->prec == TM_PREC_FP64)
-        TM_CHECK(bt->sN64.enqueue(bt->rhsN.p, bt->u1.p, v.tol, bt->bud_outer[0], bt->bud_inner[0], s, fail, track));
+        TM_CHECK(bt->sN64.enqueue(bt->rhsN.p, bt->u1.p, v.tol, bt->bud_outer[0], bt->bud_inner[0], s, fail, bad, track));
     else
-        TM_CHECK(bt->sN32.enqueue(bt->rhsN.p, bt->u1.p, v.tol, bt->bud_outer[0], bt->bud_inner[0], s, fail, track));
+        TM_CHECK(bt->sN32.enqueue(bt->rhsN.p, bt->u1.p, v.tol, bt->bud_outer[0], bt->bud_inner[0], s, fail, bad, track));
     TM_CHECK(boundary_product(bt, v.bnodes, bt->u1.p, bt->rhsD.p));
     if (bt->prec == TM_PREC_FP64)
-        TM_CHECK(bt->sD64.enqueue(bt->rhsD.p, bt->u2.p, v.tol, bt->bud_outer[1], bt->bud_inner[1], s, fail, track + kMaxBud));
+        TM_CHECK(bt->sD64.enqueue(bt->rhsD.p, bt->u2.p, v.tol, bt->bud_outer[1], bt->bud_inner[1], s, fail, bad,
+                                  track + kMaxBud));
     else
-        TM_CHECK(bt->sD32.enqueue(bt->rhsD.p, bt->u2.p, v.tol, bt->bud_outer[1], bt->bud_inner[1], s, fail, track + kMaxBud));
+        TM_CHECK(bt->sD32.enqueue(bt->rhsD.p, bt->u2.p, v.tol, bt->bud_outer[1], bt->bud_inner[1], s, fail, bad,
+                                  track + kMaxBud));
     hipLaunchKernelGGL(k_b_sum2, dim3(elem_grid(NS)), dim3(kBlock), 0, s, NS, (const double*)bt->u1.p,
                        (const double*)bt->u2.p, bt->usum.p);
     return launch_fields(bt, alpha, variant, dmdt, nullptr, false);
@@ -4000,6 +4011,14 @@ int tm_batch_get_timers(tm_batch* bt, tm_phase_times* out, int reset) {
 
 namespace {
 
+// Statuses after which every sample has its result: some may have missed the
+// tolerance, some may not be finite (the others are as without them).
+bool solved(int st) { return st == TM_OK || st == TM_ERR_MAXITER || st == TM_ERR_NONFINITE; }
+int worse(int a, int b) {
+    if (a == TM_ERR_NONFINITE || b == TM_ERR_NONFINITE) return TM_ERR_NONFINITE;
+    return a != TM_OK ? a : b;
+}
+
 // tm_batch_eval_rhs; with euler_dt > 0 the field kernel also writes the
 // Euler step of m into m2, which then becomes the batch's m
 int batch_eval(tm_batch* bt, const double* m, int mwhere, double alpha, int variant, double* dmdt, int dwhere,
@@ -4021,7 +4040,7 @@ int batch_eval(tm_batch* bt, const double* m, int mwhere, double alpha, int vari
     double rN = 0, rD = 0;
     int stN = bt->prec == TM_PREC_FP64 ? bt->sN64.solve(bt->rhsN.p, bt->u1.p, v.tol, v.maxit, s, &oN, &iN, &rN)
                                        : bt->sN32.solve(bt->rhsN.p, bt->u1.p, v.tol, v.maxit, s, &oN, &iN, &rN);
-    if (stN != TM_OK && stN != TM_ERR_MAXITER) return stN;
+    if (!solved(stN)) return stN;
     if (bt->timers) TM_HIP(hipEventRecord(bt->ev[2], s));
     // boundary integral (DemagField.cpp:184-201) as a GEMM: G = B U^T, U the
     // gathered boundary potentials of every sample
@@ -4029,7 +4048,7 @@ int batch_eval(tm_batch* bt, const double* m, int mwhere, double alpha, int vari
     if (bt->timers) TM_HIP(hipEventRecord(bt->ev[3], s));
     int stD = bt->prec == TM_PREC_FP64 ? bt->sD64.solve(bt->rhsD.p, bt->u2.p, v.tol, v.maxit, s, &oD, &iD, &rD)
                                        : bt->sD32.solve(bt->rhsD.p, bt->u2.p, v.tol, v.maxit, s, &oD, &iD, &rD);
-    if (stD != TM_OK && stD != TM_ERR_MAXITER) return stD;
+    if (!solved(stD)) return stD;
     if (bt->timers) TM_HIP(hipEventRecord(bt->ev[4], s));
     // total potential, gathered once per entry by the field kernel
     hipLaunchKernelGGL(k_b_sum2, dim3(elem_grid(NS)), dim3(kBlock), 0, s, NS, (const double*)bt->u1.p,
@@ -4068,7 +4087,7 @@ int batch_eval(tm_batch* bt, const double* m, int mwhere, double alpha, int vari
         TM_HIP(hipMemcpyAsync(stats->max_torque, bt->torque.p, sizeof(double) * S, hipMemcpyDeviceToHost, s));
         TM_HIP(hipStreamSynchronize(s));
     }
-    return stN != TM_OK ? stN : stD;
+    return worse(stN, stD);
 }
 
 }  // namespace
@@ -4093,7 +4112,7 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
     const size_t NS = (size_t)bt->n * bt->S, N3 = 3 * NS;
     for (auto& k : bt->rk_k) TM_CHECK(k.alloc(N3));
     TM_CHECK(bt->rk_base.alloc(N3));
-    constexpr int kMaxBud = tm_batch::kMaxBud, kCount = 1 + 2 * kMaxBud;
+    constexpr int kMaxBud = tm_batch::kMaxBud, kCount = tm_batch::kCounts;
     TM_CHECK(bt->rk_fail.alloc(kCount));
     hipStream_t s = bt->stream;
     const dim3 g(elem_grid(N3));
@@ -4156,8 +4175,8 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
             const bool fin = final_step && k == 3;
             const int r = tm_batch_eval_rhs(bt, nullptr, TM_DEVICE, alpha, variant, bt->rk_k[k].p, TM_DEVICE, nullptr,
                                             TM_DEVICE, &es);
-            if (r != TM_OK && r != TM_ERR_MAXITER) return r;
-            if (r == TM_ERR_MAXITER) st = r;
+            if (!solved(r)) return r;
+            st = worse(st, r);
             R.max_iters_neumann = std::max(R.max_iters_neumann, es.inner_neumann);
             R.max_iters_dirichlet = std::max(R.max_iters_dirichlet, es.inner_dirichlet);
             if (fin && last) *last = es;
@@ -4237,7 +4256,7 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
                 break;
             }
             for (int w = 0; w < 2; ++w) {
-                const int* took = reinterpret_cast<const int*>(counts) + 1 + w * kMaxBud;
+                const int* took = reinterpret_cast<const int*>(counts) + 2 + w * kMaxBud;
                 int sum = 0;
                 for (int k = 0; k < kMaxBud; ++k) sum += took[k];
                 (w == 0 ? R.max_iters_neumann : R.max_iters_dirichlet) =
@@ -4246,8 +4265,9 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
                     seen[w * kMaxBud + k] = std::max(seen[w * kMaxBud + k], took[k]);
             }
             ++replays;
-            if (counts[0] == 0) {
+            if (counts[0] == 0) {  // (no redo for samples that are not finite: they would end the same way)
                 R.graph_steps += 1;
+                if (counts[1] != 0) status = TM_ERR_NONFINITE;
                 if (fin && last) last->nsamples = bt->S;
                 continue;
             }
@@ -4260,11 +4280,11 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
             std::fill(seen, seen + 2 * kMaxBud, 0);
         }
         const int r = polled_step(fin, missed);
-        if (r != TM_OK && r != TM_ERR_MAXITER) {
+        if (!solved(r)) {
             status = r;
             break;
         }
-        if (r == TM_ERR_MAXITER) status = r;
+        status = worse(status, r);
     }
     tighten();
     for (int w = 0; w < 2; ++w) {
