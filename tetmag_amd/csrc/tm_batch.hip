@@ -2659,7 +2659,6 @@ __global__ void k_b_win_advance(int S, WinState* ws, const OState* os) {
 
 template <typename T>
 struct BatchSolver {
-    const CgSolver* cg = nullptr;
     int n = 0, S = 0, G = 0;
     SlotOp sl0;                   // level-0 operator in slots
     DevBuf<T> wA0;                // its weights
@@ -2687,6 +2686,12 @@ struct BatchSolver {
         DevBuf<T> wU;
     };
     std::vector<LvOps> lo;
+    // the coarsest level: its C^-1 (nc x nc), or that folded into the last
+    // restriction (nc x dense_m, see k_b_dmv for the line); a copy, since a captured step holds its
+    // address and the context's solvers may be set anew while this batch lives
+    DevBuf<double> dense;
+    int nc = 0, dense_m = 0;
+    bool folded = false;
     DevBuf<unsigned char> fixed;
     DevBuf<T> rT, q;              // rT: [r | x_c]
     static constexpr int kRing = 40;  // iterations per inner solve (a longer one is cut there; the outer loop goes on)
@@ -2717,12 +2722,17 @@ struct BatchSolver {
     }
 
     int setup(const CgSolver& solver, int S_, hipStream_t s) {
-        cg = &solver;
         n = solver.n;
         S = S_;
         G = row_grid(n);
         const AmgPrecond& M = solver.amg;
         const int L = (int)M.levels.size();
+        nc = M.nc;
+        folded = M.D.p != nullptr && !wide();
+        dense_m = folded ? M.levels[L - 1].n : nc;
+        TM_CHECK(dense.alloc((size_t)nc * dense_m));
+        TM_HIP(hipMemcpyAsync(dense.p, folded ? M.D.p : M.Cinv.p, (size_t)nc * dense_m * sizeof(double),
+                              hipMemcpyDeviceToDevice, s));
         TM_CHECK(sl0.build(n, n, solver.pat.h_rowptr.data(), solver.pat.h_csrcol.data(), S, s));
         TM_CHECK(sl0.values(solver.h_val, wA0, s));
         TM_CHECK(sl0.values(solver.h_val, wA64, s));
@@ -2735,7 +2745,7 @@ struct BatchSolver {
             const int nnext = l + 1 < L ? M.levels[l + 1].n : M.nc;
             HostCsr down, up;
             TM_CHECK(fetch_csr(V.down, down, s));
-            if (l + 1 < L || !fold()) {
+            if (l + 1 < L || !folded) {
                 TM_CHECK(lo[l].RA.build(nnext, V.n, down.rp.data(), down.ci.data(), S, s));
                 TM_CHECK(lo[l].RA.values(down.v, lo[l].wRA, s));
             }
@@ -2787,26 +2797,23 @@ struct BatchSolver {
     // z = M r (AMG V-cycle, batched) for r = [r | x_c], partial (r, z) into prz:
     // one product per level in each direction, as the single-sample solver's
     int precond(T* r, T* zout, double* prz, hipStream_t s) {
-        const AmgPrecond& M = cg->amg;
-        const int L = (int)M.levels.size();
+        const int L = (int)lo.size();
         if (L == 0) return TM_ERR_UNSUPPORTED;  // the batched solve needs at least one AMG level
         auto vec = [&](int l) { return l == 0 ? r : bx[l].p; };  // [b | x_c] of level l
-        auto tail = [&](int l) { return vec(l) + (size_t)M.levels[l].n * S; };
-        const bool dense = fold();
-        for (int l = 0; l < (dense ? L - 1 : L); ++l)
+        auto tail = [&](int l) { return vec(l) + (size_t)lo[l].U.n * S; };
+        for (int l = 0; l < (folded ? L - 1 : L); ++l)
             spmm(lo[l].RA, lo[l].wRA.p, vec(l), l + 1 < L ? vec(l + 1) : bc.p, s);
-        if (dense) dmv(M.nc, M.levels[L - 1].n, M.D.p, vec(L - 1), tail(L - 1), s);
-        else dmv(M.nc, M.nc, M.Cinv.p, bc.p, tail(L - 1), s);
+        dmv(folded ? vec(L - 1) : bc.p, tail(L - 1), s);
         for (int l = L - 1; l > 0; --l) spmm(lo[l].U, lo[l].wU.p, vec(l), tail(l - 1), s);
         up0(r, zout, prz, s);
         TM_HIP(hipGetLastError());
         return TM_OK;
     }
 
-    // C^-1 folded into the last restriction (see k_b_dmv for the line)
-    bool fold() const { return cg->amg.D.p != nullptr && !wide(); }
-    // y = D x, dense
-    void dmv(int rows, int m, const double* D, const T* x, T* y, hipStream_t s) {
+    // y = the coarsest level's dense matrix times x
+    void dmv(const T* x, T* y, hipStream_t s) {
+        const int rows = nc, m = dense_m;
+        const double* D = dense.p;
         auto run = [&](auto vec) {
             constexpr int VEC = decltype(vec)::value;
             const int nch = (S + 16 * VEC - 1) / (16 * VEC);
@@ -2949,7 +2956,7 @@ struct BatchSolver {
     // Solves A x = b for all samples ([n][S] FP64); x is the warm start.
     int solve(const double* b, double* x, double tol, int maxit, hipStream_t s, int* outer_out, int* inner_out,
               double* maxrel) {
-        if (cg->precond != TM_PRECOND_AMG || cg->amg.levels.empty()) return TM_ERR_UNSUPPORTED;
+        if (lo.empty()) return TM_ERR_UNSUPPORTED;
         const size_t NS = (size_t)n * S;
         double* pbb = part.p;
         double* prr = part.p + (size_t)S * gmax();
@@ -3084,7 +3091,7 @@ struct BatchSolver {
     // offsets (4 B) and weights once, every vector read or written once.
     template <class Timer>
     int time_kernels(hipStream_t s, Timer&& timeit, std::vector<tm_batch_kernel_time>& out) {
-        if (cg->amg.levels.empty()) return TM_ERR_UNSUPPORTED;
+        if (lo.empty()) return TM_ERR_UNSUPPORTED;
         const int e = (int)sizeof(T);
         const double nS = (double)n * S;
         double* pzq = part.p + (size_t)3 * S * gmax();
@@ -3103,17 +3110,15 @@ struct BatchSolver {
         add(sizeof(T) == 4 ? "k_b_cg_update<float>" : "k_b_cg_update<double>",
             timeit([&] { cg_update(part.p + (size_t)S * gmax(), s); }), 3.0 * nS * e);
         const LvOps& O = lo[0];
-        const AmgPrecond& M = cg->amg;
-        const double n1 = M.levels.size() > 1 ? M.levels[1].n : M.nc;
+        const double n1 = lo.size() > 1 ? lo[1].U.n : nc;
         if (O.RA.n > 0) {
-            T* y1 = M.levels.size() > 1 ? bx[1].p : bc.p;
+            T* y1 = lo.size() > 1 ? bx[1].p : bc.p;
             add(O.RA.long_rows() && wide() ? "k_b_spmm_w<long> (R(I-AwD^-1), level 0)"
                                            : "k_b_spmm (R(I-AwD^-1), level 0)",
                 timeit([&] { spmm(O.RA, O.wRA.p, rT.p, y1, s); }), slots(O.RA) * (4 + e) + nS * e + n1 * S * e);
         } else {
             add("k_b_dmv (C^-1 R(I-AwD^-1), level 0)",
-                timeit([&] { dmv(M.nc, n, M.D.p, rT.p, rT.p + (size_t)n * S, s); }),
-                8.0 * M.nc * n + nS * e + n1 * S * e);
+                timeit([&] { dmv(rT.p, rT.p + (size_t)n * S, s); }), 8.0 * nc * n + nS * e + n1 * S * e);
         }
         add(tiled() ? "k_b_up_t (level 0)" : wide() ? "k_b_up_w (level 0)" : "k_b_up (level 0)",
             timeit([&] { up0(rT.p, ring.p, prz, s); }), slots(O.U) * (4 + e) + 2.0 * nS * e + n1 * S * e);
@@ -3141,7 +3146,7 @@ struct BatchSolver {
     // refinement step o.
     int enqueue(const double* b, double* x, double tol, int nouter, const int* ninner, hipStream_t s,
                 unsigned* fail, unsigned* bad, int* track) {
-        if (cg->precond != TM_PRECOND_AMG || cg->amg.levels.empty()) return TM_ERR_UNSUPPORTED;
+        if (lo.empty()) return TM_ERR_UNSUPPORTED;
         if (nouter < 0 || nouter > kMaxOuter || !fail || !bad || !track) return TM_ERR_BAD_ARG;
         const size_t NS = (size_t)n * S;
         double* pbb = part.p;
