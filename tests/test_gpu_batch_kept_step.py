@@ -61,3 +61,58 @@ def test_survives_new_solvers_of_the_context(gpu_available, prec, precond):
         b.close()
         ca.close()
         cb.close()
+
+
+@pytest.mark.parametrize("prec", ["FP64", "MIXED_BEMI8"])
+def test_replayed_only_for_what_it_was_captured_for(gpu_available, prec):
+    """One batch runs captured, another the same calls host-polled, while what
+    the step depends on changes from call to call: the time step, the damping,
+    the LLG form, the samples' fields, the per-node field (set, changed,
+    cleared) and the buffer that holds m (an odd number of fused Euler steps
+    swaps it).  Each is returned to its first value, so that the kept step of
+    another call would fit in all but one of them."""
+    from tetmag_amd import _native as N
+    from tetmag_amd import problem as P
+    from tetmag_amd.batch import BatchContext, to_batch
+    from tetmag_amd.context import FieldContext
+    prob, dt = _problem()
+    S, n = 64, prob.n
+    m = to_batch(P.smooth_random_fields(prob.mesh, S, seed=31, lam_min=10.0, lam_max=60.0))
+    ctx = FieldContext(prob, tol=1e-12)
+    a, b = BatchContext(ctx, S, getattr(N, "TM_PREC_" + prec)), BatchContext(ctx, S, getattr(N, "TM_PREC_" + prec))
+    g = np.random.default_rng(2)
+    field = 2e5 * g.standard_normal(3 * n)
+    H0 = np.stack([np.linspace(-3e4, 3e4, S), np.zeros(S), np.full(S, 1e4)])
+    tol = 1e-11 if prec == "FP64" else 1e-9
+    calls = [("first", {}), ("again", {}), ("dt", {"dtau": 0.4 * dt}), ("dt back", {}), ("alpha", {"alpha": 0.02}),
+             ("alpha back", {}), ("form", {"variant": N.TM_LLG_NOPREC}), ("form back", {}),
+             ("samples' fields", {"H": -40 * H0}), ("samples' fields back", {}), ("node field", {"field": field}),
+             ("other node field", {"field": -field}), ("cleared", {}), ("node field again", {"field": field}),
+             ("m swapped", {"euler": 1}), ("m swapped back", {"euler": 1})]
+    replayed = 0
+    try:
+        for bc in (a, b):
+            bc.set_mag(m)
+        for name, c in calls:
+            before = a.get_mag()
+            ctx.set_hext(prob.hext, c.get("field"))
+            for bc in (a, b):
+                bc.set_zeeman(c.get("H", H0))
+                for _ in range(c.get("euler", 0)):
+                    bc.eval_euler(dt, stats=False)
+            kw = {"alpha": c.get("alpha", prob.alpha), "variant": c.get("variant", N.TM_LLG_CLASSIC)}
+            _, ra = a.run_rk4(c.get("dtau", dt), 2, use_graph=True, **kw)
+            b.run_rk4(c.get("dtau", dt), 2, **kw)
+            ctx.synchronize()
+            ma, mb = a.get_mag(), b.get_mag()
+            d, moved = rel_l2(ma, mb), rel_l2(ma, before)
+            print(f"{prec} {name}: replayed {ra['graph_steps']}, captured {ra['captures']}, apart {d:.1e}, "
+                  f"moved {moved:.1e}", flush=True)
+            replayed += ra["graph_steps"]
+            # the two drift apart from call to call: each call's own bound adds up
+            assert d < tol * (1 + [x for x, _ in calls].index(name)) and moved > 1e-4
+        assert replayed >= len(calls)
+    finally:
+        a.close()
+        b.close()
+        ctx.close()
