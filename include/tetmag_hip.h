@@ -469,8 +469,9 @@ int tm_batch_eval_euler(tm_batch* b, double alpha, int variant, double dtau, dou
  * after each step), each stage a full batched evaluation.  The hysteresis
  * driver of the reference steps one field value at a time through CVODE
  * (Hysteresis.cpp:43-169, TheLLG.cpp:578-711).  use_graph = 1: after a first
- * host-polled step has set the solver budgets (refinement steps and inner
- * iterations per step, per solve), one whole step -- four evaluations with
+ * host-polled step (of the batch, and again after tm_batch_set_mag or an
+ * evaluation of a given m) has set the solver budgets (refinement steps and
+ * inner iterations per step, per solve), one whole step -- four evaluations with
  * fixed-budget solves whose kernels return at once past convergence -- is
  * captured in a HIP graph and replayed with one host synchronisation per
  * step; a step in which a sample missed the tolerance is restored and redone

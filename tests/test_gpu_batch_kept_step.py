@@ -116,3 +116,38 @@ def test_replayed_only_for_what_it_was_captured_for(gpu_available, prec):
         a.close()
         b.close()
         ctx.close()
+
+
+@pytest.mark.parametrize("prec", ["FP64", "MIXED"])
+@pytest.mark.parametrize("how", ["set_mag", "eval_rhs"])
+def test_first_step_of_a_given_state_is_host_polled(gpu_available, prec, how):
+    """The budgets and kept solutions of one state say nothing about another: a
+    replay would miss the tolerance, be redone host-polled and be captured
+    anew.  Replays go on as soon as the state is the batch's own again."""
+    from tetmag_amd import _native as N
+    from tetmag_amd import problem as P
+    from tetmag_amd.batch import BatchContext, to_batch
+    from tetmag_amd.context import FieldContext
+    prob, dt = _problem()
+    fields = [to_batch(P.smooth_random_fields(prob.mesh, 64, seed=k, lam_min=10.0, lam_max=60.0)) for k in range(4)]
+    ctx = FieldContext(prob, tol=1e-12)
+    a, b = BatchContext(ctx, 64, getattr(N, "TM_PREC_" + prec)), BatchContext(ctx, 64, getattr(N, "TM_PREC_" + prec))
+    try:
+        for k, m in enumerate(fields):
+            for bc in (a, b):
+                if how == "set_mag":
+                    bc.set_mag(m)
+                else:
+                    bc.eval_rhs_host(m)
+            _, ra = a.run_rk4(dt, 1, use_graph=True)
+            b.run_rk4(dt, 1)
+            print(prec, how, k, {x: ra[x] for x in ("sync_steps", "graph_steps", "redone_steps", "captures")}, flush=True)
+            assert (ra["sync_steps"], ra["graph_steps"], ra["redone_steps"], ra["captures"]) == (1, 0, 0, 0)
+            replayed = sum(a.run_rk4(dt, 2, use_graph=True)[1]["graph_steps"] for _ in range(3))
+            b.run_rk4(dt, 6)
+            assert replayed >= 4
+            assert rel_l2(a.get_mag(), b.get_mag()) < (1e-11 if prec == "FP64" else 1e-9)
+    finally:
+        a.close()
+        b.close()
+        ctx.close()

@@ -3232,6 +3232,7 @@ struct tm_batch {
     static constexpr int kCounts = 2 + 2 * kMaxBud;  // missed, not finite, iterations
     DevBuf<unsigned> rk_fail;
     bool bud_set = false;
+    bool m_replaced = false;  // m was set from outside since the last step
     int bud_outer[2] = {0, 0};
     int bud_inner[2][kMaxBud] = {};
     // The captured step is kept for the next call with the same arguments
@@ -3959,6 +3960,7 @@ int tm_batch_set_zeeman(tm_batch* bt, const double* h3s) {
 
 int tm_batch_set_mag(tm_batch* bt, const double* m, int where) {
     if (!bt) return TM_ERR_BAD_ARG;
+    bt->m_replaced = true;
     return copy_in(bt->m.p, m, where, (size_t)3 * bt->n * bt->S, bt->stream);
 }
 
@@ -4035,7 +4037,10 @@ int batch_eval(tm_batch* bt, const double* m, int mwhere, double alpha, int vari
     const size_t NS = (size_t)n * S;
     hipStream_t s = bt->stream;
     const CtxView& v = bt->cv;
-    if (m) TM_CHECK(copy_in(bt->m.p, m, mwhere, 3 * NS, s));
+    if (m) {
+        bt->m_replaced = true;
+        TM_CHECK(copy_in(bt->m.p, m, mwhere, 3 * NS, s));
+    }
     if (bt->timers) TM_HIP(hipEventRecord(bt->ev[0], s));
     // Poisson right-hand side (DemagField.cpp:124-136), all samples
     launch_div(bt);
@@ -4192,6 +4197,7 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
                            (const double*)bt->rk_k[3].p, dtau, bt->m.p);
         TM_HIP(hipGetLastError());
         R.sync_steps += 1;
+        bt->m_replaced = false;
         return st;
     };
     int status = TM_OK;
@@ -4199,7 +4205,10 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
     for (int step = 0; step < nsteps; ++step) {
         const bool fin = step == nsteps - 1;
         bool missed = false;
-        if (graph_ok && bt->bud_set) {
+        // A state from outside has nothing to do with the kept solutions or the
+        // budgets: its first step is host-polled (a replay would run to its end,
+        // miss the tolerance and be redone)
+        if (graph_ok && bt->bud_set && !bt->m_replaced) {
             if (replays >= 8) tighten();
             tm_batch::StepKey key;
             key.dtau = dtau;
