@@ -509,11 +509,11 @@ int tm_batch_bem_apply(tm_batch* b, const double* x, int xwhere, double* y, int 
 /* Kernel timing of a batch (no reference counterpart): the hot kernels of an
  * evaluation -- the divergence, the fused field + LLG kernel, the tuned
  * boundary GEMM (FP64 forms), and of the Neumann solve the level-0 kernels
- * of one inner CG iteration (SpMM, update, the pre-smoothing restriction,
- * the prolongation, the post-smoother) and the FP64 outer residual -- each
- * launched `reps` times alone on the batch's
- * stream (all samples active) and timed with HIP events.  For each: its
- * name, the mean ms per launch and its algorithmic bytes per launch (slot
+ * of one inner CG iteration (the product with the search direction, the
+ * update, the V-cycle's product down and its product up) and the FP64 outer
+ * residual -- each launched `reps` times alone on the batch's
+ * stream (all samples active) and timed with HIP events.  For each: the
+ * name of the kernel that runs for this mesh and batch, the mean ms per launch and its algorithmic bytes per launch (slot
  * offsets and weights read once, every vector read or written once, the
  * gathered rows counted once).  Leaves the batch's solver state undefined
  * until the next evaluation; *count receives the number written (<= cap). */

@@ -100,3 +100,26 @@ def test_coarsest_level_product(gpu_available, S, nx, ny, nz, prec):
         bc.close()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("S, nz, prec, names", [
+    (18, 15, "FP64", {"k_b_div", "k_b_eval_t<DMI>", "k_b_resid_t<double>", "k_b_cg_spmv_t", "k_b_up_t (level 0)"}),
+    (64, 15, "MIXED", {"k_b_div", "k_b_eval_t<DMI>", "k_b_resid_t<float>", "k_b_cg_spmv_t", "k_b_up_t (level 0)"}),
+    (18, 3, "FP64", {"k_b_div_l2", "k_b_eval<DMI>", "k_b_resid<double>", "k_b_cg_spmv", "k_b_up (level 0)"}),
+    (64, 3, "MIXED", {"k_b_div_l2", "k_b_eval_w<DMI>", "k_b_resid<float>", "k_b_cg_spmv_w", "k_b_up_w (level 0)"})])
+def test_kernel_times_name_what_runs(gpu_available, S, nz, prec, names):
+    """17,424 and 4,356 nodes: with tiles and gathering from L2."""
+    from tetmag_amd import _native as N
+    from tetmag_amd import problem as P
+    from tetmag_amd.batch import BatchContext
+    from tetmag_amd.context import FieldContext
+    prob = P.cuboid_problem("names", 32, 32, nz, 3.0, 0.1, 3, P.Material(D=1e-3))
+    ctx = FieldContext(prob, tol=1e-12)
+    try:
+        bc = BatchContext(ctx, S, getattr(N, "TM_PREC_" + prec))
+        got = [k["kernel"] for k in bc.time_kernels(1)]
+        print(S, prob.n, prec, got, flush=True)
+        assert names <= set(got)
+        bc.close()
+    finally:
+        ctx.close()

@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <cstddef>
 #include <cmath>
+#include <string>
 #include <type_traits>
 #include <utility>
 #include <vector>
@@ -752,7 +753,7 @@ __device__ inline double buf_ld8(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
 
 // b = sum_d tGrad_d (Js m_d) / mu0 for every sample (DemagField.cpp:124-136);
 // the slot weights hold tGrad_d(i, j) Js_j / mu0 (set at batch creation)
-__global__ __launch_bounds__(kBlock) void k_b_div(SlotArgs P, const double* __restrict__ wty,
+__global__ __launch_bounds__(kBlock) void k_b_div_l2(SlotArgs P, const double* __restrict__ wty,
                                                   const double* __restrict__ wtz, int S,
                                                   const double* __restrict__ m, double* __restrict__ out) {
     const int n = P.n;
@@ -1073,10 +1074,10 @@ __device__ inline void tile_partial(typename TT::T* lds, double* part, int S, co
     part[(size_t)sm * gridDim.x + blockIdx.x] = s;
 }
 
-// b = sum_d tGrad_d (Js m_d) / mu0, as k_b_div
+// b = sum_d tGrad_d (Js m_d) / mu0, as k_b_div_l2 (which gathers from L2)
 constexpr int kDivPerCu = 2;
 template <bool EVEN>
-__global__ __launch_bounds__(kTileThreads, 2 * kDivPerCu) void k_b_div_t(TileArgs t, const double* __restrict__ wx,
+__global__ __launch_bounds__(kTileThreads, 2 * kDivPerCu) void k_b_div(TileArgs t, const double* __restrict__ wx,
                                                                         const double* __restrict__ wy,
                                                                         const double* __restrict__ wz, int n,
                                                                         const double* __restrict__ m,
@@ -3124,9 +3125,9 @@ struct BatchSolver {
             timeit([&] { up0(rT.p, ring.p, prz, s); }), slots(O.U) * (4 + e) + 2.0 * nS * e + n1 * S * e);
         double* pbb = part.p;
         double* prr = part.p + (size_t)S * gmax();
-        add(sizeof(T) == 4 ? "k_b_resid<float>" : "k_b_resid<double>", timeit([&] {
-                resid(lv0_b64(), lv0_x64(), pbb, prr, s);
-            }),
+        const char* resid_name = t0.nt > 0 ? (sizeof(T) == 4 ? "k_b_resid_t<float>" : "k_b_resid_t<double>")
+                                           : (sizeof(T) == 4 ? "k_b_resid<float>" : "k_b_resid<double>");
+        add(resid_name, timeit([&] { resid(lv0_b64(), lv0_x64(), pbb, prr, s); }),
             slots(sl0) * (4 + 8) + 2.0 * nS * 8 + nS * e);
         return TM_OK;
     }
@@ -3703,16 +3704,16 @@ void launch_div(tm_batch* bt) {
     if (bt->et.nt > 0) {
         const TileArgs t = bt->et.args(bt->eo);
         if (S % 2 == 0)
-            hipLaunchKernelGGL(k_b_div_t<true>, dim3(tile_blocks(t.nch, kDivPerCu)), dim3(kTileThreads), 0, bt->stream, t,
+            hipLaunchKernelGGL(k_b_div<true>, dim3(tile_blocks(t.nch, kDivPerCu)), dim3(kTileThreads), 0, bt->stream, t,
                                (const double*)bt->tx.p, (const double*)bt->ty.p, (const double*)bt->tz.p, n,
                                (const double*)bt->m.p, bt->rhsN.p);
         else
-            hipLaunchKernelGGL(k_b_div_t<false>, dim3(tile_blocks(t.nch, kDivPerCu)), dim3(kTileThreads), 0, bt->stream, t,
+            hipLaunchKernelGGL(k_b_div<false>, dim3(tile_blocks(t.nch, kDivPerCu)), dim3(kTileThreads), 0, bt->stream, t,
                                (const double*)bt->tx.p, (const double*)bt->ty.p, (const double*)bt->tz.p, n,
                                (const double*)bt->m.p, bt->rhsN.p);
         return;
     }
-    hipLaunchKernelGGL(k_b_div, dim3(row_grid(n)), dim3(kBlock), 0, bt->stream, bt->eo.args(8, bt->tx.p),
+    hipLaunchKernelGGL(k_b_div_l2, dim3(row_grid(n)), dim3(kBlock), 0, bt->stream, bt->eo.args(8, bt->tx.p),
                        (const double*)bt->ty.p, (const double*)bt->tz.p, S, (const double*)bt->m.p, bt->rhsN.p);
 }
 
@@ -4365,14 +4366,15 @@ int tm_batch_time_kernels(tm_batch* bt, int reps, tm_batch_kernel_time* out, int
         v.push_back(k);
     };
     const double eslots = (double)bt->eo.h_sp[n];
-    add("k_b_div", timeit([&] {
+    add(bt->et.nt > 0 ? "k_b_div" : "k_b_div_l2", timeit([&] {
             launch_div(bt);
         }),
         eslots * (4 + 3 * 8) + 3 * nS * 8 + nS * 8);
     const int nw = (bt->exch ? 1 : 0) + 3 + (bt->dmi ? 3 : 0);
     const double per_node = 8.0 * n * (1 + (bt->cv.has_ku ? 4 : 0) + (bt->dmi ? 4 : 0));
-    add(S == kMaxS ? (bt->dmi ? "k_b_eval_w<DMI>" : "k_b_eval_w") : (bt->dmi ? "k_b_eval<DMI>" : "k_b_eval"),
-        timeit([&] {
+    const std::string eval = std::string(bt->et.nt > 0 ? "k_b_eval_t" : S == kMaxS ? "k_b_eval_w" : "k_b_eval") +
+                             (bt->dmi ? "<DMI>" : "");  // as launch_fields chooses
+    add(eval.c_str(), timeit([&] {
             (void)launch_fields(bt, 0.5, TM_LLG_CLASSIC, bt->dmdt.p, nullptr, false);
         }),
         eslots * (4 + 8.0 * nw) + 3 * nS * 8 + nS * 8 + 3 * nS * 8 + per_node);
