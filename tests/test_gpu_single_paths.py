@@ -48,6 +48,47 @@ def test_solver_forms(gpu_available, cells, which):
         L.tm_solver_destroy(h)
 
 
+@pytest.mark.parametrize("seed", [8, 9])
+def test_attainable_residual(gpu_available, seed):
+    """The residual that some 450 Jacobi-preconditioned iterations to 1e-13 leave:
+    rounding, above all, and not above that of the same iteration in numpy with
+    q = A p.  Another order of the sums moves it by 1 % either way; q kept by a
+    recurrence raises it by 10 to 19 % (right-hand sides 8 to 11): 5 % tell them apart."""
+    import scipy.sparse as sp
+    from tetmag_amd import _native as N
+    from tetmag_amd import problem as P
+    prob = P.cuboid_problem("forms", 39, 37, 21, 3.0, 0.1, 5)
+    n, tol = prob.n, 1e-13
+    rp, col, val = prob.neumann_matrix()
+    A = sp.csr_matrix((val, col, rp), shape=(n, n))
+    d = A.diagonal()
+    b = np.random.default_rng(seed).standard_normal(n)
+    x = np.where(np.diff(rp) == 1, b, 0.0)
+    r = b - A @ x
+    z = r / d
+    p, rz = z.copy(), r @ z
+    for _ in range(1000):
+        q = A @ p
+        a = rz / (p @ q)
+        x, r = x + a * p, r - a * q
+        if r @ r <= tol * tol * (b @ b):
+            break
+        z = r / d
+        new = r @ z
+        p, rz = z + new / rz * p, new
+    ref = np.linalg.norm(b - A @ x)
+    h, L = C.c_void_p(), N.lib()
+    N.check(L.tm_solver_create(n, N.ptr(rp), N.ptr(col), N.ptr(val), N.TM_PRECOND_JACOBI, C.byref(h)), "create")
+    try:
+        y, it = np.zeros(n), C.c_int()
+        N.check(L.tm_solver_solve(h, N.ptr(b), N.TM_HOST, N.ptr(y), N.TM_HOST, tol, 1000, 0, C.byref(it), None), "solve")
+        got = np.linalg.norm(b - A @ y)
+        print("seed", seed, "iterations", it.value, "residual", got, "numpy", ref, "ratio", got / ref, flush=True)
+        assert got <= 1.05 * ref
+    finally:
+        L.tm_solver_destroy(h)
+
+
 @pytest.mark.parametrize("b", [1, 2, 17, 255, 1122, 2049, 4111])
 def test_boundary_product_splits(gpu_available, b):
     """y = B x against torch: both sum b products, so they differ by at most

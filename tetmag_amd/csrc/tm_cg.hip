@@ -13,8 +13,8 @@
 // Each iteration is two kernels, the second of which also forms the first
 // product of the next V-cycle, with no host round trip and no device-scope
 // fence:
-//   k_cg_spmv(k) : gamma_k, (r,r) from the partials; beta; q = A z + beta q
-//                  (= A p, the gathers read z only); p = z + beta p; partial (p,q)
+//   k_cg_spmv(k) : gamma_k, (r,r) from the partials; beta; p' = z + beta p;
+//                  q = A p', with p' formed in the gathers; partial (p',q)
 //   k_cg_step(k) : alpha = gamma_k / (p,q); x += alpha p; r' = r - alpha q;
 //                  partial (r',r'); and on further blocks F r' = F r - alpha F q
 //                  for the preconditioner's first product F
@@ -293,10 +293,13 @@ __device__ inline bool cg_beta(int k, const double* part, int G, CgState* st, do
     return true;
 }
 
-// p = z + beta p, q = A p = A z + beta q, partial (p, q); one lane per row (SELL)
+// p_new = z + beta p_old, q = A p_new, partial (p_new, q); one lane per row (SELL).
+// (q = A z + beta q would gather z alone, but its rounding errors add up over the
+// iterations: the residual that a Jacobi solve to 1e-13 leaves grew by up to 18 %.)
 __global__ __launch_bounds__(kBlock) void k_cg_spmv(SellView A, const double* __restrict__ val,
-                                                    const double* __restrict__ z, double* __restrict__ p,
-                                                    double* __restrict__ q, int k, double* part, CgState* st) {
+                                                    const double* __restrict__ z, const double* __restrict__ p_old,
+                                                    double* __restrict__ p_new, double* __restrict__ q, int k,
+                                                    double* part, CgState* st) {
     if (st->done) return;
     const int G = gridDim.x;
     double beta;
@@ -304,45 +307,55 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv(SellView A, const double* __
     double v = 0.0;
     CG_SLICE_LOOP(A) {
         double acc = 0.0;
-        sell_row(A, s, lane, [&](int64_t e, int c) { acc += val[e] * z[c]; });
+        if (k == 0) sell_row(A, s, lane, [&](int64_t e, int c) { acc += val[e] * z[c]; });
+        else sell_row(A, s, lane, [&](int64_t e, int c) { acc += val[e] * (z[c] + beta * p_old[c]); });
         const int row = s * kWave + lane;
         if (row < A.n) {
-            const double pi = k == 0 ? z[row] : z[row] + beta * p[row];
-            const double qi = k == 0 ? acc : acc + beta * q[row];
-            p[row] = pi;
-            q[row] = qi;
-            v += pi * qi;
+            const double pi = k == 0 ? z[row] : z[row] + beta * p_old[row];
+            p_new[row] = pi;
+            q[row] = acc;
+            v += pi * acc;
         }
     }
     block_partials(part + 3 * G, G, v, 0.0, 1);
 }
 
-// the same with LPR lanes per row
+// the same with LPR lanes per row; A z and A p_old are summed apart, so that the
+// gathers do not wait for beta
 template <int LPR>
 __global__ __launch_bounds__(kBlock) void k_cg_spmv_l(int n, const int* __restrict__ rp, const int* __restrict__ ci,
                                                       const double* __restrict__ v, const double* __restrict__ z,
-                                                      double* __restrict__ p, double* __restrict__ q, int k,
-                                                      double* part, CgState* st) {
+                                                      const double* __restrict__ p_old, double* __restrict__ p_new,
+                                                      double* __restrict__ q, int k, double* part, CgState* st) {
     if (st->done) return;
     const int G = gridDim.x;
     const RowShare R = row_share<LPR>(n, xcd_block(), G);
     const int sub = threadIdx.x & (LPR - 1);
     int row = R.r0 + threadIdx.x / LPR;
-    double s[1] = {0.0};
-    if (row < R.r1) csr_row<LPR, 1>(rp, ci, v, {z}, row, sub, s);
+    double s[2] = {0.0, 0.0};
+    auto sums = [&]() {
+        if (k > 0) {
+            csr_row<LPR, 2>(rp, ci, v, {z, p_old}, row, sub, s);
+        } else {
+            double s0[1];
+            csr_row<LPR, 1>(rp, ci, v, {z}, row, sub, s0);
+            s[0] = s0[0];
+        }
+    };
+    if (row < R.r1) sums();
     double beta;
     if (!cg_beta(k, part, G, st, beta)) return;
     double dot = 0.0;
     while (row < R.r1) {
         if (sub == 0) {
-            const double pi = k == 0 ? z[row] : z[row] + beta * p[row];
-            const double qi = k == 0 ? s[0] : s[0] + beta * q[row];
-            p[row] = pi;
+            const double pi = k == 0 ? z[row] : z[row] + beta * p_old[row];
+            const double qi = k == 0 ? s[0] : s[0] + beta * s[1];
+            p_new[row] = pi;
             q[row] = qi;
             dot += pi * qi;
         }
         row += kBlock / LPR;
-        if (row < R.r1) csr_row<LPR, 1>(rp, ci, v, {z}, row, sub, s);
+        if (row < R.r1) sums();
     }
     block_partials(part + 3 * G, G, dot, 0.0, 1);
 }
@@ -613,7 +626,7 @@ int CgSolver::setup(int n_, const int* rowptr, const int* colidx, const double* 
     TM_CHECK(fixed.upload(fx.data(), fx.size(), s));
     TM_CHECK(z.alloc(n));
     TM_CHECK(q.alloc(n));
-    TM_CHECK(p.alloc(n));
+    for (auto& v : p) TM_CHECK(v.alloc(n));
     lanes = precond == TM_PRECOND_AMG && n <= kLaneRows;
     if (lanes) {
         // lanes per row: what fills the chip (1,024 blocks) once, at most 16
@@ -663,7 +676,7 @@ int CgSolver::start(Seq& sq, const double* b, double* x, double tol, hipStream_t
     } else {
         hipLaunchKernelGGL(k_cg_init_fixed, dim3(grid), dim3(kBlock), 0, s, n, fixed.p, b, x, part.p);
     }
-    sq = Seq{rb[0].p, rb[1].p, false, true};
+    sq = Seq{rb[0].p, rb[1].p, p[0].p, p[1].p, false, true};
     if (lanes)
         with_lanes(A.lpr, [&](auto lpr) {
             hipLaunchKernelGGL(k_cg_init_res_l<decltype(lpr)::value>, dim3(grid), dim3(kBlock), 0, s, n, A.rp.p,
@@ -692,35 +705,36 @@ int CgSolver::precondition(Seq& sq, hipStream_t s) {
 int CgSolver::iteration(Seq& sq, double* x, int k, bool another, hipStream_t s) {
     const int G = grid;
     const bool jac = precond == TM_PRECOND_JACOBI;
+    std::swap(sq.pcur, sq.pold);
     if (lanes)
         with_lanes(A.lpr, [&](auto lpr) {
             hipLaunchKernelGGL(k_cg_spmv_l<decltype(lpr)::value>, dim3(G), dim3(kBlock), 0, s, n, A.rp.p, A.ci.p,
-                               A.v.p, (const double*)z.p, p.p, q.p, k, part.p, st.p);
+                               A.v.p, (const double*)z.p, (const double*)sq.pold, sq.pcur, q.p, k, part.p, st.p);
         });
     else
-        hipLaunchKernelGGL(k_cg_spmv, dim3(G), dim3(kBlock), 0, s, view(pat), val.p, (const double*)z.p, p.p, q.p, k,
-                           part.p, st.p);
+        hipLaunchKernelGGL(k_cg_spmv, dim3(G), dim3(kBlock), 0, s, view(pat), val.p, (const double*)z.p,
+                           (const double*)sq.pold, sq.pcur, q.p, k, part.p, st.p);
     sq.first_done = lanes && another && !amg.levels.empty();
     if (sq.first_done) {
         const AmgPrecond::First F = amg.first();
         double* out = F.out ? F.out : sq.rnext + n;
         if (F.dense)
-            hipLaunchKernelGGL(k_cg_step<0>, dim3(G + F.rows), dim3(kBlock), 0, s, n, G, (const double*)p.p,
+            hipLaunchKernelGGL(k_cg_step<0>, dim3(G + F.rows), dim3(kBlock), 0, s, n, G, (const double*)sq.pcur,
                                (const double*)q.p, x, (const double*)sq.rcur, sq.rnext, F.rows, (const int*)nullptr,
                                (const int*)nullptr, F.dense, out, k, part.p, st.p);
         else
             with_lanes(F.csr->lpr, [&](auto lpr) {
                 constexpr int kL = decltype(lpr)::value;
                 hipLaunchKernelGGL(k_cg_step<kL>, dim3(G + (F.rows + kBlock / kL - 1) / (kBlock / kL)), dim3(kBlock),
-                                   0, s, n, G, (const double*)p.p, (const double*)q.p, x, (const double*)sq.rcur,
+                                   0, s, n, G, (const double*)sq.pcur, (const double*)q.p, x, (const double*)sq.rcur,
                                    sq.rnext, F.rows, F.csr->rp.p, F.csr->ci.p, F.csr->v.p, out, k, part.p, st.p);
             });
         std::swap(sq.rcur, sq.rnext);
     } else if (jac) {
-        hipLaunchKernelGGL(k_cg_update<true>, dim3(G), dim3(kBlock), 0, s, n, dinv.p, p.p, q.p, x, sq.rcur, z.p, k,
+        hipLaunchKernelGGL(k_cg_update<true>, dim3(G), dim3(kBlock), 0, s, n, dinv.p, sq.pcur, q.p, x, sq.rcur, z.p, k,
                            part.p, st.p);
     } else {
-        hipLaunchKernelGGL(k_cg_update<false>, dim3(G), dim3(kBlock), 0, s, n, dinv.p, p.p, q.p, x, sq.rcur, z.p, k,
+        hipLaunchKernelGGL(k_cg_update<false>, dim3(G), dim3(kBlock), 0, s, n, dinv.p, sq.pcur, q.p, x, sq.rcur, z.p, k,
                            part.p, st.p);
     }
     sq.rr_new = true;

@@ -599,7 +599,7 @@ struct CgSolver {
     // the two swapped by each fused update
     bool lanes = false;
     AmgPrecond::CsrDev A;
-    DevBuf<double> rb[2], z, q, p;
+    DevBuf<double> rb[2], z, q, p[2];
     DevBuf<double> part;     // partial sums: bb | rz | rr | pq, grid entries each
     DevBuf<CgState> st;
     CgState* h_st = nullptr;  // pinned; written by the device at the end of a chunk of iterations
@@ -642,6 +642,8 @@ private:
     struct Seq {
         double* rcur;
         double* rnext;
+        double* pcur;     // the search direction of the last iteration, and
+        double* pold;     // of the one before
         bool first_done;  // the V-cycle's first product of rcur is formed already
         bool rr_new;      // the (r, r) partials of rcur have not been tested yet
     };
