@@ -496,7 +496,8 @@ int tm_batch_gemm_info(tm_batch* b, int* solution, int* own_kernel, int* candida
                        double* ms_tuned, int* ksplit);
 /* In-pipeline timing of the boundary GEMM (no reference counterpart): on = 1
  * starts recording a HIP event pair around the GEMM launch of each following
- * evaluation on the batch's stream (no host wait; the first 256 are kept);
+ * evaluation on the batch's stream (no host wait; the first 256 are kept;
+ * those of captured RK4 steps, replayed without the host, are left out);
  * on = 0 stops, waits for the last recorded event and returns the mean
  * duration in ms of the launches recorded since the last start and their
  * number (either output may be NULL). */

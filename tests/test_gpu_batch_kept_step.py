@@ -151,3 +151,31 @@ def test_first_step_of_a_given_state_is_host_polled(gpu_available, prec, how):
         a.close()
         b.close()
         ctx.close()
+
+
+@pytest.mark.parametrize("prec", ["FP64", "MIXED_BEMI8"])
+def test_live_gemm_events_leave_captured_steps_out(gpu_available, prec):
+    """tm_batch_gemm_live while a step is captured and replayed: the host-polled
+    step's four products are recorded, the replays' are not, and nothing that
+    follows fails."""
+    from tetmag_amd import _native as N
+    from tetmag_amd import problem as P
+    from tetmag_amd.batch import BatchContext, to_batch
+    from tetmag_amd.context import FieldContext
+    prob, dt = _problem()
+    ctx = FieldContext(prob, tol=1e-12)
+    bc = BatchContext(ctx, 64, getattr(N, "TM_PREC_" + prec))
+    try:
+        bc.set_mag(to_batch(P.smooth_random_fields(prob.mesh, 64, seed=31, lam_min=10.0, lam_max=60.0)))
+        for _ in range(2):
+            bc.gemm_live(True)
+            _, rk = bc.run_rk4(dt, 4, use_graph=True)
+            ms, count = bc.gemm_live(False)
+            print(prec, rk, ms, count, flush=True)
+            assert rk["graph_steps"] >= 3 and count == 4 * rk["sync_steps"] and (ms > 0) == (count > 0)
+        bc.gemm_live(True)
+        bc.eval_euler(dt, stats=False)
+        assert bc.gemm_live(False)[1] == 1
+    finally:
+        bc.close()
+        ctx.close()

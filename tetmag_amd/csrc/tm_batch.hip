@@ -3284,9 +3284,10 @@ struct tm_batch {
     hipEvent_t lev[2 * kLivePairs] = {};
     int lev_n = 0;
     bool lev_on = false;
+    bool capturing = false;  // a step is being captured: an event recorded now could not be read
     // marks the start (0) or end (1) of a boundary GEMM launch while recording
     void live_mark(int which) {
-        if (!lev_on || lev_n >= kLivePairs) return;
+        if (!lev_on || capturing || lev_n >= kLivePairs) return;
         (void)hipEventRecord(lev[2 * lev_n + which], stream);
         if (which == 1) ++lev_n;
     }
@@ -4231,6 +4232,7 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
                 bt->gemm_shape = bt->own_shape;
                 bt->gemm_ks = bt->own_ks;
                 TM_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+                bt->capturing = true;
                 int r = TM_OK;
                 hipLaunchKernelGGL(k_b_reset_fail, dim3(1), dim3(64), 0, s, kCount, bt->rk_fail.p);
                 hipLaunchKernelGGL(k_b_copy, g, dim3(kBlock), 0, s, N3, (const double*)bt->m.p, bt->rk_base.p);
@@ -4245,6 +4247,7 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
                                    (const double*)bt->rk_k[1].p, (const double*)bt->rk_k[2].p,
                                    (const double*)bt->rk_k[3].p, dtau, bt->m.p);
                 const hipError_t ec = hipStreamEndCapture(s, &gr);
+                bt->capturing = false;
                 bt->gemm_own = k_own;
                 bt->gemm_shape = k_shape;
                 bt->gemm_ks = k_ks;
