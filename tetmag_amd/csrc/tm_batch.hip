@@ -2177,8 +2177,7 @@ __global__ void k_b_zero_small(int cnt, double* p) {
     if ((int)threadIdx.x < cnt) p[threadIdx.x] = 0.0;
 }
 
-// *fail += number of samples whose outer residual missed the tolerance
-// *fail, *bad: the samples that missed the tolerance, and those that are not finite
+// *fail, *bad += the samples whose outer residual missed the tolerance, and those that are not finite
 __global__ void k_b_count_undone(int S, const OState* os, unsigned* fail, unsigned* bad) {
     const int s = threadIdx.x;
     if (s < S && os->done[s] != 1) atomicAdd(os->done[s] == 0 ? fail : bad, 1u);
@@ -3373,6 +3372,28 @@ __global__ __launch_bounds__(kBlock) void k_b_fill_pattern(size_t n, double* __r
         x[e] = sin(0.37 * (double)(e % 100003)) + 0.25;
 }
 
+// out[0] = max |own - ref|, out[1] = max |ref| (both zero before) for own b x S
+// row-major and ref column-major; a difference that is not a number is infinite
+__global__ __launch_bounds__(kBlock) void k_b_max_diff(int b, int S, const double* __restrict__ own,
+                                                       const double* __restrict__ ref, double* out) {
+    double d = 0.0, r = 0.0;
+    const size_t tot = (size_t)b * S;
+    for (size_t e = (size_t)blockIdx.x * kBlock + threadIdx.x; e < tot; e += (size_t)gridDim.x * kBlock) {
+        const double x = ref[(e % S) * b + e / S], y = fabs(own[e] - x);
+        d = fmax(d, y == y ? y : INFINITY);
+        r = fmax(r, fabs(x));
+    }
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        d = fmax(d, __shfl_xor(d, o));
+        r = fmax(r, __shfl_xor(r, o));
+    }
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        atomic_max_nonneg(out, d);
+        atomic_max_nonneg(out + 1, r);
+    }
+}
+
 // K splits worth timing for a tile shape: the one that gives ~1024 blocks,
 // and those that fill j = 1..6 rounds of the resident block slots (all
 // blocks carry the same work, so a last round that is only partly filled
@@ -3480,30 +3501,27 @@ int tune_gemm(tm_batch* bt) {
         if (bt->Pd.alloc((size_t)ksmax * b * S) == TM_OK) {
             hipLaunchKernelGGL(k_b_fill_pattern, dim3(elem_grid((size_t)b * S)), dim3(kBlock), 0, bt->stream,
                                (size_t)b * S, bt->U.p);
-            std::vector<double> ref((size_t)b * S), own((size_t)b * S);
-            DevBuf<double> G2;
-            bool ok = G2.alloc((size_t)b * S) == TM_OK && gemm_run(bt, bt->gemm_sol) == TM_OK &&
-                      hipMemcpyAsync(ref.data(), bt->Gm.p, ref.size() * sizeof(double), hipMemcpyDeviceToHost,
-                                     bt->stream) == hipSuccess &&
-                      hipStreamSynchronize(bt->stream) == hipSuccess;
-            double rmax = 0.0;
-            for (size_t e = 0; ok && e < ref.size(); ++e) rmax = std::max(rmax, std::fabs(ref[e]));
+            // compared on the device: copying every candidate's product back and comparing
+            // it on the host was most of the tuning's time (6,000 rows, 63 samples: 30 ms)
+            DevBuf<double> G2, dmax;
+            const bool ok = G2.alloc((size_t)b * S) == TM_OK && dmax.alloc(2) == TM_OK &&
+                            gemm_run(bt, bt->gemm_sol) == TM_OK;
             const int keep_shape = bt->gemm_shape, keep_ks = bt->gemm_ks;
             int best_shape = -1, best_ks = 1;
             for (size_t ci = 0; ok && ci < cand.size(); ++ci) {
                 bt->gemm_shape = cand[ci].first;
                 bt->gemm_ks = cand[ci].second;
-                if (gemm_own_run(bt, G2.p) != TM_OK ||
-                    hipMemcpyAsync(own.data(), G2.p, own.size() * sizeof(double), hipMemcpyDeviceToHost,
-                                   bt->stream) != hipSuccess ||
+                double m[2] = {};
+                hipLaunchKernelGGL(k_b_zero_small, dim3(1), dim3(kMaxS), 0, bt->stream, 2, dmax.p);
+                if (gemm_own_run(bt, G2.p) != TM_OK) break;
+                hipLaunchKernelGGL(k_b_max_diff, dim3(elem_grid((size_t)b * S)), dim3(kBlock), 0, bt->stream, b, S,
+                                   (const double*)G2.p, (const double*)bt->Gm.p, dmax.p);
+                if (hipMemcpyAsync(m, dmax.p, sizeof(m), hipMemcpyDeviceToHost, bt->stream) != hipSuccess ||
                     hipStreamSynchronize(bt->stream) != hipSuccess)
                     break;
-                double dmax = 0.0;
-                for (size_t e = 0; e < ref.size(); ++e)  // own: b x S row-major; ref: column-major
-                    dmax = std::max(dmax, std::fabs(own[e] - ref[(e % S) * b + e / S]));
-                const double err = rmax > 0 ? dmax / rmax : dmax;
+                const double err = m[1] > 0 ? m[0] / m[1] : m[0];
                 bt->gemm_own_err = std::max(bt->gemm_own_err, err);
-                if (err > 1e-12) continue;  // never choose a kernel that disagrees with the library
+                if (!(err <= 1e-12)) continue;  // never choose a kernel that disagrees with the library
                 float ms = 0.0f;
                 bool run_ok = hipEventRecord(e0, bt->stream) == hipSuccess;
                 for (int k = 0; k < 2 && run_ok; ++k) run_ok = gemm_own_run(bt, nullptr) == TM_OK;
