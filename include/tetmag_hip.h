@@ -476,9 +476,10 @@ int tm_batch_eval_euler(tm_batch* b, double alpha, int variant, double dtau, dou
  * captured in a HIP graph and replayed with one host synchronisation per
  * step; a step in which a sample missed the tolerance is restored and redone
  * with host-polled solves, and the budgets grow.  The captured steps run the
- * boundary product on the fastest of the library's own FP64 GEMM kernels that
- * agreed with rocBLAS at tm_batch_create (S = 64, FP64 boundary product);
- * other batches run every step host-polled.
+ * boundary product from int8 digits (any S), or on the fastest of the
+ * library's own FP64 GEMM kernels that agreed with rocBLAS at tm_batch_create
+ * (S = 64); batches of fewer samples with the FP64 product, and those with the
+ * FP32 copy of B, run every step host-polled.
  * `last` (may be null): statistics of the final evaluation when it was
  * host-polled (only nsamples is set after a replayed final step); `rk` (may
  * be null): step counts, budgets (summed inner iterations per solve) and the
@@ -490,7 +491,7 @@ int tm_batch_run_rk4(tm_batch* b, double dtau, int nsteps, double alpha, int var
  * index (0 = library default; rocBLAS indices may be negative).
  * *own_kernel = 1: the library's own FP64 MFMA kernel (only chosen when it
  * agrees with rocBLAS to 1e-12), *solution its tile shape, run with `ksplit`
- * partial products over K.  Also the number of candidates timed and the
+ * partial products over K; with int8 digits the wavefronts per block (4 or 8).  Also the number of candidates timed and the
  * timings of the library default and of the choice.  Any output may be NULL. */
 int tm_batch_gemm_info(tm_batch* b, int* solution, int* own_kernel, int* candidates, double* ms_default,
                        double* ms_tuned, int* ksplit);

@@ -215,9 +215,8 @@ def test_trajectory_with_kept_solutions(base, prec):
                                     ("bemi8", 3)])
 def test_batch_bem_apply(base, prec, S):
     """tm_batch_bem_apply against the dense FP64 product B X on the host: the
-    boundary GEMM the batched evaluation runs (tuned MFMA kernel or rocBLAS for
-    S = 64, rocBLAS otherwise; the int8 digit-slice kernel), host and device
-    operands."""
+    boundary GEMM the batched evaluation runs (tuned MFMA kernel or rocBLAS;
+    the int8 digit-slice kernel), host and device operands."""
     import torch
     from tetmag_amd.batch import BatchContext
     prob, ctx, _ = base
@@ -229,8 +228,8 @@ def test_batch_bem_apply(base, prec, S):
     ref = B @ X
     Y = bc.bem_apply(X)
     # bem32: FP32 products summed in FP64 per 512-column chunk; bemi8: five
-    # base-2^7 digits per value (~2^-35 of the row / column maxima per
-    # entry) and the digit products with p + q <= 4
+    # base-2^7 digits (~2^-35 of the row / column maxima per
+    # entry) for B, six for U, and the digit products with p + q <= 5
     tol = {"bem32": 1e-5, "bemi8": 2e-7}.get(prec, 1e-13)
     print("rel err", rel_l2(Y, ref))
     assert rel_l2(Y, ref) < tol

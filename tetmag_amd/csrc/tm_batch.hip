@@ -834,8 +834,9 @@ __device__ inline double pair_sum(d2v s) {
 // from L2).  64 samples at 282,897 nodes, against the gathers from L2: fields
 // 1,006 -> 591 us, divergence 513 -> 282, FP64 residual 216 -> 134; 24 samples
 // at 38,025 nodes 102 -> 39, 55 -> 20 and 25 -> 12.  A third of the lanes' time
-// goes into vector instructions, a third into LDS; two (fields, divergence) and
-// four (residual) blocks per CU were the fastest.
+// goes into vector instructions, a third into LDS.  Two (fields, divergence) and
+// three (residual) blocks per CU; the residual with 2, 3 and 4 of them: 129.2,
+// 129.9 and 132.7 us for 64 samples at 282,897 nodes, 10.6, 10.8 and 11.8 for 24 at 38,440.
 constexpr int kTileThreads = 512;
 constexpr int kTileRows = kTileThreads / 16;
 constexpr int kTileS = 16;       // samples of a unit
@@ -2040,10 +2041,12 @@ __global__ __launch_bounds__(kBlock) void k_b_i8_uslice(int b, int S, int nC, co
 // chunk c + 1 are in flight into registers, stored to the other buffer
 // afterwards, and B's digits of chunks c + 1 and c + 2 into a rotation of three
 // register sets: 8 wavefronts then keep 80 KB per CU in flight, with one chunk
-// ahead (40 KB) every wavefront waited for memory.  Bound by HBM and the
-// matrix cores alike: 40,962 boundary nodes and 64 samples 1,700 -> 1,440 us (up
-// to 1,530 from box to box), B's 8.4 GB of digits at 5.8 TB/s (the 131 M products alone: 1.5 ms at the 2.86
-// POPS that the instruction sustains over long runs, 0.86 at its peak).
+// ahead (40 KB) every wavefront waited for memory.  40,962 boundary nodes and 64
+// samples 1,700 -> 1,440 us (up to 1,530 from box to box): B's 8.4 GB of digits at
+// 5.8 TB/s, and 4.3 T operations (the 131 M MFMAs) at 2.98 POPS.  Near both limits:
+// 6.5 TB/s is the best streaming read here; the operations alone take 0.86 ms at
+// the nominal 5 POPS, but the instruction by itself settles at 2.86 POPS when it
+// runs for long, under the power limit, which a launch of 1.4 ms can exceed.
 // v_mfma_i32_16x16x64_i8: A lane l = row l % 16, B lane l = column l % 16,
 // both the 16 k of block l / 16; D lane l register r = C[4 (l / 16) + r][l % 16].
 template <int NW>
@@ -2326,9 +2329,16 @@ struct SlotOp {
 // numbering when none of those fits: 31.7 of 32 rows per tile on the 282,897-node
 // cuboid (28 without the next row, and the kernels 5 to 30 per cent slower), 4
 // nodes per row where 32 consecutive rows of its Z-order numbering need 5.
-// None (nt = 0) when a row alone refers to too many nodes, or when there are fewer
-// than 1,024 units, two for each block (the smaller problems sit in L2, where a
-// gather's latency is all it costs).
+// None (nt = 0) when a row alone refers to too many nodes, or below 1,024 units of
+// 32 rows and 16 samples: two for each of the 512 blocks of the fields and the
+// divergence, 1.3 for the 768 of the residual and of the products with 16 samples
+// per unit.  The FP32 products for 64 samples take one unit per tile, 256 for 512
+// blocks at the line, half of which then return at once.  An evaluation in us, from L2 / with tiles:
+//   64 samples, mixed  364 units 395 / 403, 608 495 / 470, 848 595 / 545, 1,052 660 / 601
+//   64 samples, FP64   364 units 429 / 417, 608 498 / 462, 848 589 / 534, 1,052 657 / 583
+//   24 samples, FP64   360 units 455 / 402, 640 597 / 477, 856 698 / 549, 1,052 801 / 605
+//   7 samples, mixed   383 units 525 / 429, 633 686 / 505, 878 866 / 604, 1,016 950 / 631
+// So the line is on the safe side: tiles are the faster form from about 400 units on.
 struct TileOp {
     int nt = 0;
     DevBuf<int> row0, node0, nodes;
@@ -4188,8 +4198,11 @@ int tm_batch_run_rk4(tm_batch* bt, double dtau, int nsteps, double alpha, int va
     hipStream_t s = bt->stream;
     const dim3 g(elem_grid(N3));
     const double cst[4] = {0.0, 0.5 * dtau, 0.5 * dtau, dtau};
-    // graphs need kernel-only boundary products (the own MFMA GEMM); the
-    // rocBLAS paths run eagerly
+    // graphs need kernel-only boundary products (the own GEMMs): from int8 digits
+    // for any number of samples, in FP64 for 64; other batches run every step
+    // host-polled.  (The FP64 kernel takes fewer samples too, and captured steps
+    // with it measured faster: 7 samples at 2,205 nodes 1.29 against 1.46 ms a
+    // step, 24 at 38,440 4.31 against 4.93.  Not set up: own_ok asks for 64.)
     const bool graph_ok =
         use_graph && (bt->prec == TM_PREC_MIXED_BEMI8 || (bt->prec != TM_PREC_MIXED_BEM32 && bt->own_ok));
     tm_rk4_stats R = {};

@@ -29,9 +29,8 @@
 // product per level (tm_amg.hip) an iteration of a two-level solve is three
 // launches (of a four-level one eight), where separate smoothing, restriction,
 // prolongation and update kernels took eight (fifteen): a cold Neumann solve
-// of 71,825 nodes 1,178 -> 791 us, one FP64 evaluation at 29,760 nodes 710 ->
-// 303 us, at 282,897 nodes 3.43 -> 2.79 ms (2.06 ms of it the boundary
-// product), the other kernels' changes included.
+// of 71,825 nodes 1,150 -> 789 us, one FP64 evaluation at 29,760 nodes 710 ->
+// 352 us, at 282,897 nodes 3.47 -> 2.89 ms (2.06 ms of it the boundary product).
 #include <algorithm>
 #include <cmath>
 

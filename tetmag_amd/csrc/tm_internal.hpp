@@ -170,7 +170,7 @@ __device__ inline void block_sum(double (&v)[NV], double* smem /* NV * kBlock/kW
 }
 
 // Every block of a consumer kernel reduces the partials written by the
-// producer kernel (one per producer block, at most a few hundred) itself; the
+// producer kernel (one per producer block, at most kMaxCgBlocks) itself; the
 // sum is then known to every thread of the block.  Kernel boundaries order
 // producer and consumer, so no device-scope fence is needed, and every block
 // computes bit-identical totals (same data, same order), so decisions taken on
@@ -271,7 +271,11 @@ struct SellLanes {
 // idle on small meshes and too few loads in flight on large ones.  Fields /
 // divergence in us with 1, 4 and 16 lanes (8 at 29,760 nodes): 2,205 nodes 8.0 / 7.6,
 // 5.1 / 4.1, 4.3 / 3.2; 29,760 nodes (DMI) 13.4 / 9.9, 9.5 / 5.7, 14.8 / 7.8;
-// 282,897 nodes 68 / 48 and 56 / 35.
+// 282,897 nodes 68 / 48 and 56 / 35.  Around the line (DMI, kernel times, 4 and 16
+// lanes): 3,920 nodes 5.1 / 3.2 and 4.8 / 2.8; 5,832 5.2 / 3.3 and 5.6 / 3.1; 8,192
+// 5.3 / 3.4 and 5.6 / 3.0; 9,800 5.2 / 3.4 and 6.5 / 3.3; 16,000 5.1 / 3.2 and 7.4 / 3.8:
+// up to the line the sum of both is as good with 16 or better.  The sparse product
+// takes 2.7 to 3.0 us with either.
 template <class F>
 void with_row_lanes(int n, F&& f) {
     if (n <= 8192) f(std::integral_constant<int, 16>{});
@@ -655,9 +659,14 @@ private:
 
 constexpr int kMaxCgBlocks = 2048;
 // Rows up to which several lanes share a matrix row in the single-sample
-// solver's level-0 kernels (above, one lane per row in SELL order fills the
-// chip, and the fused step's two gathers per entry cost more than the launch
-// they save).
+// solver's level-0 kernels and the update forms the V-cycle's first product as
+// well.  Above, one lane per row in SELL order fills the chip, and the two
+// gathers per entry of that product cost more than the launch they save.  A cold
+// Neumann solve in us, several lanes / one lane: 8,228 rows 389 / 499; 29,988 517 /
+// 533; 49,572 633 / 641; 59,177 676 / 664; 71,825 767 / 736; 108,800 1,009 / 868;
+// 131,648 1,375 / 963 (more rows than the 2,048 blocks take at once); 220,932
+// 1,652 / 1,326.  The two meet at about 55,000 rows; from there to this line one
+// lane per row would be the faster form, by up to a seventh.
 constexpr int kLaneRows = 1 << 17;
 
 // Read-only view of a field context's device data (tm_field.hip), used by
