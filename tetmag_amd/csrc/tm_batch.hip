@@ -2045,8 +2045,8 @@ __global__ __launch_bounds__(kBlock) void k_b_i8_uslice(int b, int S, int nC, co
 // samples 1,700 -> 1,440 us (up to 1,530 from box to box): B's 8.4 GB of digits at
 // 5.8 TB/s, and 4.3 T operations (the 131 M MFMAs) at 2.98 POPS.  Near both limits:
 // 6.5 TB/s is the best streaming read here; the operations alone take 0.86 ms at
-// the nominal 5 POPS, but the instruction by itself settles at 2.86 POPS when it
-// runs for long, under the power limit, which a launch of 1.4 ms can exceed.
+// the nominal 5 POPS, while the instruction by itself settles at 2.86 POPS when it
+// runs for long (a launch of 1.4 ms can exceed that).
 // v_mfma_i32_16x16x64_i8: A lane l = row l % 16, B lane l = column l % 16,
 // both the 16 k of block l / 16; D lane l register r = C[4 (l / 16) + r][l % 16].
 template <int NW>
